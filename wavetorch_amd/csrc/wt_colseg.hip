@@ -171,7 +171,11 @@ __device__ __forceinline__ void cs_snapshot(const CsGeom &g, const float *Q, flo
 
 // One forward step of this thread's segment; REC records lap(u_n) (and u_n
 // for the nonlinear cell) of the output rows through range-checked buffers.
-template <int R, int NL, bool REC>
+// UH: grid step 1, where each product with t1 = h^-2 is the value itself and
+// -4*ctr is exact.  Otherwise the five products are formed and added in
+// conv2d's order, one v_mul per neighbour (the centre's is the product the
+// rows above and below use): 15 VALU operations per row instead of 11.
+template <int R, int NL, bool REC, bool UH>
 __device__ __forceinline__ void cs_fwd_rows(const FwdArgs &a, const float *__restrict__ P,
                                             float *__restrict__ Q,
                                             float (&Uc)[R], float (&Up)[R], const float (&KA)[R],
@@ -181,16 +185,30 @@ __device__ __forceinline__ void cs_fwd_rows(const FwdArgs &a, const float *__res
                                             __amdgpu_buffer_rsrc_t rsl, __amdgpu_buffer_rsrc_t rsu,
                                             uint32_t voff, int Ny) {
   const int lfb = base - CS, rtb = base + CS;
-  float upv = P[base - 1];
+  // the row above and, for UH = false, this row times t1
+  float upv = UH ? P[base - 1] : a.t1 * P[base - 1];
+  float ctv = UH ? 0.0f : a.t1 * Uc[0];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const float ct = Uc[r];
     const float dn = (r < R - 1) ? Uc[r + 1] : P[base + R];
     const float lf = P[lfb + r], rt = P[rtb + r];
-    float sacc = upv + lf;
-    sacc = __builtin_fmaf(-4.0f, ct, sacc);
-    sacc = sacc + rt;
-    const float lap = sacc + dn;
+    float lap;
+    if (UH) {
+      float sacc = upv + lf;
+      sacc = __builtin_fmaf(-4.0f, ct, sacc);
+      sacc = sacc + rt;
+      lap = sacc + dn;
+      upv = ct;
+    } else {
+      const float dnv = a.t1 * dn;
+      float sacc = upv + a.t1 * lf;
+      sacc = sacc + a.t4 * ct;
+      sacc = sacc + a.t1 * rt;
+      lap = sacc + dnv;
+      upv = ctv;
+      ctv = dnv;
+    }
     float A, Bm, C2;
     if (NL == 0) {
       A = KA[r]; Bm = KB[r]; C2 = KC[r];
@@ -219,7 +237,6 @@ __device__ __forceinline__ void cs_fwd_rows(const FwdArgs &a, const float *__res
     // source: weight 1 at source pixels, 0 elsewhere; fma(1, x, v) rounds
     // once, exactly like the reference's v + x (source.py:22)
     v = __builtin_fmaf(KS[r], xv, v);
-    upv = ct;
     Up[r] = v;
     Q[base + r] = v;
     if (REC) {
@@ -238,7 +255,7 @@ __device__ unsigned long long *wt_phase_ts = nullptr;
 // described by `a`; shared by the single-configuration kernel and the
 // batched kernel (one launch over several configurations; BATCH compiles in
 // the per-sample lengths and record slots).
-template <int NT, int R, int NL, bool REC, bool BATCH>
+template <int NT, int R, int NL, bool REC, bool BATCH, bool UH>
 __device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
   WT_TS(0);
   extern __shared__ float smem[];
@@ -361,7 +378,7 @@ __device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
         cs_rsrc((REC && NL) ? a.rec_u + ro : a.in1, (REC && NL) ? rbytes : 0);
     const float xv = blk_src ? xs[s] : 0.0f;
     if (need)
-      cs_fwd_rows<R, NL, REC>(a, P, Q, Uc, Up, KA, KB, KC, KD, KS, g.base, g.CS, vmask, xv, rsl,
+      cs_fwd_rows<R, NL, REC, UH>(a, P, Q, Uc, Up, KA, KB, KC, KD, KS, g.base, g.CS, vmask, xv, rsl,
                               rsu, voff, Ny);
     __syncthreads();
     if (pidx >= 0) {
@@ -403,9 +420,9 @@ __device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
   WT_TS(3);
 }
 
-template <int NT, int R, int NL, bool REC>
+template <int NT, int R, int NL, bool REC, bool UH = true>
 __global__ __launch_bounds__(NT) void k_fwd_cs(FwdArgs a) {
-  fwd_cs_body<NT, R, NL, REC, false>(a, xcd_remap(blockIdx.x, gridDim.x));
+  fwd_cs_body<NT, R, NL, REC, false, UH>(a, xcd_remap(blockIdx.x, gridDim.x));
 }
 
 // Group of a batched launch that work item w belongs to.
@@ -420,7 +437,7 @@ template <int NT, int R, int NL, bool REC>
 __global__ __launch_bounds__(NT) void k_fwd_cs_batch(BatchFwd bl) {
   const int w = xcd_remap(blockIdx.x, gridDim.x);
   const int gi = batch_group(bl.start, bl.ngrp, w);
-  fwd_cs_body<NT, R, NL, REC, true>(bl.grp[gi], w - bl.start[gi]);
+  fwd_cs_body<NT, R, NL, REC, true, true>(bl.grp[gi], w - bl.start[gi]);
 }
 
 // ------------------------------------------------------------------ adjoint
@@ -530,9 +547,9 @@ __device__ __forceinline__ void adj_cs_body(const AdjArgs &a, const int w) {
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const float A = KA1[r];
-    KA1[r] = A * s2; KW[r] = A * KC2[r];
+    // w carries the Laplacian's h^-2 (exactly 1 at h = 1): no step pays for it
+    KA1[r] = A * s2; KW[r] = (A * KC2[r]) * a.t1;
     G[r] = 0.0f; SG1[r] = 0.0f;
-
   }
   __syncthreads();
   if (tid == 0) {
@@ -929,7 +946,7 @@ __global__ __launch_bounds__(NT) void k_adj_cs_nl(AdjArgs a, NlCarry cy) {
         Gc[r] = __builtin_fmaf(dvdc, lam, Gc[r]);
         if (GB) Gb[r] = __builtin_fmaf(dvdb, lam, Gb[r]);
         Gr[r] = __builtin_fmaf(dvdb * sd + dvdc * c2raw, lam, Gr[r]);
-        const float wn = A * (cc * cc);
+        const float wn = (A * (cc * cc)) * a.t1;  // with the Laplacian's h^-2
         Wm[r] = wn;
         Pm[r] = s2 * A + dvdb * dbdu + dvdc * dcdu;
         A2a[r] = A2b[r];
@@ -1035,20 +1052,26 @@ int cs_threads(int R, int RH, int RW) {
 }
 
 template <int NT, int R>
-static hipError_t cs_fwd_dispatch(int nl, bool rec, const FwdArgs &a, int nblocks,
+static hipError_t cs_fwd_dispatch(bool unit_h, int nl, bool rec, const FwdArgs &a, int nblocks,
                                   int nthreads, size_t shmem, hipStream_t s) {
-#define FT(NL, REC)                                                                   \
+#define FT(NL, REC, UH)                                                               \
   do {                                                                                \
-    auto kfn = k_fwd_cs<NT, R, NL, REC>;                                              \
+    auto kfn = k_fwd_cs<NT, R, NL, REC, UH>;                                           \
     static std::atomic<uint64_t> done{0};                                             \
     hipError_t e = allow_dyn_lds((const void *)kfn, done);                            \
     if (e != hipSuccess) return e;                                                    \
     hipLaunchKernelGGL(kfn, dim3(nblocks), dim3(nthreads), shmem, s, a);              \
   } while (0)
   if (nl == 0) {
-    if (rec) FT(0, true); else FT(0, false);
+    if (unit_h) {
+      if (rec) FT(0, true, true); else FT(0, false, true);
+    } else {
+      if (rec) FT(0, true, false); else FT(0, false, false);
+    }
+  } else if (unit_h) {
+    if (rec) FT(8, true, true); else FT(8, false, true);
   } else {
-    if (rec) FT(8, true); else FT(8, false);
+    if (rec) FT(8, true, false); else FT(8, false, false);
   }
 #undef FT
   return hipGetLastError();
@@ -1067,14 +1090,15 @@ static hipError_t cs_adj_dispatch(const AdjArgs &a, int nblocks, int nthreads, s
 
 // The region geometry (RH, RW) of the largest tile decides the block size
 // and LDS of the launch; smaller tiles leave threads idle.
-hipError_t launch_fwd_cs(int nt, int R, int nl, bool rec, const FwdArgs &a, int RHmax,
-                         int RWmax, hipStream_t s) {
+hipError_t launch_fwd_cs(int nt, int R, bool unit_h, int nl, bool rec, const FwdArgs &a,
+                         int RHmax, int RWmax, hipStream_t s) {
   int nblocks = a.B * a.ntiles;
   size_t shmem = cs_shmem_bytes(R, RHmax, RWmax, true);
   int nthreads = cs_threads(R, RHmax, RWmax);
   if (shmem + 1024 > (size_t)cs_max_dyn_lds() || nthreads > nt) return hipErrorInvalidConfiguration;
 #define X(A, B) \
-  if (nt == A && R == B) return cs_fwd_dispatch<A, B>(nl, rec, a, nblocks, nthreads, shmem, s);
+  if (nt == A && R == B)                                                                \
+    return cs_fwd_dispatch<A, B>(unit_h, nl, rec, a, nblocks, nthreads, shmem, s);
   WT_CS_VARIANTS(X)
 #undef X
   return hipErrorInvalidValue;

@@ -90,8 +90,8 @@ size_t tiled_shmem_bytes(int nt, int cpt, int LW);
 bool cs_variant_exists(int nt, int r);
 size_t cs_shmem_bytes(int R, int RH, int RW, bool padded);
 int cs_threads(int R, int RH, int RW);
-hipError_t launch_fwd_cs(int nt, int R, int nl, bool rec, const FwdArgs &a, int RHmax,
-                         int RWmax, hipStream_t s);
+hipError_t launch_fwd_cs(int nt, int R, bool unit_h, int nl, bool rec, const FwdArgs &a,
+                         int RHmax, int RWmax, hipStream_t s);
 hipError_t launch_adj_cs(int nt, int R, const AdjArgs &a, int RHmax, int RWmax, hipStream_t s);
 bool cs_nl_variant_exists(int nt, int r);
 size_t cs_nl_shmem_bytes(int R, int RH, int RW);
@@ -683,7 +683,12 @@ static int plan_build(const wt_config *cfg, int32_t B, int32_t T, float cmax_geo
   p->K = tun.ck_every > 0 ? tun.ck_every : 64;
   if (p->K > T) p->K = T;
   p->nseg = (T + p->K - 1) / p->K;
-  bool tiled = !tun.plain && p->unit_h;
+  // Every grid step runs blocked: off h = 1 the forward pays four more VALU
+  // operations per cell-step and the adjoint none, against one launch and
+  // three field passes per step (150x150, batch 32, 1500 steps, h = 1.43,
+  // training step: 27.0 ms plain, 5.9 ms blocked).  The flat family's
+  // kernels take h = 1 only.
+  bool tiled = !tun.plain && (p->unit_h || tun.kind == 0);
   if (tiled) {
     int strips = tun.strips, tb = tun.tblock, nt = tun.nt, cpt = tun.cpt;
     // the nonlinear cell forms its coefficients (three divisions) per cell
@@ -1107,7 +1112,8 @@ int run_forward(const Plan &p, FwdArgs a, int n0, int n1, const float *in1, cons
       if (p.tun.kind == 1)
         WT_HIP(launch_fwd_tiled(p.tun.nt, p.tun.cpt, p.unit_h, p.nl, rec, a, p.LWmax, s));
       else
-        WT_HIP(launch_fwd_cs(p.tun.nt, p.tun.cpt, p.nl, rec, a, p.RHmax, p.RWmax, s));
+        WT_HIP(launch_fwd_cs(p.tun.nt, p.tun.cpt, p.unit_h, p.nl, rec, a, p.RHmax,
+                             p.RWmax, s));
       i1 = o1;
       i2 = o2;
       pp ^= 1;
