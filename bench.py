@@ -86,13 +86,13 @@ def log(*a):
 #   bytes    algorithmic HBM bytes per cell-step of one step
 WORKLOADS = {
     "train_150_b64": dict(
-        kind="train", bytes=28.0,
+        kind="train", bytes=28.0, K=64,
         metric="fwd+adjoint Gcell-steps/s (150x150, batch 64, 3000 steps, training step)",
         desc="150x150 grid incl. 20-cell PML, free-form rho on the 110x110 interior, batch 64, "
              "3000 steps, 3 intensity probes, CE loss, adjoint with checkpoints every 64 steps, "
              "Adam"),
     "nonlinear_150_b32": dict(
-        kind="train", bytes=28.0,
+        kind="train", bytes=28.0, K=64,
         metric="fwd+adjoint Gcell-steps/s (150x150, batch 32, 3000 steps, nonlinear cell)",
         desc="as train_150_b64 at batch 32 with saturable damping b_nl=0.5, I_sat=0.1 and Kerr "
              "speed c_nl=0.05 clamped to [0.4, 1.1], dt=0.64"),
@@ -129,6 +129,8 @@ def build(dev, tuning=None, workload="train_150_b64", T=None):
     model = model.to(dev)
     if tuning is not None:
         model.tuning = tuning
+    if WORKLOADS[workload].get("K"):  # the workload's checkpoint interval
+        model.checkpoint_every = WORKLOADS[workload]["K"]
     fs = WORKLOADS[workload].get("field_stride")
     if fs:
         model.field_stride = fs

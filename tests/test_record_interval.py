@@ -1,0 +1,51 @@
+"""The checkpoint interval of a call that leaves it open: the rule on the
+host, and on the device the plans that forwards take while an earlier
+forward's whole record waits for its backward."""
+import pytest
+import torch
+
+from tests.helpers import rel
+from wavetorch_amd import (WaveCell, WaveGeometryFreeForm, WaveIntensityProbe, WaveRNN,
+                           WaveSource)
+from wavetorch_amd._loop import LoopConfig, auto_interval
+
+
+@pytest.mark.parametrize("nonlinear", [False, True])
+def test_auto_interval(nonlinear):
+    cfg = LoopConfig(Nx=50, Ny=39, dt=0.6, h=1.0, src_px=((9, 9, 0),), taps=((20, 20, 1),),
+                     c_nl=0.05 if nonlinear else 0.0)
+    step = (8 if nonlinear else 4) * 3 * 50 * 40  # batch 3
+    K = lambda T, steps: auto_interval(cfg, 3, T, steps * step, 64)
+    assert K(1000, 1000) == 1000                  # fits whole
+    assert K(1000, 999) == 500 and K(1001, 501) == 501
+    assert K(1000, 334) == 334 and K(1000, 333) == 250 and K(1000, 250) == 250
+    assert K(1000, 249) == 64                     # less than a quarter: not worth its memory
+    assert K(64, 1) == 64 and K(10, 0) == 10      # no longer than the default interval
+    assert K(100, 99) == 64                       # a half is shorter than the default
+
+
+@pytest.mark.gpu
+def test_forward_while_a_record_waits(cuda):
+    geom = WaveGeometryFreeForm((60, 52), 1.0, c0=1.0, c1=0.5, abs_N=8, abs_sig=1.0, abs_p=2,
+                                rho="half")
+    model = WaveRNN(WaveCell(0.7, geom), WaveSource(16, 26),
+                    [WaveIntensityProbe(44, 20), WaveIntensityProbe(44, 30)]).to(cuda)
+    n = torch.arange(150.0)
+    x = torch.stack([torch.sin(0.3 * n + k) * torch.exp(-((n - 60) / 25) ** 2)
+                     for k in range(3)]).to(cuda)
+
+    def grad(y):
+        model.zero_grad(set_to_none=True)
+        y.sum().backward()
+        return geom.rho.grad.cpu().numpy()
+
+    y1 = model(x)
+    y2 = model(x)  # y1's record waits: checkpoints every 64 steps
+    assert sorted(p.tuning["ck_every"] for p in model._plans.values()) == [64, 150]
+    assert torch.equal(y1, y2)
+    g2, g1 = grad(y2), grad(y1)
+    assert rel(g1, g2) < 1e-5  # the same lambdas, summed over other launches
+    y3 = model(x)              # nothing waits any more
+    assert model.plan(3, 150, x.device).record_waits()
+    assert rel(grad(y3), g1) == 0.0
+    assert not model.plan(3, 150, x.device).record_waits()

@@ -153,8 +153,9 @@ def tune(model, x, labels=None, steps=2, verbose=False, budget_s=300.0, rounds=2
     Nx, Ny = model.cell.geom.domain_shape
     K = int(model.checkpoint_every)
     user_k = model._checkpoint_every
-    if tune_k:
-        model.checkpoint_every = None
+    # the interval searched for is the model's, not the one an open model
+    # would choose per call
+    model.checkpoint_every = None if tune_k else K
     t_start = time.perf_counter()
 
     def step():

@@ -12,7 +12,7 @@ from __future__ import annotations
 import numpy as np
 import torch
 
-from ._loop import LoopConfig, Plan, WaveLoop
+from ._loop import LoopConfig, Plan, WaveLoop, auto_interval
 from .probe import WaveProbe
 
 
@@ -32,7 +32,8 @@ class WaveRNN(torch.nn.Module):
         # wavetorch_amd.autotune.tune(model, ...) or by hand.
         self.tuning = None
         # checkpoint interval K of the adjoint (steps); None = the tuning's
-        # ck_every, else 64.  A value set here overrides the tuning's.
+        # ck_every, else chosen per call (plan).  A value set here overrides
+        # the tuning's.
         self._checkpoint_every = None
         # extension: keep only every field_stride-th field when output_fields
         self.field_stride = 1
@@ -46,7 +47,8 @@ class WaveRNN(torch.nn.Module):
     @property
     def checkpoint_every(self) -> int:
         """Checkpoint interval K of the adjoint: the value set on the model,
-        else the tuning's ``ck_every``, else 64."""
+        else the tuning's ``ck_every``, else 64 (the interval of a call whose
+        record is not kept whole, see ``plan``)."""
         if self._checkpoint_every is not None:
             return self._checkpoint_every
         return int((self.tuning or {}).get("ck_every") or 64)
@@ -119,10 +121,18 @@ class WaveRNN(torch.nn.Module):
         self._cfg_cache = (key, cfg)
         return cfg
 
-    def plan(self, B: int, T: int, device) -> Plan:
+    def plan(self, B: int, T: int, device, lean: bool = False) -> Plan:
+        """The plan of a (B, T) batch.  When neither the model nor its tuning
+        names a checkpoint interval, the longest one whose record fits an
+        eighth of the device's memory is taken (``auto_interval``): the
+        forward then records the steps that the adjoint would otherwise
+        recompute.  `lean` asks for K = 64 there instead."""
         cfg = self.loop_config()
         tun = dict(self.tuning) if self.tuning else {}
         tun["ck_every"] = self.checkpoint_every
+        if not lean and self._checkpoint_every is None and not (self.tuning or {}).get("ck_every"):
+            total = torch.cuda.get_device_properties(device).total_memory
+            tun["ck_every"] = auto_interval(cfg, B, T, total // 8, tun["ck_every"])
         tkey = tuple(sorted(tun.items()))
         key = (cfg, B, T, str(device), tkey)
         p = self._plans.get(key)
@@ -159,9 +169,20 @@ class WaveRNN(torch.nn.Module):
         c = geom.c
         b = geom.b
         rho = geom.rho if self.loop_config().nonlinear else None
-        plan = self.plan(B, T, x.device)
-        out = WaveLoop.apply(x, c, b, rho, plan, fields_mode, stride,
-                             self._nonfinite_flags(x.device))
+        # one whole record per model at a time: while a forward's record waits
+        # for its backward, further forwards keep checkpoints every 64 steps
+        # (the float64 loop keeps every field and has no interval)
+        plan = self.plan(B, T, x.device, lean=x.dtype == torch.float64)
+        if torch.is_grad_enabled() and plan.record_waits():
+            plan = self.plan(B, T, x.device, lean=True)
+        args = (fields_mode, stride, self._nonfinite_flags(x.device))
+        try:
+            out = WaveLoop.apply(x, c, b, rho, plan, *args)
+        except torch.cuda.OutOfMemoryError:
+            lean = self.plan(B, T, x.device, lean=True)
+            if lean is plan:
+                raise
+            out = WaveLoop.apply(x, c, b, rho, lean, *args)
         if fields_mode:
             return out
         shp = self.probes[0].out_shape()  # from tensor shapes: no device read
