@@ -1,9 +1,11 @@
 """The checkpoint interval of a call that leaves it open: the rule on the
 host, and on the device the plans that forwards take while an earlier
 forward's whole record waits for its backward."""
+import numpy as np
 import pytest
 import torch
 
+import oracle.c_oracle as co
 from tests.helpers import rel
 from wavetorch_amd import (WaveCell, WaveGeometryFreeForm, WaveIntensityProbe, WaveRNN,
                            WaveSource)
@@ -49,3 +51,20 @@ def test_forward_while_a_record_waits(cuda):
     assert model.plan(3, 150, x.device).record_waits()
     assert rel(grad(y3), g1) == 0.0
     assert not model.plan(3, 150, x.device).record_waits()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,T", [(7, 300), (14, 257), (20, 1000)])
+def test_launch_longer_than_its_block(N, T, cuda):
+    """A small grid is one tile whose launches take up to 256 steps with 64
+    or 128 threads: the staged input samples outnumber the threads."""
+    geom = WaveGeometryFreeForm((N, N), 1.0, c0=1.0, c1=0.5, abs_N=2, abs_sig=1.0, abs_p=2,
+                                rho="half")
+    model = WaveRNN(WaveCell(0.7, geom), WaveSource(3, 3),
+                    [WaveIntensityProbe(N - 3, N - 3)]).to(cuda)
+    x = np.random.default_rng(N).standard_normal((2, T)).astype(np.float32)
+    with torch.no_grad():
+        y = model(torch.from_numpy(x).to(cuda)).cpu().numpy()
+        c = geom.c.cpu().numpy()
+    yo, _ = co.forward(geom.b.cpu().numpy(), c, x, 0.7, 1.0, [[3, 3, 0]], [[N - 3, N - 3, 1]])
+    assert np.array_equal(y, yo)

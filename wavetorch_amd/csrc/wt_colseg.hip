@@ -321,6 +321,13 @@ __device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
     tb_tp[4 * tid] = tpv0; tb_tp[4 * tid + 1] = tpv1;
     tb_tp[4 * tid + 2] = tpv2; tb_tp[4 * tid + 3] = tpv3;
   }
+  // blocks of fewer threads than steps or table entries (small grids)
+  for (int i = tid + blockDim.x; i < a.nsteps; i += blockDim.x)
+    xs[i] = a.x[(int64_t)b * a.T + a.n0 + i];
+  for (int i = tid + blockDim.x; i < nsp; i += blockDim.x) {
+    const int32_t *e = a.spx + (td[8] + i) * SPX_W;
+    for (int j = 0; j < 3; ++j) tb_sp[3 * i + j] = e[j];
+  }
   __syncthreads();
   WT_TS(5);
   if (g.active) {
@@ -543,6 +550,10 @@ __device__ __forceinline__ void adj_cs_body(const AdjArgs &a, const int w) {
   if (tid < nsp) {
     int *t = tb_sp + 6 * tid;
     t[0] = e0; t[1] = e1; t[2] = e2; t[3] = e3; t[4] = e4; t[5] = e5;
+  }
+  for (int i = tid + blockDim.x; i < nsp; i += blockDim.x) {
+    const int32_t *e = a.spx + (td[8] + i) * SPX_W;
+    for (int j = 0; j < 6; ++j) tb_sp[6 * i + j] = e[j];
   }
 #pragma unroll
   for (int r = 0; r < R; ++r) {
@@ -806,6 +817,10 @@ __global__ __launch_bounds__(NT) void k_adj_cs_nl(AdjArgs a, NlCarry cy) {
   if (tid < nsp) {
     int *t = tb_sp + 6 * tid;
     t[0] = e0; t[1] = e1; t[2] = e2; t[3] = e3; t[4] = e4; t[5] = e5;
+  }
+  for (int i = tid + blockDim.x; i < nsp; i += blockDim.x) {
+    const int32_t *e = a.spx + (td[8] + i) * SPX_W;
+    for (int j = 0; j < 6; ++j) tb_sp[6 * i + j] = e[j];
   }
   __syncthreads();
   if (tid == 0) {
