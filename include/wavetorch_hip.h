@@ -295,6 +295,23 @@ int wt_loop_adj_f64(void *plan, const wt_scalars_f64 *sc, const double *b, const
                     void *temp, double *grad_c, double *grad_b, double *grad_rho,
                     double *grad_x, void *stream);
 
+/* The float64 loop of the linear cell in temporally blocked launches.  The
+ * forward with gradients keeps lap(u_n) of every step instead of u_n, which
+ * is what the adjoint of the linear cell reads; dJ/db and gradients of the
+ * fields are not formed here (wt_loop_fwd_f64 / wt_loop_adj_f64 form them).
+ * Outputs equal wt_loop_fwd_f64's bit for bit.  WT_EUNSUPPORTED for plans
+ * that do not run it (the nonlinear cell, tuning.plain, pixels shared by
+ * several sources): use the entry points above.  Replaces the same reference
+ * code as those. */
+int wt_workspace_bytes_rec_f64(const void *plan, int32_t with_grad, int64_t *saved,
+                               int64_t *temp);
+int wt_loop_fwd_rec_f64(void *plan, const wt_scalars_f64 *sc, const double *b, const double *c,
+                        const double *x, double *y, double *fields, int32_t field_stride,
+                        int32_t with_grad, void *saved, void *temp, void *stream);
+int wt_loop_adj_rec_f64(void *plan, const wt_scalars_f64 *sc, const double *c,
+                        const double *ybar, void *saved, void *temp, double *grad_c,
+                        double *grad_x, void *stream);
+
 /* ------------------------------------------------------------------------ */
 /* Batched instances                                                         */
 /* ------------------------------------------------------------------------ */

@@ -130,6 +130,12 @@ _SIGS = {
                                        c_p, c_i32, c_i32, c_p, c_p, c_p]),
     "wt_loop_adj_f64": (ctypes.c_int, [c_p, ctypes.POINTER(WtScalarsF64), c_p, c_p, c_p, c_p, c_p,
                                        c_p, c_p, c_p, c_p, c_p, c_p, c_p]),
+    "wt_workspace_bytes_rec_f64": (ctypes.c_int, [c_p, c_i32, ctypes.POINTER(c_i64),
+                                                  ctypes.POINTER(c_i64)]),
+    "wt_loop_fwd_rec_f64": (ctypes.c_int, [c_p, ctypes.POINTER(WtScalarsF64), c_p, c_p, c_p, c_p,
+                                           c_p, c_i32, c_i32, c_p, c_p, c_p]),
+    "wt_loop_adj_rec_f64": (ctypes.c_int, [c_p, ctypes.POINTER(WtScalarsF64), c_p, c_p, c_p, c_p,
+                                           c_p, c_p, c_p]),
     "wt_autotune": (ctypes.c_int, [ctypes.POINTER(WtConfig), c_i32, c_i32, c_f32,
                                    ctypes.POINTER(WtTuning), c_i32, c_p, c_p, c_p, c_p, c_i32,
                                    ctypes.c_double, ctypes.POINTER(WtTuning),

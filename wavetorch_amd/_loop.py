@@ -138,6 +138,21 @@ class Plan:
                    "wt_workspace_bytes_f64")
         return s0.value, t0.value
 
+    def bytes_rec_f64(self):
+        """{with_grad: (saved, temp)} bytes of the blocked float64 loop of the
+        linear cell (wt_workspace_bytes_rec_f64), or None when this plan does
+        not run it."""
+        out = {}
+        for g in (0, 1):
+            s0, t0 = _lib.c_i64(), _lib.c_i64()
+            rc = _lib.lib().wt_workspace_bytes_rec_f64(self.handle, g, ctypes.byref(s0),
+                                                       ctypes.byref(t0))
+            if rc == _lib.WT_EUNSUPPORTED:
+                return None
+            _lib.check(rc, "wt_workspace_bytes_rec_f64")
+            out[g] = (s0.value, t0.value)
+        return out
+
     def __del__(self):
         h = getattr(self, "handle", None)
         if h is not None and h.value:
@@ -194,7 +209,21 @@ class WaveLoop(torch.autograd.Function):
         else:
             y = torch.empty((B, T, ntap), dtype=dtype, device=dev)
         s = _lib.stream_ptr(dev)
-        if f64:
+        # float64: blocked launches, unless dJ/db or the fields' gradient is
+        # wanted (the per-step loop forms those from every field)
+        rec64 = None
+        if f64 and not need[2] and not (with_grad and output_fields):
+            rec64 = plan.bytes_rec_f64()
+        if rec64 is not None:
+            sb, tb = rec64[int(with_grad)]
+            saved = _buf(sb, dev) if with_grad else None
+            temp = _buf(tb, dev)
+            sc = scalars_f64(plan.cfg)
+            _lib.check(_lib.lib().wt_loop_fwd_rec_f64(
+                plan.handle, ctypes.byref(sc), b.data_ptr(), c.data_ptr(), x.data_ptr(),
+                _lib.ptr(y), _lib.ptr(fields), int(field_stride), int(with_grad),
+                _lib.ptr(saved), temp.data_ptr(), s), "wt_loop_fwd_rec_f64")
+        elif f64:
             sb, tb = plan.bytes_f64(with_grad)
             saved = _buf(sb, dev) if with_grad else None
             # three rotating fields without gradients; the tape holds every
@@ -220,6 +249,7 @@ class WaveLoop(torch.autograd.Function):
             ctx.ws = saved
             plan._record = weakref.ref(saved)
             ctx.plan = plan
+            ctx.rec64 = rec64
             ctx.has_rho = rho_c is not None
             ctx.output_fields = output_fields
             ctx.field_stride = field_stride
@@ -246,7 +276,15 @@ class WaveLoop(torch.autograd.Function):
         s = _lib.stream_ptr(dev)
         ybar = None if ctx.output_fields else g.data_ptr()
         fbar = g.data_ptr() if ctx.output_fields else None
-        if f64:
+        if ctx.rec64 is not None:
+            temp = _buf(ctx.rec64[1][1], dev)
+            sc = scalars_f64(plan.cfg)
+            _lib.check(_lib.lib().wt_loop_adj_rec_f64(
+                plan.handle, ctypes.byref(sc), c.data_ptr(), ybar, ctx.ws.data_ptr(),
+                temp.data_ptr(), _lib.ptr(gc), _lib.ptr(gx), s), "wt_loop_adj_rec_f64")
+            if grho is not None:
+                grho.zero_()  # the linear cell does not read rho
+        elif f64:
             temp = _buf(plan.bytes_f64(True)[1], dev)
             sc = scalars_f64(plan.cfg)
             _lib.check(_lib.lib().wt_loop_adj_f64(

@@ -1,0 +1,118 @@
+// wt_colseg.h -- region geometry and memory access shared by the temporally
+// blocked column-segment kernels (wt_colseg.hip in float, wt_f64.hip in
+// double; the thread mapping is described in wt_colseg.hip).  Not part of the
+// public ABI.
+#pragma once
+
+#include "wt_internal.h"
+
+namespace wt {
+
+// Largest number of steps one launch of these kernels may take (the input
+// samples of a launch are staged in LDS).
+constexpr int CS_MAX_TBLOCK = 256;
+// Largest number of special pixels / probe taps one tile may hold.
+constexpr int CS_MAX_TABLE = 256;
+// Probe-seed table: at most this many probe pixels per region.
+constexpr int CS_MAX_SEEDS = 16;
+
+struct CsGeom {
+  int R0, RH, C0, RW;     // region
+  int or0, or1, oc0, oc1; // output rows / cols (domain)
+  int k, c;               // segment, column of this thread
+  bool active;            // thread owns cells
+  int CS;                 // LDS column stride (odd)
+  int base;               // LDS index of this thread's first cell
+};
+
+// LAYOUT: take the thread-mapping width and LDS column stride the host chose
+// (cs_layout, descriptor words 12 and 13; the plain mapping unless they fit
+// this launch's rows per thread and threads) -- the forward kernels, whose
+// LDS allocation holds the padded stride.  Otherwise (the adjoints, which
+// wait little on LDS) the plain mapping t -> (t / RW, t % RW).
+template <int R, bool LAYOUT = false>
+__device__ __forceinline__ CsGeom cs_geom(const int32_t *td, int tid) {
+  CsGeom g;
+  g.R0 = td[0]; g.RH = td[1]; g.C0 = td[2]; g.RW = td[3];
+  g.or0 = td[4]; g.or1 = td[5]; g.oc0 = td[6]; g.oc1 = td[7];
+  const int nseg = (g.RH + R - 1) / R;
+  if constexpr (LAYOUT) {
+    int RWm = td[12], CS = td[13];
+    if (RWm < g.RW || CS < nseg * R + 2 || CS > ((nseg * R + 2) | 1) + cs_lds_slack(R) ||
+        RWm * nseg > (int)blockDim.x) {
+      RWm = g.RW;
+      CS = (nseg * R + 2) | 1;
+    }
+    g.CS = CS;
+    g.k = tid / RWm;
+    g.c = tid - g.k * RWm;
+    g.active = g.k < nseg && g.c < g.RW;
+  } else {
+    g.k = tid / g.RW;
+    g.c = tid - g.k * g.RW;
+    g.active = g.k < nseg;
+    g.CS = (nseg * R + 2) | 1;
+  }
+  g.base = (g.c + 1) * g.CS + g.k * R + 1;
+  return g;
+}
+
+// Rows [lo, hi) of the region that still influence the output after step s
+// of a launch of n steps.
+__device__ __forceinline__ void cone(const CsGeom &g, int s, int n, int &lo, int &hi) {
+  const int rem = n - 1 - s;
+  const int olo = g.or0 - g.R0, ohi = g.or1 - g.R0;
+  lo = olo > 0 ? max(0, olo - rem) : 0;
+  hi = ohi < g.RH ? min(g.RH, ohi + rem) : g.RH;
+}
+
+// Raw buffer access with hardware range checking (gfx9 descriptor word 3 =
+// 0x00020000): a load outside [0, num_records) bytes returns 0 and a store
+// there is dropped.  The slices below put the buffer base at the first
+// output row of the tile, so rows above the output rows give negative byte
+// offsets (huge as unsigned) and rows below give offsets >= num_records:
+// both fall outside the range without any per-row predicate.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t cs_rsrc(const void *p, int64_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void *)p, (short)0, (int)bytes, 0x00020000);
+}
+__device__ __forceinline__ float cs_bload(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, (int)off, 0, 0));
+}
+__device__ __forceinline__ void cs_bstore(__amdgpu_buffer_rsrc_t rs, uint32_t off, float v) {
+  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rs, (int)off, 0, 0);
+}
+// Byte offset of this thread's first cell relative to the first output row
+// of its tile (column C0 + c); an out-of-range marker if the thread's column
+// is outside the tile's output columns.
+template <typename T>
+__device__ __forceinline__ uint32_t cs_out_voff(const CsGeom &g, int row0, int Ny) {
+  const int gc = g.C0 + g.c;
+  if (!g.active || gc < g.oc0 || gc >= g.oc1) return 0x80000000u;
+  return (uint32_t)(((g.R0 + row0 - g.or0) * Ny + gc) * (int)sizeof(T));
+}
+
+// Zeroes LDS buffer b1 and, of b0, only the cells that the workgroup's fill
+// of b0 (every cell of every segment of the region's columns) leaves alone:
+// the ring columns 0 and RW+1 and, in the region's columns, the ring row 0
+// and the rows past the last segment (CS - nrows cells per column).
+template <typename T>
+__device__ __forceinline__ void cs_zero_lds(T *b0, T *b1, const CsGeom &g, int nrows,
+                                            int NBUF) {
+  for (int i = threadIdx.x; i < NBUF; i += blockDim.x) b1[i] = T(0);
+  const int tail = g.CS - nrows;
+  const int nring = 2 * g.CS + g.RW * tail;
+  for (int i = threadIdx.x; i < nring; i += blockDim.x) {
+    int idx;
+    if (i < g.CS) {
+      idx = i;
+    } else if (i < 2 * g.CS) {
+      idx = (g.RW + 1) * g.CS + (i - g.CS);
+    } else {
+      const int j = i - 2 * g.CS, col = j / tail, r = j - col * tail;
+      idx = (col + 1) * g.CS + (r == 0 ? 0 : nrows + r);
+    }
+    b0[idx] = T(0);
+  }
+}
+
+}  // namespace wt

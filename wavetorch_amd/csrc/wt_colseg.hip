@@ -28,81 +28,10 @@
 //     gacc += lap(u_{m-1}) * lam_m
 // Cells with a source pixel or a probe tap take a slower code path that only
 // the waves containing them execute (wave-uniform branch).
-#include "wt_internal.h"
+#include "wt_colseg.h"
 
 namespace wt {
 
-// Largest number of steps one launch of these kernels may take (the input
-// samples of a launch are staged in LDS).
-constexpr int CS_MAX_TBLOCK = 256;
-// Largest number of special pixels / probe taps one tile may hold.
-constexpr int CS_MAX_TABLE = 256;
-
-struct CsGeom {
-  int R0, RH, C0, RW;     // region
-  int or0, or1, oc0, oc1; // output rows / cols (domain)
-  int k, c;               // segment, column of this thread
-  bool active;            // thread owns cells
-  int CS;                 // LDS column stride (odd)
-  int base;               // LDS index of this thread's first cell
-};
-
-// LAYOUT: take the thread-mapping width and LDS column stride the host chose
-// (cs_layout, descriptor words 12 and 13; the plain mapping unless they fit
-// this launch's rows per thread and threads) -- the forward kernels, whose
-// LDS allocation holds the padded stride.  Otherwise (the adjoints, which
-// wait little on LDS) the plain mapping t -> (t / RW, t % RW).
-template <int R, bool LAYOUT = false>
-__device__ __forceinline__ CsGeom cs_geom(const int32_t *td, int tid) {
-  CsGeom g;
-  g.R0 = td[0]; g.RH = td[1]; g.C0 = td[2]; g.RW = td[3];
-  g.or0 = td[4]; g.or1 = td[5]; g.oc0 = td[6]; g.oc1 = td[7];
-  const int nseg = (g.RH + R - 1) / R;
-  if constexpr (LAYOUT) {
-    int RWm = td[12], CS = td[13];
-    if (RWm < g.RW || CS < nseg * R + 2 || CS > ((nseg * R + 2) | 1) + cs_lds_slack(R) ||
-        RWm * nseg > (int)blockDim.x) {
-      RWm = g.RW;
-      CS = (nseg * R + 2) | 1;
-    }
-    g.CS = CS;
-    g.k = tid / RWm;
-    g.c = tid - g.k * RWm;
-    g.active = g.k < nseg && g.c < g.RW;
-  } else {
-    g.k = tid / g.RW;
-    g.c = tid - g.k * g.RW;
-    g.active = g.k < nseg;
-    g.CS = (nseg * R + 2) | 1;
-  }
-  g.base = (g.c + 1) * g.CS + g.k * R + 1;
-  return g;
-}
-
-// Rows [lo, hi) of the region that still influence the output after step s
-// of a launch of n steps.
-__device__ __forceinline__ void cone(const CsGeom &g, int s, int n, int &lo, int &hi) {
-  const int rem = n - 1 - s;
-  const int olo = g.or0 - g.R0, ohi = g.or1 - g.R0;
-  lo = olo > 0 ? max(0, olo - rem) : 0;
-  hi = ohi < g.RH ? min(g.RH, ohi + rem) : g.RH;
-}
-
-// Raw buffer access with hardware range checking (gfx9 descriptor word 3 =
-// 0x00020000): a load outside [0, num_records) bytes returns 0 and a store
-// there is dropped.  The slices below put the buffer base at the first
-// output row of the tile, so rows above the output rows give negative byte
-// offsets (huge as unsigned) and rows below give offsets >= num_records:
-// both fall outside the range without any per-row predicate.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t cs_rsrc(const float *p, int64_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc((void *)p, (short)0, (int)bytes, 0x00020000);
-}
-__device__ __forceinline__ float cs_bload(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, (int)off, 0, 0));
-}
-__device__ __forceinline__ void cs_bstore(__amdgpu_buffer_rsrc_t rs, uint32_t off, float v) {
-  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rs, (int)off, 0, 0);
-}
 // The segment record (lap u, u) is written once by the recompute and read
 // once by the adjoint.  Cache policies of those accesses (the buffer
 // instructions' cache-policy operand: 2 = nt, 16 = sc1).  Measured on MI355X
@@ -122,38 +51,6 @@ __device__ __forceinline__ float cs_rec_load(__amdgpu_buffer_rsrc_t rs, uint32_t
 __device__ __forceinline__ void cs_rec_store(__amdgpu_buffer_rsrc_t rs, uint32_t off, float v) {
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rs, (int)off, 0,
                                         WT_RECORD_STORE_CPOL);
-}
-
-// Byte offset of this thread's first cell relative to the first output row
-// of its tile (column C0 + c); an out-of-range marker if the thread's column
-// is outside the tile's output columns.
-__device__ __forceinline__ uint32_t cs_out_voff(const CsGeom &g, int row0, int Ny) {
-  const int gc = g.C0 + g.c;
-  if (!g.active || gc < g.oc0 || gc >= g.oc1) return 0x80000000u;
-  return (uint32_t)(((g.R0 + row0 - g.or0) * Ny + gc) * 4);
-}
-
-// Zeroes LDS buffer b1 and, of b0, only the cells that the workgroup's fill
-// of b0 (every cell of every segment of the region's columns) leaves alone:
-// the ring columns 0 and RW+1 and, in the region's columns, the ring row 0
-// and the rows past the last segment (CS - nrows cells per column).
-__device__ __forceinline__ void cs_zero_lds(float *b0, float *b1, const CsGeom &g, int nrows,
-                                            int NBUF) {
-  for (int i = threadIdx.x; i < NBUF; i += blockDim.x) b1[i] = 0.0f;
-  const int tail = g.CS - nrows;
-  const int nring = 2 * g.CS + g.RW * tail;
-  for (int i = threadIdx.x; i < nring; i += blockDim.x) {
-    int idx;
-    if (i < g.CS) {
-      idx = i;
-    } else if (i < 2 * g.CS) {
-      idx = (g.RW + 1) * g.CS + (i - g.CS);
-    } else {
-      const int j = i - 2 * g.CS, col = j / tail, r = j - col * tail;
-      idx = (col + 1) * g.CS + (r == 0 ? 0 : nrows + r);
-    }
-    b0[idx] = 0.0f;
-  }
 }
 
 // ------------------------------------------------------------------ forward
@@ -313,7 +210,7 @@ __device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
     tpv0 = t[0]; tpv1 = t[1]; tpv2 = t[2]; tpv3 = t[3];
   }
   // 2) LDS (buf0's region cells are filled from U0 below)
-  cs_zero_lds(buf0, buf1, g, ((g.RH + R - 1) / R) * R, NBUF);
+  cs_zero_lds<float>(buf0, buf1, g, ((g.RH + R - 1) / R) * R, NBUF);
   WT_TS(4);
   if (tid < a.nsteps) xs[tid] = xsv;
   if (tid < nsp) { tb_sp[3 * tid] = spv0; tb_sp[3 * tid + 1] = spv1; tb_sp[3 * tid + 2] = spv2; }
@@ -363,7 +260,7 @@ __device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
       ++kk;
     }
   }
-  const uint32_t voff = cs_out_voff(g, row0, Ny);
+  const uint32_t voff = cs_out_voff<float>(g, row0, Ny);
   const int64_t out_bytes = (int64_t)(g.or1 - g.or0) * Ny * 4;
   // record slots of this sample; steps at or past its length are not
   // recorded (empty slice: the stores are dropped)
@@ -448,9 +345,6 @@ __global__ __launch_bounds__(NT) void k_fwd_cs_batch(BatchFwd bl) {
 }
 
 // ------------------------------------------------------------------ adjoint
-
-// Probe-seed table: at most this many probe pixels per region.
-constexpr int CS_MAX_SEEDS = 16;
 
 // One reverse step of this thread's segment.  SP: the wave holds
 // probe/source pixels (sr0, sr1).  a2 = A*Bm is formed as a1 - 1 (with
@@ -546,7 +440,7 @@ __device__ __forceinline__ void adj_cs_body(const AdjArgs &a, const int w) {
     e0 = e[0]; e1 = e[1]; e2 = e[2]; e3 = e[3]; e4 = e[4]; e5 = e[5];
   }
   // 2) LDS (buf0's region cells are filled from the lambda pair below)
-  cs_zero_lds(buf0, buf1, g, ((g.RH + R - 1) / R) * R, NBUF);
+  cs_zero_lds<float>(buf0, buf1, g, ((g.RH + R - 1) / R) * R, NBUF);
   if (tid < nsp) {
     int *t = tb_sp + 6 * tid;
     t[0] = e0; t[1] = e1; t[2] = e2; t[3] = e3; t[4] = e4; t[5] = e5;
@@ -621,7 +515,7 @@ __device__ __forceinline__ void adj_cs_body(const AdjArgs &a, const int w) {
       if (row0 + r < g.RH && gr >= g.or0 && gr < g.or1) omask |= 1u << r;
     }
   }
-  const uint32_t voff = cs_out_voff(g, row0, Ny);
+  const uint32_t voff = cs_out_voff<float>(g, row0, Ny);
   const int64_t out_bytes = (int64_t)(g.or1 - g.or0) * Ny * 4;
   // record of step j (read at reverse step m = j + 1): a sample's steps at or
   // past its length are not recorded, and lambda_m is exactly 0 there, so

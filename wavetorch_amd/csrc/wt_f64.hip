@@ -285,10 +285,17 @@ __global__ void k64_finalize_gx(const double *__restrict__ gsrc, int B, int T, i
 
 static inline unsigned nblk64(int64_t n) { return (unsigned)((n + 255) / 256); }
 
-static hipError_t fill64(double *p, int64_t n, double v, hipStream_t s) {
+hipError_t launch_fill64(double *p, int64_t n, double v, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   const unsigned g = (unsigned)std::min<int64_t>((n + 255) / 256, 4096);
   hipLaunchKernelGGL(k64_fill, dim3(g), dim3(256), 0, s, p, n, v);
+  return hipGetLastError();
+}
+
+hipError_t launch_finalize_gx64(const double *gsrc, int B, int T, int nslot, const int32_t *mult,
+                                double *gx, hipStream_t s) {
+  hipLaunchKernelGGL(k64_finalize_gx, dim3(nblk64((int64_t)B * T)), dim3(256), 0, s, gsrc, B, T,
+                     nslot, mult, gx);
   return hipGetLastError();
 }
 
@@ -369,7 +376,7 @@ extern "C" int wt_loop_fwd_f64(void *plan, const wt_scalars_f64 *sc, const doubl
   const unsigned g = nblk64(w.BF);
   if (with_grad) {
     double *U = (double *)saved;
-    WT_HIP(fill64(U, 2 * w.BF, 0.0, s));  // u_{-1} = u_0 = 0 (rnn.py:39-41)
+    WT_HIP(launch_fill64(U, 2 * w.BF, 0.0, s));  // u_{-1} = u_0 = 0 (rnn.py:39-41)
     for (int n = 0; n < v.T; ++n) {
       hipLaunchKernelGGL(k64_fwd, dim3(g), dim3(256), 0, s, a, U + (int64_t)(n + 1) * w.BF,
                          U + (int64_t)n * w.BF, U + (int64_t)(n + 2) * w.BF, y, fields,
@@ -378,7 +385,7 @@ extern "C" int wt_loop_fwd_f64(void *plan, const wt_scalars_f64 *sc, const doubl
     }
   } else {
     double *st = (double *)temp;
-    WT_HIP(fill64(st, 2 * w.BF, 0.0, s));
+    WT_HIP(launch_fill64(st, 2 * w.BF, 0.0, s));
     double *p1 = st, *p2 = st + w.BF, *p3 = st + 2 * w.BF;  // u_n, u_{n-1}, u_{n+1}
     for (int n = 0; n < v.T; ++n) {
       hipLaunchKernelGGL(k64_fwd, dim3(g), dim3(256), 0, s, a, p1, p2, p3, y, fields,
@@ -410,7 +417,7 @@ extern "C" int wt_loop_adj_f64(void *plan, const wt_scalars_f64 *sc, const doubl
   double *lam[3] = {t, t + BF, t + 2 * BF};
   double *gc = t + 3 * BF, *gb = t + 4 * BF, *gr = t + 5 * BF;
   double *gsrc = t + 6 * BF;
-  WT_HIP(fill64(t, w.adj_temp, 0.0, s));  // lambda_{T+1} = lambda_{T+2} = 0
+  WT_HIP(launch_fill64(t, w.adj_temp, 0.0, s));  // lambda_{T+1} = lambda_{T+2} = 0
   const int tiles_x = (v.Nx + K64_TX - 1) / K64_TX, tiles_y = (v.Ny + K64_TY - 1) / K64_TY;
   const unsigned g = (unsigned)((int64_t)v.B * tiles_x * tiles_y);
   double *l1 = lam[0], *l2 = lam[1], *l0 = lam[2];
@@ -437,16 +444,14 @@ extern "C" int wt_loop_adj_f64(void *plan, const wt_scalars_f64 *sc, const doubl
       hipLaunchKernelGGL(k64_batch_sum, dim3(gf), dim3(256), 0, s, gr, v.B, F, grad_rho);
       WT_HIP(hipGetLastError());
     } else {
-      WT_HIP(fill64(grad_rho, F, 0.0, s));
+      WT_HIP(launch_fill64(grad_rho, F, 0.0, s));
     }
   }
   if (grad_x) {
     if (v.nslot > 0) {
-      hipLaunchKernelGGL(k64_finalize_gx, dim3(nblk64((int64_t)v.B * v.T)), dim3(256), 0, s,
-                         gsrc, v.B, v.T, v.nslot, v.mult, grad_x);
-      WT_HIP(hipGetLastError());
+      WT_HIP(launch_finalize_gx64(gsrc, v.B, v.T, v.nslot, v.mult, grad_x, s));
     } else {
-      WT_HIP(fill64(grad_x, (int64_t)v.B * v.T, 0.0, s));
+      WT_HIP(launch_fill64(grad_x, (int64_t)v.B * v.T, 0.0, s));
     }
   }
   return WT_OK;

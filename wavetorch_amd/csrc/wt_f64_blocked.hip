@@ -1,0 +1,609 @@
+// wt_f64_blocked.hip -- the linear WaveRNN loop in double precision,
+// temporally blocked (gfx950).
+//
+// The thread mapping and the launches are those of the float kernels
+// (wt_colseg.hip): one workgroup advances one tile of one sample plus a halo
+// by `nsteps` steps, a thread's R rows of one column in registers and the
+// field in LDS.  Double vector instructions issue at the rate of the
+// non-packed float ones on this chip, so a step costs what it costs in
+// float; registers and LDS hold half the cells.
+//
+// The forward with gradients records lap(u_n) of every step (the tape's size:
+// T x B x Nx x Ny doubles), which is all of the field that the adjoint of the
+// linear cell reads:
+//   lambda_m = a1 lambda_{m+1} + L(w lambda_{m+1}) - a2 lambda_{m+2} + seeds
+//   dJ/dc    = 2 A c sum_m lap(u_{m-1}) lambda_m
+// so nothing is recomputed, and each step of the adjoint reads 8 bytes per
+// cell instead of the fields u_{m+1} .. u_{m-2}, both lambdas and the
+// gradient sum (the per-step kernels of wt_f64.hip, which stay for the
+// nonlinear cell, for dJ/db and for field seeds).  The forward follows the
+// reference's operation order (cell.py:12-17, operators.py:5-11), bitwise
+// equal to the per-step kernel's.
+#include <algorithm>
+
+#include "wt_colseg.h"
+
+namespace wt {
+
+struct F64Blk {
+  int B, Nx, Ny, T, ntiles, ntap, nslot;
+  const int32_t *tiles, *spx, *taps;
+  const double *A, *Bm, *C2;
+  double s2, t1, t4;
+  const double *in1, *in2;  // null: zero fields
+  double *out1, *out2;
+  int n0, nsteps;           // forward: first step of the launch
+  const double *x;
+  double *y, *yraw, *fields, *rec;
+  int fstride;
+  const double *ybar;       // adjoint: reverse steps m_hi .. m_hi - nsteps + 1
+  double *gacc, *gsrc;
+  int m_hi;
+  int first;                // adjoint: gacc holds nothing yet
+};
+
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ double b64_load(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
+  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, (int)off, 0, 0));
+}
+__device__ __forceinline__ void b64_store(__amdgpu_buffer_rsrc_t rs, uint32_t off, double v) {
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), rs, (int)off, 0, 0);
+}
+
+template <int NT, int R, bool REC, bool UH>
+__global__ __launch_bounds__(NT) void k64_fwd_cs(F64Blk a) {
+  extern __shared__ double smem64[];
+  __shared__ int tb_sp[CS_MAX_TABLE * 3];  // source pixels of the region: x, y, multiplicity
+  __shared__ int tb_tp[CS_MAX_TABLE * 4];
+  const int tid = threadIdx.x;
+  const int w = xcd_remap(blockIdx.x, gridDim.x);
+  const int b = w / a.ntiles, ti = w - (w / a.ntiles) * a.ntiles;
+  const int32_t *td = a.tiles + ti * TILE_W;
+  const CsGeom g = cs_geom<R>(td, tid);
+  const int NBUF = (g.RW + 2) * g.CS;
+  double *buf0 = smem64, *buf1 = smem64 + NBUF, *xs = smem64 + 2 * NBUF;
+  const int Ny = a.Ny;
+  const int64_t F = (int64_t)a.Nx * Ny, boff = (int64_t)b * F;
+  const int nsp = min(td[9] - td[8], CS_MAX_TABLE), ntp = min(td[11] - td[10], CS_MAX_TABLE);
+  const int row0 = g.k * R;
+  double U0[R], U1[R], KA[R], KB[R], KC[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    double u1 = 0., u2 = 0., v0 = 0., v1 = 0., v2 = 0.;
+    if (g.active && row0 + r < g.RH) {
+      const int64_t q = (int64_t)(g.R0 + row0 + r) * Ny + (g.C0 + g.c);
+      v0 = a.A[q]; v1 = a.Bm[q]; v2 = a.C2[q];
+      if (a.in1) { u1 = a.in1[boff + q]; u2 = a.in2[boff + q]; }
+    }
+    U0[r] = u1; U1[r] = u2; KA[r] = v0; KB[r] = v1; KC[r] = v2;
+  }
+  for (int i = tid; i < a.nsteps; i += blockDim.x) xs[i] = a.x[(int64_t)b * a.T + a.n0 + i];
+  for (int i = tid; i < nsp; i += blockDim.x) {
+    const int32_t *e = a.spx + (td[8] + i) * SPX_W;
+    for (int j = 0; j < 3; ++j) tb_sp[3 * i + j] = e[j];
+  }
+  for (int i = tid; i < ntp; i += blockDim.x) {
+    const int32_t *e = a.taps + (td[10] + i) * TAP_W;
+    for (int j = 0; j < 4; ++j) tb_tp[4 * i + j] = e[j];
+  }
+  cs_zero_lds<double>(buf0, buf1, g, ((g.RH + R - 1) / R) * R, NBUF);
+  __syncthreads();
+  if (g.active) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) buf0[g.base + r] = U0[r];
+  }
+  // rows of this thread that hold a source pixel (at most two; the host sends
+  // other source sets to the per-step kernels)
+  int sr0 = -1, sr1 = -1;
+  for (int k = 0; k < nsp; ++k) {
+    const int rr = tb_sp[3 * k] - g.R0 - row0;
+    if (tb_sp[3 * k + 2] <= 0 || !g.active || tb_sp[3 * k + 1] - g.C0 != g.c || rr < 0 ||
+        rr >= R || row0 + rr >= g.RH)
+      continue;
+    if (sr0 < 0) sr0 = rr; else sr1 = rr;
+  }
+  const bool wave_src = __ballot(sr0 >= 0) != 0;
+  // probe tap of this thread (taps in the output region)
+  int pidx = -1, pkind = 0, pcol = 0;
+  for (int t = 0, kk = 0; t < ntp; ++t) {
+    const int tx = tb_tp[4 * t], ty = tb_tp[4 * t + 1];
+    if (ty < g.oc0 || ty >= g.oc1) continue;
+    if (kk++ == tid) {
+      pidx = (ty - g.C0 + 1) * g.CS + (tx - g.R0) + 1;
+      pkind = tb_tp[4 * t + 2];
+      pcol = tb_tp[4 * t + 3];
+    }
+  }
+  const uint32_t voff = cs_out_voff<double>(g, row0, Ny);
+  const int64_t out_bytes = (int64_t)(g.or1 - g.or0) * Ny * 8;
+  __syncthreads();
+
+  auto step = [&](const double *P, double *Q, double(&Uc)[R], double(&Up)[R], int s) {
+    const int n = a.n0 + s;
+    int lo, hi;
+    cone(g, s, a.nsteps, lo, hi);
+    const bool snap = a.fields && ((n + 1) % a.fstride) == 0;
+    if (g.active && row0 < hi && row0 + R > lo) {
+      const __amdgpu_buffer_rsrc_t rsl = cs_rsrc(
+          REC ? a.rec + ((int64_t)b * a.T + n) * F + (int64_t)g.or0 * Ny : a.A,
+          REC ? out_bytes : 0);
+      const int lfb = g.base - g.CS, rtb = g.base + g.CS;
+      double upv = UH ? P[g.base - 1] : a.t1 * P[g.base - 1];
+      double ctv = UH ? 0.0 : a.t1 * Uc[0];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const double ct = Uc[r];
+        const double dn = (r < R - 1) ? Uc[r + 1] : P[g.base + R];
+        const double lf = P[lfb + r], rt = P[rtb + r];
+        double lap;
+        if (UH) {  // products with t1 = 1 and t4 = -4 are exact
+          double s0 = upv + lf;
+          s0 = __builtin_fma(-4.0, ct, s0);
+          s0 = s0 + rt;
+          lap = s0 + dn;
+          upv = ct;
+        } else {
+          const double dnv = a.t1 * dn;
+          double s0 = upv + a.t1 * lf;
+          s0 = s0 + a.t4 * ct;
+          s0 = s0 + a.t1 * rt;
+          lap = s0 + dnv;
+          upv = ctv;
+          ctv = dnv;
+        }
+        const double p1 = a.s2 * ct;
+        const double p2 = KB[r] * Up[r];
+        const double p3 = KC[r] * lap;
+        const double v = KA[r] * ((p1 - p2) + p3);
+        Up[r] = v;
+        Q[g.base + r] = v;
+        if (REC) b64_store(rsl, voff + (uint32_t)(r * Ny * 8), lap);
+      }
+      if (wave_src && sr0 >= 0) {
+        const double xv = xs[s];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          if (r == sr0 || r == sr1) {
+            Up[r] = Up[r] + xv;
+            Q[g.base + r] = Up[r];
+          }
+      }
+      if (snap) {  // the thread's own rows: consecutive lanes, consecutive columns
+        const int64_t nf = a.T / a.fstride;
+        const __amdgpu_buffer_rsrc_t rf = cs_rsrc(
+            a.fields + ((int64_t)b * nf + (n + 1) / a.fstride - 1) * F + (int64_t)g.or0 * Ny,
+            out_bytes);
+#pragma unroll
+        for (int r = 0; r < R; ++r) b64_store(rf, voff + (uint32_t)(r * Ny * 8), Up[r]);
+      }
+    }
+    __syncthreads();
+    if (pidx >= 0) {
+      const double v = Q[pidx];
+      const int64_t o = ((int64_t)b * a.T + n) * a.ntap + pcol;
+      if (a.y) a.y[o] = pkind ? v * v : v;
+      if (a.yraw) a.yraw[o] = v;
+    }
+  };
+  int s = 0;
+  for (; s + 1 < a.nsteps; s += 2) {
+    step(buf0, buf1, U0, U1, s);
+    step(buf1, buf0, U1, U0, s + 1);
+  }
+  if (s < a.nsteps) step(buf0, buf1, U0, U1, s);
+  const bool odd = (a.nsteps & 1) != 0;
+  const __amdgpu_buffer_rsrc_t r1 = cs_rsrc(a.out1 + boff + (int64_t)g.or0 * Ny, out_bytes);
+  const __amdgpu_buffer_rsrc_t r2 = cs_rsrc(a.out2 + boff + (int64_t)g.or0 * Ny, out_bytes);
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    b64_store(r1, voff + (uint32_t)(r * Ny * 8), odd ? U1[r] : U0[r]);
+    b64_store(r2, voff + (uint32_t)(r * Ny * 8), odd ? U0[r] : U1[r]);
+  }
+}
+
+// LDS holds w * lambda (w with the Laplacian's h^-2); the gradient sum and
+// the record values of the next two steps live in registers, the record read
+// two steps ahead at one issue point (as in the float kernel).
+template <int NT, int R>
+__global__ __launch_bounds__(NT) void k64_adj_cs(F64Blk a) {
+  extern __shared__ double smem64[];
+  __shared__ int tb_sp[CS_MAX_TABLE * 6];
+  __shared__ int seed_px[CS_MAX_SEEDS];
+  __shared__ int nseeds;
+  const int tid = threadIdx.x;
+  const int w = xcd_remap(blockIdx.x, gridDim.x);
+  const int b = w / a.ntiles, ti = w - (w / a.ntiles) * a.ntiles;
+  const int32_t *td = a.tiles + ti * TILE_W;
+  const CsGeom g = cs_geom<R>(td, tid);
+  const int NBUF = (g.RW + 2) * g.CS;
+  double *buf0 = smem64, *buf1 = smem64 + NBUF, *seeds = smem64 + 2 * NBUF;
+  const int Ny = a.Ny;
+  const int64_t F = (int64_t)a.Nx * Ny, boff = (int64_t)b * F;
+  const int nsp = min(td[9] - td[8], CS_MAX_TABLE);
+  const int row0 = g.k * R;
+  double L1[R], L2[R], KA1[R], KW[R], G[R], SG0[R], SG1[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    double A = 0., C2 = 0., u1 = 0., u2 = 0.;
+    if (g.active && row0 + r < g.RH) {
+      const int64_t q = (int64_t)(g.R0 + row0 + r) * Ny + (g.C0 + g.c);
+      A = a.A[q]; C2 = a.C2[q];
+      if (a.in1) { u1 = a.in1[boff + q]; u2 = a.in2[boff + q]; }
+    }
+    KA1[r] = A * a.s2; KW[r] = (A * C2) * a.t1;
+    L1[r] = u1; L2[r] = u2;
+    G[r] = 0.0; SG1[r] = 0.0;
+  }
+  for (int i = tid; i < nsp; i += blockDim.x) {
+    const int32_t *e = a.spx + (td[8] + i) * SPX_W;
+    for (int j = 0; j < 6; ++j) tb_sp[6 * i + j] = e[j];
+  }
+  cs_zero_lds<double>(buf0, buf1, g, ((g.RH + R - 1) / R) * R, NBUF);
+  __syncthreads();
+  if (tid == 0) {
+    int n = 0;
+    for (int k = 0; k < nsp && n < CS_MAX_SEEDS; ++k)
+      if (tb_sp[6 * k + 5] > tb_sp[6 * k + 4]) seed_px[n++] = k;
+    nseeds = n;
+  }
+  if (g.active) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) buf0[g.base + r] = KW[r] * L1[r];
+  }
+  __syncthreads();
+  for (int i = tid; i < nseeds * a.nsteps; i += blockDim.x) {
+    const int k = i / a.nsteps, s = i - k * a.nsteps, m = a.m_hi - s;
+    const int *e = tb_sp + 6 * seed_px[k];
+    double gs = 0.0;
+    if (a.ybar)
+      for (int t = e[4]; t < e[5]; ++t) {
+        const int32_t *tp = a.taps + t * TAP_W;
+        const int64_t o = ((int64_t)b * a.T + (m - 1)) * a.ntap + tp[3];
+        gs += tp[2] ? 2.0 * a.yraw[o] * a.ybar[o] : a.ybar[o];
+      }
+    seeds[i] = gs;
+  }
+  // special rows of this thread (at most two): seed slot, source slot
+  int sr0 = -1, sr1 = -1, sd0 = -1, sd1 = -1, sl0 = -1, sl1 = -1;
+  for (int k = 0, nseed = 0; k < nsp; ++k) {
+    const int *e = tb_sp + 6 * k;
+    const int sd = e[5] > e[4] ? nseed++ : -1;
+    const int rr = e[0] - g.R0 - row0;
+    if (!g.active || e[1] - g.C0 != g.c || rr < 0 || rr >= R || row0 + rr >= g.RH) continue;
+    const int sl = e[2] > 0 ? e[3] : -1;
+    if (sr0 < 0) { sr0 = rr; sd0 = sd; sl0 = sl; }
+    else { sr1 = rr; sd1 = sd; sl1 = sl; }
+  }
+  const bool wave_sp = __ballot(sr0 >= 0) != 0;
+  const uint32_t voff = cs_out_voff<double>(g, row0, Ny);
+  const int64_t out_bytes = (int64_t)(g.or1 - g.or0) * Ny * 8;
+  const bool out_col = voff != 0x80000000u;
+  const int olo = g.or0 - g.R0 - row0, ohi = g.or1 - g.R0 - row0;  // output rows, thread's count
+  __syncthreads();
+  auto rec_rsrc = [&](int m) {
+    return cs_rsrc(a.rec + ((int64_t)b * a.T + (m - 1)) * F + (int64_t)g.or0 * Ny, out_bytes);
+  };
+  {
+    const __amdgpu_buffer_rsrc_t rs0 = rec_rsrc(a.m_hi);
+#pragma unroll
+    for (int r = 0; r < R; ++r) SG0[r] = b64_load(rs0, voff + (uint32_t)(r * Ny * 8));
+    const bool two = a.nsteps > 1;
+    const __amdgpu_buffer_rsrc_t rs1 = rec_rsrc(two ? a.m_hi - 1 : a.m_hi);
+    const uint32_t v1 = two ? voff : 0x80000000u;
+#pragma unroll
+    for (int r = 0; r < R; ++r) SG1[r] = b64_load(rs1, v1 + (uint32_t)(r * Ny * 8));
+  }
+  auto step = [&](const double *P, double *Q, double(&Lc)[R], double(&Ln)[R], double(&SG)[R],
+                  int s) {
+    const int m = a.m_hi - s;
+    int lo, hi;
+    cone(g, s, a.nsteps, lo, hi);
+    const bool prefetch = s + 2 < a.nsteps;
+    const __amdgpu_buffer_rsrc_t rsn = rec_rsrc(prefetch ? m - 2 : m);
+    const uint32_t pvoff = prefetch ? voff : 0x80000000u;
+    if (g.active && row0 < hi && row0 + R > lo) {
+      const int lfb = g.base - g.CS, rtb = g.base + g.CS;
+      double upv = P[g.base - 1];
+      double ct = KW[0] * Lc[0];
+      double gs0 = 0.0, gs1 = 0.0;
+      if (wave_sp) {
+        if (sd0 >= 0) gs0 = seeds[sd0 * a.nsteps + s];
+        if (sd1 >= 0) gs1 = seeds[sd1 * a.nsteps + s];
+      }
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const double dn = (r < R - 1) ? KW[r + 1] * Lc[r + 1] : P[g.base + R];
+        const double lf = P[lfb + r], rt = P[rtb + r];
+        double lapw = upv + lf;
+        lapw = __builtin_fma(-4.0, ct, lapw);
+        lapw = lapw + rt;
+        lapw = lapw + dn;
+        // a1 L1 + lapw - a2 L2 with a2 = a1 - 1
+        double lam = __builtin_fma(KA1[r], Lc[r] - Ln[r], lapw + Ln[r]);
+        if (wave_sp) {
+          if (r == sr0) lam += gs0;
+          if (r == sr1) lam += gs1;
+        }
+        upv = ct;
+        ct = dn;
+        Ln[r] = lam;
+        Q[g.base + r] = KW[r] * lam;
+      }
+      if (wave_sp) {
+        double v0 = Ln[0], v1 = Ln[0];
+#pragma unroll
+        for (int r = 1; r < R; ++r) {
+          v0 = (r == sr0) ? Ln[r] : v0;
+          v1 = (r == sr1) ? Ln[r] : v1;
+        }
+        double *gsrc_row = a.gsrc + ((int64_t)b * a.T + (m - 1)) * a.nslot;
+        if (sl0 >= 0 && out_col && sr0 >= olo && sr0 < ohi) gsrc_row[sl0] = v0;
+        if (sl1 >= 0 && out_col && sr1 >= olo && sr1 < ohi) gsrc_row[sl1] = v1;
+      }
+    }
+    // gradient sum, then the record of two steps later into the same
+    // registers: one issue point outside the branches, always issued (see
+    // the float kernel in wt_colseg.hip)
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      G[r] = __builtin_fma(SG[r], Ln[r], G[r]);
+      asm volatile("" : "+v"(G[r]));
+      SG[r] = b64_load(rsn, pvoff + (uint32_t)(r * Ny * 8));
+    }
+    __syncthreads();
+  };
+  int s = 0;
+  for (; s + 1 < a.nsteps; s += 2) {
+    step(buf0, buf1, L1, L2, SG0, s);
+    step(buf1, buf0, L2, L1, SG1, s + 1);
+  }
+  if (s < a.nsteps) step(buf0, buf1, L1, L2, SG0, s);
+  const bool odd = (a.nsteps & 1) != 0;
+  const __amdgpu_buffer_rsrc_t r1 = cs_rsrc(a.out1 + boff + (int64_t)g.or0 * Ny, out_bytes);
+  const __amdgpu_buffer_rsrc_t r2 = cs_rsrc(a.out2 + boff + (int64_t)g.or0 * Ny, out_bytes);
+  const __amdgpu_buffer_rsrc_t rg = cs_rsrc(a.gacc + boff + (int64_t)g.or0 * Ny, out_bytes);
+  if (!a.first) {
+    double gold[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) gold[r] = b64_load(rg, voff + (uint32_t)(r * Ny * 8));
+#pragma unroll
+    for (int r = 0; r < R; ++r) G[r] = gold[r] + G[r];
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    b64_store(r1, voff + (uint32_t)(r * Ny * 8), odd ? L2[r] : L1[r]);
+    b64_store(r2, voff + (uint32_t)(r * Ny * 8), odd ? L1[r] : L2[r]);
+    b64_store(rg, voff + (uint32_t)(r * Ny * 8), G[r]);
+  }
+}
+
+// A = 1/(dt^-2 + b dt^-1), Bm = dt^-2 - b dt^-1, C2 = c^2 of the clamped c
+__global__ void k64_coef(const double *__restrict__ b, const double *__restrict__ c, int64_t n,
+                         double dtm1, double dtm2, int clamp, double cmin, double cmax,
+                         double *__restrict__ A, double *__restrict__ Bm,
+                         double *__restrict__ C2) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const double bd = b[i] * dtm1;
+  double cc = c[i];
+  if (clamp) {
+    if (cc < cmin) cc = cmin;
+    if (cc > cmax) cc = cmax;
+  }
+  A[i] = 1.0 / (dtm2 + bd);
+  Bm[i] = dtm2 - bd;
+  C2[i] = cc * cc;
+}
+
+// dJ/dc = 2 A c sum_b gacc, zero where the clamp holds c
+__global__ void k64_finalize_gc(const double *__restrict__ gacc, int B, int64_t F,
+                                const double *__restrict__ c, const double *__restrict__ A,
+                                int clamp, double cmin, double cmax, double *__restrict__ gc) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= F) return;
+  double s = 0.0;
+  for (int b = 0; b < B; ++b) s += gacc[(int64_t)b * F + q];
+  const double cc = c[q];
+  const bool held = clamp && (cc < cmin || cc > cmax);
+  gc[q] = held ? 0.0 : A[q] * 2.0 * cc * s;
+}
+
+size_t cs64_shmem_bytes(int R, int RH, int RW, int tb) {
+  const int nseg = (RH + R - 1) / R;
+  // field double buffer + staged inputs (forward) or probe seeds (adjoint)
+  return ((size_t)2 * (RW + 2) * ((nseg * R + 2) | 1) + (size_t)CS_MAX_SEEDS * tb) *
+         sizeof(double);
+}
+
+bool cs64_variant_exists(int R, bool fwd) { return R == 4 || (fwd ? R == 6 || R == 8 : R == 5); }
+
+template <typename K>
+static hipError_t launch64(K kfn, std::atomic<uint64_t> &done, const F64Blk &a, int nthreads,
+                           size_t shmem, hipStream_t s) {
+  hipError_t e = allow_dyn_lds((const void *)kfn, done);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kfn, dim3(a.B * a.ntiles), dim3(nthreads), shmem, s, a);
+  return hipGetLastError();
+}
+
+template <int R, bool REC, bool UH>
+static hipError_t launch64_fwd(const F64Blk &a, int nthreads, size_t shmem, hipStream_t s) {
+  static std::atomic<uint64_t> done{0};
+  return launch64(k64_fwd_cs<1024, R, REC, UH>, done, a, nthreads, shmem, s);
+}
+
+template <int R>
+static hipError_t launch64_fwd(bool rec, bool uh, const F64Blk &a, int nthreads, size_t shmem,
+                               hipStream_t s) {
+  if (uh)
+    return rec ? launch64_fwd<R, true, true>(a, nthreads, shmem, s)
+               : launch64_fwd<R, false, true>(a, nthreads, shmem, s);
+  return rec ? launch64_fwd<R, true, false>(a, nthreads, shmem, s)
+             : launch64_fwd<R, false, false>(a, nthreads, shmem, s);
+}
+
+template <int R>
+static hipError_t launch64_adj(const F64Blk &a, int nthreads, size_t shmem, hipStream_t s) {
+  static std::atomic<uint64_t> done{0};
+  return launch64(k64_adj_cs<1024, R>, done, a, nthreads, shmem, s);
+}
+
+// Workspace layout in doubles.  saved: A, Bm, C2, the probe amplitudes and
+// lap(u_n) of every step; temp: two state pairs and, forward without
+// gradients, the coefficients, or, adjoint, the gradient sum and lambda at
+// the source slots.
+struct Blk64 {
+  int64_t F, BF, yraw, rec, gsrc;
+  int64_t saved() const { return 3 * F + yraw + rec; }
+  int64_t fwd_temp() const { return 4 * BF + 3 * F; }
+  int64_t adj_temp() const { return 5 * BF + gsrc; }
+};
+static Blk64 blk64(const PlanView &v) {
+  Blk64 w;
+  w.F = (int64_t)v.Nx * v.Ny;
+  w.BF = v.B * w.F;
+  w.yraw = (int64_t)v.B * v.T * std::max(v.ntap, 1);
+  w.rec = (int64_t)v.T * w.BF;
+  w.gsrc = (int64_t)v.B * v.T * std::max(v.nslot, 1);
+  return w;
+}
+
+static F64Blk args64(const PlanView &v, const wt_scalars_f64 &sc, const TileView &t) {
+  F64Blk a{};
+  a.B = v.B; a.Nx = v.Nx; a.Ny = v.Ny; a.T = v.T; a.ntap = v.ntap;
+  a.nslot = std::max(v.nslot, 1);
+  a.ntiles = t.ntiles; a.tiles = t.tiles; a.spx = v.spx; a.taps = v.taps;
+  a.s2 = 2.0 * (1.0 / (sc.dt * sc.dt));
+  a.t1 = 1.0 / (sc.h * sc.h);
+  a.t4 = -4.0 * a.t1;
+  a.fstride = 1;
+  return a;
+}
+
+}  // namespace wt
+
+using namespace wt;
+
+// Common argument checks: a plan whose linear cell runs blocked in double
+// precision.
+static int check64(const char *what, const void *plan, const wt_scalars_f64 *sc, PlanView *v) {
+  if (!plan || plan_view(plan, v) != WT_OK || (sc && (!(sc->dt > 0) || !(sc->h > 0)))) {
+    set_error("%s: invalid argument", what);
+    return WT_EINVAL;
+  }
+  if (v->f64.R == 0) {
+    set_error("%s: the plan does not run blocked in double precision", what);
+    return WT_EUNSUPPORTED;
+  }
+  return WT_OK;
+}
+
+extern "C" int wt_workspace_bytes_rec_f64(const void *plan, int32_t with_grad, int64_t *saved,
+                                          int64_t *temp) {
+  PlanView v;
+  if (!saved || !temp) {
+    set_error("wt_workspace_bytes_rec_f64: invalid argument");
+    return WT_EINVAL;
+  }
+  const int rc = check64("wt_workspace_bytes_rec_f64", plan, nullptr, &v);
+  if (rc) return rc;
+  const Blk64 w = blk64(v);
+  *saved = with_grad ? w.saved() * 8 : 0;
+  *temp = (with_grad ? std::max(w.fwd_temp(), w.adj_temp()) : w.fwd_temp()) * 8;
+  return WT_OK;
+}
+
+extern "C" int wt_loop_fwd_rec_f64(void *plan, const wt_scalars_f64 *sc, const double *b,
+                                   const double *c, const double *x, double *y, double *fields,
+                                   int32_t field_stride, int32_t with_grad, void *saved,
+                                   void *temp, void *stream) {
+  PlanView v;
+  if (!sc || !b || !c || !x || !temp || (with_grad && !saved)) {
+    set_error("wt_loop_fwd_rec_f64: invalid argument");
+    return WT_EINVAL;
+  }
+  const int rc = check64("wt_loop_fwd_rec_f64", plan, sc, &v);
+  if (rc) return rc;
+  if (field_stride < 1 || (fields && v.T % field_stride != 0)) {
+    set_error("wt_loop_fwd_rec_f64: field_stride %d must divide T = %d", field_stride, v.T);
+    return WT_EINVAL;
+  }
+  hipStream_t s = (hipStream_t)stream;
+  const Blk64 w = blk64(v);
+  const TileView &t = v.f64;
+  F64Blk a = args64(v, *sc, t);
+  double *st = (double *)temp;
+  double *coef = with_grad ? (double *)saved : st + 4 * w.BF;
+  a.A = coef; a.Bm = coef + w.F; a.C2 = coef + 2 * w.F;
+  hipLaunchKernelGGL(k64_coef, dim3((unsigned)((w.F + 255) / 256)), dim3(256), 0, s, b, c, w.F,
+                     1.0 / sc->dt, 1.0 / (sc->dt * sc->dt), (v.nlf & 4) != 0, sc->c_min,
+                     sc->c_max, coef, coef + w.F, coef + 2 * w.F);
+  WT_HIP(hipGetLastError());
+  a.x = x; a.y = y; a.fields = fields; a.fstride = field_stride;
+  if (with_grad) {
+    a.yraw = coef + 3 * w.F;
+    a.rec = a.yraw + w.yraw;
+  }
+  const size_t shmem = cs64_shmem_bytes(t.R, t.RHmax, t.RWmax, t.tb);
+  int pp = 0;
+  for (int n = 0; n < v.T; n += t.tb, pp ^= 1) {
+    a.n0 = n;
+    a.nsteps = std::min(t.tb, v.T - n);
+    a.out1 = st + 2 * pp * w.BF;
+    a.out2 = a.out1 + w.BF;
+    hipError_t e = t.R == 4   ? launch64_fwd<4>(with_grad, sc->h == 1.0, a, t.nthreads, shmem, s)
+                   : t.R == 6 ? launch64_fwd<6>(with_grad, sc->h == 1.0, a, t.nthreads, shmem, s)
+                              : launch64_fwd<8>(with_grad, sc->h == 1.0, a, t.nthreads, shmem, s);
+    WT_HIP(e);
+    a.in1 = a.out1;
+    a.in2 = a.out2;
+  }
+  return WT_OK;
+}
+
+extern "C" int wt_loop_adj_rec_f64(void *plan, const wt_scalars_f64 *sc, const double *c,
+                                   const double *ybar, void *saved, void *temp, double *grad_c,
+                                   double *grad_x, void *stream) {
+  PlanView v;
+  if (!sc || !c || !saved || !temp) {
+    set_error("wt_loop_adj_rec_f64: invalid argument");
+    return WT_EINVAL;
+  }
+  const int rc = check64("wt_loop_adj_rec_f64", plan, sc, &v);
+  if (rc) return rc;
+  hipStream_t s = (hipStream_t)stream;
+  const Blk64 w = blk64(v);
+  const TileView &t = v.f64_a;
+  F64Blk a = args64(v, *sc, t);
+  double *coef = (double *)saved, *st = (double *)temp;
+  a.A = coef; a.Bm = coef + w.F; a.C2 = coef + 2 * w.F;
+  a.yraw = coef + 3 * w.F;
+  a.rec = a.yraw + w.yraw;
+  a.ybar = ybar;
+  a.gacc = st + 4 * w.BF;
+  a.gsrc = st + 5 * w.BF;
+  a.first = 1;
+  const size_t shmem = cs64_shmem_bytes(t.R, t.RHmax, t.RWmax, t.tb);
+  int pp = 0;
+  for (int m = v.T; m > 0; m -= t.tb, pp ^= 1) {
+    a.m_hi = m;
+    a.nsteps = std::min(t.tb, m);
+    a.out1 = st + 2 * pp * w.BF;
+    a.out2 = a.out1 + w.BF;
+    WT_HIP(t.R == 4 ? launch64_adj<4>(a, t.nthreads, shmem, s)
+                    : launch64_adj<5>(a, t.nthreads, shmem, s));
+    a.in1 = a.out1;
+    a.in2 = a.out2;
+    a.first = 0;
+  }
+  if (grad_c) {
+    hipLaunchKernelGGL(k64_finalize_gc, dim3((unsigned)((w.F + 255) / 256)), dim3(256), 0, s,
+                       a.gacc, v.B, w.F, c, coef, (v.nlf & 4) != 0, sc->c_min, sc->c_max,
+                       grad_c);
+    WT_HIP(hipGetLastError());
+  }
+  if (grad_x)
+    WT_HIP(v.nslot > 0 ? launch_finalize_gx64(a.gsrc, v.B, v.T, v.nslot, v.mult, grad_x, s)
+                       : launch_fill64(grad_x, (int64_t)v.B * v.T, 0.0, s));
+  return WT_OK;
+}

@@ -186,6 +186,13 @@ struct NlAdjBufs {
   int64_t rec_slice;   // stride of one (sample, step) slice of the record
 };
 
+// One tiling of a plan on the device, with the block that runs it: `tb` steps
+// per launch, R rows per thread, `nthreads` threads (R = 0: none).
+struct TileView {
+  int ntiles = 0, RHmax = 0, RWmax = 0, tb = 0, R = 0, nthreads = 0;
+  const int32_t *tiles = nullptr;
+};
+
 // Read-only view of a plan's configuration and device tables, for code
 // outside the runtime (the double-precision loop).
 struct PlanView {
@@ -193,6 +200,7 @@ struct PlanView {
   int nlf;  // nonlinear flags as in FwdArgs (bit2 also for a clamp-only cell)
   int nspx, ntap, nslot;
   const int32_t *spx, *taps, *spmap, *mult;
+  TileView f64, f64_a;  // blocked double-precision forward and adjoint
 };
 int plan_view(const void *plan, PlanView *out);
 
@@ -245,6 +253,11 @@ __device__ __forceinline__ int xcd_remap(int bid, int nb) {
 namespace wt {
 void set_error(const char *fmt, ...);
 int hip_fail(hipError_t e, const char *what);
+
+// implemented in wt_f64.hip
+hipError_t launch_fill64(double *p, int64_t n, double v, hipStream_t s);
+hipError_t launch_finalize_gx64(const double *gsrc, int B, int T, int nslot, const int32_t *mult,
+                                double *gx, hipStream_t s);
 
 // Largest dynamic LDS a workgroup may request on the current device (cached
 // per device id below 64).

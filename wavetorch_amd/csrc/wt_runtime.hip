@@ -93,6 +93,8 @@ int cs_threads(int R, int RH, int RW);
 hipError_t launch_fwd_cs(int nt, int R, bool unit_h, int nl, bool rec, const FwdArgs &a,
                          int RHmax, int RWmax, hipStream_t s);
 hipError_t launch_adj_cs(int nt, int R, const AdjArgs &a, int RHmax, int RWmax, hipStream_t s);
+size_t cs64_shmem_bytes(int R, int RH, int RW, int tb);
+bool cs64_variant_exists(int R, bool fwd);
 bool cs_nl_variant_exists(int nt, int r);
 size_t cs_nl_shmem_bytes(int R, int RH, int RW);
 hipError_t launch_adj_cs_nl(int nt, int R, bool gb, const AdjArgs &a, const NlCarry &cy,
@@ -174,6 +176,10 @@ struct Plan {
   int32_t *d_tiles_a = nullptr;
   int ntiles_a = 1, RHmax_a = 0, RWmax_a = 0, tb_a = 1, nt_a = 0, cpt_a = 0;
   bool tiled = false;
+  // blocked double-precision loop of the linear cell (R = 0: per-step kernels)
+  TileView t64, t64_a;
+  std::vector<int32_t> h_t64, h_t64_a;
+  int32_t *d_t64 = nullptr, *d_t64_a = nullptr;
   // batched instances: one c (hence C2) per sample instead of one per plan
   bool c2ps = false;
   // step slots of the saved record (0 = B * K; batched instances in one
@@ -197,6 +203,8 @@ static void free_plan(Plan *p) {
   if (p->d_mult) (void)hipFree(p->d_mult);
   if (p->d_tiles) (void)hipFree(p->d_tiles);
   if (p->d_tiles_a) (void)hipFree(p->d_tiles_a);
+  if (p->d_t64) (void)hipFree(p->d_t64);
+  if (p->d_t64_a) (void)hipFree(p->d_t64_a);
   delete p;
 }
 
@@ -292,15 +300,28 @@ static bool tiles_ok(const Plan &p, int nt, int cpt) {
 // Column-segment family: block of cs_threads() threads, R rows per thread;
 // per thread at most 2 special rows (adjoint) and source multiplicity <= 2.
 // `fwd`: forward tiles (their LDS allocation holds the padded layout).
+static bool tables_ok_cs(const Plan &p, int R, int nthr);
 static bool tiles_ok_cs(const Plan &p, int nt, int R, bool fwd = true) {
   if (!cs_variant_exists(nt, R)) return false;
+  if (cs_shmem_bytes(R, p.RHmax, p.RWmax, fwd) + 1024 > LDS_LIMIT) return false;
+  int nthr = cs_threads(R, p.RHmax, p.RWmax);
+  return nthr <= nt && tables_ok_cs(p, R, nthr);
+}
+
+// The same for the double-precision block of R rows and tb steps, whose
+// static LDS (tables) is 7.2 KB.
+static bool tiles_ok_64(const Plan &p, int R, int tb, bool fwd) {
+  if (!cs64_variant_exists(R, fwd)) return false;
+  if (cs64_shmem_bytes(R, p.RHmax, p.RWmax, tb) + 8 * 1024 > LDS_LIMIT) return false;
+  const int nthr = cs_threads(R, p.RHmax, p.RWmax);
+  return nthr <= 1024 && tables_ok_cs(p, R, nthr);
+}
+
+static bool tables_ok_cs(const Plan &p, int R, int nthr) {
   for (int ti = 0; ti < p.ntiles; ++ti) {  // tables staged in LDS per tile
     const int32_t *t = &p.h_tiles[ti * TILE_W];
     if (t[9] - t[8] > 256 || t[11] - t[10] > 256) return false;
   }
-  if (cs_shmem_bytes(R, p.RHmax, p.RWmax, fwd) + 1024 > LDS_LIMIT) return false;
-  int nthr = cs_threads(R, p.RHmax, p.RWmax);
-  if (nthr > nt) return false;
   for (int ti = 0; ti < p.ntiles; ++ti) {
     const int32_t *t = &p.h_tiles[ti * TILE_W];
     int RH = t[1], RW = t[3];
@@ -559,6 +580,50 @@ int wt_step_bwd(const float *b, const float *c, int32_t bc_per_sample, const flo
 }  // extern "C"
 
 static int plan_upload(Plan *p);
+
+// Tilings of the blocked double-precision loop.  A tiling given by the caller
+// is used when a block holds it; otherwise the cheapest by block_cost.
+static void plan_f64(Plan &p, const wt_tuning *tuning) {
+  const std::vector<int32_t> ft = p.h_tiles;
+  const int fnt = p.ntiles, fRH = p.RHmax, fRW = p.RWmax, fLW = p.LWmax;
+  auto take = [&](int s, int c, int tb, int R, bool fwd) {
+    build_tiles(p, s, c, tb);
+    if (!tiles_ok_64(p, R, tb, fwd)) return false;
+    TileView &t = fwd ? p.t64 : p.t64_a;
+    t.ntiles = p.ntiles; t.RHmax = p.RHmax; t.RWmax = p.RWmax;
+    t.tb = tb; t.R = R;
+    t.nthreads = cs_threads(R, p.RHmax, p.RWmax);
+    (fwd ? p.h_t64 : p.h_t64_a) = p.h_tiles;
+    return true;
+  };
+  for (int fwd = 1; fwd >= 0; --fwd) {
+    bool ok = false;
+    if (tuning && tuning->strips > 0) {
+      const int s = fwd || tuning->a_strips <= 0 ? tuning->strips : tuning->a_strips;
+      const int c = fwd || tuning->a_tcols <= 0 ? tuning->tcols : tuning->a_tcols;
+      const int tb = fwd || tuning->a_tblock <= 0 ? tuning->tblock : tuning->a_tblock;
+      const int R = fwd || tuning->a_cpt <= 0 ? tuning->cpt : tuning->a_cpt;
+      ok = tb > 0 && tb <= 256 && take(s, std::max(c, 1), std::min(tb, p.T), R, fwd);
+    }
+    if (!ok) {
+      for (const auto &t : tile_order(p.Nx, p.Ny)) {
+        if ((int64_t)p.B * t.first * t.second < 256 &&
+            std::min(p.Nx / t.first, p.Ny / t.second) > 24)
+          continue;
+        for (int tb : {12, 8, 4})
+          for (int R : {4, 5, 6, 8})
+            if (!ok) ok = take(t.first, t.second, std::min(tb, p.T), R, fwd);
+        if (ok) break;
+      }
+    }
+    if (!ok) {
+      p.t64.R = p.t64_a.R = 0;
+      break;
+    }
+  }
+  p.h_tiles = ft;
+  p.ntiles = fnt; p.RHmax = fRH; p.RWmax = fRW; p.LWmax = fLW;
+}
 
 // Host half of plan creation: validation, special-pixel tables, tiling and
 // variant choice, workspace layout.  No device call except hipGetDevice.
@@ -889,6 +954,7 @@ static int plan_build(const wt_config *cfg, int32_t B, int32_t T, float cmax_geo
   }
   p->tun = tun;
   p->tiled = tiled;
+  if (p->nl == 0 && !(tuning && tuning->plain) && tun.kind == 0) plan_f64(*p, tuning);
   plan_layout(*p);
   *plan_out = p;
   return WT_OK;
@@ -972,8 +1038,11 @@ static int plan_upload(Plan *p) {
   int rc;
   if ((rc = up(&p->d_spx, p->h_spx)) || (rc = up(&p->d_taps, p->h_taps)) ||
       (rc = up(&p->d_spmap, spmap)) || (rc = up(&p->d_mult, p->h_mult)) ||
-      (rc = up(&p->d_tiles, p->h_tiles)) || (rc = up(&p->d_tiles_a, p->h_tiles_a)))
+      (rc = up(&p->d_tiles, p->h_tiles)) || (rc = up(&p->d_tiles_a, p->h_tiles_a)) ||
+      (rc = up(&p->d_t64, p->h_t64)) || (rc = up(&p->d_t64_a, p->h_t64_a)))
     return rc;
+  p->t64.tiles = p->d_t64;
+  p->t64_a.tiles = p->d_t64_a;
   return WT_OK;
 }
 
@@ -985,6 +1054,7 @@ int plan_view(const void *plan, PlanView *out) {
   out->nlf = p->nl | (p->clamp_only ? 4 : 0);
   out->nspx = p->nspx; out->ntap = p->ntap; out->nslot = p->nslot;
   out->spx = p->d_spx; out->taps = p->d_taps; out->spmap = p->d_spmap; out->mult = p->d_mult;
+  out->f64 = p->t64; out->f64_a = p->t64_a;
   return WT_OK;
 }
 }  // namespace wt
