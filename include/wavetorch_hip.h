@@ -178,6 +178,24 @@ typedef struct wt_tuning {
 int wt_plan_create(const wt_config *cfg, int32_t B, int32_t T, float cmax,
                    const wt_tuning *tuning, void **plan_out);
 
+/* The tiling, depth and rows per thread, forward and adjoint, that the
+ * library's model of a launch's time finds fastest for this configuration,
+ * batch, length and checkpoint interval, as a tuning to pass to
+ * wt_plan_create (all fields but ck_every zero, the default plan, when no
+ * block holds it).  `group`: the steps that wt_plan_group will be given, or 0.
+ * At h = 1 the adjoint's depth is that of the default plan with a checkpoint
+ * interval of `group` (0: ck_every), so that gradients keep its rounding.
+ * Host only. */
+int wt_plan_suggest(const wt_config *cfg, int32_t B, int32_t T, float cmax_geom, int32_t ck_every,
+                    int32_t group, wt_tuning *out);
+
+/* Ends the adjoint launches of a plan at multiples of `steps` steps (0, the
+ * state after wt_plan_create: only at checkpoint segments), so that a
+ * gradient summed launch by launch rounds as with a checkpoint interval of
+ * `steps`.  Host only; not to be called while a loop of the plan is being
+ * launched. */
+int wt_plan_group(void *plan, int32_t steps);
+
 /* Host-only half of wt_plan_create: the same validation (including the CFL
  * check of cell.py:66-73) and tiling/variant choice, with no device work.
  * Writes the resolved tuning to *out and the with-grad workspace sizes of
@@ -301,9 +319,10 @@ int wt_loop_adj_f64(void *plan, const wt_scalars_f64 *sc, const double *b, const
  * fields are not formed here (wt_loop_fwd_f64 / wt_loop_adj_f64 form them).
  * Outputs equal wt_loop_fwd_f64's bit for bit.  WT_EUNSUPPORTED for plans
  * that do not run it (the nonlinear cell, tuning.plain, pixels shared by
- * several sources): use the entry points above.  Replaces the same reference
- * code as those. */
-int wt_workspace_bytes_rec_f64(const void *plan, int32_t with_grad, int64_t *saved,
+ * several sources): use the entry points above.  The first of these calls on
+ * a plan builds and uploads the tilings (synchronously).  Replaces the same
+ * reference code as those. */
+int wt_workspace_bytes_rec_f64(void *plan, int32_t with_grad, int64_t *saved,
                                int64_t *temp);
 int wt_loop_fwd_rec_f64(void *plan, const wt_scalars_f64 *sc, const double *b, const double *c,
                         const double *x, double *y, double *fields, int32_t field_stride,

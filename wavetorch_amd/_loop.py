@@ -60,6 +60,17 @@ def scalars_f64(cfg: LoopConfig):
                              c_nl=cfg.c_nl, c_min=cmin, c_max=cmax)
 
 
+def suggest(cfg: LoopConfig, B: int, T: int, cmax: float, K: int, group: int = 0) -> dict:
+    """The tuning that the library's launch-time model finds fastest
+    (``wt_plan_suggest``), as the fields to pass to ``Plan``."""
+    c, keep = cfg.to_c()
+    out = _lib.WtTuning()
+    _lib.check(_lib.lib().wt_plan_suggest(ctypes.byref(c), B, T, float(cmax), int(K),
+                                          int(group), ctypes.byref(out)), "wt_plan_suggest")
+    del keep
+    return {k: v for k, v in out.as_dict().items() if v}
+
+
 def resolve(cfg: LoopConfig, B: int, T: int, cmax: float, tuning=None):
     """Host-only plan resolution (``wt_plan_resolve``): validates ``cfg``
     (ValueError on CFL or bad indices, as the reference's constructors raise)
@@ -98,7 +109,8 @@ def auto_interval(cfg: LoopConfig, B: int, T: int, budget: int, K0: int) -> int:
 class Plan:
     """Owner of a library plan (validated config + device tables + tiling)."""
 
-    def __init__(self, cfg: LoopConfig, B: int, T: int, cmax: float, device, tuning=None):
+    def __init__(self, cfg: LoopConfig, B: int, T: int, cmax: float, device, tuning=None,
+                 group: int = 0):
         self.cfg, self.B, self.T, self.device = cfg, B, T, device
         c, keep = cfg.to_c()
         tun = None
@@ -112,6 +124,8 @@ class Plan:
                                         ctypes.byref(handle)), "wt_plan_create")
         self.handle = handle
         del keep
+        if group:
+            _lib.check(L.wt_plan_group(handle, int(group)), "wt_plan_group")
         t = _lib.WtTuning()
         _lib.check(L.wt_plan_tuning(handle, ctypes.byref(t)), "wt_plan_tuning")
         self.tuning = t.as_dict()

@@ -486,7 +486,9 @@ using namespace wt;
 
 // Common argument checks: a plan whose linear cell runs blocked in double
 // precision.
-static int check64(const char *what, const void *plan, const wt_scalars_f64 *sc, PlanView *v) {
+static int check64(const char *what, void *plan, const wt_scalars_f64 *sc, PlanView *v) {
+  const int rc = plan ? plan_use_f64(plan) : WT_EINVAL;
+  if (plan && rc) return rc;
   if (!plan || plan_view(plan, v) != WT_OK || (sc && (!(sc->dt > 0) || !(sc->h > 0)))) {
     set_error("%s: invalid argument", what);
     return WT_EINVAL;
@@ -498,7 +500,7 @@ static int check64(const char *what, const void *plan, const wt_scalars_f64 *sc,
   return WT_OK;
 }
 
-extern "C" int wt_workspace_bytes_rec_f64(const void *plan, int32_t with_grad, int64_t *saved,
+extern "C" int wt_workspace_bytes_rec_f64(void *plan, int32_t with_grad, int64_t *saved,
                                           int64_t *temp) {
   PlanView v;
   if (!saved || !temp) {

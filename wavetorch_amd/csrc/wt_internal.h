@@ -203,6 +203,7 @@ struct PlanView {
   TileView f64, f64_a;  // blocked double-precision forward and adjoint
 };
 int plan_view(const void *plan, PlanView *out);
+int plan_use_f64(void *plan);  // builds f64 and f64_a on first use
 
 // Optional phase timestamps (diagnostic builds compiled with
 // -DWT_PHASE_TIMING): thread 0 of every workgroup records the 100 MHz wall
@@ -240,11 +241,13 @@ __device__ __forceinline__ float adj_div(float a, float b) {
 // XCD-aware work-item order.  Workgroups are dispatched round-robin over the
 // 8 XCDs of the chip (workgroup i runs on XCD i % 8); remap so that
 // consecutive work items (the strips of one sample, which exchange halos
-// through L2 between launches) land on the same XCD and share its L2.
+// through L2 between launches) land on the same XCD and share its L2.  XCD x
+// gets ceil or floor of nb/8 items: the first nb % 8 of them one more.
+// (1024x1024, one sample, 14x18 tiles, recording forward: 45 us per 18-step
+// launch in dispatch order, 30 us remapped.)
 __device__ __forceinline__ int xcd_remap(int bid, int nb) {
-  if ((nb & 7) != 0) return bid;
-  int per = nb >> 3;
-  return (bid & 7) * per + (bid >> 3);
+  const int x = bid & 7, per = nb >> 3, more = nb & 7;
+  return x * per + min(x, more) + (bid >> 3);
 }
 
 }  // namespace wt

@@ -166,6 +166,7 @@ struct Plan {
   float dtm1 = 0, dtm2 = 0, s2 = 0, t1 = 1, t4 = -4;
   wt_tuning tun{};
   int K = 64, nseg = 1;
+  int group = 0;  // adjoint launches end at multiples of this many steps (0: any)
   int nspx = 0, ntap = 0, nslot = 0;
   std::vector<int32_t> h_spx, h_taps, h_tiles, h_mult;
   int32_t *d_spx = nullptr, *d_taps = nullptr, *d_spmap = nullptr, *d_mult = nullptr;
@@ -177,6 +178,11 @@ struct Plan {
   int ntiles_a = 1, RHmax_a = 0, RWmax_a = 0, tb_a = 1, nt_a = 0, cpt_a = 0;
   bool tiled = false;
   // blocked double-precision loop of the linear cell (R = 0: per-step kernels)
+  // built by the first use (plan_use_f64); `given`: the tuning asked for
+  bool may64 = false;
+  std::once_flag once64;
+  int rc64 = WT_OK;
+  wt_tuning given{};
   TileView t64, t64_a;
   std::vector<int32_t> h_t64, h_t64_a;
   int32_t *d_t64 = nullptr, *d_t64_a = nullptr;
@@ -248,12 +254,13 @@ static void build_tiles(Plan &p, int strips, int cols, int halo) {
 // Heuristic tilings of an Nx x Ny grid (s strips x c columns of tiles per
 // sample): by tile count, then by how far the tiles are from square
 // (|log2 of (Nx/s)/(Ny/c)|), then more strips first.  Tilings whose tiles
-// are more than 2:1 are left out, except the single tile.
-static std::vector<std::pair<int, int>> tile_order(int Nx, int Ny) {
+// are more than 2:1 are left out, except the single tile; `most`: no more
+// tiles than that (the whole list takes a millisecond to sort).
+static std::vector<std::pair<int, int>> tile_order(int Nx, int Ny, int most) {
   struct Cand { int s, c; double bad; };
   std::vector<Cand> v;
   for (int s = 1; s <= std::min(Nx, 128); ++s)
-    for (int c = 1; c <= std::min(Ny, 128); ++c) {
+    for (int c = 1; c <= std::min(Ny, 128) && s * c <= most; ++c) {
       const double bad = std::fabs(std::log2(((double)Nx / s) / ((double)Ny / c)));
       if (s * c == 1 || bad <= 1.0 + 1e-9) v.push_back({s, c, bad});
     }
@@ -579,26 +586,134 @@ int wt_step_bwd(const float *b, const float *c, int32_t bc_per_sample, const flo
 
 }  // extern "C"
 
+// ---------------------------------------------------------------- plan model
+//
+// Time of one launch of a blocked kernel in us, fitted to launches measured on
+// MI355X: random tilings, grids, batches, depths and rows per thread (4000 of
+// the float linear kernels, 2500 each of the double-precision and the
+// nonlinear ones) and the cheapest tilings of 160 random problems.  A CU runs
+// `occ` workgroups at once (registers, LDS); n of them, of w waves each, take
+//   ts + tR R n ceil(w/4)                           set-up
+//   lat + cw (R + c0) (n ceil(w/4) + kb)            per step
+// (kb: a row's own latency, in waves per SIMD of issue), and the launch the
+// rounds its fullest CU needs, plus t0 and the traffic of the record and of
+// the state.  On the cheapest tilings the model is off by 5-6% rms (adjoint in
+// double precision 9%), and its choice is on average 2% (5%) slower than the
+// fastest of 14 candidates measured.
+struct BlockModel {
+  double t0, ts, tR, lat, cw, kb, c0, rec, state;
+  int rows[5], waves[5];  // rows per thread; waves per SIMD that its registers leave
+};
+// forward (the recording kernel, which also ranks the plain one), adjoint
+static const BlockModel kModelLin = {4.25, 1.42, 0.0164, 0.0, 0.00849, 3.66, 4.02, 0.21, 4.25e-6,
+                                     {4, 6, 8, 10, 12}, {8, 6, 5, 4, 4}};
+static const BlockModel kModelLinAdj = {5.68, 0.51, 0.0666, 0.0, 0.00754, 5.91, 2.59, 0.17,
+                                        4.54e-6, {4, 6, 8, 10, 0}, {7, 5, 4, 4, 0}};
+static const BlockModel kModelNl = {5.3, 0.0, 0.0, 0.0, 0.063, 1.65, 0.56, 0.66, 4.1e-6,
+                                    {4, 6, 8, 0, 0}, {7, 6, 5, 0, 0}};
+static const BlockModel kModelNlAdj = {7.27, 1.58, 0.0655, 0.07, 0.0485, 1.72, 4.89, 1.21, 8.94e-6,
+                                       {4, 0, 0, 0, 0}, {4, 0, 0, 0, 0}};
+static const BlockModel kModel64 = {4.49, 0.43, 0.037, 0.0, 0.0143, 3.66, 1.89, 0.16, 9.1e-6,
+                                    {4, 6, 8, 0, 0}, {6, 5, 4, 0, 0}};
+static const BlockModel kModel64Adj = {3.11, 2.35, 0.0442, 0.256, 0.00338, 1.19, 30.0, 0.57,
+                                       5.4e-6, {4, 5, 0, 0, 0}, {4, 4, 0, 0, 0}};
+
+struct BlockChoice {
+  double us;
+  int s, c, tb, R;
+};
+
+// The `top` cheapest (strips, columns, steps per launch, rows per thread) for
+// B samples of an Nx x Ny grid over `len` steps, cheapest first; `depth` > 0:
+// that many steps per launch.  shmem(R, RH, RW, tb): LDS of the block, static
+// part included.
+template <typename Shmem>
+static std::vector<BlockChoice> cheapest_blocks(const BlockModel &m, int Nx, int Ny, int B,
+                                                int len, int depth, int top, Shmem shmem) {
+  static const int depths[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 14, 16, 18, 20, 24, 28, 32, 40, 48};
+  std::vector<BlockChoice> best;
+  auto consider = [&](int s, int c, int tb) {
+    const int th = (Nx + s - 1) / s, tw = (Ny + c - 1) / c;
+    const int RH = std::min(Nx, th + (s > 2 ? 2 * tb : s == 2 ? tb : 0));
+    const int RW = std::min(Ny, tw + (c > 2 ? 2 * tb : c == 2 ? tb : 0));
+    const int percu = (int)(((int64_t)B * s * c + 255) / 256);
+    for (int v = 0; v < 5 && m.rows[v]; ++v) {
+      const int R = m.rows[v], waves = cs_threads(R, RH, RW) / 64;
+      if (waves > 16) continue;
+      const size_t lds = shmem(R, RH, RW, tb);
+      if (lds > LDS_LIMIT) continue;
+      const int occ = std::max(1, std::min((int)(LDS_LIMIT / lds), m.waves[v] * 4 / waves));
+      const double cells = (double)B * Nx * Ny;
+      auto launch = [&](int n) {
+        auto round = [&](int wg) {
+          const int k = wg * ((waves + 3) / 4);
+          return m.ts + m.tR * R * k + n * (m.lat + m.cw * (R + m.c0) * (k + m.kb));
+        };
+        return m.t0 + percu / occ * round(occ) + (percu % occ ? round(percu % occ) : 0.0) +
+               cells * (m.rec * n * 1e-6 + m.state);
+      };
+      // among tilings that the model's whole waves and rounds call equal, the
+      // one with the least area computed (halos clipped at the domain's edge;
+      // halo rows drop out of the cone step by step, halo columns stay)
+      const double area = (Nx + (s > 1 ? 1.0 * tb * (s - 1) : 0.0)) *
+                          (Ny + (c > 1 ? 2.0 * tb * (c - 1) : 0.0)) * B;
+      const double us = (len / tb * launch(tb) + (len % tb ? launch(len % tb) : 0.0)) *
+                        (1.0 + 0.06 * area / (256.0 * 1024.0 * R * percu));
+      if ((int)best.size() == top && us >= best.back().us) continue;
+      const BlockChoice ch{us, s, c, tb, R};
+      best.insert(std::upper_bound(best.begin(), best.end(), ch,
+                                   [](const BlockChoice &a, const BlockChoice &b) {
+                                     return a.us < b.us;
+                                   }),
+                  ch);
+      if ((int)best.size() > top) best.pop_back();
+    }
+  };
+  consider(1, 1, depth > 0 ? depth : std::min(len, 256));  // no halo: any depth
+  // near-square tilings (at most 2:1) of up to two workgroups per CU, or of
+  // four times the tiles that 64 x 64 cells each would make of a large batch
+  const int64_t most = std::max<int64_t>(512, (int64_t)B * Nx * Ny / 1024);
+  for (int s = 1; s <= std::min(Nx / 2, 96); ++s) {
+    if (s > 1 && (Nx + s - 1) / s == (Nx + s - 2) / (s - 1)) continue;  // no lower tiles
+    const int c0 = std::max(1, (int)((int64_t)s * Ny / (2 * (int64_t)Nx)));
+    const int c1 = std::min<int64_t>(std::min(Ny / 2, 96), 2 * (int64_t)s * Ny / Nx + 1);
+    for (int c = c0; c <= c1; ++c) {
+      if (s * c == 1 || (int64_t)B * s * c > most) continue;
+      if (c > 1 && (Ny + c - 1) / c == (Ny + c - 2) / (c - 1)) continue;
+      const int own = std::min(s > 1 ? Nx / s : Nx, c > 1 ? Ny / c : Ny);
+      if (depth > 0) {
+        consider(s, c, depth);
+      } else {
+        for (int tb : depths)
+          if (tb <= len && tb <= 2 * own) consider(s, c, tb);
+      }
+    }
+  }
+  return best;
+}
+
 static int plan_upload(Plan *p);
 
 // Tilings of the blocked double-precision loop.  A tiling given by the caller
-// is used when a block holds it; otherwise the cheapest by block_cost.
-static void plan_f64(Plan &p, const wt_tuning *tuning) {
-  const std::vector<int32_t> ft = p.h_tiles;
-  const int fnt = p.ntiles, fRH = p.RHmax, fRW = p.RWmax, fLW = p.LWmax;
+// is used when a block holds it; otherwise the cheapest by the model above.
+static void plan_f64(Plan &plan) {
+  const wt_tuning *tuning = &plan.given;
+  Plan p;  // scratch for build_tiles
+  p.B = plan.B; p.T = plan.T; p.Nx = plan.Nx; p.Ny = plan.Ny;
+  p.nspx = plan.nspx; p.ntap = plan.ntap; p.h_spx = plan.h_spx; p.h_taps = plan.h_taps;
   auto take = [&](int s, int c, int tb, int R, bool fwd) {
     build_tiles(p, s, c, tb);
     if (!tiles_ok_64(p, R, tb, fwd)) return false;
-    TileView &t = fwd ? p.t64 : p.t64_a;
+    TileView &t = fwd ? plan.t64 : plan.t64_a;
     t.ntiles = p.ntiles; t.RHmax = p.RHmax; t.RWmax = p.RWmax;
     t.tb = tb; t.R = R;
     t.nthreads = cs_threads(R, p.RHmax, p.RWmax);
-    (fwd ? p.h_t64 : p.h_t64_a) = p.h_tiles;
+    (fwd ? plan.h_t64 : plan.h_t64_a) = p.h_tiles;
     return true;
   };
   for (int fwd = 1; fwd >= 0; --fwd) {
     bool ok = false;
-    if (tuning && tuning->strips > 0) {
+    if (tuning->strips > 0) {
       const int s = fwd || tuning->a_strips <= 0 ? tuning->strips : tuning->a_strips;
       const int c = fwd || tuning->a_tcols <= 0 ? tuning->tcols : tuning->a_tcols;
       const int tb = fwd || tuning->a_tblock <= 0 ? tuning->tblock : tuning->a_tblock;
@@ -606,23 +721,20 @@ static void plan_f64(Plan &p, const wt_tuning *tuning) {
       ok = tb > 0 && tb <= 256 && take(s, std::max(c, 1), std::min(tb, p.T), R, fwd);
     }
     if (!ok) {
-      for (const auto &t : tile_order(p.Nx, p.Ny)) {
-        if ((int64_t)p.B * t.first * t.second < 256 &&
-            std::min(p.Nx / t.first, p.Ny / t.second) > 24)
-          continue;
-        for (int tb : {12, 8, 4})
-          for (int R : {4, 5, 6, 8})
-            if (!ok) ok = take(t.first, t.second, std::min(tb, p.T), R, fwd);
+      for (const BlockChoice &ch : cheapest_blocks(
+               fwd ? kModel64 : kModel64Adj, p.Nx, p.Ny, p.B, p.T, 0, 32,
+               [](int R, int RH, int RW, int tb) {
+                 return cs64_shmem_bytes(R, RH, RW, tb) + 8 * 1024;
+               })) {
+        ok = take(ch.s, ch.c, ch.tb, ch.R, fwd);
         if (ok) break;
       }
     }
     if (!ok) {
-      p.t64.R = p.t64_a.R = 0;
+      plan.t64.R = plan.t64_a.R = 0;
       break;
     }
   }
-  p.h_tiles = ft;
-  p.ntiles = fnt; p.RHmax = fRH; p.RWmax = fRW; p.LWmax = fLW;
 }
 
 // Host half of plan creation: validation, special-pixel tables, tiling and
@@ -772,7 +884,7 @@ static int plan_build(const wt_config *cfg, int32_t B, int32_t T, float cmax_geo
     std::vector<std::pair<int, int>> order;
     size_t oi = 0;
     if (square) {
-      order = tile_order(p->Nx, p->Ny);
+      order = tile_order(p->Nx, p->Ny, 1024);
       for (size_t i = 1; i < order.size(); ++i) {
         if ((int64_t)B * order[oi].first * order[oi].second >= 256) break;
         if (std::min(p->Nx / order[i].first, p->Ny / order[i].second) >= 2 * tb) oi = i;
@@ -786,6 +898,8 @@ static int plan_build(const wt_config *cfg, int32_t B, int32_t T, float cmax_geo
     int tcols = (tun.kind == 0 && tun.tcols > 0) ? tun.tcols : 1;
     bool ok = false;
     for (; square ? oi < order.size() : strips <= p->Nx; square ? (void)++oi : (void)++strips) {
+      if (square && oi + 1 == order.size() && order[oi].first * order[oi].second <= 1024)
+        order = tile_order(p->Nx, p->Ny, 128 * 128);  // nothing up to there holds: the rest
       if (square) {
         strips = order[oi].first;
         tcols = order[oi].second;
@@ -905,7 +1019,7 @@ static int plan_build(const wt_config *cfg, int32_t B, int32_t T, float cmax_geo
         if (!aok) atb = dmax;
       }
       if (!aok && !fixed) {
-        for (const auto &t : tile_order(p->Nx, p->Ny)) {
+        for (const auto &t : tile_order(p->Nx, p->Ny, 128 * 128)) {
           if (t.first * t.second <= as * ac) continue;
           if (fits(t.first, t.second, atb)) {
             as = t.first;
@@ -954,13 +1068,72 @@ static int plan_build(const wt_config *cfg, int32_t B, int32_t T, float cmax_geo
   }
   p->tun = tun;
   p->tiled = tiled;
-  if (p->nl == 0 && !(tuning && tuning->plain) && tun.kind == 0) plan_f64(*p, tuning);
+  p->may64 = p->nl == 0 && !(tuning && tuning->plain) && tun.kind == 0;
+  if (tuning) p->given = *tuning;
   plan_layout(*p);
   *plan_out = p;
   return WT_OK;
 }
 
 extern "C" {
+
+int wt_plan_suggest(const wt_config *cfg, int32_t B, int32_t T, float cmax_geom, int32_t ck_every,
+                    int32_t group, wt_tuning *out) {
+  if (!out) {
+    set_error("wt_plan_suggest: null argument");
+    return WT_EINVAL;
+  }
+  // the library's default plan: validates, builds the tables, and names the
+  // adjoint's depth
+  wt_tuning def{};
+  def.ck_every = group > 0 ? group : ck_every;
+  Plan *p = nullptr;
+  const int rc = plan_build(cfg, B, T, cmax_geom, &def, &p);
+  if (rc) return rc;
+  const int K = std::min(T, ck_every > 0 ? ck_every : 64);
+  // At h = 1 the adjoint keeps the default plan's depth, and wt_plan_group
+  // ends its launches at the default segments: the float32 gradient is summed
+  // launch by launch, so another grouping would change its rounding (by 1e-7
+  // of it on the training shapes, by 1e-4 where the terms cancel).
+  const int a_depth = p->tiled && p->unit_h ? p->tb_a : 0;
+  *out = wt_tuning{};
+  out->ck_every = K;
+  bool ok = false;
+  for (const BlockChoice &ch : cheapest_blocks(
+           p->nl ? kModelNl : kModelLin, p->Nx, p->Ny, B, K, 0, 32,
+           [](int R, int RH, int RW, int) { return cs_shmem_bytes(R, RH, RW, true) + 8192; })) {
+    build_tiles(*p, ch.s, ch.c, ch.tb);
+    if (!tiles_ok_cs(*p, 1024, ch.R)) continue;
+    out->strips = ch.s; out->tcols = ch.c; out->tblock = ch.tb;
+    out->nt = 1024; out->cpt = ch.R;
+    ok = true;
+    break;
+  }
+  bool aok = false;
+  if (ok) {
+    const bool nl = p->nl != 0;
+    for (const BlockChoice &ch : cheapest_blocks(
+             nl ? kModelNlAdj : kModelLinAdj, p->Nx, p->Ny, B, K, a_depth, 32,
+             [nl](int R, int RH, int RW, int) {
+               return (nl ? cs_nl_shmem_bytes(R, RH, RW) : cs_shmem_bytes(R, RH, RW, false)) +
+                      8192;
+             })) {
+      build_tiles(*p, ch.s, ch.c, ch.tb);
+      if (!tiles_ok_cs(*p, 1024, ch.R, false)) continue;
+      out->a_strips = ch.s; out->a_tcols = ch.c; out->a_tblock = ch.tb;
+      out->a_nt = 1024; out->a_cpt = ch.R;
+      aok = true;
+      break;
+    }
+  }
+  if (!aok) {  // no block holds this configuration: the library's default
+    const int k = out->ck_every;
+    *out = wt_tuning{};
+    out->ck_every = k;
+  }
+  free_plan(p);
+  return WT_OK;
+}
 
 int wt_plan_resolve(const wt_config *cfg, int32_t B, int32_t T, float cmax_geom,
                     const wt_tuning *tuning, wt_tuning *out, int64_t *saved, int64_t *temp) {
@@ -1016,33 +1189,55 @@ static void set_tile_layouts(std::vector<int32_t> &tiles, int R, int RHmax, int 
   }
 }
 
+static int upload_table(int32_t **dst, const std::vector<int32_t> &v) {
+  size_t n = std::max<size_t>(v.size(), 1) * sizeof(int32_t);
+  hipError_t e = hipMalloc((void **)dst, n);
+  if (e != hipSuccess) return hip_fail(e, "hipMalloc(plan table)");
+  if (!v.empty()) {
+    e = hipMemcpy(*dst, v.data(), v.size() * sizeof(int32_t), hipMemcpyHostToDevice);
+    if (e != hipSuccess) return hip_fail(e, "hipMemcpy(plan table)");
+  }
+  return WT_OK;
+}
+
+namespace wt {
+// The tilings of the blocked double-precision loop and their device copies,
+// once per plan and only for plans that run it.
+int plan_use_f64(void *plan) {
+  Plan *p = (Plan *)plan;
+  if (!p) return WT_EINVAL;
+  std::call_once(p->once64, [p] {
+    if (!p->may64) return;
+    plan_f64(*p);
+    if (p->t64.R == 0) return;
+    int cur = p->dev;
+    (void)hipGetDevice(&cur);
+    if (cur != p->dev) (void)hipSetDevice(p->dev);
+    p->rc64 = upload_table(&p->d_t64, p->h_t64);
+    if (!p->rc64) p->rc64 = upload_table(&p->d_t64_a, p->h_t64_a);
+    if (cur != p->dev) (void)hipSetDevice(cur);
+    p->t64.tiles = p->d_t64;
+    p->t64_a.tiles = p->d_t64_a;
+  });
+  return p->rc64;
+}
+}  // namespace wt
+
 // Device copies of a plan's tables (synchronous).
 static int plan_upload(Plan *p) {
   if (p->tiled && p->tun.kind == 0) {
     // forward tiles only: the adjoints wait little on LDS (measured: no gain)
     set_tile_layouts(p->h_tiles, p->tun.cpt, p->RHmax, p->RWmax);
   }
-  auto up = [&](int32_t **dst, const std::vector<int32_t> &v) -> int {
-    size_t n = std::max<size_t>(v.size(), 1) * sizeof(int32_t);
-    hipError_t e = hipMalloc((void **)dst, n);
-    if (e != hipSuccess) return hip_fail(e, "hipMalloc(plan table)");
-    if (!v.empty()) {
-      e = hipMemcpy(*dst, v.data(), v.size() * sizeof(int32_t), hipMemcpyHostToDevice);
-      if (e != hipSuccess) return hip_fail(e, "hipMemcpy(plan table)");
-    }
-    return WT_OK;
-  };
+  auto up = upload_table;
   std::vector<int32_t> spmap((size_t)p->Nx * p->Ny, -1);
   for (int k = 0; k < p->nspx; ++k)
     spmap[(size_t)p->h_spx[k * SPX_W] * p->Ny + p->h_spx[k * SPX_W + 1]] = k;
   int rc;
   if ((rc = up(&p->d_spx, p->h_spx)) || (rc = up(&p->d_taps, p->h_taps)) ||
       (rc = up(&p->d_spmap, spmap)) || (rc = up(&p->d_mult, p->h_mult)) ||
-      (rc = up(&p->d_tiles, p->h_tiles)) || (rc = up(&p->d_tiles_a, p->h_tiles_a)) ||
-      (rc = up(&p->d_t64, p->h_t64)) || (rc = up(&p->d_t64_a, p->h_t64_a)))
+      (rc = up(&p->d_tiles, p->h_tiles)) || (rc = up(&p->d_tiles_a, p->h_tiles_a)))
     return rc;
-  p->t64.tiles = p->d_t64;
-  p->t64_a.tiles = p->d_t64_a;
   return WT_OK;
 }
 
@@ -1060,6 +1255,15 @@ int plan_view(const void *plan, PlanView *out) {
 }  // namespace wt
 
 extern "C" {
+
+int wt_plan_group(void *plan, int32_t steps) {
+  if (!plan || steps < 0) {
+    set_error("wt_plan_group: invalid argument");
+    return WT_EINVAL;
+  }
+  ((Plan *)plan)->group = steps;
+  return WT_OK;
+}
 
 int wt_plan_destroy(void *plan) {
   free_plan((Plan *)plan);
@@ -1165,9 +1369,10 @@ FwdArgs base_fwd(const Plan &p, const Ws &w, const float *b, const float *c, con
 // when given.  Plain: one launch per step rotating through tmp[0..2]; the
 // final state is copied to (out1, out2) when given.
 int run_forward(const Plan &p, FwdArgs a, int n0, int n1, const float *in1, const float *in2,
-                float *out1, float *out2, float *tmp[4], bool rec, int prof_cls, hipStream_t s) {
+                float *out1, float *out2, float *tmp[4], bool rec, int prof_cls, hipStream_t s,
+                bool blocked = true) {
   const int64_t BF = (int64_t)p.B * p.F;
-  if (p.tiled) {
+  if (p.tiled && blocked) {
     const float *i1 = in1, *i2 = in2;
     int pp = 0;
     int n = n0;
@@ -1221,6 +1426,13 @@ int prepare_coef(const Plan &p, const Ws &w, const float *b, const float *c, con
     WT_HIP(launch_coef_linear(b, cc, F, p.dtm1, p.dtm2, w.A, w.Bm, w.C2, s));
   }
   return WT_OK;
+}
+
+// Steps of the adjoint launch that starts at reverse step m of the segment
+// from n0.
+int adj_steps(const Plan &p, int m, int n0) {
+  const int lo = p.group > 0 ? std::max(n0, (m - 1) / p.group * p.group) : n0;
+  return std::min(p.tb_a, m - lo);
 }
 
 // Reverse sweep of the nonlinear cell: per segment, recompute from the
@@ -1293,7 +1505,7 @@ int adj_nonlinear(const Plan &p, const float *b, const float *c, const float *rh
       aa.seg_u = from_fwd ? w.rec + segcells : fa.rec_u;
       aa.seg_n0 = n0;
       for (int m = n1; m > n0;) {
-        const int k = std::min(p.tb_a, m - n0);
+        const int k = adj_steps(p, m, n0);
         aa.in1 = l[0]; aa.in2 = l[1]; aa.out1 = l[2]; aa.out2 = l[3];
         aa.m_hi = m;
         aa.nsteps = k;
@@ -1457,9 +1669,7 @@ int wt_loop_adj(void *plan, const float *b, const float *c, const float *rho, co
       if (use_tiled) {
         rc = run_forward(*p, fa, n0, n1, ck, ck + BF, nullptr, nullptr, tmp, true, 1, s);
       } else {
-        Plan q = *p;
-        q.tiled = false;
-        rc = run_forward(q, fa, n0, n1, ck, ck + BF, nullptr, nullptr, tmp, true, 1, s);
+        rc = run_forward(*p, fa, n0, n1, ck, ck + BF, nullptr, nullptr, tmp, true, 1, s, false);
       }
       if (rc) return rc;
     }
@@ -1469,7 +1679,7 @@ int wt_loop_adj(void *plan, const float *b, const float *c, const float *rho, co
     int m = n1;
     if (use_tiled) {
       while (m > n0) {
-        int k = std::min(p->tb_a, m - n0);
+        int k = adj_steps(*p, m, n0);
         aa.in1 = l1; aa.in2 = l2; aa.out1 = l3; aa.out2 = l4;
         aa.m_hi = m; aa.nsteps = k;
         ProfScope ps(2, s, (int64_t)p->B * p->Nx * p->Ny * k);

@@ -12,7 +12,7 @@ from __future__ import annotations
 import numpy as np
 import torch
 
-from ._loop import LoopConfig, Plan, WaveLoop, auto_interval
+from ._loop import LoopConfig, Plan, WaveLoop, auto_interval, suggest
 from .probe import WaveProbe
 
 
@@ -130,16 +130,20 @@ class WaveRNN(torch.nn.Module):
         cfg = self.loop_config()
         tun = dict(self.tuning) if self.tuning else {}
         tun["ck_every"] = self.checkpoint_every
+        group = 0
         if not lean and self._checkpoint_every is None and not (self.tuning or {}).get("ck_every"):
+            group = tun["ck_every"]  # the gradient sums of the default interval
             total = torch.cuda.get_device_properties(device).total_memory
             tun["ck_every"] = auto_interval(cfg, B, T, total // 8, tun["ck_every"])
         tkey = tuple(sorted(tun.items()))
-        key = (cfg, B, T, str(device), tkey)
+        key = (cfg, B, T, str(device), tkey, group)
         p = self._plans.get(key)
         if p is None:
             if len(self._plans) > 8:
                 self._plans.clear()
-            p = Plan(cfg, B, T, self.cell.geom.cmax, device, tun)
+            if not self.tuning:  # no tiling asked for
+                tun = suggest(cfg, B, T, self.cell.geom.cmax, tun["ck_every"], group)
+            p = Plan(cfg, B, T, self.cell.geom.cmax, device, tun, group)
             self._plans[key] = p
         return p
 
