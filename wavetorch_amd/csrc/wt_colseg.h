@@ -13,6 +13,8 @@ namespace wt {
 constexpr int CS_MAX_TBLOCK = 256;
 // Largest number of special pixels / probe taps one tile may hold.
 constexpr int CS_MAX_TABLE = 256;
+// Static LDS of the float kernels next to the launch's dynamic LDS, at most.
+constexpr int CS_STATIC_LDS = 7424;
 // Probe-seed table: at most this many probe pixels per region.
 constexpr int CS_MAX_SEEDS = 16;
 
@@ -20,6 +22,7 @@ struct CsGeom {
   int R0, RH, C0, RW;     // region
   int or0, or1, oc0, oc1; // output rows / cols (domain)
   int k, c;               // segment, column of this thread
+  int RWm;                // thread-mapping width: t = k * RWm + c
   bool active;            // thread owns cells
   int CS;                 // LDS column stride (odd)
   int base;               // LDS index of this thread's first cell
@@ -44,10 +47,12 @@ __device__ __forceinline__ CsGeom cs_geom(const int32_t *td, int tid) {
       CS = (nseg * R + 2) | 1;
     }
     g.CS = CS;
+    g.RWm = RWm;
     g.k = tid / RWm;
     g.c = tid - g.k * RWm;
     g.active = g.k < nseg && g.c < g.RW;
   } else {
+    g.RWm = g.RW;
     g.k = tid / g.RW;
     g.c = tid - g.k * g.RW;
     g.active = g.k < nseg;
@@ -64,6 +69,130 @@ __device__ __forceinline__ void cone(const CsGeom &g, int s, int n, int &lo, int
   const int olo = g.or0 - g.R0, ohi = g.or1 - g.R0;
   lo = olo > 0 ? max(0, olo - rem) : 0;
   hi = ohi < g.RH ? min(g.RH, ohi + rem) : g.RH;
+}
+
+// Owner of the region cell (x, y): thread k * RWm + c, its row r in [0, R);
+// -1 outside the region.
+template <int R>
+__device__ __forceinline__ int cs_owner(const CsGeom &g, int x, int y, int &r) {
+  const int rr = x - g.R0, cc = y - g.C0;
+  if (rr < 0 || rr >= g.RH || cc < 0 || cc >= g.RW) return -1;
+  const int k = rr / R;
+  r = rr - k * R;
+  return k * g.RWm + cc;
+}
+
+// Special pixels of a region for the adjoints.  The table's entries find
+// their owners (a scan of the whole table in every thread, and in one thread
+// for the probe pixels, took about half of a launch with a line source of 100
+// pixels): entry kk lowers own[owner] and raises own[n + owner] (n =
+// blockDim.x; at most two entries per thread, so the two extremes are both of
+// them), and its probe-seed slot is its rank among the probe pixels, which
+// the host stored as a prefix count (word 6).  Phases, a barrier between each:
+// cs_special_load, then cs_special_stage, cs_special_scatter, cs_special_read.
+constexpr int CS_SP_W = 7;
+struct CsSpecials {
+  int sr0 = -1, sr1 = -1, sd0 = -1, sd1 = -1, sl0 = -1, sl1 = -1;  // row, seed slot, source slot
+};
+// This thread's entry of the table (loads only: they travel with the set-up's
+// other loads), then table and owners' extremes in LDS.
+__device__ __forceinline__ void cs_special_load(const int32_t *spx, int lo, int nsp,
+                                                int (&e)[CS_SP_W]) {
+#pragma unroll
+  for (int j = 0; j < CS_SP_W; ++j) e[j] = 0;
+  if ((int)threadIdx.x < nsp) {
+    const int32_t *p = spx + (lo + threadIdx.x) * SPX_W;
+#pragma unroll
+    for (int j = 0; j < CS_SP_W; ++j) e[j] = p[j];
+  }
+}
+__device__ __forceinline__ void cs_special_stage(const int32_t *spx, int lo, int nsp,
+                                                 const int (&e)[CS_SP_W], int *tb_sp, int *own) {
+  own[threadIdx.x] = 0x7fffffff;
+  own[blockDim.x + threadIdx.x] = -1;
+  if ((int)threadIdx.x < nsp) {
+#pragma unroll
+    for (int j = 0; j < CS_SP_W; ++j) tb_sp[CS_SP_W * threadIdx.x + j] = e[j];
+  }
+  for (int i = threadIdx.x + blockDim.x; i < nsp; i += blockDim.x)  // more entries than threads
+    for (int j = 0; j < CS_SP_W; ++j) tb_sp[CS_SP_W * i + j] = spx[(lo + i) * SPX_W + j];
+}
+template <int R>
+__device__ __forceinline__ void cs_special_scatter(const CsGeom &g, int nsp, const int *tb_sp,
+                                                   int *own, int *seed_px, int *nseeds) {
+  for (int kk = threadIdx.x; kk < nsp; kk += blockDim.x) {
+    const int *e = tb_sp + CS_SP_W * kk;
+    int r;
+    const int t = cs_owner<R>(g, e[0], e[1], r);
+    if (t >= 0) {
+      atomicMin(&own[t], kk);
+      atomicMax(&own[blockDim.x + t], kk);
+    }
+    const int slot = e[6] - tb_sp[6];
+    const bool has_tap = e[5] > e[4];
+    if (has_tap && slot < CS_MAX_SEEDS) seed_px[slot] = kk;
+    if (kk == nsp - 1) *nseeds = min(slot + (has_tap ? 1 : 0), CS_MAX_SEEDS);
+  }
+  if (nsp == 0 && threadIdx.x == 0) *nseeds = 0;
+}
+__device__ __forceinline__ CsSpecials cs_special_read(const CsGeom &g, int row0, const int *tb_sp,
+                                                      const int *own) {
+  CsSpecials sp;
+  const int k0 = own[threadIdx.x], k1 = own[blockDim.x + threadIdx.x];
+  if (k1 >= 0) {
+    const int *e = tb_sp + CS_SP_W * k0;
+    sp.sr0 = e[0] - g.R0 - row0;
+    sp.sd0 = e[5] > e[4] ? e[6] - tb_sp[6] : -1;
+    sp.sl0 = e[2] > 0 ? e[3] : -1;
+    if (k1 > k0) {
+      e = tb_sp + CS_SP_W * k1;
+      sp.sr1 = e[0] - g.R0 - row0;
+      sp.sd1 = e[5] > e[4] ? e[6] - tb_sp[6] : -1;
+      sp.sl1 = e[2] > 0 ? e[3] : -1;
+    }
+  }
+  return sp;
+}
+
+// Probe tap handled by this thread (taps in the output region): LDS index of
+// its cell, kind and output column, or pidx = -1.  Thread t takes tap t;
+// blocks of fewer threads than the tile's row range has taps count the ones
+// in its columns.  `e`: this thread's row of the table, loaded with the
+// set-up's other loads (cs_tap_load).
+struct CsTap {
+  int pidx = -1, pkind = 0, pcol = 0;
+};
+__device__ __forceinline__ void cs_tap_load(const int32_t *taps, int lo, int ntp,
+                                            int (&e)[TAP_W]) {
+#pragma unroll
+  for (int j = 0; j < TAP_W; ++j) e[j] = 0;
+  if ((int)threadIdx.x < ntp) {
+    const int32_t *p = taps + (lo + threadIdx.x) * TAP_W;
+#pragma unroll
+    for (int j = 0; j < TAP_W; ++j) e[j] = p[j];
+  }
+}
+__device__ __forceinline__ CsTap cs_tap(const CsGeom &g, const int32_t *taps, int lo, int ntp,
+                                        int (&e)[TAP_W]) {
+  CsTap p;
+  bool mine = (int)threadIdx.x < ntp && e[1] >= g.oc0 && e[1] < g.oc1;
+  if (ntp > (int)blockDim.x) {
+    mine = false;
+    for (int t = 0, kk = 0; t < ntp; ++t) {
+      const int32_t *q = taps + (lo + t) * TAP_W;
+      if (q[1] < g.oc0 || q[1] >= g.oc1) continue;
+      if (kk++ == (int)threadIdx.x) {
+        mine = true;
+        for (int j = 0; j < TAP_W; ++j) e[j] = q[j];
+      }
+    }
+  }
+  if (mine) {
+    p.pidx = (e[1] - g.C0 + 1) * g.CS + (e[0] - g.R0) + 1;
+    p.pkind = e[2];
+    p.pcol = e[3];
+  }
+  return p;
 }
 
 // Raw buffer access with hardware range checking (gfx9 descriptor word 3 =

@@ -171,10 +171,9 @@ __device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
   const int64_t F = (int64_t)a.Nx * Ny;
   const int64_t boff = (int64_t)b * F;
 
-  // tables of this tile staged in LDS (one parallel load, then scans hit
-  // LDS): special pixels (x, y, multiplicity) and probe taps (x, y, kind, col)
-  __shared__ int tb_sp[CS_MAX_TABLE * 3];
-  __shared__ int tb_tp[CS_MAX_TABLE * 4];
+  // source rows of each thread as a bit mask, filled by the table's entries
+  // (behind the input samples, in the space sized for the adjoint's seeds)
+  int *own = (int *)(xs + CS_MAX_TBLOCK);
   const int nsp = min(td[9] - td[8], CS_MAX_TABLE), ntp = min(td[11] - td[10], CS_MAX_TABLE);
 
   float U0[R], U1[R], KA[R], KB[R], KC[R], KD[R], KS[R];
@@ -196,70 +195,49 @@ __device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
       u2 = a.in2[boff + q];
     }
     U0[r] = u1; U1[r] = u2;
-    KA[r] = v0; KB[r] = v1; KC[r] = v2; KD[r] = v3; KS[r] = 0.0f;
+    KA[r] = v0; KB[r] = v1; KC[r] = v2; KD[r] = v3;
   }
   float xsv = 0.0f;
   if (tid < a.nsteps) xsv = a.x[(int64_t)b * a.T + a.n0 + tid];
-  int spv0 = 0, spv1 = 0, spv2 = 0, tpv0 = 0, tpv1 = 0, tpv2 = 0, tpv3 = 0;
+  int spv0 = 0, spv1 = 0, spv2 = 0;
   if (tid < nsp) {
     const int32_t *e = a.spx + (td[8] + tid) * SPX_W;
     spv0 = e[0]; spv1 = e[1]; spv2 = e[2];
   }
-  if (tid < ntp) {
-    const int32_t *t = a.taps + (td[10] + tid) * TAP_W;
-    tpv0 = t[0]; tpv1 = t[1]; tpv2 = t[2]; tpv3 = t[3];
-  }
+  int te[TAP_W];
+  cs_tap_load(a.taps, td[10], ntp, te);
   // 2) LDS (buf0's region cells are filled from U0 below)
   cs_zero_lds<float>(buf0, buf1, g, ((g.RH + R - 1) / R) * R, NBUF);
+  own[tid] = 0;
   WT_TS(4);
   if (tid < a.nsteps) xs[tid] = xsv;
-  if (tid < nsp) { tb_sp[3 * tid] = spv0; tb_sp[3 * tid + 1] = spv1; tb_sp[3 * tid + 2] = spv2; }
-  if (tid < ntp) {
-    tb_tp[4 * tid] = tpv0; tb_tp[4 * tid + 1] = tpv1;
-    tb_tp[4 * tid + 2] = tpv2; tb_tp[4 * tid + 3] = tpv3;
-  }
-  // blocks of fewer threads than steps or table entries (small grids)
+  // blocks of fewer threads than steps (small grids)
   for (int i = tid + blockDim.x; i < a.nsteps; i += blockDim.x)
     xs[i] = a.x[(int64_t)b * a.T + a.n0 + i];
-  for (int i = tid + blockDim.x; i < nsp; i += blockDim.x) {
-    const int32_t *e = a.spx + (td[8] + i) * SPX_W;
-    for (int j = 0; j < 3; ++j) tb_sp[3 * i + j] = e[j];
-  }
   __syncthreads();
   WT_TS(5);
   if (g.active) {
 #pragma unroll
     for (int r = 0; r < R; ++r) buf0[g.base + r] = U0[r];
   }
-  // source pixels of this thread (multiplicity 1; the host routes pixels
-  // shared by several sources to the other kernels)
-  bool any_src = false;
-  for (int kk = 0; kk < nsp; ++kk) {
-    if (tb_sp[3 * kk + 2] <= 0) continue;
-    const int rr = tb_sp[3 * kk] - g.R0 - row0, cc = tb_sp[3 * kk + 1] - g.C0;
-    if (!g.active || cc != g.c || rr < 0 || rr >= R || row0 + rr >= g.RH) continue;
-    any_src = true;
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-      if (r == rr) KS[r] = 1.0f;
-  }
-  const bool blk_src = __syncthreads_or(any_src);
-  WT_TS(6);
-  // probe tap handled by this thread (taps in the output region)
-  int pidx = -1, pkind = 0, pcol = 0;
-  {
-    int kk = 0;
-    for (int t = 0; t < ntp; ++t) {
-      const int tx = tb_tp[4 * t], ty = tb_tp[4 * t + 1];
-      if (ty < g.oc0 || ty >= g.oc1) continue;
-      if (kk == tid) {
-        pidx = (ty - g.C0 + 1) * g.CS + (tx - g.R0) + 1;
-        pkind = tb_tp[4 * t + 2];
-        pcol = tb_tp[4 * t + 3];
-      }
-      ++kk;
+  // source pixels (multiplicity 1; the host routes pixels shared by several
+  // sources to the other kernels) mark the rows of their owners
+  for (int kk = tid; kk < nsp; kk += blockDim.x) {
+    if (kk != tid) {  // more entries than threads
+      const int32_t *e = a.spx + (td[8] + kk) * SPX_W;
+      spv0 = e[0]; spv1 = e[1]; spv2 = e[2];
     }
+    int rr;
+    const int t = spv2 > 0 ? cs_owner<R>(g, spv0, spv1, rr) : -1;
+    if (t >= 0) atomicOr(&own[t], 1 << rr);
   }
+  __syncthreads();
+  WT_TS(6);
+  const CsTap tap = cs_tap(g, a.taps, td[10], ntp, te);
+  const int srows = own[tid];
+#pragma unroll
+  for (int r = 0; r < R; ++r) KS[r] = (srows >> r) & 1 ? 1.0f : 0.0f;
+  const bool wave_src = __ballot(srows != 0) != 0;
   const uint32_t voff = cs_out_voff<float>(g, row0, Ny);
   const int64_t out_bytes = (int64_t)(g.or1 - g.or0) * Ny * 4;
   // record slots of this sample; steps at or past its length are not
@@ -267,7 +245,6 @@ __device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
   const int64_t rslot0 =
       (BATCH && a.rec_soff) ? (int64_t)a.rec_soff[b] : (int64_t)b * a.rec_K;
   const int Lb = (BATCH && a.Tlim) ? a.Tlim[b] : 0x7fffffff;
-  __syncthreads();
 
   auto step = [&](const float *P, float *Q, float(&Uc)[R], float(&Up)[R], int s) {
     const int n = a.n0 + s;
@@ -280,15 +257,15 @@ __device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
     const __amdgpu_buffer_rsrc_t rsl = cs_rsrc(REC ? a.rec_lap + ro : a.in1, REC ? rbytes : 0);
     const __amdgpu_buffer_rsrc_t rsu =
         cs_rsrc((REC && NL) ? a.rec_u + ro : a.in1, (REC && NL) ? rbytes : 0);
-    const float xv = blk_src ? xs[s] : 0.0f;
+    const float xv = wave_src ? xs[s] : 0.0f;
     if (need)
       cs_fwd_rows<R, NL, REC, UH>(a, P, Q, Uc, Up, KA, KB, KC, KD, KS, g.base, g.CS, vmask, xv, rsl,
                               rsu, voff, Ny);
     __syncthreads();
-    if (pidx >= 0) {
-      const float v = Q[pidx];
-      const int64_t o = ((int64_t)b * a.T + n) * a.ntap + pcol;
-      if (a.y) a.y[o] = pkind ? v * v : v;
+    if (tap.pidx >= 0) {
+      const float v = Q[tap.pidx];
+      const int64_t o = ((int64_t)b * a.T + n) * a.ntap + tap.pcol;
+      if (a.y) a.y[o] = tap.pkind ? v * v : v;
       if (a.yraw) a.yraw[o] = v;
     }
     if (a.fields && ((n + 1) % a.fstride) == 0) {
@@ -415,7 +392,7 @@ __device__ __forceinline__ void adj_cs_body(const AdjArgs &a, const int w) {
   const int64_t boff = (int64_t)b * F;
   const float s2 = a.s2;
 
-  __shared__ int tb_sp[CS_MAX_TABLE * 6];  // x, y, mult, slot, tap_lo, tap_hi
+  __shared__ int tb_sp[CS_MAX_TABLE * CS_SP_W];
   const int nsp = min(td[9] - td[8], CS_MAX_TABLE);
 
   float L1[R], L2[R], KA1[R], KW[R], G[R], SG0[R], SG1[R];
@@ -434,21 +411,14 @@ __device__ __forceinline__ void adj_cs_body(const AdjArgs &a, const int w) {
     KA1[r] = A; KC2[r] = C2;
     L1[r] = u1; L2[r] = u2;
   }
-  int e0 = 0, e1 = 0, e2 = 0, e3 = 0, e4 = 0, e5 = 0;
-  if (tid < nsp) {
-    const int32_t *e = a.spx + (td[8] + tid) * SPX_W;
-    e0 = e[0]; e1 = e[1]; e2 = e[2]; e3 = e[3]; e4 = e[4]; e5 = e[5];
-  }
+  // (the owners' table lies behind the seeds, or under them in launches of
+  // more than 128 steps, with a barrier more)
+  int *own = (int *)(seeds + (a.nsteps > 128 ? 0 : 128 * CS_MAX_SEEDS));
+  int spe[CS_SP_W];
+  cs_special_load(a.spx, td[8], nsp, spe);
   // 2) LDS (buf0's region cells are filled from the lambda pair below)
   cs_zero_lds<float>(buf0, buf1, g, ((g.RH + R - 1) / R) * R, NBUF);
-  if (tid < nsp) {
-    int *t = tb_sp + 6 * tid;
-    t[0] = e0; t[1] = e1; t[2] = e2; t[3] = e3; t[4] = e4; t[5] = e5;
-  }
-  for (int i = tid + blockDim.x; i < nsp; i += blockDim.x) {
-    const int32_t *e = a.spx + (td[8] + i) * SPX_W;
-    for (int j = 0; j < 6; ++j) tb_sp[6 * i + j] = e[j];
-  }
+  cs_special_stage(a.spx, td[8], nsp, spe, tb_sp, own);
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const float A = KA1[r];
@@ -457,23 +427,21 @@ __device__ __forceinline__ void adj_cs_body(const AdjArgs &a, const int w) {
     G[r] = 0.0f; SG1[r] = 0.0f;
   }
   __syncthreads();
-  if (tid == 0) {
-    // probe pixels of the region, in table order
-    int n = 0;
-    for (int kk = 0; kk < nsp && n < CS_MAX_SEEDS; ++kk)
-      if (tb_sp[6 * kk + 5] > tb_sp[6 * kk + 4]) seed_px[n++] = kk;
-    nseeds = n;
-  }
+  cs_special_scatter<R>(g, nsp, tb_sp, own, seed_px, &nseeds);
   if (g.active) {
 #pragma unroll
     for (int r = 0; r < R; ++r) buf0[g.base + r] = KW[r] * L1[r];
   }
   __syncthreads();
+  // special rows of this thread: probe taps (seed slot) / source pixels (slot)
+  const CsSpecials sp = cs_special_read(g, row0, tb_sp, own);
+  const int sr0 = sp.sr0, sr1 = sp.sr1, sd0 = sp.sd0, sd1 = sp.sd1, sl0 = sp.sl0, sl1 = sp.sl1;
+  if (a.nsteps > 128) __syncthreads();
   // seeds[k][s] = sum over taps of pixel k of dy/du * ybar at step m = m_hi - s
   for (int i = tid; i < nseeds * a.nsteps; i += blockDim.x) {
     const int k = i / a.nsteps, s = i - (i / a.nsteps) * a.nsteps;
     const int m = a.m_hi - s;
-    const int *e = tb_sp + 6 * seed_px[k];
+    const int *e = tb_sp + CS_SP_W * seed_px[k];
     float gs = 0.0f;
     if (a.ybar && (!a.Tlim || m - 1 < a.Tlim[b])) {
       for (int t = e[4]; t < e[5]; ++t) {
@@ -484,22 +452,6 @@ __device__ __forceinline__ void adj_cs_body(const AdjArgs &a, const int w) {
       }
     }
     seeds[i] = gs;
-  }
-  // special rows of this thread: probe taps (seed slot) / source pixels (slot)
-  int sr0 = -1, sr1 = -1, sd0 = -1, sd1 = -1, sl0 = -1, sl1 = -1;
-  {
-    int nseed = 0;
-    for (int kk = 0; kk < nsp; ++kk) {
-      const int *e = tb_sp + 6 * kk;
-      const bool has_tap = e[5] > e[4];
-      const int seed_slot = has_tap ? nseed : -1;
-      if (has_tap) ++nseed;
-      const int rr = e[0] - g.R0 - row0;
-      if (!g.active || e[1] - g.C0 != g.c || rr < 0 || rr >= R || row0 + rr >= g.RH) continue;
-      const int src_slot = e[2] > 0 ? e[3] : -1;
-      if (sr0 < 0) { sr0 = rr; sd0 = seed_slot; sl0 = src_slot; }
-      else { sr1 = rr; sd1 = seed_slot; sl1 = src_slot; }
-    }
   }
   // wave-uniform special-pixel path: none, one slot, two slots; source
   // gradient stores only in waves that hold a source pixel
@@ -667,7 +619,7 @@ __global__ __launch_bounds__(NT) void k_adj_cs_nl(AdjArgs a, NlCarry cy) {
   float4 *mat = (float4 *)(smem + ((2 * NBUF + CS_MAX_SEEDS * CS_MAX_TBLOCK + 3) & ~3));
   __shared__ int seed_px[CS_MAX_SEEDS];
   __shared__ int nseeds;
-  __shared__ int tb_sp[CS_MAX_TABLE * 6];
+  __shared__ int tb_sp[CS_MAX_TABLE * CS_SP_W];
   const int Ny = a.Ny;
   const int64_t F = (int64_t)a.Nx * Ny;
   const int64_t boff = (int64_t)b * F;
@@ -701,37 +653,29 @@ __global__ __launch_bounds__(NT) void k_adj_cs_nl(AdjArgs a, NlCarry cy) {
       if (g.active) mat[g.base + r] = mt;
     }
   }
-  int e0 = 0, e1 = 0, e2 = 0, e3 = 0, e4 = 0, e5 = 0;
-  if (tid < nsp) {
-    const int32_t *e = a.spx + (td[8] + tid) * SPX_W;
-    e0 = e[0]; e1 = e[1]; e2 = e[2]; e3 = e[3]; e4 = e[4]; e5 = e[5];
-  }
+  // (the owners' table lies behind the seeds, or under them in launches of
+  // more than 128 steps, with a barrier more)
+  int *own = (int *)(seeds + (a.nsteps > 128 ? 0 : 128 * CS_MAX_SEEDS));
+  int spe[CS_SP_W];
+  cs_special_load(a.spx, td[8], nsp, spe);
   // 2) LDS: w_m * lambda_{m+1} of the region, tables, probe seeds
   for (int i = tid; i < 2 * NBUF; i += blockDim.x) smem[i] = 0.0f;
-  if (tid < nsp) {
-    int *t = tb_sp + 6 * tid;
-    t[0] = e0; t[1] = e1; t[2] = e2; t[3] = e3; t[4] = e4; t[5] = e5;
-  }
-  for (int i = tid + blockDim.x; i < nsp; i += blockDim.x) {
-    const int32_t *e = a.spx + (td[8] + i) * SPX_W;
-    for (int j = 0; j < 6; ++j) tb_sp[6 * i + j] = e[j];
-  }
+  cs_special_stage(a.spx, td[8], nsp, spe, tb_sp, own);
   __syncthreads();
-  if (tid == 0) {
-    int n = 0;
-    for (int kk = 0; kk < nsp && n < CS_MAX_SEEDS; ++kk)
-      if (tb_sp[6 * kk + 5] > tb_sp[6 * kk + 4]) seed_px[n++] = kk;
-    nseeds = n;
-  }
+  cs_special_scatter<R>(g, nsp, tb_sp, own, seed_px, &nseeds);
   if (g.active) {
 #pragma unroll
     for (int r = 0; r < R; ++r) buf0[g.base + r] = Wm[r] * Lc[r];
   }
   __syncthreads();
+  // special rows of this thread: probe taps (seed slot) / source pixels (slot)
+  const CsSpecials sp = cs_special_read(g, row0, tb_sp, own);
+  const int sr0 = sp.sr0, sr1 = sp.sr1, sd0 = sp.sd0, sd1 = sp.sd1, sl0 = sp.sl0, sl1 = sp.sl1;
+  if (a.nsteps > 128) __syncthreads();
   for (int i = tid; i < nseeds * a.nsteps; i += blockDim.x) {
     const int k = i / a.nsteps, s = i - (i / a.nsteps) * a.nsteps;
     const int m = a.m_hi - s;
-    const int *e = tb_sp + 6 * seed_px[k];
+    const int *e = tb_sp + CS_SP_W * seed_px[k];
     float gs = 0.0f;
     if (a.ybar) {
       for (int t = e[4]; t < e[5]; ++t) {
@@ -742,21 +686,6 @@ __global__ __launch_bounds__(NT) void k_adj_cs_nl(AdjArgs a, NlCarry cy) {
       }
     }
     seeds[i] = gs;
-  }
-  int sr0 = -1, sr1 = -1, sd0 = -1, sd1 = -1, sl0 = -1, sl1 = -1;
-  {
-    int nseed = 0;
-    for (int kk = 0; kk < nsp; ++kk) {
-      const int *e = tb_sp + 6 * kk;
-      const bool has_tap = e[5] > e[4];
-      const int seed_slot = has_tap ? nseed : -1;
-      if (has_tap) ++nseed;
-      const int rr = e[0] - g.R0 - row0;
-      if (!g.active || e[1] - g.C0 != g.c || rr < 0 || rr >= R || row0 + rr >= g.RH) continue;
-      const int src_slot = e[2] > 0 ? e[3] : -1;
-      if (sr0 < 0) { sr0 = rr; sd0 = seed_slot; sl0 = src_slot; }
-      else { sr1 = rr; sd1 = seed_slot; sl1 = src_slot; }
-    }
   }
   uint32_t omask = 0;
   if (g.active && col >= g.oc0 && col < g.oc1) {
@@ -1004,7 +933,7 @@ hipError_t launch_fwd_cs(int nt, int R, bool unit_h, int nl, bool rec, const Fwd
   int nblocks = a.B * a.ntiles;
   size_t shmem = cs_shmem_bytes(R, RHmax, RWmax, true);
   int nthreads = cs_threads(R, RHmax, RWmax);
-  if (shmem + 1024 > (size_t)cs_max_dyn_lds() || nthreads > nt) return hipErrorInvalidConfiguration;
+  if (shmem + CS_STATIC_LDS > (size_t)cs_max_dyn_lds() || nthreads > nt) return hipErrorInvalidConfiguration;
 #define X(A, B) \
   if (nt == A && R == B)                                                                \
     return cs_fwd_dispatch<A, B>(unit_h, nl, rec, a, nblocks, nthreads, shmem, s);
@@ -1017,7 +946,7 @@ hipError_t launch_adj_cs(int nt, int R, const AdjArgs &a, int RHmax, int RWmax, 
   int nblocks = a.B * a.ntiles;
   size_t shmem = cs_shmem_bytes(R, RHmax, RWmax, false);
   int nthreads = cs_threads(R, RHmax, RWmax);
-  if (shmem + 1024 > (size_t)cs_max_dyn_lds() || nthreads > nt) return hipErrorInvalidConfiguration;
+  if (shmem + CS_STATIC_LDS > (size_t)cs_max_dyn_lds() || nthreads > nt) return hipErrorInvalidConfiguration;
 #define X(A, B) if (nt == A && R == B) return cs_adj_dispatch<A, B>(a, nblocks, nthreads, shmem, s);
   WT_CS_VARIANTS(X)
 #undef X
@@ -1038,7 +967,7 @@ hipError_t launch_adj_cs_nl(int nt, int R, bool gb, const AdjArgs &a, const NlCa
   int nblocks = a.B * a.ntiles;
   size_t shmem = cs_nl_shmem_bytes(R, RHmax, RWmax);
   int nthreads = cs_threads(R, RHmax, RWmax);
-  if (shmem + 1024 > (size_t)cs_max_dyn_lds() || nthreads > nt || !cs_nl_variant_exists(nt, R))
+  if (shmem + CS_STATIC_LDS > (size_t)cs_max_dyn_lds() || nthreads > nt || !cs_nl_variant_exists(nt, R))
     return hipErrorInvalidConfiguration;
 #define NLK(RR, G)                                                                     \
   do {                                                                                 \
@@ -1088,7 +1017,7 @@ hipError_t launch_fwd_cs_batch(int nt, int R, bool rec, const BatchFwd &bl, int 
   if (nblocks <= 0) return hipSuccess;
   size_t shmem = cs_shmem_bytes(R, RHmax, RWmax, true);
   int nthreads = cs_threads(R, RHmax, RWmax);
-  if (shmem + 1024 > (size_t)cs_max_dyn_lds() || nthreads > nt) return hipErrorInvalidConfiguration;
+  if (shmem + CS_STATIC_LDS > (size_t)cs_max_dyn_lds() || nthreads > nt) return hipErrorInvalidConfiguration;
 #define X(A, B) \
   if (nt == A && R == B) return cs_fwd_batch_dispatch<A, B>(rec, bl, nblocks, nthreads, shmem, s);
   WT_CS_VARIANTS(X)
@@ -1102,7 +1031,7 @@ hipError_t launch_adj_cs_batch(int nt, int R, const BatchAdj &bl, int RHmax, int
   if (nblocks <= 0) return hipSuccess;
   size_t shmem = cs_shmem_bytes(R, RHmax, RWmax, false);
   int nthreads = cs_threads(R, RHmax, RWmax);
-  if (shmem + 1024 > (size_t)cs_max_dyn_lds() || nthreads > nt) return hipErrorInvalidConfiguration;
+  if (shmem + CS_STATIC_LDS > (size_t)cs_max_dyn_lds() || nthreads > nt) return hipErrorInvalidConfiguration;
 #define X(A, B) \
   if (nt == A && R == B) return cs_adj_batch_dispatch<A, B>(bl, nblocks, nthreads, shmem, s);
   WT_CS_VARIANTS(X)

@@ -53,8 +53,7 @@ __device__ __forceinline__ void b64_store(__amdgpu_buffer_rsrc_t rs, uint32_t of
 template <int NT, int R, bool REC, bool UH>
 __global__ __launch_bounds__(NT) void k64_fwd_cs(F64Blk a) {
   extern __shared__ double smem64[];
-  __shared__ int tb_sp[CS_MAX_TABLE * 3];  // source pixels of the region: x, y, multiplicity
-  __shared__ int tb_tp[CS_MAX_TABLE * 4];
+  __shared__ int own[NT];  // source rows of each thread, a bit mask
   const int tid = threadIdx.x;
   const int w = xcd_remap(blockIdx.x, gridDim.x);
   const int b = w / a.ntiles, ti = w - (w / a.ntiles) * a.ntiles;
@@ -78,45 +77,35 @@ __global__ __launch_bounds__(NT) void k64_fwd_cs(F64Blk a) {
     U0[r] = u1; U1[r] = u2; KA[r] = v0; KB[r] = v1; KC[r] = v2;
   }
   for (int i = tid; i < a.nsteps; i += blockDim.x) xs[i] = a.x[(int64_t)b * a.T + a.n0 + i];
-  for (int i = tid; i < nsp; i += blockDim.x) {
-    const int32_t *e = a.spx + (td[8] + i) * SPX_W;
-    for (int j = 0; j < 3; ++j) tb_sp[3 * i + j] = e[j];
+  int spx0 = 0, spx1 = 0, spx2 = 0, te[TAP_W];
+  if (tid < nsp) {
+    const int32_t *e = a.spx + (td[8] + tid) * SPX_W;
+    spx0 = e[0]; spx1 = e[1]; spx2 = e[2];
   }
-  for (int i = tid; i < ntp; i += blockDim.x) {
-    const int32_t *e = a.taps + (td[10] + i) * TAP_W;
-    for (int j = 0; j < 4; ++j) tb_tp[4 * i + j] = e[j];
-  }
+  cs_tap_load(a.taps, td[10], ntp, te);
+  own[tid] = 0;
   cs_zero_lds<double>(buf0, buf1, g, ((g.RH + R - 1) / R) * R, NBUF);
   __syncthreads();
   if (g.active) {
 #pragma unroll
     for (int r = 0; r < R; ++r) buf0[g.base + r] = U0[r];
   }
-  // rows of this thread that hold a source pixel (at most two; the host sends
-  // other source sets to the per-step kernels)
-  int sr0 = -1, sr1 = -1;
-  for (int k = 0; k < nsp; ++k) {
-    const int rr = tb_sp[3 * k] - g.R0 - row0;
-    if (tb_sp[3 * k + 2] <= 0 || !g.active || tb_sp[3 * k + 1] - g.C0 != g.c || rr < 0 ||
-        rr >= R || row0 + rr >= g.RH)
-      continue;
-    if (sr0 < 0) sr0 = rr; else sr1 = rr;
-  }
-  const bool wave_src = __ballot(sr0 >= 0) != 0;
-  // probe tap of this thread (taps in the output region)
-  int pidx = -1, pkind = 0, pcol = 0;
-  for (int t = 0, kk = 0; t < ntp; ++t) {
-    const int tx = tb_tp[4 * t], ty = tb_tp[4 * t + 1];
-    if (ty < g.oc0 || ty >= g.oc1) continue;
-    if (kk++ == tid) {
-      pidx = (ty - g.C0 + 1) * g.CS + (tx - g.R0) + 1;
-      pkind = tb_tp[4 * t + 2];
-      pcol = tb_tp[4 * t + 3];
+  // source pixels mark the rows of their owners
+  for (int kk = tid; kk < nsp; kk += blockDim.x) {
+    if (kk != tid) {  // more entries than threads
+      const int32_t *e = a.spx + (td[8] + kk) * SPX_W;
+      spx0 = e[0]; spx1 = e[1]; spx2 = e[2];
     }
+    int rr;
+    const int t = spx2 > 0 ? cs_owner<R>(g, spx0, spx1, rr) : -1;
+    if (t >= 0) atomicOr(&own[t], 1 << rr);
   }
+  __syncthreads();
+  const CsTap tap = cs_tap(g, a.taps, td[10], ntp, te);
+  const int srows = own[tid];
+  const bool wave_src = __ballot(srows != 0) != 0;
   const uint32_t voff = cs_out_voff<double>(g, row0, Ny);
   const int64_t out_bytes = (int64_t)(g.or1 - g.or0) * Ny * 8;
-  __syncthreads();
 
   auto step = [&](const double *P, double *Q, double(&Uc)[R], double(&Up)[R], int s) {
     const int n = a.n0 + s;
@@ -159,11 +148,11 @@ __global__ __launch_bounds__(NT) void k64_fwd_cs(F64Blk a) {
         Q[g.base + r] = v;
         if (REC) b64_store(rsl, voff + (uint32_t)(r * Ny * 8), lap);
       }
-      if (wave_src && sr0 >= 0) {
+      if (wave_src && srows) {
         const double xv = xs[s];
 #pragma unroll
         for (int r = 0; r < R; ++r)
-          if (r == sr0 || r == sr1) {
+          if ((srows >> r) & 1) {
             Up[r] = Up[r] + xv;
             Q[g.base + r] = Up[r];
           }
@@ -178,10 +167,10 @@ __global__ __launch_bounds__(NT) void k64_fwd_cs(F64Blk a) {
       }
     }
     __syncthreads();
-    if (pidx >= 0) {
-      const double v = Q[pidx];
-      const int64_t o = ((int64_t)b * a.T + n) * a.ntap + pcol;
-      if (a.y) a.y[o] = pkind ? v * v : v;
+    if (tap.pidx >= 0) {
+      const double v = Q[tap.pidx];
+      const int64_t o = ((int64_t)b * a.T + n) * a.ntap + tap.pcol;
+      if (a.y) a.y[o] = tap.pkind ? v * v : v;
       if (a.yraw) a.yraw[o] = v;
     }
   };
@@ -207,7 +196,8 @@ __global__ __launch_bounds__(NT) void k64_fwd_cs(F64Blk a) {
 template <int NT, int R>
 __global__ __launch_bounds__(NT) void k64_adj_cs(F64Blk a) {
   extern __shared__ double smem64[];
-  __shared__ int tb_sp[CS_MAX_TABLE * 6];
+  __shared__ int tb_sp[CS_MAX_TABLE * CS_SP_W];
+  __shared__ int own[2 * NT];
   __shared__ int seed_px[CS_MAX_SEEDS];
   __shared__ int nseeds;
   const int tid = threadIdx.x;
@@ -234,18 +224,12 @@ __global__ __launch_bounds__(NT) void k64_adj_cs(F64Blk a) {
     L1[r] = u1; L2[r] = u2;
     G[r] = 0.0; SG1[r] = 0.0;
   }
-  for (int i = tid; i < nsp; i += blockDim.x) {
-    const int32_t *e = a.spx + (td[8] + i) * SPX_W;
-    for (int j = 0; j < 6; ++j) tb_sp[6 * i + j] = e[j];
-  }
+  int spe[CS_SP_W];
+  cs_special_load(a.spx, td[8], nsp, spe);
   cs_zero_lds<double>(buf0, buf1, g, ((g.RH + R - 1) / R) * R, NBUF);
+  cs_special_stage(a.spx, td[8], nsp, spe, tb_sp, own);
   __syncthreads();
-  if (tid == 0) {
-    int n = 0;
-    for (int k = 0; k < nsp && n < CS_MAX_SEEDS; ++k)
-      if (tb_sp[6 * k + 5] > tb_sp[6 * k + 4]) seed_px[n++] = k;
-    nseeds = n;
-  }
+  cs_special_scatter<R>(g, nsp, tb_sp, own, seed_px, &nseeds);
   if (g.active) {
 #pragma unroll
     for (int r = 0; r < R; ++r) buf0[g.base + r] = KW[r] * L1[r];
@@ -253,7 +237,7 @@ __global__ __launch_bounds__(NT) void k64_adj_cs(F64Blk a) {
   __syncthreads();
   for (int i = tid; i < nseeds * a.nsteps; i += blockDim.x) {
     const int k = i / a.nsteps, s = i - k * a.nsteps, m = a.m_hi - s;
-    const int *e = tb_sp + 6 * seed_px[k];
+    const int *e = tb_sp + CS_SP_W * seed_px[k];
     double gs = 0.0;
     if (a.ybar)
       for (int t = e[4]; t < e[5]; ++t) {
@@ -264,16 +248,8 @@ __global__ __launch_bounds__(NT) void k64_adj_cs(F64Blk a) {
     seeds[i] = gs;
   }
   // special rows of this thread (at most two): seed slot, source slot
-  int sr0 = -1, sr1 = -1, sd0 = -1, sd1 = -1, sl0 = -1, sl1 = -1;
-  for (int k = 0, nseed = 0; k < nsp; ++k) {
-    const int *e = tb_sp + 6 * k;
-    const int sd = e[5] > e[4] ? nseed++ : -1;
-    const int rr = e[0] - g.R0 - row0;
-    if (!g.active || e[1] - g.C0 != g.c || rr < 0 || rr >= R || row0 + rr >= g.RH) continue;
-    const int sl = e[2] > 0 ? e[3] : -1;
-    if (sr0 < 0) { sr0 = rr; sd0 = sd; sl0 = sl; }
-    else { sr1 = rr; sd1 = sd; sl1 = sl; }
-  }
+  const CsSpecials sp = cs_special_read(g, row0, tb_sp, own);
+  const int sr0 = sp.sr0, sr1 = sp.sr1, sd0 = sp.sd0, sd1 = sp.sd1, sl0 = sp.sl0, sl1 = sp.sl1;
   const bool wave_sp = __ballot(sr0 >= 0) != 0;
   const uint32_t voff = cs_out_voff<double>(g, row0, Ny);
   const int64_t out_bytes = (int64_t)(g.or1 - g.or0) * Ny * 8;

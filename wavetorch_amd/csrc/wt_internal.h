@@ -17,7 +17,8 @@ namespace wt {
 // deduplicated, sorted by (x, y).  One row of 8 int32:
 //   [0] x  [1] y  [2] source multiplicity (number of sources containing it)
 //   [3] source slot (index among pixels with multiplicity > 0, or -1)
-//   [4] tap_lo [5] tap_hi  (range in the sorted tap table)  [6..7] unused
+//   [4] tap_lo [5] tap_hi  (range in the sorted tap table)
+//   [6] rows before this one that carry probe taps  [7] unused
 constexpr int SPX_W = 8;
 // Sorted taps: (x, y, kind, column) -- column = output index in y[b, n, :].
 constexpr int TAP_W = 4;

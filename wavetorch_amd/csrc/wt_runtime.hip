@@ -15,7 +15,7 @@
 #include <string>
 #include <vector>
 
-#include "wt_internal.h"
+#include "wt_colseg.h"
 
 namespace wt {
 
@@ -310,16 +310,16 @@ static bool tiles_ok(const Plan &p, int nt, int cpt) {
 static bool tables_ok_cs(const Plan &p, int R, int nthr);
 static bool tiles_ok_cs(const Plan &p, int nt, int R, bool fwd = true) {
   if (!cs_variant_exists(nt, R)) return false;
-  if (cs_shmem_bytes(R, p.RHmax, p.RWmax, fwd) + 1024 > LDS_LIMIT) return false;
+  if (cs_shmem_bytes(R, p.RHmax, p.RWmax, fwd) + CS_STATIC_LDS > LDS_LIMIT) return false;
   int nthr = cs_threads(R, p.RHmax, p.RWmax);
   return nthr <= nt && tables_ok_cs(p, R, nthr);
 }
 
 // The same for the double-precision block of R rows and tb steps, whose
-// static LDS (tables) is 7.2 KB.
+// static LDS (tables) is up to 15.3 KB.
 static bool tiles_ok_64(const Plan &p, int R, int tb, bool fwd) {
   if (!cs64_variant_exists(R, fwd)) return false;
-  if (cs64_shmem_bytes(R, p.RHmax, p.RWmax, tb) + 8 * 1024 > LDS_LIMIT) return false;
+  if (cs64_shmem_bytes(R, p.RHmax, p.RWmax, tb) + 16 * 1024 > LDS_LIMIT) return false;
   const int nthr = cs_threads(R, p.RHmax, p.RWmax);
   return nthr <= 1024 && tables_ok_cs(p, R, nthr);
 }
@@ -618,6 +618,18 @@ static const BlockModel kModel64 = {4.49, 0.43, 0.037, 0.0, 0.0143, 3.66, 1.89, 
 static const BlockModel kModel64Adj = {3.11, 2.35, 0.0442, 0.256, 0.00338, 1.19, 30.0, 0.57,
                                        5.4e-6, {4, 5, 0, 0, 0}, {4, 4, 0, 0, 0}};
 
+// Modelled time of a launch of n steps: `percu` workgroups of `waves` waves on
+// the fullest CU, `occ` of them at once, `cells` cells in all.
+static double launch_us(const BlockModel &m, int R, int waves, int occ, int percu, int n,
+                        double cells) {
+  auto round = [&](int wg) {
+    const int k = wg * ((waves + 3) / 4);
+    return m.ts + m.tR * R * k + n * (m.lat + m.cw * (R + m.c0) * (k + m.kb));
+  };
+  return m.t0 + percu / occ * round(occ) + (percu % occ ? round(percu % occ) : 0.0) +
+         cells * (m.rec * n * 1e-6 + m.state);
+}
+
 struct BlockChoice {
   double us;
   int s, c, tb, R;
@@ -644,14 +656,7 @@ static std::vector<BlockChoice> cheapest_blocks(const BlockModel &m, int Nx, int
       if (lds > LDS_LIMIT) continue;
       const int occ = std::max(1, std::min((int)(LDS_LIMIT / lds), m.waves[v] * 4 / waves));
       const double cells = (double)B * Nx * Ny;
-      auto launch = [&](int n) {
-        auto round = [&](int wg) {
-          const int k = wg * ((waves + 3) / 4);
-          return m.ts + m.tR * R * k + n * (m.lat + m.cw * (R + m.c0) * (k + m.kb));
-        };
-        return m.t0 + percu / occ * round(occ) + (percu % occ ? round(percu % occ) : 0.0) +
-               cells * (m.rec * n * 1e-6 + m.state);
-      };
+      auto launch = [&](int n) { return launch_us(m, R, waves, occ, percu, n, cells); };
       // among tilings that the model's whole waves and rounds call equal, the
       // one with the least area computed (halos clipped at the domain's edge;
       // halo rows drop out of the cone step by step, halo columns stay)
@@ -724,7 +729,7 @@ static void plan_f64(Plan &plan) {
       for (const BlockChoice &ch : cheapest_blocks(
                fwd ? kModel64 : kModel64Adj, p.Nx, p.Ny, p.B, p.T, 0, 32,
                [](int R, int RH, int RW, int tb) {
-                 return cs64_shmem_bytes(R, RH, RW, tb) + 8 * 1024;
+                 return cs64_shmem_bytes(R, RH, RW, tb) + 16 * 1024;
                })) {
         ok = take(ch.s, ch.c, ch.tb, ch.R, fwd);
         if (ok) break;
@@ -845,8 +850,10 @@ static int plan_build(const wt_config *cfg, int32_t B, int32_t T, float cmax_geo
     q.thi = hi;
   }
   p->nslot = nslot;
+  int ntappx = 0;
   for (auto &q : px) {
-    int32_t r[SPX_W] = {q.x, q.y, q.mult, q.slot, q.tlo, q.thi, 0, 0};
+    int32_t r[SPX_W] = {q.x, q.y, q.mult, q.slot, q.tlo, q.thi, ntappx, 0};
+    ntappx += q.thi > q.tlo;
     p->h_spx.insert(p->h_spx.end(), r, r + SPX_W);
   }
   for (auto &t : tp) {
@@ -1004,7 +1011,7 @@ static int plan_build(const wt_config *cfg, int32_t B, int32_t T, float cmax_geo
       auto fits = [&](int q, int qc, int d) {
         build_tiles(*p, q, qc, d);
         return tiles_ok_cs(*p, ant, acp, false) &&
-               cs_nl_shmem_bytes(acp, p->RHmax, p->RWmax) + 1024 <= LDS_LIMIT;
+               cs_nl_shmem_bytes(acp, p->RHmax, p->RWmax) + CS_STATIC_LDS <= LDS_LIMIT;
       };
       const bool fixed = tun.a_strips > 0;
       const int dmax = std::min(8, p->K), dmin = fixed ? 1 : std::min(4, p->K);
