@@ -399,6 +399,9 @@ int wt_batch_adj(void *plan, const wt_batch_group_io *io, void *saved,
  * can capture whole. */
 int wt_batch_fwd_adj(void *plan, const wt_batch_group_io *io, void *saved,
                      void *temp, void *stream);
+
+/* As wt_plan_group, for a batch plan. */
+int wt_batch_plan_group(void *plan, int32_t steps);
 int wt_batch_plan_destroy(void *plan);
 
 /* ------------------------------------------------------------------------ */

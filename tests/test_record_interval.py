@@ -68,3 +68,31 @@ def test_launch_longer_than_its_block(N, T, cuda):
         c = geom.c.cpu().numpy()
     yo, _ = co.forward(geom.b.cpu().numpy(), c, x, 0.7, 1.0, [[3, 3, 0]], [[N - 3, N - 3, 1]])
     assert np.array_equal(y, yo)
+
+
+@pytest.mark.gpu
+def test_open_batch_equals_checkpointed(cuda):
+    """A batch whose interval is left open records every step; its outputs and
+    gradients are those of checkpoints every 64 steps, bit for bit (launches
+    end at the same steps), also in several parts."""
+    from wavetorch_amd.batch import Instance, InstanceBatch
+    rng = np.random.default_rng(3)
+    insts, cs, xs, ys = [], [], [], []
+    for N, T in [(40, 150), (56, 131), (40, 70), (56, 64)]:
+        cfg = LoopConfig(Nx=N, Ny=N, dt=0.7, h=1.0, taps=((N - 12, N // 2, 1),),
+                         src_px=tuple((9, j, 0) for j in range(N // 4, 3 * N // 4)))
+        insts.append(Instance(cfg, torch.zeros(N, N), T, 1.0))
+        for lst, a in ((cs, rng.uniform(0.5, 1.0, (N, N))), (xs, rng.standard_normal(T)),
+                       (ys, rng.standard_normal((T, 1)))):
+            lst.append(torch.from_numpy(a.astype(np.float32)).to(cuda))
+    ref = None
+    for kw in (dict(checkpoint_every=64), {}, dict(tuning={"streams": 2})):
+        bt = InstanceBatch(insts, cuda, **kw)
+        print("case", kw, bt.tuning[0]["ck_every"], flush=True)
+        assert bt.tuning[0]["ck_every"] == (64 if "checkpoint_every" in kw else 150)
+        bt.set_inputs(cs, xs, ys)
+        bt.fwd_adj()
+        out = [t.clone() for o in bt.outputs() for t in o]
+        ref = ref or out
+        assert all(torch.equal(a, b) for a, b in zip(ref, out))
+    assert float(ref[1].abs().max()) > 0

@@ -153,6 +153,7 @@ _SIGS = {
     "wt_batch_fwd": (ctypes.c_int, [c_p, ctypes.POINTER(WtBatchIO), c_i32, c_p, c_p, c_p]),
     "wt_batch_adj": (ctypes.c_int, [c_p, ctypes.POINTER(WtBatchIO), c_p, c_p, c_p]),
     "wt_batch_fwd_adj": (ctypes.c_int, [c_p, ctypes.POINTER(WtBatchIO), c_p, c_p, c_p]),
+    "wt_batch_plan_group": (ctypes.c_int, [c_p, c_i32]),
     "wt_batch_plan_destroy": (ctypes.c_int, [c_p]),
     "wt_profile": (ctypes.c_int, [c_i32]),
     "wt_profile_read": (ctypes.c_int, [ctypes.POINTER(ctypes.c_double), ctypes.POINTER(c_i64),

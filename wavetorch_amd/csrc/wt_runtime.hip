@@ -1755,6 +1755,7 @@ struct BatchPlan {
   std::vector<int> ord_f, ord_a;  // groups in a launch's table: largest regions
                                   // first (forward, adjoint tilings)
   int T = 0, K = 64, nseg = 1;
+  int group = 0;  // adjoint launches end at multiples of this many steps (0: any)
   int tb = 24, nt = 1024, R = 10, tb_a = 24, nt_a = 1024, R_a = 10;
   int RHmax = 0, RWmax = 0, RHmax_a = 0, RWmax_a = 0;
   std::vector<size_t> soff, toff;
@@ -1943,7 +1944,8 @@ int batch_adjoint(const BatchPlan &bp, const wt_batch_group_io *io, char *saved,
     }
     // adjoint over m = n1 .. n0+1
     for (int m = n1; m > n0;) {
-      const int k = std::min(bp.tb_a, m - n0);
+      const int lo = bp.group > 0 ? std::max(n0, (m - 1) / bp.group * bp.group) : n0;
+      const int k = std::min(bp.tb_a, m - lo);
       BatchAdj bl{};
       int64_t work = 0;
       for (int j = 0; j < G; ++j) {
@@ -2309,6 +2311,15 @@ int wt_batch_plan_create(int32_t ngroups, const wt_config *cfgs, const int32_t *
     }
   }
   *plan_out = h;
+  return WT_OK;
+}
+
+int wt_batch_plan_group(void *plan, int32_t steps) {
+  if (!plan || steps < 0) {
+    set_error("wt_batch_plan_group: invalid argument");
+    return WT_EINVAL;
+  }
+  for (BatchPlan *bp : ((BatchHandle *)plan)->parts) bp->group = steps;
   return WT_OK;
 }
 
