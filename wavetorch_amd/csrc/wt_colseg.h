@@ -62,13 +62,16 @@ __device__ __forceinline__ CsGeom cs_geom(const int32_t *td, int tid) {
   return g;
 }
 
-// Rows [lo, hi) of the region that still influence the output after step s
-// of a launch of n steps.
-__device__ __forceinline__ void cone(const CsGeom &g, int s, int n, int &lo, int &hi) {
-  const int rem = n - 1 - s;
+// Steps of a launch of n in which this thread's rows still influence the
+// output rows: the halo shrinks by a row a step, so they are its first ones
+// (0 for a thread without cells).
+template <int R>
+__device__ __forceinline__ int cs_live_steps(const CsGeom &g, int row0, int n) {
   const int olo = g.or0 - g.R0, ohi = g.or1 - g.R0;
-  lo = olo > 0 ? max(0, olo - rem) : 0;
-  hi = ohi < g.RH ? min(g.RH, ohi + rem) : g.RH;
+  int q = 0;  // steps that must be left
+  if (ohi < g.RH) q = max(q, row0 - ohi + 1);
+  if (olo > 0) q = max(q, olo - row0 - R + 1);
+  return g.active ? n - q : 0;
 }
 
 // Owner of the region cell (x, y): thread k * RWm + c, its row r in [0, R);

@@ -55,17 +55,6 @@ __device__ __forceinline__ void cs_rec_store(__amdgpu_buffer_rsrc_t rs, uint32_t
 
 // ------------------------------------------------------------------ forward
 
-// Writes the output tile of the field in LDS buffer Q to fields[(b,idx)]:
-// a flat loop over the tile (used only at snapshot steps).
-__device__ __forceinline__ void cs_snapshot(const CsGeom &g, const float *Q, float *fo, int Ny) {
-  const int th = g.or1 - g.or0, tw = g.oc1 - g.oc0;
-  for (int i = threadIdx.x; i < th * tw; i += blockDim.x) {
-    const int rr = i / tw, cc = i - (i / tw) * tw;
-    const int row = g.or0 - g.R0 + rr, col = g.oc0 - g.C0 + cc;
-    fo[(int64_t)(g.or0 + rr) * Ny + (g.oc0 + cc)] = Q[(col + 1) * g.CS + row + 1];
-  }
-}
-
 // One forward step of this thread's segment; REC records lap(u_n) (and u_n
 // for the nonlinear cell) of the output rows through range-checked buffers.
 // UH: grid step 1, where each product with t1 = h^-2 is the value itself and
@@ -246,31 +235,56 @@ __device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
       (BATCH && a.rec_soff) ? (int64_t)a.rec_soff[b] : (int64_t)b * a.rec_K;
   const int Lb = (BATCH && a.Tlim) ? a.Tlim[b] : 0x7fffffff;
 
+  // What a step needs beyond its rows is a pointer that moves: the per-step
+  // address arithmetic of every wave is on the path between two barriers.
+  const int live = cs_live_steps<R>(g, row0, a.nsteps);
+  const float *recl = REC ? a.rec_lap + (rslot0 + (a.n0 - a.rec_n0)) * F + (int64_t)g.or0 * Ny
+                          : a.in1;
+  const float *recu = (REC && NL) ? a.rec_u + (rslot0 + (a.n0 - a.rec_n0)) * F +
+                                        (int64_t)g.or0 * Ny
+                                  : a.in1;
+  const int64_t yo = ((int64_t)b * a.T + a.n0) * a.ntap + tap.pcol;
+  float *yp = a.y ? a.y + yo : nullptr, *yrp = a.yraw ? a.yraw + yo : nullptr;
+  // next snapshot: at step `snap`, written by the threads from their registers
+  int snap = a.fields ? a.fstride - 1 - a.n0 % a.fstride : -1;
+  const float *fp = a.fields ? a.fields +
+                                   ((int64_t)b * (a.T / a.fstride) + a.n0 / a.fstride) * F +
+                                   (int64_t)g.or0 * Ny
+                             : a.in1;
+
   auto step = [&](const float *P, float *Q, float(&Uc)[R], float(&Up)[R], int s) {
-    const int n = a.n0 + s;
-    int lo, hi;
-    cone(g, s, a.nsteps, lo, hi);
-    const bool need = g.active && row0 < hi && row0 + R > lo;
-    // the (sample, step) slice of the record, based at the first output row
-    const int64_t ro = (rslot0 + (n - a.rec_n0)) * F + (int64_t)g.or0 * Ny;
-    const int64_t rbytes = n < Lb ? out_bytes : 0;
-    const __amdgpu_buffer_rsrc_t rsl = cs_rsrc(REC ? a.rec_lap + ro : a.in1, REC ? rbytes : 0);
-    const __amdgpu_buffer_rsrc_t rsu =
-        cs_rsrc((REC && NL) ? a.rec_u + ro : a.in1, (REC && NL) ? rbytes : 0);
+    // the (sample, step) slice of the record, based at the first output row;
+    // steps at or past the sample's length: an empty slice
+    const int64_t rbytes = (!BATCH || a.n0 + s < Lb) ? out_bytes : 0;
+    const __amdgpu_buffer_rsrc_t rsl = cs_rsrc(recl, REC ? rbytes : 0);
+    const __amdgpu_buffer_rsrc_t rsu = cs_rsrc(recu, (REC && NL) ? rbytes : 0);
     const float xv = wave_src ? xs[s] : 0.0f;
-    if (need)
-      cs_fwd_rows<R, NL, REC, UH>(a, P, Q, Uc, Up, KA, KB, KC, KD, KS, g.base, g.CS, vmask, xv, rsl,
-                              rsu, voff, Ny);
+    if (s < live) {
+      cs_fwd_rows<R, NL, REC, UH>(a, P, Q, Uc, Up, KA, KB, KC, KD, KS, g.base, g.CS, vmask, xv,
+                                  rsl, rsu, voff, Ny);
+      if (s == snap) {
+        const __amdgpu_buffer_rsrc_t rf = cs_rsrc(fp, out_bytes);
+#pragma unroll
+        for (int r = 0; r < R; ++r) cs_bstore(rf, voff + (uint32_t)(r * Ny * 4), Up[r]);
+      }
+    }
+    if (s == snap) {
+      snap += a.fstride;
+      fp += F;
+    }
+    if (REC) recl += F;
+    if (REC && NL) recu += F;
     __syncthreads();
     if (tap.pidx >= 0) {
       const float v = Q[tap.pidx];
-      const int64_t o = ((int64_t)b * a.T + n) * a.ntap + tap.pcol;
-      if (a.y) a.y[o] = tap.pkind ? v * v : v;
-      if (a.yraw) a.yraw[o] = v;
-    }
-    if (a.fields && ((n + 1) % a.fstride) == 0) {
-      const int64_t nf = a.T / a.fstride;
-      cs_snapshot(g, Q, a.fields + ((int64_t)b * nf + (n + 1) / a.fstride - 1) * F, Ny);
+      if (yp) {
+        *yp = tap.pkind ? v * v : v;
+        yp += a.ntap;
+      }
+      if (yrp) {
+        *yrp = v;
+        yrp += a.ntap;
+      }
     }
   };
 
@@ -478,42 +492,43 @@ __device__ __forceinline__ void adj_cs_body(const AdjArgs &a, const int w) {
 
   const int64_t sslot0 =
       (BATCH && a.seg_soff) ? (int64_t)a.seg_soff[b] : (int64_t)b * a.seg_K;
-  auto seg_rsrc = [&](int m) {
-    return cs_rsrc(a.seg_lap + (sslot0 + (m - 1 - a.seg_n0)) * F + (int64_t)g.or0 * Ny,
-                   out_bytes);
-  };
+  // slice of the record read at reverse step m_hi (the steps below it lie F
+  // values before each other)
+  const float *rec0 =
+      a.seg_lap + (sslot0 + (a.m_hi - 1 - a.seg_n0)) * F + (int64_t)g.or0 * Ny;
   // lap(u_{m-1}) of the first two steps of this launch (SG0: even steps,
   // SG1: odd steps)
   {
-    const __amdgpu_buffer_rsrc_t rs0 = seg_rsrc(a.m_hi);
+    const __amdgpu_buffer_rsrc_t rs0 = cs_rsrc(rec0, out_bytes);
     const uint32_t voff0 = rec_off(a.m_hi - 1);
 #pragma unroll
     for (int r = 0; r < R; ++r) SG0[r] = cs_rec_load(rs0, voff0 + (uint32_t)(r * Ny * 4));
     // issued even for a one-step launch (out of range, reads nothing) so
     // that the loop's wait counts need not cover a path without them
     const bool two = a.nsteps > 1;
-    const __amdgpu_buffer_rsrc_t rs1 = seg_rsrc(two ? a.m_hi - 1 : a.m_hi);
+    const __amdgpu_buffer_rsrc_t rs1 = cs_rsrc(two ? rec0 - F : rec0, out_bytes);
     const uint32_t voff1 = two ? rec_off(a.m_hi - 2) : 0x80000000u;
 #pragma unroll
     for (int r = 0; r < R; ++r) SG1[r] = cs_rec_load(rs1, voff1 + (uint32_t)(r * Ny * 4));
   }
+  const int live = cs_live_steps<R>(g, row0, a.nsteps);
+  const float *recp = rec0 - 2 * F;  // the step after next
+  float *gsrc_row = a.gsrc + ((int64_t)b * a.T + (a.m_hi - 1)) * a.nsrcslot;
+
+  const float *sd0p = seeds + (sd0 >= 0 ? sd0 * a.nsteps : 0);
+  const float *sd1p = seeds + (sd1 >= 0 ? sd1 * a.nsteps : 0);
 
   auto step = [&](const float *P, float *Q, float(&Lc)[R], float(&Ln)[R], float(&SG)[R],
                   int s) {
-    const int m = a.m_hi - s;
-    int lo, hi;
-    cone(g, s, a.nsteps, lo, hi);
-    const bool need = g.active && row0 < hi && row0 + R > lo;
     // record index m-3-seg_n0 >= 0: m-2 >= m_hi-nsteps+1 >= seg_n0+1
     const bool prefetch = s + 2 < a.nsteps;
-    const __amdgpu_buffer_rsrc_t rsn = seg_rsrc(prefetch ? m - 2 : m);
-    const uint32_t pvoff = prefetch ? rec_off(m - 3) : 0x80000000u;
-    float *gsrc_row = a.gsrc + ((int64_t)b * a.T + (m - 1)) * a.nsrcslot;
-    if (need) {
+    const __amdgpu_buffer_rsrc_t rsn = cs_rsrc(recp, out_bytes);
+    const uint32_t pvoff = prefetch ? rec_off(a.m_hi - s - 3) : 0x80000000u;
+    if (s < live) {
       if (wave_sp) {
-        const float gs0 = sd0 >= 0 ? seeds[sd0 * a.nsteps + s] : 0.0f;
+        const float gs0 = sd0 >= 0 ? sd0p[s] : 0.0f;
         if (wave_sp2) {
-          const float gs1 = sd1 >= 0 ? seeds[sd1 * a.nsteps + s] : 0.0f;
+          const float gs1 = sd1 >= 0 ? sd1p[s] : 0.0f;
           cs_adj_rows<R, 2, true>(P, Q, Lc, Ln, KA1, KW, g.base, g.CS, omask, sr0, sr1, gs0,
                                   gs1, sl0, sl1, gsrc_row);
         } else if (wave_gs) {
@@ -545,6 +560,8 @@ __device__ __forceinline__ void adj_cs_body(const AdjArgs &a, const int w) {
       asm volatile("" : "+v"(G[r]));
       SG[r] = cs_rec_load(rsn, pvoff + (uint32_t)(r * Ny * 4));
     }
+    recp -= F;
+    gsrc_row -= a.nsrcslot;
     __syncthreads();
   };
 
@@ -723,13 +740,12 @@ __global__ __launch_bounds__(NT) void k_adj_cs_nl(AdjArgs a, NlCarry cy) {
     }
   };
   load_record(a.m_hi, true);
+  const int live = cs_live_steps<R>(g, row0, a.nsteps);
+  float *gsrc0 = a.gsrc + ((int64_t)b * a.T + (a.m_hi - 1)) * a.nsrcslot;
   auto step = [&](const float *P, float *Q, float(&Lx)[R], float(&Ly)[R], int s) {
     // Lx = lambda_{m+1}, Ly = lambda_{m+2} on entry, lambda_m on exit
     const int m = a.m_hi - s;
-    int lo, hi;
-    cone(g, s, a.nsteps, lo, hi);
-    const bool need = g.active && row0 < hi && row0 + R > lo;
-    if (need) {
+    if (s < live) {
       const float gs0 = sd0 >= 0 ? seeds[sd0 * a.nsteps + s] : 0.0f;
       const float gs1 = sd1 >= 0 ? seeds[sd1 * a.nsteps + s] : 0.0f;
       const int lfb = g.base - g.CS, rtb = g.base + g.CS;
@@ -795,7 +811,7 @@ __global__ __launch_bounds__(NT) void k_adj_cs_nl(AdjArgs a, NlCarry cy) {
       if (sr0 >= 0) {
         // lambda_m at source pixels of the output rows -> dJ/dx[b, m-1]:
         // picked with selects, at most two stores
-        float *gsrc_row = a.gsrc + ((int64_t)b * a.T + (m - 1)) * a.nsrcslot;
+        float *gsrc_row = gsrc0 - (int64_t)s * a.nsrcslot;
         float v0 = Ly[0], v1 = Ly[0];
 #pragma unroll
         for (int r = 1; r < R; ++r) {

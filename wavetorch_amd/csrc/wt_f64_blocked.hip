@@ -107,15 +107,20 @@ __global__ __launch_bounds__(NT) void k64_fwd_cs(F64Blk a) {
   const uint32_t voff = cs_out_voff<double>(g, row0, Ny);
   const int64_t out_bytes = (int64_t)(g.or1 - g.or0) * Ny * 8;
 
+  const int live = cs_live_steps<R>(g, row0, a.nsteps);
+  const double *recp = REC ? a.rec + ((int64_t)b * a.T + a.n0) * F + (int64_t)g.or0 * Ny : a.A;
+  const int64_t yo = ((int64_t)b * a.T + a.n0) * a.ntap + tap.pcol;
+  double *yp = a.y ? a.y + yo : nullptr, *yrp = a.yraw ? a.yraw + yo : nullptr;
+  // next snapshot: at step `snap`
+  int snap = a.fields ? a.fstride - 1 - a.n0 % a.fstride : -1;
+  const double *fp = a.fields ? a.fields +
+                                    ((int64_t)b * (a.T / a.fstride) + a.n0 / a.fstride) * F +
+                                    (int64_t)g.or0 * Ny
+                              : a.A;
+
   auto step = [&](const double *P, double *Q, double(&Uc)[R], double(&Up)[R], int s) {
-    const int n = a.n0 + s;
-    int lo, hi;
-    cone(g, s, a.nsteps, lo, hi);
-    const bool snap = a.fields && ((n + 1) % a.fstride) == 0;
-    if (g.active && row0 < hi && row0 + R > lo) {
-      const __amdgpu_buffer_rsrc_t rsl = cs_rsrc(
-          REC ? a.rec + ((int64_t)b * a.T + n) * F + (int64_t)g.or0 * Ny : a.A,
-          REC ? out_bytes : 0);
+    if (s < live) {
+      const __amdgpu_buffer_rsrc_t rsl = cs_rsrc(recp, REC ? out_bytes : 0);
       const int lfb = g.base - g.CS, rtb = g.base + g.CS;
       double upv = UH ? P[g.base - 1] : a.t1 * P[g.base - 1];
       double ctv = UH ? 0.0 : a.t1 * Uc[0];
@@ -157,21 +162,28 @@ __global__ __launch_bounds__(NT) void k64_fwd_cs(F64Blk a) {
             Q[g.base + r] = Up[r];
           }
       }
-      if (snap) {  // the thread's own rows: consecutive lanes, consecutive columns
-        const int64_t nf = a.T / a.fstride;
-        const __amdgpu_buffer_rsrc_t rf = cs_rsrc(
-            a.fields + ((int64_t)b * nf + (n + 1) / a.fstride - 1) * F + (int64_t)g.or0 * Ny,
-            out_bytes);
+      if (s == snap) {  // the thread's own rows: consecutive lanes, consecutive columns
+        const __amdgpu_buffer_rsrc_t rf = cs_rsrc(fp, out_bytes);
 #pragma unroll
         for (int r = 0; r < R; ++r) b64_store(rf, voff + (uint32_t)(r * Ny * 8), Up[r]);
       }
     }
+    if (s == snap) {
+      snap += a.fstride;
+      fp += F;
+    }
+    if (REC) recp += F;
     __syncthreads();
     if (tap.pidx >= 0) {
       const double v = Q[tap.pidx];
-      const int64_t o = ((int64_t)b * a.T + n) * a.ntap + tap.pcol;
-      if (a.y) a.y[o] = tap.pkind ? v * v : v;
-      if (a.yraw) a.yraw[o] = v;
+      if (yp) {
+        *yp = tap.pkind ? v * v : v;
+        yp += a.ntap;
+      }
+      if (yrp) {
+        *yrp = v;
+        yrp += a.ntap;
+      }
     }
   };
   int s = 0;
@@ -256,28 +268,27 @@ __global__ __launch_bounds__(NT) void k64_adj_cs(F64Blk a) {
   const bool out_col = voff != 0x80000000u;
   const int olo = g.or0 - g.R0 - row0, ohi = g.or1 - g.R0 - row0;  // output rows, thread's count
   __syncthreads();
-  auto rec_rsrc = [&](int m) {
-    return cs_rsrc(a.rec + ((int64_t)b * a.T + (m - 1)) * F + (int64_t)g.or0 * Ny, out_bytes);
-  };
+  // slice of the record read at reverse step m_hi
+  const double *rec0 = a.rec + ((int64_t)b * a.T + (a.m_hi - 1)) * F + (int64_t)g.or0 * Ny;
   {
-    const __amdgpu_buffer_rsrc_t rs0 = rec_rsrc(a.m_hi);
+    const __amdgpu_buffer_rsrc_t rs0 = cs_rsrc(rec0, out_bytes);
 #pragma unroll
     for (int r = 0; r < R; ++r) SG0[r] = b64_load(rs0, voff + (uint32_t)(r * Ny * 8));
     const bool two = a.nsteps > 1;
-    const __amdgpu_buffer_rsrc_t rs1 = rec_rsrc(two ? a.m_hi - 1 : a.m_hi);
+    const __amdgpu_buffer_rsrc_t rs1 = cs_rsrc(two ? rec0 - F : rec0, out_bytes);
     const uint32_t v1 = two ? voff : 0x80000000u;
 #pragma unroll
     for (int r = 0; r < R; ++r) SG1[r] = b64_load(rs1, v1 + (uint32_t)(r * Ny * 8));
   }
+  const int live = cs_live_steps<R>(g, row0, a.nsteps);
+  const double *recp = rec0 - 2 * F;  // the step after next
+  double *gsrc_row = a.gsrc + ((int64_t)b * a.T + (a.m_hi - 1)) * a.nslot;
   auto step = [&](const double *P, double *Q, double(&Lc)[R], double(&Ln)[R], double(&SG)[R],
                   int s) {
-    const int m = a.m_hi - s;
-    int lo, hi;
-    cone(g, s, a.nsteps, lo, hi);
     const bool prefetch = s + 2 < a.nsteps;
-    const __amdgpu_buffer_rsrc_t rsn = rec_rsrc(prefetch ? m - 2 : m);
+    const __amdgpu_buffer_rsrc_t rsn = cs_rsrc(recp, out_bytes);
     const uint32_t pvoff = prefetch ? voff : 0x80000000u;
-    if (g.active && row0 < hi && row0 + R > lo) {
+    if (s < live) {
       const int lfb = g.base - g.CS, rtb = g.base + g.CS;
       double upv = P[g.base - 1];
       double ct = KW[0] * Lc[0];
@@ -312,7 +323,6 @@ __global__ __launch_bounds__(NT) void k64_adj_cs(F64Blk a) {
           v0 = (r == sr0) ? Ln[r] : v0;
           v1 = (r == sr1) ? Ln[r] : v1;
         }
-        double *gsrc_row = a.gsrc + ((int64_t)b * a.T + (m - 1)) * a.nslot;
         if (sl0 >= 0 && out_col && sr0 >= olo && sr0 < ohi) gsrc_row[sl0] = v0;
         if (sl1 >= 0 && out_col && sr1 >= olo && sr1 < ohi) gsrc_row[sl1] = v1;
       }
@@ -326,6 +336,8 @@ __global__ __launch_bounds__(NT) void k64_adj_cs(F64Blk a) {
       asm volatile("" : "+v"(G[r]));
       SG[r] = b64_load(rsn, pvoff + (uint32_t)(r * Ny * 8));
     }
+    recp -= F;
+    gsrc_row -= a.nslot;
     __syncthreads();
   };
   int s = 0;
