@@ -4,6 +4,8 @@
 // public ABI.
 #pragma once
 
+#include <utility>
+
 #include "wt_internal.h"
 
 namespace wt {
@@ -196,6 +198,62 @@ __device__ __forceinline__ CsTap cs_tap(const CsGeom &g, const int32_t *taps, in
     p.pcol = e[3];
   }
   return p;
+}
+
+// Special rows after a step's rows are done: one code path computes every
+// row, and the waves that hold a special pixel then pick its row with selects,
+// change it and put it back (registers and LDS), instead of carrying the
+// addition through every row of every wave.
+// (Written out by expansion: of a loop over r == row the compiler makes an
+// indexed access, which moves the rows from registers to scratch memory.)
+template <int R, typename T, int... I>
+__device__ __forceinline__ T cs_pick_(const T (&v)[R], int row,
+                                      std::integer_sequence<int, I...>) {
+  T x = v[0];
+  ((x = (I == row) ? v[I] : x), ...);
+  return x;
+}
+template <int R, typename T>
+__device__ __forceinline__ T cs_pick(const T (&v)[R], int row) {
+  return cs_pick_<R>(v, row, std::make_integer_sequence<int, R>{});
+}
+template <int R, typename T, int... I>
+__device__ __forceinline__ void cs_put_(T (&v)[R], int row, T x,
+                                        std::integer_sequence<int, I...>) {
+  ((v[I] = (I == row) ? x : v[I]), ...);
+}
+template <int R, typename T>
+__device__ __forceinline__ void cs_put(T (&v)[R], int row, T x) {
+  cs_put_<R>(v, row, x, std::make_integer_sequence<int, R>{});
+}
+// Adds x_n to the rows in the mask `srows` (bit r: row r is a source pixel):
+// `one`: no lane of the wave holds more than one.
+template <int R, typename T>
+__device__ __forceinline__ void cs_add_source(T (&v)[R], T *Q, int srows, bool one, T xv) {
+  if (one) {
+    const int row = __ffs(srows) - 1;
+    const T x = cs_pick<R>(v, row) + xv;
+    cs_put<R>(v, row, x);
+    if (row >= 0) Q[row] = x;
+  } else {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if ((srows >> r) & 1) {
+        v[r] = v[r] + xv;
+        Q[r] = v[r];
+      }
+  }
+}
+
+// A special pixel of this thread in a reverse step: seed `gs` added to its
+// row (LDS too, as w * lambda), and lambda_m stored for dJ/dx where the pixel
+// is a source of the output rows (`gx`, else null).
+template <int R, typename T>
+__device__ __forceinline__ void cs_adj_special(T (&Ln)[R], T *Q, int row, T kw, T gs, T *gx) {
+  const T v = cs_pick<R>(Ln, row) + gs;
+  cs_put<R>(Ln, row, v);
+  if (row >= 0) Q[row] = kw * v;
+  if (gx) *gx = v;
 }
 
 // Raw buffer access with hardware range checking (gfx9 descriptor word 3 =

@@ -66,9 +66,8 @@ __device__ __forceinline__ void cs_fwd_rows(const FwdArgs &a, const float *__res
                                             float *__restrict__ Q,
                                             float (&Uc)[R], float (&Up)[R], const float (&KA)[R],
                                             const float (&KB)[R], const float (&KC)[R],
-                                            const float (&KD)[R], const float (&KS)[R],
-                                            int base, int CS, uint32_t vmask, float xv,
-                                            __amdgpu_buffer_rsrc_t rsl, __amdgpu_buffer_rsrc_t rsu,
+                                            const float (&KD)[R], int base, int CS,
+                                            uint32_t vmask, __amdgpu_buffer_rsrc_t rsl, __amdgpu_buffer_rsrc_t rsu,
                                             uint32_t voff, int Ny) {
   const int lfb = base - CS, rtb = base + CS;
   // the row above and, for UH = false, this row times t1
@@ -119,10 +118,7 @@ __device__ __forceinline__ void cs_fwd_rows(const FwdArgs &a, const float *__res
     const float p1 = a.s2 * ct;
     const float p2 = Bm * Up[r];
     const float p3 = C2 * lap;
-    float v = A * ((p1 - p2) + p3);
-    // source: weight 1 at source pixels, 0 elsewhere; fma(1, x, v) rounds
-    // once, exactly like the reference's v + x (source.py:22)
-    v = __builtin_fmaf(KS[r], xv, v);
+    const float v = A * ((p1 - p2) + p3);
     Up[r] = v;
     Q[base + r] = v;
     if (REC) {
@@ -165,7 +161,7 @@ __device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
   int *own = (int *)(xs + CS_MAX_TBLOCK);
   const int nsp = min(td[9] - td[8], CS_MAX_TABLE), ntp = min(td[11] - td[10], CS_MAX_TABLE);
 
-  float U0[R], U1[R], KA[R], KB[R], KC[R], KD[R], KS[R];
+  float U0[R], U1[R], KA[R], KB[R], KC[R], KD[R];
   const int row0 = g.k * R;  // region row of cell 0
   uint32_t vmask = 0;        // cells that are inside the region
   // 1) all global loads first (one round trip for the whole set-up)
@@ -224,9 +220,8 @@ __device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
   WT_TS(6);
   const CsTap tap = cs_tap(g, a.taps, td[10], ntp, te);
   const int srows = own[tid];
-#pragma unroll
-  for (int r = 0; r < R; ++r) KS[r] = (srows >> r) & 1 ? 1.0f : 0.0f;
   const bool wave_src = __ballot(srows != 0) != 0;
+  const bool one_src = __ballot((srows & (srows - 1)) != 0) == 0;
   const uint32_t voff = cs_out_voff<float>(g, row0, Ny);
   const int64_t out_bytes = (int64_t)(g.or1 - g.or0) * Ny * 4;
   // record slots of this sample; steps at or past its length are not
@@ -258,10 +253,11 @@ __device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
     const int64_t rbytes = (!BATCH || a.n0 + s < Lb) ? out_bytes : 0;
     const __amdgpu_buffer_rsrc_t rsl = cs_rsrc(recl, REC ? rbytes : 0);
     const __amdgpu_buffer_rsrc_t rsu = cs_rsrc(recu, (REC && NL) ? rbytes : 0);
-    const float xv = wave_src ? xs[s] : 0.0f;
     if (s < live) {
-      cs_fwd_rows<R, NL, REC, UH>(a, P, Q, Uc, Up, KA, KB, KC, KD, KS, g.base, g.CS, vmask, xv,
-                                  rsl, rsu, voff, Ny);
+      cs_fwd_rows<R, NL, REC, UH>(a, P, Q, Uc, Up, KA, KB, KC, KD, g.base, g.CS, vmask, rsl, rsu,
+                                  voff, Ny);
+      // v + x_n at the source pixels (source.py:22)
+      if (wave_src) cs_add_source<R>(Up, Q + g.base, srows, one_src, xs[s]);
       if (s == snap) {
         const __amdgpu_buffer_rsrc_t rf = cs_rsrc(fp, out_bytes);
 #pragma unroll
@@ -337,17 +333,16 @@ __global__ __launch_bounds__(NT) void k_fwd_cs_batch(BatchFwd bl) {
 
 // ------------------------------------------------------------------ adjoint
 
-// One reverse step of this thread's segment.  SP: the wave holds
-// probe/source pixels (sr0, sr1).  a2 = A*Bm is formed as a1 - 1 (with
-// a1 = A*s2 = 2/(1+b*dt), a2 = (1-b*dt)/(1+b*dt)).  The thread's own w*lambda
-// values (up/centre/down neighbours) are re-formed as KW*Lc -- the same fp32
-// product the previous step stored to LDS -- instead of being kept in R more
-// registers.
-template <int R, int NSP, bool GS>
-__device__ __forceinline__ void cs_adj_rows(
-    const float *__restrict__ P, float *__restrict__ Q, float (&Lc)[R], float (&Ln)[R],
-    const float (&KA1)[R], const float (&KW)[R], int base, int CS, uint32_t omask, int sr0,
-    int sr1, float gs0, float gs1, int sl0, int sl1, float *__restrict__ gsrc_row) {
+// One reverse step of this thread's segment, without probe seeds.  a2 = A*Bm
+// is formed as a1 - 1 (with a1 = A*s2 = 2/(1+b*dt), a2 = (1-b*dt)/(1+b*dt)).
+// The thread's own w*lambda values (up/centre/down neighbours) are re-formed
+// as KW*Lc -- the same fp32 product the previous step stored to LDS --
+// instead of being kept in R more registers.
+template <int R>
+__device__ __forceinline__ void cs_adj_rows(const float *__restrict__ P, float *__restrict__ Q,
+                                            float (&Lc)[R], float (&Ln)[R],
+                                            const float (&KA1)[R], const float (&KW)[R],
+                                            int base, int CS) {
   const int lfb = base - CS, rtb = base + CS;
   float upv = P[base - 1];
   float ct = KW[0] * Lc[0];
@@ -360,27 +355,11 @@ __device__ __forceinline__ void cs_adj_rows(
     lapw = lapw + rt;
     lapw = lapw + dn;
     // a1*L1 + lapw - (a1-1)*L2 = a1*(L1 - L2) + (lapw + L2)
-    float lam = __builtin_fmaf(KA1[r], Lc[r] - Ln[r], lapw + Ln[r]);
-    if (NSP >= 1 && r == sr0) lam += gs0;
-    if (NSP >= 2 && r == sr1) lam += gs1;
+    const float lam = __builtin_fmaf(KA1[r], Lc[r] - Ln[r], lapw + Ln[r]);
     upv = ct;
     ct = dn;
     Ln[r] = lam;
     Q[base + r] = KW[r] * lam;
-  }
-  if (GS) {
-    // lambda_m at source pixels of the output rows -> dJ/dx[b, m-1]: pick
-    // the rows' values with selects, then at most NSP stores (one masked
-    // store per row would put R branches on every step of the waves that
-    // hold special pixels, which the step's barrier waits for)
-    float v0 = Ln[0], v1 = Ln[0];
-#pragma unroll
-    for (int r = 1; r < R; ++r) {
-      v0 = (r == sr0) ? Ln[r] : v0;
-      if (NSP >= 2) v1 = (r == sr1) ? Ln[r] : v1;
-    }
-    if (sl0 >= 0 && sr0 >= 0 && ((omask >> sr0) & 1u)) gsrc_row[sl0] = v0;
-    if (NSP >= 2 && sl1 >= 0 && sr1 >= 0 && ((omask >> sr1) & 1u)) gsrc_row[sl1] = v1;
   }
 }
 
@@ -467,11 +446,9 @@ __device__ __forceinline__ void adj_cs_body(const AdjArgs &a, const int w) {
     }
     seeds[i] = gs;
   }
-  // wave-uniform special-pixel path: none, one slot, two slots; source
-  // gradient stores only in waves that hold a source pixel
+  // waves with special pixels, with two in a thread
   const bool wave_sp = __ballot(sr0 >= 0) != 0;
   const bool wave_sp2 = __ballot(sr1 >= 0) != 0;
-  const bool wave_gs = __ballot(sl0 >= 0 || sl1 >= 0) != 0;
   // output cells of this thread (gradient write-back, dJ/dx)
   uint32_t omask = 0;
   if (g.active && g.C0 + g.c >= g.oc0 && g.C0 + g.c < g.oc1) {
@@ -513,6 +490,9 @@ __device__ __forceinline__ void adj_cs_body(const AdjArgs &a, const int w) {
   }
   const int live = cs_live_steps<R>(g, row0, a.nsteps);
   const float *recp = rec0 - 2 * F;  // the step after next
+  const float kw0 = cs_pick<R>(KW, sr0), kw1 = cs_pick<R>(KW, sr1);
+  const bool gx0 = sl0 >= 0 && sr0 >= 0 && ((omask >> sr0) & 1u);
+  const bool gx1 = sl1 >= 0 && sr1 >= 0 && ((omask >> sr1) & 1u);
   float *gsrc_row = a.gsrc + ((int64_t)b * a.T + (a.m_hi - 1)) * a.nsrcslot;
 
   const float *sd0p = seeds + (sd0 >= 0 ? sd0 * a.nsteps : 0);
@@ -525,22 +505,13 @@ __device__ __forceinline__ void adj_cs_body(const AdjArgs &a, const int w) {
     const __amdgpu_buffer_rsrc_t rsn = cs_rsrc(recp, out_bytes);
     const uint32_t pvoff = prefetch ? rec_off(a.m_hi - s - 3) : 0x80000000u;
     if (s < live) {
+      cs_adj_rows<R>(P, Q, Lc, Ln, KA1, KW, g.base, g.CS);
       if (wave_sp) {
-        const float gs0 = sd0 >= 0 ? sd0p[s] : 0.0f;
-        if (wave_sp2) {
-          const float gs1 = sd1 >= 0 ? sd1p[s] : 0.0f;
-          cs_adj_rows<R, 2, true>(P, Q, Lc, Ln, KA1, KW, g.base, g.CS, omask, sr0, sr1, gs0,
-                                  gs1, sl0, sl1, gsrc_row);
-        } else if (wave_gs) {
-          cs_adj_rows<R, 1, true>(P, Q, Lc, Ln, KA1, KW, g.base, g.CS, omask, sr0, -1, gs0,
-                                  0.f, sl0, -1, gsrc_row);
-        } else {
-          cs_adj_rows<R, 1, false>(P, Q, Lc, Ln, KA1, KW, g.base, g.CS, omask, sr0, -1, gs0,
-                                   0.f, -1, -1, gsrc_row);
-        }
-      } else {
-        cs_adj_rows<R, 0, false>(P, Q, Lc, Ln, KA1, KW, g.base, g.CS, omask, -1, -1, 0.f, 0.f,
-                                 -1, -1, gsrc_row);
+        cs_adj_special<R>(Ln, Q + g.base, sr0, kw0, sd0 >= 0 ? sd0p[s] : 0.0f,
+                          gx0 ? gsrc_row + sl0 : nullptr);
+        if (wave_sp2)
+          cs_adj_special<R>(Ln, Q + g.base, sr1, kw1, sd1 >= 0 ? sd1p[s] : 0.0f,
+                            gx1 ? gsrc_row + sl1 : nullptr);
       }
     }
     // gradient sum, then refill SG with lap(u) of step m-2 (the record is

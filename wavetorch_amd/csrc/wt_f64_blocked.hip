@@ -104,6 +104,7 @@ __global__ __launch_bounds__(NT) void k64_fwd_cs(F64Blk a) {
   const CsTap tap = cs_tap(g, a.taps, td[10], ntp, te);
   const int srows = own[tid];
   const bool wave_src = __ballot(srows != 0) != 0;
+  const bool one_src = __ballot((srows & (srows - 1)) != 0) == 0;
   const uint32_t voff = cs_out_voff<double>(g, row0, Ny);
   const int64_t out_bytes = (int64_t)(g.or1 - g.or0) * Ny * 8;
 
@@ -153,15 +154,7 @@ __global__ __launch_bounds__(NT) void k64_fwd_cs(F64Blk a) {
         Q[g.base + r] = v;
         if (REC) b64_store(rsl, voff + (uint32_t)(r * Ny * 8), lap);
       }
-      if (wave_src && srows) {
-        const double xv = xs[s];
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-          if ((srows >> r) & 1) {
-            Up[r] = Up[r] + xv;
-            Q[g.base + r] = Up[r];
-          }
-      }
+      if (wave_src) cs_add_source<R>(Up, Q + g.base, srows, one_src, xs[s]);
       if (s == snap) {  // the thread's own rows: consecutive lanes, consecutive columns
         const __amdgpu_buffer_rsrc_t rf = cs_rsrc(fp, out_bytes);
 #pragma unroll
@@ -265,8 +258,12 @@ __global__ __launch_bounds__(NT) void k64_adj_cs(F64Blk a) {
   const bool wave_sp = __ballot(sr0 >= 0) != 0;
   const uint32_t voff = cs_out_voff<double>(g, row0, Ny);
   const int64_t out_bytes = (int64_t)(g.or1 - g.or0) * Ny * 8;
-  const bool out_col = voff != 0x80000000u;
+  const bool wave_sp2 = __ballot(sr1 >= 0) != 0;
   const int olo = g.or0 - g.R0 - row0, ohi = g.or1 - g.R0 - row0;  // output rows, thread's count
+  const bool out_col = voff != 0x80000000u;
+  const bool gx0 = sl0 >= 0 && out_col && sr0 >= olo && sr0 < ohi;
+  const bool gx1 = sl1 >= 0 && out_col && sr1 >= olo && sr1 < ohi;
+  const double kw0 = cs_pick<R>(KW, sr0), kw1 = cs_pick<R>(KW, sr1);
   __syncthreads();
   // slice of the record read at reverse step m_hi
   const double *rec0 = a.rec + ((int64_t)b * a.T + (a.m_hi - 1)) * F + (int64_t)g.or0 * Ny;
@@ -292,11 +289,6 @@ __global__ __launch_bounds__(NT) void k64_adj_cs(F64Blk a) {
       const int lfb = g.base - g.CS, rtb = g.base + g.CS;
       double upv = P[g.base - 1];
       double ct = KW[0] * Lc[0];
-      double gs0 = 0.0, gs1 = 0.0;
-      if (wave_sp) {
-        if (sd0 >= 0) gs0 = seeds[sd0 * a.nsteps + s];
-        if (sd1 >= 0) gs1 = seeds[sd1 * a.nsteps + s];
-      }
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         const double dn = (r < R - 1) ? KW[r + 1] * Lc[r + 1] : P[g.base + R];
@@ -306,25 +298,18 @@ __global__ __launch_bounds__(NT) void k64_adj_cs(F64Blk a) {
         lapw = lapw + rt;
         lapw = lapw + dn;
         // a1 L1 + lapw - a2 L2 with a2 = a1 - 1
-        double lam = __builtin_fma(KA1[r], Lc[r] - Ln[r], lapw + Ln[r]);
-        if (wave_sp) {
-          if (r == sr0) lam += gs0;
-          if (r == sr1) lam += gs1;
-        }
+        const double lam = __builtin_fma(KA1[r], Lc[r] - Ln[r], lapw + Ln[r]);
         upv = ct;
         ct = dn;
         Ln[r] = lam;
         Q[g.base + r] = KW[r] * lam;
       }
       if (wave_sp) {
-        double v0 = Ln[0], v1 = Ln[0];
-#pragma unroll
-        for (int r = 1; r < R; ++r) {
-          v0 = (r == sr0) ? Ln[r] : v0;
-          v1 = (r == sr1) ? Ln[r] : v1;
-        }
-        if (sl0 >= 0 && out_col && sr0 >= olo && sr0 < ohi) gsrc_row[sl0] = v0;
-        if (sl1 >= 0 && out_col && sr1 >= olo && sr1 < ohi) gsrc_row[sl1] = v1;
+        cs_adj_special<R>(Ln, Q + g.base, sr0, kw0, sd0 >= 0 ? seeds[sd0 * a.nsteps + s] : 0.0,
+                          gx0 ? gsrc_row + sl0 : nullptr);
+        if (wave_sp2)
+          cs_adj_special<R>(Ln, Q + g.base, sr1, kw1, sd1 >= 0 ? seeds[sd1 * a.nsteps + s] : 0.0,
+                            gx1 ? gsrc_row + sl1 : nullptr);
       }
     }
     // gradient sum, then the record of two steps later into the same
