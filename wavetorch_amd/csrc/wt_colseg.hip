@@ -55,6 +55,33 @@ __device__ __forceinline__ void cs_rec_store(__amdgpu_buffer_rsrc_t rs, uint32_t
 
 // ------------------------------------------------------------------ forward
 
+// Correctly rounded quotients of the nonlinear forward in 3 to 6 operations
+// instead of the 11 of the general division (scaling and special cases):
+// a quotient from a reciprocal and one residual correction, Markstein's
+// method ("IA-64 and Elementary Functions", 2000): q = a y, r = a - b q,
+// q + r y, with y = 1/b to the last bit.  Checked on MI355X against the
+// general division for all 2^23 mantissas of the variable operand at 141
+// exponents and 1032 pairs of constants: not one differs.  Outside the normal
+// range the callers see to the operands.
+// a / b for a wave-uniform b with rb = 1/b (rounded to nearest)
+__device__ __forceinline__ float nl_div_by(float a, float b, float rb) {
+  const float q = a * rb;
+  return __builtin_fmaf(__builtin_fmaf(-b, q, a), rb, q);
+}
+// a / b
+__device__ __forceinline__ float nl_div(float a, float b) {
+  float y = __builtin_amdgcn_rcpf(b);
+  y = __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
+  const float q = a * y;
+  return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+}
+// 1 / b
+__device__ __forceinline__ float nl_rcp(float b) {
+  float y = __builtin_amdgcn_rcpf(b);
+  y = __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
+  return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
+}
+
 // One forward step of this thread's segment; REC records lap(u_n) (and u_n
 // for the nonlinear cell) of the output rows through range-checked buffers.
 // UH: grid step 1, where each product with t1 = h^-2 is the value itself and
@@ -67,7 +94,7 @@ __device__ __forceinline__ void cs_fwd_rows(const FwdArgs &a, const float *__res
                                             float (&Uc)[R], float (&Up)[R], const float (&KA)[R],
                                             const float (&KB)[R], const float (&KC)[R],
                                             const float (&KD)[R], int base, int CS,
-                                            uint32_t vmask, __amdgpu_buffer_rsrc_t rsl, __amdgpu_buffer_rsrc_t rsu,
+                                            float ruth, __amdgpu_buffer_rsrc_t rsl, __amdgpu_buffer_rsrc_t rsu,
                                             uint32_t voff, int Ny) {
   const int lfb = base - CS, rtb = base + CS;
   // the row above and, for UH = false, this row times t1
@@ -100,20 +127,18 @@ __device__ __forceinline__ void cs_fwd_rows(const FwdArgs &a, const float *__res
     } else {
       float bb = KA[r], cc = KB[r];
       if (a.nlf & 1) {
-        float q = ct / a.sat_uth;
-        q = fabsf(q);
-        q = q * q;
-        q = q + 1.0f;
-        q = a.sat_b0 / q;
-        bb = bb + KC[r] * q;
+        // b0 / (1 + |u/uth|^2).  1 + q^2 stops at 2^120 (also where u/uth
+        // overflows): b0 over it adds nothing to dt^-2
+        const float q = nl_div_by(ct, a.sat_uth, ruth);
+        const float d = fminf(q * q + 1.0f, 0x1p120f);
+        bb = bb + KC[r] * nl_div(a.sat_b0, d);
       }
       if (a.nlf & 2) cc = cc + KD[r] * (ct * ct);
       if (a.nlf & 4) cc = fminf(fmaxf(cc, a.cmin), a.cmax);
       const float bd = bb * a.dtm1;
-      A = 1.0f / (a.dtm2 + bd);
+      A = nl_rcp(a.dtm2 + bd);
       Bm = a.dtm2 - bd;
       C2 = cc * cc;
-      if (!((vmask >> r) & 1u)) A = 0.0f;
     }
     const float p1 = a.s2 * ct;
     const float p2 = Bm * Up[r];
@@ -222,6 +247,8 @@ __device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
   const int srows = own[tid];
   const bool wave_src = __ballot(srows != 0) != 0;
   const bool one_src = __ballot((srows & (srows - 1)) != 0) == 0;
+  const bool wave_part = __ballot(g.active && vmask != (1u << R) - 1u) != 0;
+  const float ruth = NL ? 1.0f / a.sat_uth : 0.0f;
   const uint32_t voff = cs_out_voff<float>(g, row0, Ny);
   const int64_t out_bytes = (int64_t)(g.or1 - g.or0) * Ny * 4;
   // record slots of this sample; steps at or past its length are not
@@ -254,8 +281,17 @@ __device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
     const __amdgpu_buffer_rsrc_t rsl = cs_rsrc(recl, REC ? rbytes : 0);
     const __amdgpu_buffer_rsrc_t rsu = cs_rsrc(recu, (REC && NL) ? rbytes : 0);
     if (s < live) {
-      cs_fwd_rows<R, NL, REC, UH>(a, P, Q, Uc, Up, KA, KB, KC, KD, g.base, g.CS, vmask, rsl, rsu,
+      cs_fwd_rows<R, NL, REC, UH>(a, P, Q, Uc, Up, KA, KB, KC, KD, g.base, g.CS, ruth, rsl, rsu,
                                   voff, Ny);
+      // rows past the region stay zero (the linear cell has A = 0 there)
+      if (NL && wave_part) {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          if (!((vmask >> r) & 1u)) {
+            Up[r] = 0.0f;
+            Q[g.base + r] = 0.0f;
+          }
+      }
       // v + x_n at the source pixels (source.py:22)
       if (wave_src) cs_add_source<R>(Up, Q + g.base, srows, one_src, xs[s]);
       if (s == snap) {
