@@ -158,57 +158,76 @@ __device__ __forceinline__ void cs_fwd_rows(const FwdArgs &a, const float *__res
 __device__ unsigned long long *wt_phase_ts = nullptr;
 #endif
 
-// Work item w (sample w / ntiles, tile w % ntiles) of the forward launch
-// described by `a`; shared by the single-configuration kernel and the
-// batched kernel (one launch over several configurations; BATCH compiles in
-// the per-sample lengths and record slots).
-template <int NT, int R, int NL, bool REC, bool BATCH, bool UH>
-__device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
-  WT_TS(0);
+// A forward workgroup's tile: its geometry, special pixels and cells.
+template <int R>
+struct CsFwd {
+  CsGeom g;
+  CsTap tap;
+  int b, row0, srows;   // sample, region row of cell 0, source rows (bit mask)
+  uint32_t vmask, voff; // cells inside the region; cs_out_voff
+  bool wave_src, one_src, wave_part;
+  float *buf0, *buf1, *xs;
+  float U0[R], U1[R];                    // u_n, u_{n-1}
+  float KA[R], KB[R], KC[R], KD[R];
+};
+
+// State shared between the workgroups of one launch: accessed at device
+// scope, the eight dies' L2 caches are not coherent for ordinary accesses.
+__device__ __forceinline__ float cs_dev_load(const float *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void cs_dev_store(float *p, float v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Loads tile ti of sample b (state from in1, in2; DEV: shared with other
+// workgroups of this launch) and the input samples n0 .. n0 + nsteps - 1,
+// and fills buf0.  Ends with a barrier.
+template <int R, int NL, bool DEV>
+__device__ __forceinline__ void fwd_cs_setup(const FwdArgs &a, CsFwd<R> &S, int b, int ti,
+                                             const float *in1, const float *in2, int n0,
+                                             int nsteps) {
   extern __shared__ float smem[];
   const int tid = threadIdx.x;
-  const int b = w / a.ntiles, ti = w - (w / a.ntiles) * a.ntiles;
-  // a sample whose own length ends before this launch has nothing to do (a
-  // recording launch too: the adjoint reads no record of a step at or past
-  // the sample's length)
-  if (BATCH && a.Tlim && a.n0 >= a.Tlim[b]) return;
   const int32_t *td = a.tiles + ti * TILE_W;
-  const CsGeom g = cs_geom<R, true>(td, tid);
+  S.b = b;
+  S.g = cs_geom<R, true>(td, tid);
+  const CsGeom &g = S.g;
   const int NBUF = (g.RW + 2) * g.CS;
-  float *buf0 = smem, *buf1 = smem + NBUF;
-  float *xs = smem + 2 * NBUF;  // the input samples of this launch
+  S.buf0 = smem;
+  S.buf1 = smem + NBUF;
+  S.xs = smem + 2 * NBUF;  // the input samples of this launch
   const int Ny = a.Ny;
   const int64_t F = (int64_t)a.Nx * Ny;
   const int64_t boff = (int64_t)b * F;
 
   // source rows of each thread as a bit mask, filled by the table's entries
   // (behind the input samples, in the space sized for the adjoint's seeds)
-  int *own = (int *)(xs + CS_MAX_TBLOCK);
+  int *own = (int *)(S.xs + CS_MAX_TBLOCK);
   const int nsp = min(td[9] - td[8], CS_MAX_TABLE), ntp = min(td[11] - td[10], CS_MAX_TABLE);
 
-  float U0[R], U1[R], KA[R], KB[R], KC[R], KD[R];
-  const int row0 = g.k * R;  // region row of cell 0
-  uint32_t vmask = 0;        // cells that are inside the region
+  const int row0 = S.row0 = g.k * R;
+  S.vmask = 0;
   // 1) all global loads first (one round trip for the whole set-up)
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     float u1 = 0.f, u2 = 0.f, v0 = 0.f, v1 = 0.f, v2 = 0.f, v3 = 0.f;
     if (g.active && row0 + r < g.RH) {
-      vmask |= 1u << r;
+      S.vmask |= 1u << r;
       const int64_t q = (int64_t)(g.R0 + row0 + r) * Ny + (g.C0 + g.c);
       if (NL == 0) {
         v0 = a.A[q]; v1 = a.Bm[q]; v2 = a.C2[q + (int64_t)b * a.c2_bstride];
       } else {
         v0 = a.bgeom[q]; v1 = a.clin[q]; v2 = a.rho[q]; v3 = a.rhoc[q];
       }
-      u1 = a.in1[boff + q];
-      u2 = a.in2[boff + q];
+      u1 = DEV ? cs_dev_load(in1 + boff + q) : in1[boff + q];
+      u2 = DEV ? cs_dev_load(in2 + boff + q) : in2[boff + q];
     }
-    U0[r] = u1; U1[r] = u2;
-    KA[r] = v0; KB[r] = v1; KC[r] = v2; KD[r] = v3;
+    S.U0[r] = u1; S.U1[r] = u2;
+    S.KA[r] = v0; S.KB[r] = v1; S.KC[r] = v2; S.KD[r] = v3;
   }
   float xsv = 0.0f;
-  if (tid < a.nsteps) xsv = a.x[(int64_t)b * a.T + a.n0 + tid];
+  if (tid < nsteps) xsv = a.x[(int64_t)b * a.T + n0 + tid];
   int spv0 = 0, spv1 = 0, spv2 = 0;
   if (tid < nsp) {
     const int32_t *e = a.spx + (td[8] + tid) * SPX_W;
@@ -217,18 +236,18 @@ __device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
   int te[TAP_W];
   cs_tap_load(a.taps, td[10], ntp, te);
   // 2) LDS (buf0's region cells are filled from U0 below)
-  cs_zero_lds<float>(buf0, buf1, g, ((g.RH + R - 1) / R) * R, NBUF);
+  cs_zero_lds<float>(S.buf0, S.buf1, g, ((g.RH + R - 1) / R) * R, NBUF);
   own[tid] = 0;
   WT_TS(4);
-  if (tid < a.nsteps) xs[tid] = xsv;
+  if (tid < nsteps) S.xs[tid] = xsv;
   // blocks of fewer threads than steps (small grids)
-  for (int i = tid + blockDim.x; i < a.nsteps; i += blockDim.x)
-    xs[i] = a.x[(int64_t)b * a.T + a.n0 + i];
+  for (int i = tid + blockDim.x; i < nsteps; i += blockDim.x)
+    S.xs[i] = a.x[(int64_t)b * a.T + n0 + i];
   __syncthreads();
   WT_TS(5);
   if (g.active) {
 #pragma unroll
-    for (int r = 0; r < R; ++r) buf0[g.base + r] = U0[r];
+    for (int r = 0; r < R; ++r) S.buf0[g.base + r] = S.U0[r];
   }
   // source pixels (multiplicity 1; the host routes pixels shared by several
   // sources to the other kernels) mark the rows of their owners
@@ -243,13 +262,24 @@ __device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
   }
   __syncthreads();
   WT_TS(6);
-  const CsTap tap = cs_tap(g, a.taps, td[10], ntp, te);
-  const int srows = own[tid];
-  const bool wave_src = __ballot(srows != 0) != 0;
-  const bool one_src = __ballot((srows & (srows - 1)) != 0) == 0;
-  const bool wave_part = __ballot(g.active && vmask != (1u << R) - 1u) != 0;
+  S.tap = cs_tap(g, a.taps, td[10], ntp, te);
+  S.srows = own[tid];
+  S.wave_src = __ballot(S.srows != 0) != 0;
+  S.one_src = __ballot((S.srows & (S.srows - 1)) != 0) == 0;
+  S.wave_part = __ballot(g.active && S.vmask != (1u << R) - 1u) != 0;
+  S.voff = cs_out_voff<float>(g, row0, Ny);
+}
+
+// Steps n0 .. n0 + nsteps - 1 of the tile: after an even number of them u_n is
+// in U0 and buf0, u_{n-1} in U1, after an odd number the other way round.
+template <int R, int NL, bool REC, bool BATCH, bool UH>
+__device__ __forceinline__ void fwd_cs_steps(const FwdArgs &a, CsFwd<R> &S, int n0, int nsteps) {
+  const CsGeom &g = S.g;
+  const CsTap &tap = S.tap;
+  const int b = S.b, Ny = a.Ny;
+  const int64_t F = (int64_t)a.Nx * Ny;
+  const uint32_t voff = S.voff;
   const float ruth = NL ? 1.0f / a.sat_uth : 0.0f;
-  const uint32_t voff = cs_out_voff<float>(g, row0, Ny);
   const int64_t out_bytes = (int64_t)(g.or1 - g.or0) * Ny * 4;
   // record slots of this sample; steps at or past its length are not
   // recorded (empty slice: the stores are dropped)
@@ -259,41 +289,41 @@ __device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
 
   // What a step needs beyond its rows is a pointer that moves: the per-step
   // address arithmetic of every wave is on the path between two barriers.
-  const int live = cs_live_steps<R>(g, row0, a.nsteps);
-  const float *recl = REC ? a.rec_lap + (rslot0 + (a.n0 - a.rec_n0)) * F + (int64_t)g.or0 * Ny
+  const int live = cs_live_steps<R>(g, S.row0, nsteps);
+  const float *recl = REC ? a.rec_lap + (rslot0 + (n0 - a.rec_n0)) * F + (int64_t)g.or0 * Ny
                           : a.in1;
-  const float *recu = (REC && NL) ? a.rec_u + (rslot0 + (a.n0 - a.rec_n0)) * F +
+  const float *recu = (REC && NL) ? a.rec_u + (rslot0 + (n0 - a.rec_n0)) * F +
                                         (int64_t)g.or0 * Ny
                                   : a.in1;
-  const int64_t yo = ((int64_t)b * a.T + a.n0) * a.ntap + tap.pcol;
+  const int64_t yo = ((int64_t)b * a.T + n0) * a.ntap + tap.pcol;
   float *yp = a.y ? a.y + yo : nullptr, *yrp = a.yraw ? a.yraw + yo : nullptr;
   // next snapshot: at step `snap`, written by the threads from their registers
-  int snap = a.fields ? a.fstride - 1 - a.n0 % a.fstride : -1;
+  int snap = a.fields ? a.fstride - 1 - n0 % a.fstride : -1;
   const float *fp = a.fields ? a.fields +
-                                   ((int64_t)b * (a.T / a.fstride) + a.n0 / a.fstride) * F +
+                                   ((int64_t)b * (a.T / a.fstride) + n0 / a.fstride) * F +
                                    (int64_t)g.or0 * Ny
                              : a.in1;
 
   auto step = [&](const float *P, float *Q, float(&Uc)[R], float(&Up)[R], int s) {
     // the (sample, step) slice of the record, based at the first output row;
     // steps at or past the sample's length: an empty slice
-    const int64_t rbytes = (!BATCH || a.n0 + s < Lb) ? out_bytes : 0;
+    const int64_t rbytes = (!BATCH || n0 + s < Lb) ? out_bytes : 0;
     const __amdgpu_buffer_rsrc_t rsl = cs_rsrc(recl, REC ? rbytes : 0);
     const __amdgpu_buffer_rsrc_t rsu = cs_rsrc(recu, (REC && NL) ? rbytes : 0);
     if (s < live) {
-      cs_fwd_rows<R, NL, REC, UH>(a, P, Q, Uc, Up, KA, KB, KC, KD, g.base, g.CS, ruth, rsl, rsu,
-                                  voff, Ny);
+      cs_fwd_rows<R, NL, REC, UH>(a, P, Q, Uc, Up, S.KA, S.KB, S.KC, S.KD, g.base, g.CS, ruth,
+                                  rsl, rsu, voff, Ny);
       // rows past the region stay zero (the linear cell has A = 0 there)
-      if (NL && wave_part) {
+      if (NL && S.wave_part) {
 #pragma unroll
         for (int r = 0; r < R; ++r)
-          if (!((vmask >> r) & 1u)) {
+          if (!((S.vmask >> r) & 1u)) {
             Up[r] = 0.0f;
             Q[g.base + r] = 0.0f;
           }
       }
       // v + x_n at the source pixels (source.py:22)
-      if (wave_src) cs_add_source<R>(Up, Q + g.base, srows, one_src, xs[s]);
+      if (S.wave_src) cs_add_source<R>(Up, Q + g.base, S.srows, S.one_src, S.xs[s]);
       if (s == snap) {
         const __amdgpu_buffer_rsrc_t rf = cs_rsrc(fp, out_bytes);
 #pragma unroll
@@ -322,24 +352,41 @@ __device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
 
   WT_TS(1);
   int s = 0;
-  for (; s + 1 < a.nsteps; s += 2) {
-    step(buf0, buf1, U0, U1, s);
-    step(buf1, buf0, U1, U0, s + 1);
+  for (; s + 1 < nsteps; s += 2) {
+    step(S.buf0, S.buf1, S.U0, S.U1, s);
+    step(S.buf1, S.buf0, S.U1, S.U0, s + 1);
   }
-  if (s < a.nsteps) step(buf0, buf1, U0, U1, s);
+  if (s < nsteps) step(S.buf0, S.buf1, S.U0, S.U1, s);
   WT_TS(2);
-  // final state: after an even number of steps u_n is in U0, u_{n-1} in U1
+}
+
+// Work item w (sample w / ntiles, tile w % ntiles) of the forward launch
+// described by `a`; shared by the single-configuration kernel and the
+// batched kernel (one launch over several configurations; BATCH compiles in
+// the per-sample lengths and record slots).
+template <int NT, int R, int NL, bool REC, bool BATCH, bool UH>
+__device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
+  WT_TS(0);
+  const int b = w / a.ntiles, ti = w - (w / a.ntiles) * a.ntiles;
+  // a sample whose own length ends before this launch has nothing to do (a
+  // recording launch too: the adjoint reads no record of a step at or past
+  // the sample's length)
+  if (BATCH && a.Tlim && a.n0 >= a.Tlim[b]) return;
+  CsFwd<R> S;
+  fwd_cs_setup<R, NL, false>(a, S, b, ti, a.in1, a.in2, a.n0, a.nsteps);
+  fwd_cs_steps<R, NL, REC, BATCH, UH>(a, S, a.n0, a.nsteps);
+  const CsGeom &g = S.g;
   const bool odd = (a.nsteps & 1) != 0;
   if (g.active) {
     const int gc = g.C0 + g.c;
     if (gc >= g.oc0 && gc < g.oc1) {
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        const int gr = g.R0 + row0 + r;
-        if (row0 + r < g.RH && gr >= g.or0 && gr < g.or1) {
-          const int64_t q = boff + (int64_t)gr * Ny + gc;
-          a.out1[q] = odd ? U1[r] : U0[r];
-          a.out2[q] = odd ? U0[r] : U1[r];
+        const int gr = g.R0 + S.row0 + r;
+        if (S.row0 + r < g.RH && gr >= g.or0 && gr < g.or1) {
+          const int64_t q = (int64_t)b * a.Nx * a.Ny + (int64_t)gr * a.Ny + gc;
+          a.out1[q] = odd ? S.U1[r] : S.U0[r];
+          a.out2[q] = odd ? S.U0[r] : S.U1[r];
         }
       }
     }
@@ -350,6 +397,250 @@ __device__ __forceinline__ void fwd_cs_body(const FwdArgs &a, const int w) {
 template <int NT, int R, int NL, bool REC, bool UH = true>
 __global__ __launch_bounds__(NT) void k_fwd_cs(FwdArgs a) {
   fwd_cs_body<NT, R, NL, REC, false, UH>(a, xcd_remap(blockIdx.x, gridDim.x));
+}
+
+// The resident forward: one launch walks all T steps in chunks of a.nsteps,
+// each workgroup with its own tile, whose cells and coefficients stay in its
+// registers.  Between two chunks only the halo is read again, from the state
+// that the neighbours stored: that exchange takes about 3 us (the stores'
+// and the flag's way to the memory side, a poll, the halo loads), a launch
+// and its set-up 6 to 10 us (1024 x 1024, one sample, 18-step chunks of 256
+// tiles: 5016 us per 4000 steps with a launch per chunk, 3968 us resident;
+// 141 x 141, 24 samples, 1501 steps: 1064 to 880 us).
+//
+// Word w of a.prog (CS_WALK_W ints apart, zero at the start) holds 1 + the
+// chunks that work item w's owner has done, 0 while it has no owner.  Chunk n
+// starts when every tile whose output reaches into this region has n chunks
+// done; tiles reach into each other mutually, so these are then also past
+// reading the state that chunk n overwrites (two pairs of fields alternate).
+// A workgroup raises its word when all of its stores have completed.
+//
+// The device holds all workgroups of such a launch at once, but nothing
+// relies on it (another stream's work may hold compute units): a workgroup
+// that waits for a tile without an owner takes the tile over after
+// CS_WALK_US, and an owner of several works on the one with the fewest
+// chunks.  So the least advanced of all tiles has an owner that works on it,
+// or a neighbour that will take it, or none that waits for it while its own
+// workgroup is still to start; every wait ends.
+constexpr int CS_WALK_US = 50;
+
+// A value the compiler knows nothing about: what is derived from it per row
+// is formed where it is used.  (Of loop-invariant row predicates and offsets
+// it keeps one pair of scalar registers each, and spills 100 of them.)
+template <typename T>
+__device__ __forceinline__ T cs_opaque(T v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+// First wave: waits until the tiles of sample b in `nbr` (bit q of lane l:
+// tile l + 64 q) have n chunks done.  -1: they have; -2: given up after about
+// a minute; else the work item without an owner that was taken over.
+__device__ __forceinline__ int cs_walk_wait(int *prog, int ntiles, int b, int nbr, int n) {
+  const int lane = threadIdx.x;
+  const uint64_t t0 = wall_clock64();
+  for (int polls = 0; polls < (1 << 26); ++polls) {
+    bool ok = true;
+    int unowned = -1;
+#pragma unroll
+    for (int q = 0; q < CS_WALK_MAX / 64; ++q)
+      if ((nbr >> q) & 1) {
+        const int j = b * ntiles + lane + 64 * q;
+        const int v = __hip_atomic_load(prog + j * CS_WALK_W, __ATOMIC_RELAXED,
+                                        __HIP_MEMORY_SCOPE_AGENT);
+        if (v < n + 1) ok = false;
+        if (v == 0) unowned = j;
+      }
+    if (__ballot(!ok) == 0) return -1;
+    const uint64_t cand = __ballot(unowned >= 0);
+    if (cand && wall_clock64() - t0 > 100 * CS_WALK_US) {  // the clock runs at 100 MHz
+      const int first = __ffsll((unsigned long long)cand) - 1;
+      int got = -1;
+      if (lane == first && atomicCAS(prog + unowned * CS_WALK_W, 0, 1) == 0) got = unowned;
+      got = __shfl(got, first);
+      if (got >= 0) return got;
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+  return -2;
+}
+
+// First wave: the tiles whose output rows and columns reach into tile ti's
+// region, as cs_walk_wait takes them.
+__device__ __forceinline__ int cs_walk_neighbours(const FwdArgs &a, int ti) {
+  const int32_t *td = a.tiles + ti * TILE_W;
+  int nbr = 0;
+#pragma unroll
+  for (int q = 0; q < CS_WALK_MAX / 64; ++q) {
+    const int j = threadIdx.x + 64 * q;
+    if (j < a.ntiles && j != ti) {
+      const int32_t *o = a.tiles + j * TILE_W;
+      if (o[4] < td[0] + td[1] && o[5] > td[0] && o[6] < td[2] + td[3] && o[7] > td[2])
+        nbr |= 1 << q;
+    }
+  }
+  return nbr;
+}
+
+// This thread's output rows of the tile, and its first cell.
+template <int R>
+__device__ __forceinline__ uint32_t cs_walk_out(const FwdArgs &a, const CsFwd<R> &S, int64_t &q0) {
+  const CsGeom &g = S.g;
+  uint32_t m = 0;
+  if (S.voff != 0x80000000u) {
+    const int lo = max(g.or0 - g.R0 - S.row0, 0), hi = min(g.or1 - g.R0 - S.row0, R);
+    if (hi > lo) m = ((1u << hi) - 1u) & ~((1u << lo) - 1u) & S.vmask;
+  }
+  q0 = ((int64_t)S.b * a.Nx + g.R0 + S.row0) * a.Ny + g.C0 + g.c;
+  return m;
+}
+
+// After chunk `chunk` (of nsteps steps): u_n to U0, and the output rows to
+// the state pair that the next chunk reads; then the work item's word.
+template <int R>
+__device__ __forceinline__ void cs_walk_store(const FwdArgs &a, CsFwd<R> &S, int w, int chunk,
+                                              int nsteps, uint32_t omask, int64_t q0) {
+  if (nsteps & 1) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const float u = S.U0[r];
+      S.U0[r] = S.U1[r];
+      S.U1[r] = u;
+    }
+  }
+  const int64_t BF = (int64_t)a.B * a.Nx * a.Ny;
+  float *o1 = a.out1 + (chunk & 1) * 2 * BF, *o2 = o1 + BF;
+  const uint32_t out = cs_opaque(omask);
+  int64_t q = cs_opaque(q0);
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if ((out >> r) & 1u) {
+      cs_dev_store(o1 + q, S.U0[r]);
+      cs_dev_store(o2 + q, S.U1[r]);
+    }
+    q += a.Ny;
+  }
+  // every wave's stores completed, then the word
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0)
+    __hip_atomic_store(a.prog + w * CS_WALK_W, 2 + chunk, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The wait of a workgroup was given up: probe outputs from step n0 on are NaN.
+__device__ __forceinline__ void cs_walk_failed(const FwdArgs &a, int b, int n0) {
+  const float nan = __builtin_nanf("");
+  for (int64_t i = (int64_t)n0 * a.ntap + threadIdx.x; i < (int64_t)a.T * a.ntap;
+       i += blockDim.x) {
+    if (a.y) a.y[(int64_t)b * a.T * a.ntap + i] = nan;
+    if (a.yraw) a.yraw[(int64_t)b * a.T * a.ntap + i] = nan;
+  }
+}
+
+template <int NT, int R, int NL, bool REC, bool UH>
+__global__ __launch_bounds__(NT) void k_fwd_cs_walk(FwdArgs a) {
+  const int tid = threadIdx.x;
+  const int64_t BF = (int64_t)a.B * a.Nx * a.Ny;
+  const int nchunks = (a.T + a.nsteps - 1) / a.nsteps;
+  __shared__ int msg;
+  int w = xcd_remap(blockIdx.x, gridDim.x);
+  if (tid == 0) msg = atomicCAS(a.prog + w * CS_WALK_W, 0, 1);
+  __syncthreads();
+  if (msg != 0) return;  // a neighbour took it over
+  CsFwd<R> S;
+  int64_t q0;
+  int chunk = 0, got;
+  {
+    const int b = w / a.ntiles, ti = w - b * a.ntiles;
+    const int nbr = tid < 64 ? cs_walk_neighbours(a, ti) : 0;
+    fwd_cs_setup<R, NL, true>(a, S, b, ti, a.in1, a.in2, 0, min(a.nsteps, a.T));
+    const uint32_t omask = cs_walk_out<R>(a, S, q0);
+    while (true) {
+      const int n0 = chunk * a.nsteps, nsteps = min(a.nsteps, a.T - n0);
+      fwd_cs_steps<R, NL, REC, false, UH>(a, S, n0, nsteps);
+      if (chunk + 1 == nchunks) return;
+      cs_walk_store<R>(a, S, w, chunk, nsteps, omask, q0);
+      ++chunk;
+      const int n1 = n0 + nsteps;
+      for (int i = tid; i < min(a.nsteps, a.T - n1); i += blockDim.x)
+        S.xs[i] = a.x[(int64_t)b * a.T + n1 + i];
+      if (tid < 64) {
+        const int r = cs_walk_wait(a.prog, a.ntiles, b, nbr, chunk);
+        if (tid == 0) msg = r;
+      }
+      __syncthreads();
+      got = msg;
+      if (got != -1) break;
+      const float *in1 = a.out1 + ((chunk - 1) & 1) * 2 * BF, *in2 = in1 + BF;
+      const uint32_t halo = cs_opaque(S.vmask & ~omask);
+      int64_t q = cs_opaque(q0);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        if ((halo >> r) & 1u) {
+          S.U0[r] = cs_dev_load(in1 + q);
+          S.U1[r] = cs_dev_load(in2 + q);
+        }
+        q += a.Ny;
+      }
+      if (S.g.active) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) S.buf0[S.g.base + r] = S.U0[r];
+      }
+      __syncthreads();
+    }
+  }
+  // Work items taken over: from here on every chunk of this workgroup starts
+  // with a whole set-up.
+  __shared__ int own_w[CS_WALK_MAX], own_n[CS_WALK_MAX];
+  int nown = 1, at = 0;
+  while (true) {
+    // -1: run the chunk that was waited for; >= 0: one more work item
+    if (got == -2) {
+      cs_walk_failed(a, w / a.ntiles, chunk * a.nsteps);
+      return;
+    }
+    if (got >= 0) {
+      if (tid == 0) {
+        own_w[at] = w;
+        own_n[at] = chunk;
+        own_w[nown] = got;
+        own_n[nown] = 0;
+      }
+      ++nown;
+    } else {
+      const int n0 = chunk * a.nsteps, nsteps = min(a.nsteps, a.T - n0);
+      const float *in1 = chunk ? a.out1 + ((chunk - 1) & 1) * 2 * BF : a.in1;
+      fwd_cs_setup<R, NL, true>(a, S, w / a.ntiles, w % a.ntiles, in1, in1 + BF, n0, nsteps);
+      const uint32_t omask = cs_walk_out<R>(a, S, q0);
+      fwd_cs_steps<R, NL, REC, false, UH>(a, S, n0, nsteps);
+      cs_walk_store<R>(a, S, w, chunk, nsteps, omask, q0);
+      ++chunk;
+      if (chunk == nchunks && --nown == 0) return;
+      if (tid == 0) {
+        own_n[at] = chunk;
+        if (chunk == nchunks) {
+          own_w[at] = own_w[nown];
+          own_n[at] = own_n[nown];
+        }
+      }
+    }
+    __syncthreads();
+    at = 0;  // the least advanced one next
+    for (int i = 1; i < nown; ++i)
+      if (own_n[i] < own_n[at]) at = i;
+    w = own_w[at];
+    chunk = own_n[at];
+    if (tid < 64) {
+      const int ti = w % a.ntiles;
+      const int r = chunk > 0 ? cs_walk_wait(a.prog, a.ntiles, w / a.ntiles,
+                                             cs_walk_neighbours(a, ti), chunk)
+                              : -1;
+      if (tid == 0) msg = r;
+    }
+    __syncthreads();
+    got = msg;
+  }
 }
 
 // Group of a batched launch that work item w belongs to.
@@ -939,6 +1230,32 @@ static hipError_t cs_fwd_dispatch(bool unit_h, int nl, bool rec, const FwdArgs &
 }
 
 template <int NT, int R>
+static hipError_t cs_walk_dispatch(bool unit_h, int nl, bool rec, const FwdArgs &a, int nblocks,
+                                   int nthreads, size_t shmem, hipStream_t s) {
+#define FT(NL, REC, UH)                                                               \
+  do {                                                                                \
+    auto kfn = k_fwd_cs_walk<NT, R, NL, REC, UH>;                                      \
+    static std::atomic<uint64_t> done{0};                                             \
+    hipError_t e = allow_dyn_lds((const void *)kfn, done);                            \
+    if (e != hipSuccess) return e;                                                    \
+    hipLaunchKernelGGL(kfn, dim3(nblocks), dim3(nthreads), shmem, s, a);              \
+  } while (0)
+  if (nl == 0) {
+    if (unit_h) {
+      if (rec) FT(0, true, true); else FT(0, false, true);
+    } else {
+      if (rec) FT(0, true, false); else FT(0, false, false);
+    }
+  } else if (unit_h) {
+    if (rec) FT(8, true, true); else FT(8, false, true);
+  } else {
+    if (rec) FT(8, true, false); else FT(8, false, false);
+  }
+#undef FT
+  return hipGetLastError();
+}
+
+template <int NT, int R>
 static hipError_t cs_adj_dispatch(const AdjArgs &a, int nblocks, int nthreads, size_t shmem,
                                   hipStream_t s) {
   auto kfn = k_adj_cs<NT, R>;
@@ -960,6 +1277,21 @@ hipError_t launch_fwd_cs(int nt, int R, bool unit_h, int nl, bool rec, const Fwd
 #define X(A, B) \
   if (nt == A && R == B)                                                                \
     return cs_fwd_dispatch<A, B>(unit_h, nl, rec, a, nblocks, nthreads, shmem, s);
+  WT_CS_VARIANTS(X)
+#undef X
+  return hipErrorInvalidValue;
+}
+
+hipError_t launch_fwd_cs_walk(int nt, int R, bool unit_h, int nl, bool rec, const FwdArgs &a,
+                              int RHmax, int RWmax, hipStream_t s) {
+  int nblocks = a.B * a.ntiles;
+  size_t shmem = cs_shmem_bytes(R, RHmax, RWmax, true);
+  int nthreads = cs_threads(R, RHmax, RWmax);
+  if (shmem + CS_STATIC_LDS > (size_t)cs_max_dyn_lds() || nthreads > nt || nblocks > CS_WALK_MAX)
+    return hipErrorInvalidConfiguration;
+#define X(A, B) \
+  if (nt == A && R == B)                                                                \
+    return cs_walk_dispatch<A, B>(unit_h, nl, rec, a, nblocks, nthreads, shmem, s);
   WT_CS_VARIANTS(X)
 #undef X
   return hipErrorInvalidValue;

@@ -114,7 +114,13 @@ struct FwdArgs {
   // the C2 field between samples (0 = one field shared by the batch)
   const int32_t *Tlim;
   int c2_bstride;
+  // resident launch: progress words (B * ntiles, CS_WALK_W ints apart);
+  // out1 then starts two alternating state pairs, n0 is 0 and nsteps the
+  // steps of a chunk
+  int *prog;
 };
+constexpr int CS_WALK_MAX = 256;  // work items of a resident launch, at most
+constexpr int CS_WALK_W = 16;     // ints between its progress words
 
 // Arguments of the fused adjoint kernel (row strips only: C0 = 0, RW = Ny).
 struct AdjArgs {
@@ -262,6 +268,19 @@ int hip_fail(hipError_t e, const char *what);
 hipError_t launch_fill64(double *p, int64_t n, double v, hipStream_t s);
 hipError_t launch_finalize_gx64(const double *gsrc, int B, int T, int nslot, const int32_t *mult,
                                 double *gx, hipStream_t s);
+
+// Compute units of the current device (cached per device id below 64).
+inline int device_cus() {
+  static std::atomic<int> cache[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) dev = 0;
+  const bool slot = dev >= 0 && dev < 64;
+  int v = slot ? cache[dev].load(std::memory_order_relaxed) : 0;
+  if (v > 0) return v;
+  if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) v = 0;
+  if (slot && v > 0) cache[dev].store(v, std::memory_order_relaxed);
+  return v;
+}
 
 // Largest dynamic LDS a workgroup may request on the current device (cached
 // per device id below 64).

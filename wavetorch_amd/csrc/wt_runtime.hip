@@ -92,6 +92,8 @@ size_t cs_shmem_bytes(int R, int RH, int RW, bool padded);
 int cs_threads(int R, int RH, int RW);
 hipError_t launch_fwd_cs(int nt, int R, bool unit_h, int nl, bool rec, const FwdArgs &a,
                          int RHmax, int RWmax, hipStream_t s);
+hipError_t launch_fwd_cs_walk(int nt, int R, bool unit_h, int nl, bool rec, const FwdArgs &a,
+                              int RHmax, int RWmax, hipStream_t s);
 hipError_t launch_adj_cs(int nt, int R, const AdjArgs &a, int RHmax, int RWmax, hipStream_t s);
 size_t cs64_shmem_bytes(int R, int RH, int RW, int tb);
 bool cs64_variant_exists(int R, bool fwd);
@@ -1370,6 +1372,16 @@ FwdArgs base_fwd(const Plan &p, const Ws &w, const float *b, const float *c, con
   return a;
 }
 
+// Whether a whole forward of this plan runs as one resident launch: more than
+// one chunk, a workgroup for each CU at most, and progress words that fit one
+// state buffer.
+bool walks(const Plan &p) {
+  const int64_t items = (int64_t)p.B * p.ntiles;
+  return p.tiled && p.tun.kind == 0 && p.T > p.tun.tblock &&
+         items <= std::min(CS_WALK_MAX, device_cus()) &&
+         items * CS_WALK_W <= (int64_t)p.B * (int64_t)p.F;
+}
+
 // Runs forward steps [n0, n1) from the state (in1, in2) = (u_n0, u_{n0-1}).
 // Tiled: launches of tblock steps; the first reads (in1, in2), intermediate
 // states ping-pong through tmp[0..3], and the last launch writes (out1, out2)
@@ -1595,6 +1607,32 @@ int wt_loop_fwd(void *plan, const float *b, const float *c, const float *rho, co
   // (rnn.py:39-41) lives in checkpoint 0 when recording.
   float *tmp[4] = {bufs[0], bufs[1], bufs[2], bufs[3]};
   float *z = with_grad ? w.ck : bufs[4];
+  const bool rec = with_grad && w.rec;
+  if (walks(*p) && (!with_grad || (rec && p->nseg == 1))) {
+    // the progress words take the state buffer after the (non-recording
+    // call's) zero state: one fill for both
+    const int64_t words = (int64_t)p->B * p->ntiles * CS_WALK_W;
+    if (with_grad) {
+      WT_HIP(launch_fill(z, 2 * BF, 0.0f, s));
+      WT_HIP(launch_fill(bufs[6], words, 0.0f, s));
+    } else {
+      WT_HIP(launch_fill(z, 2 * BF + words, 0.0f, s));
+    }
+    a.in1 = z;
+    a.in2 = z + BF;
+    a.out1 = bufs[0];
+    a.nsteps = p->tun.tblock;
+    a.prog = (int *)bufs[6];
+    if (rec) {
+      a.rec_lap = w.rec;
+      a.rec_u = p->nl ? w.rec + (size_t)p->B * p->K * p->Nx * (p->Ny + 1) : nullptr;
+      a.rec_K = p->K;
+    }
+    ProfScope ps(0, s, (int64_t)p->B * p->Nx * p->Ny * p->T);
+    WT_HIP(launch_fwd_cs_walk(p->tun.nt, p->tun.cpt, p->unit_h, p->nl, rec, a, p->RHmax,
+                              p->RWmax, s));
+    return WT_OK;
+  }
   WT_HIP(launch_fill(z, 2 * BF, 0.0f, s));
   const float *cur1 = z, *cur2 = z + BF;
   for (int sg = 0; sg < p->nseg; ++sg) {
