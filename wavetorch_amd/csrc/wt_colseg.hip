@@ -53,6 +53,15 @@ __device__ __forceinline__ void cs_rec_store(__amdgpu_buffer_rsrc_t rs, uint32_t
                                         WT_RECORD_STORE_CPOL);
 }
 
+// A value the compiler knows nothing about: what is derived from it per row
+// is formed where it is used.  (Of loop-invariant row predicates and offsets
+// it keeps one pair of scalar registers each, and spills 100 of them.)
+template <typename T>
+__device__ __forceinline__ T cs_opaque(T v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
 // ------------------------------------------------------------------ forward
 
 // Correctly rounded quotients of the nonlinear forward in 3 to 6 operations
@@ -424,20 +433,12 @@ __global__ __launch_bounds__(NT) void k_fwd_cs(FwdArgs a) {
 // workgroup is still to start; every wait ends.
 constexpr int CS_WALK_US = 50;
 
-// A value the compiler knows nothing about: what is derived from it per row
-// is formed where it is used.  (Of loop-invariant row predicates and offsets
-// it keeps one pair of scalar registers each, and spills 100 of them.)
-template <typename T>
-__device__ __forceinline__ T cs_opaque(T v) {
-  asm volatile("" : "+v"(v));
-  return v;
-}
-
 // First wave: waits until the tiles of sample b in `nbr` (bit q of lane l:
 // tile l + 64 q) have n chunks done.  -1: they have; -2: given up after about
 // a minute; else the work item without an owner that was taken over.
 __device__ __forceinline__ int cs_walk_wait(int *prog, int ntiles, int b, int nbr, int n) {
-  const int lane = threadIdx.x;
+  const int lane = cs_opaque((int)threadIdx.x);
+  nbr = cs_opaque(nbr);
   const uint64_t t0 = wall_clock64();
   for (int polls = 0; polls < (1 << 26); ++polls) {
     bool ok = true;
@@ -467,14 +468,14 @@ __device__ __forceinline__ int cs_walk_wait(int *prog, int ntiles, int b, int nb
 
 // First wave: the tiles whose output rows and columns reach into tile ti's
 // region, as cs_walk_wait takes them.
-__device__ __forceinline__ int cs_walk_neighbours(const FwdArgs &a, int ti) {
-  const int32_t *td = a.tiles + ti * TILE_W;
+__device__ __forceinline__ int cs_walk_neighbours(const int32_t *tiles, int ntiles, int ti) {
+  const int32_t *td = tiles + ti * TILE_W;
   int nbr = 0;
 #pragma unroll
   for (int q = 0; q < CS_WALK_MAX / 64; ++q) {
     const int j = threadIdx.x + 64 * q;
-    if (j < a.ntiles && j != ti) {
-      const int32_t *o = a.tiles + j * TILE_W;
+    if (j < ntiles && j != ti) {
+      const int32_t *o = tiles + j * TILE_W;
       if (o[4] < td[0] + td[1] && o[5] > td[0] && o[6] < td[2] + td[3] && o[7] > td[2])
         nbr |= 1 << q;
     }
@@ -495,17 +496,17 @@ __device__ __forceinline__ uint32_t cs_walk_out(const FwdArgs &a, const CsFwd<R>
   return m;
 }
 
-// After chunk `chunk` (of nsteps steps): u_n to U0, and the output rows to
-// the state pair that the next chunk reads; then the work item's word.
-template <int R>
-__device__ __forceinline__ void cs_walk_store(const FwdArgs &a, CsFwd<R> &S, int w, int chunk,
-                                              int nsteps, uint32_t omask, int64_t q0) {
+// After chunk `chunk` (of nsteps steps): the later state to V0, and the output
+// rows to the state pair that the next chunk reads; then the work item's word.
+template <int R, typename Args>
+__device__ __forceinline__ void cs_walk_store(const Args &a, float (&V0)[R], float (&V1)[R], int w,
+                                              int chunk, int nsteps, uint32_t omask, int64_t q0) {
   if (nsteps & 1) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const float u = S.U0[r];
-      S.U0[r] = S.U1[r];
-      S.U1[r] = u;
+      const float u = V0[r];
+      V0[r] = V1[r];
+      V1[r] = u;
     }
   }
   const int64_t BF = (int64_t)a.B * a.Nx * a.Ny;
@@ -515,8 +516,8 @@ __device__ __forceinline__ void cs_walk_store(const FwdArgs &a, CsFwd<R> &S, int
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     if ((out >> r) & 1u) {
-      cs_dev_store(o1 + q, S.U0[r]);
-      cs_dev_store(o2 + q, S.U1[r]);
+      cs_dev_store(o1 + q, V0[r]);
+      cs_dev_store(o2 + q, V1[r]);
     }
     q += a.Ny;
   }
@@ -553,14 +554,14 @@ __global__ __launch_bounds__(NT) void k_fwd_cs_walk(FwdArgs a) {
   int chunk = 0, got;
   {
     const int b = w / a.ntiles, ti = w - b * a.ntiles;
-    const int nbr = tid < 64 ? cs_walk_neighbours(a, ti) : 0;
+    const int nbr = tid < 64 ? cs_walk_neighbours(a.tiles, a.ntiles, ti) : 0;
     fwd_cs_setup<R, NL, true>(a, S, b, ti, a.in1, a.in2, 0, min(a.nsteps, a.T));
     const uint32_t omask = cs_walk_out<R>(a, S, q0);
     while (true) {
       const int n0 = chunk * a.nsteps, nsteps = min(a.nsteps, a.T - n0);
       fwd_cs_steps<R, NL, REC, false, UH>(a, S, n0, nsteps);
       if (chunk + 1 == nchunks) return;
-      cs_walk_store<R>(a, S, w, chunk, nsteps, omask, q0);
+      cs_walk_store<R>(a, S.U0, S.U1, w, chunk, nsteps, omask, q0);
       ++chunk;
       const int n1 = n0 + nsteps;
       for (int i = tid; i < min(a.nsteps, a.T - n1); i += blockDim.x)
@@ -614,7 +615,7 @@ __global__ __launch_bounds__(NT) void k_fwd_cs_walk(FwdArgs a) {
       fwd_cs_setup<R, NL, true>(a, S, w / a.ntiles, w % a.ntiles, in1, in1 + BF, n0, nsteps);
       const uint32_t omask = cs_walk_out<R>(a, S, q0);
       fwd_cs_steps<R, NL, REC, false, UH>(a, S, n0, nsteps);
-      cs_walk_store<R>(a, S, w, chunk, nsteps, omask, q0);
+      cs_walk_store<R>(a, S.U0, S.U1, w, chunk, nsteps, omask, q0);
       ++chunk;
       if (chunk == nchunks && --nown == 0) return;
       if (tid == 0) {
@@ -634,7 +635,7 @@ __global__ __launch_bounds__(NT) void k_fwd_cs_walk(FwdArgs a) {
     if (tid < 64) {
       const int ti = w % a.ntiles;
       const int r = chunk > 0 ? cs_walk_wait(a.prog, a.ntiles, w / a.ntiles,
-                                             cs_walk_neighbours(a, ti), chunk)
+                                             cs_walk_neighbours(a.tiles, a.ntiles, ti), chunk)
                               : -1;
       if (tid == 0) msg = r;
     }
@@ -690,33 +691,44 @@ __device__ __forceinline__ void cs_adj_rows(const float *__restrict__ P, float *
   }
 }
 
-// Linear cell.  LDS holds w*lambda.  Work item w of the launch `a` (BATCH:
-// the batched kernel, with per-sample lengths and record slots).
-template <int NT, int R, bool BATCH>
-__device__ __forceinline__ void adj_cs_body(const AdjArgs &a, const int w) {
-  WT_TS(0);
+// An adjoint workgroup's tile.
+template <int R>
+struct CsAdj {
+  CsGeom g;
+  CsSpecials sp;        // this thread's special pixels
+  int b, row0, Lb;      // sample, region row of cell 0, the sample's length (batches)
+  uint32_t omask, voff; // output rows of this thread; cs_out_voff
+  bool wave_sp, wave_sp2;
+  float kw0, kw1;       // w of the special rows
+  float *buf0, *buf1, *seeds;
+  float L1[R], L2[R];   // lambda_{m+1}, lambda_{m+2}
+  float KA1[R], KW[R];
+  float G[R];           // gradient sum of this launch or chunk
+  float SG0[R], SG1[R]; // lap(u) of its even and odd steps
+};
+
+// Loads tile ti of sample b; DEV: the state is shared with other workgroups of
+// this launch.  `tb_sp`, `seed_px`, `nseeds`: the tile's special pixels in LDS.
+// Ends before the barrier that must follow adj_cs_start.
+template <int R, bool DEV>
+__device__ __forceinline__ void adj_cs_setup(const AdjArgs &a, CsAdj<R> &S, int b, int ti,
+                                             const float *in1, const float *in2, int *tb_sp,
+                                             int *seed_px, int *nseeds) {
   extern __shared__ float smem[];
-  const int tid = threadIdx.x;
-  const int b = w / a.ntiles, ti = w - (w / a.ntiles) * a.ntiles;
-  // lambda_m = 0 for every m of this launch when the sample ends before it
-  if (BATCH && a.Tlim && a.m_hi - a.nsteps + 1 > a.Tlim[b]) return;
   const int32_t *td = a.tiles + ti * TILE_W;
-  const CsGeom g = cs_geom<R>(td, tid);
+  S.b = b;
+  S.g = cs_geom<R>(td, threadIdx.x);
+  const CsGeom &g = S.g;
   const int NBUF = (g.RW + 2) * g.CS;
-  float *buf0 = smem, *buf1 = smem + NBUF;
-  float *seeds = smem + 2 * NBUF;  // (CS_MAX_SEEDS, nsteps) probe seeds
-  __shared__ int seed_px[CS_MAX_SEEDS];
-  __shared__ int nseeds;
+  S.buf0 = smem;
+  S.buf1 = smem + NBUF;
+  S.seeds = smem + 2 * NBUF;  // (CS_MAX_SEEDS, nsteps) probe seeds
   const int Ny = a.Ny;
-  const int64_t F = (int64_t)a.Nx * Ny;
-  const int64_t boff = (int64_t)b * F;
+  const int64_t boff = (int64_t)b * a.Nx * Ny;
   const float s2 = a.s2;
 
-  __shared__ int tb_sp[CS_MAX_TABLE * CS_SP_W];
   const int nsp = min(td[9] - td[8], CS_MAX_TABLE);
-
-  float L1[R], L2[R], KA1[R], KW[R], G[R], SG0[R], SG1[R];
-  const int row0 = g.k * R;
+  const int row0 = S.row0 = g.k * R;
   // 1) all global loads first
   float KC2[R];
 #pragma unroll
@@ -725,42 +737,80 @@ __device__ __forceinline__ void adj_cs_body(const AdjArgs &a, const int w) {
     if (g.active && row0 + r < g.RH) {
       const int64_t q = (int64_t)(g.R0 + row0 + r) * Ny + (g.C0 + g.c);
       A = a.A[q]; C2 = a.C2[q + (int64_t)b * a.c2_bstride];
-      u1 = a.in1[boff + q];
-      u2 = a.in2[boff + q];
+      u1 = DEV ? cs_dev_load(in1 + boff + q) : in1[boff + q];
+      u2 = DEV ? cs_dev_load(in2 + boff + q) : in2[boff + q];
     }
-    KA1[r] = A; KC2[r] = C2;
-    L1[r] = u1; L2[r] = u2;
+    S.KA1[r] = A; KC2[r] = C2;
+    S.L1[r] = u1; S.L2[r] = u2;
   }
   // (the owners' table lies behind the seeds, or under them in launches of
   // more than 128 steps, with a barrier more)
-  int *own = (int *)(seeds + (a.nsteps > 128 ? 0 : 128 * CS_MAX_SEEDS));
+  int *own = (int *)(S.seeds + (a.nsteps > 128 ? 0 : 128 * CS_MAX_SEEDS));
   int spe[CS_SP_W];
   cs_special_load(a.spx, td[8], nsp, spe);
   // 2) LDS (buf0's region cells are filled from the lambda pair below)
-  cs_zero_lds<float>(buf0, buf1, g, ((g.RH + R - 1) / R) * R, NBUF);
+  cs_zero_lds<float>(S.buf0, S.buf1, g, ((g.RH + R - 1) / R) * R, NBUF);
   cs_special_stage(a.spx, td[8], nsp, spe, tb_sp, own);
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const float A = KA1[r];
+    const float A = S.KA1[r];
     // w carries the Laplacian's h^-2 (exactly 1 at h = 1): no step pays for it
-    KA1[r] = A * s2; KW[r] = (A * KC2[r]) * a.t1;
-    G[r] = 0.0f; SG1[r] = 0.0f;
+    S.KA1[r] = A * s2; S.KW[r] = (A * KC2[r]) * a.t1;
   }
   __syncthreads();
-  cs_special_scatter<R>(g, nsp, tb_sp, own, seed_px, &nseeds);
+  cs_special_scatter<R>(g, nsp, tb_sp, own, seed_px, nseeds);
   if (g.active) {
 #pragma unroll
-    for (int r = 0; r < R; ++r) buf0[g.base + r] = KW[r] * L1[r];
+    for (int r = 0; r < R; ++r) S.buf0[g.base + r] = S.KW[r] * S.L1[r];
   }
   __syncthreads();
   // special rows of this thread: probe taps (seed slot) / source pixels (slot)
-  const CsSpecials sp = cs_special_read(g, row0, tb_sp, own);
-  const int sr0 = sp.sr0, sr1 = sp.sr1, sd0 = sp.sd0, sd1 = sp.sd1, sl0 = sp.sl0, sl1 = sp.sl1;
+  S.sp = cs_special_read(g, row0, tb_sp, own);
   if (a.nsteps > 128) __syncthreads();
+  // waves with special pixels, with two in a thread
+  S.wave_sp = __ballot(S.sp.sr0 >= 0) != 0;
+  S.wave_sp2 = __ballot(S.sp.sr1 >= 0) != 0;
+  S.kw0 = cs_pick<R>(S.KW, S.sp.sr0);
+  S.kw1 = cs_pick<R>(S.KW, S.sp.sr1);
+  // output cells of this thread (gradient write-back, dJ/dx)
+  S.omask = 0;
+  if (g.active && g.C0 + g.c >= g.oc0 && g.C0 + g.c < g.oc1) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int gr = g.R0 + row0 + r;
+      if (row0 + r < g.RH && gr >= g.or0 && gr < g.or1) S.omask |= 1u << r;
+    }
+  }
+  S.voff = cs_out_voff<float>(g, row0, Ny);
+}
+
+// Record of step j (read at reverse step m = j + 1): a sample's steps at or
+// past its length are not recorded, and lambda_m is exactly 0 there, so
+// those reads are sent out of range (they return 0).
+template <int R, bool BATCH>
+__device__ __forceinline__ uint32_t adj_cs_rec_off(const CsAdj<R> &S, uint32_t voff, int j) {
+  return (!BATCH || j < S.Lb) ? voff : 0x80000000u;
+}
+// Slice of the record read at reverse step m (the steps below it lie F values
+// before each other).
+template <int R, bool BATCH>
+__device__ __forceinline__ const float *adj_cs_rec(const AdjArgs &a, const CsAdj<R> &S, int m) {
+  const int64_t sslot0 =
+      (BATCH && a.seg_soff) ? (int64_t)a.seg_soff[S.b] : (int64_t)S.b * a.seg_K;
+  return a.seg_lap + (sslot0 + (m - 1 - a.seg_n0)) * ((int64_t)a.Nx * a.Ny) +
+         (int64_t)S.g.or0 * a.Ny;
+}
+
+// What the reverse steps m_hi .. m_hi - nsteps + 1 read besides the state:
+// probe seeds (a barrier must follow) and the record of the first two.
+template <int R, bool BATCH>
+__device__ __forceinline__ void adj_cs_start(const AdjArgs &a, CsAdj<R> &S, int m_hi, int nsteps,
+                                             const int *tb_sp, const int *seed_px, int nseeds) {
+  const int b = S.b, Ny = a.Ny;
   // seeds[k][s] = sum over taps of pixel k of dy/du * ybar at step m = m_hi - s
-  for (int i = tid; i < nseeds * a.nsteps; i += blockDim.x) {
-    const int k = i / a.nsteps, s = i - (i / a.nsteps) * a.nsteps;
-    const int m = a.m_hi - s;
+  for (int i = cs_opaque((int)threadIdx.x); i < nseeds * nsteps; i += blockDim.x) {
+    const int k = i / nsteps, s = i - (i / nsteps) * nsteps;
+    const int m = m_hi - s;
     const int *e = tb_sp + CS_SP_W * seed_px[k];
     float gs = 0.0f;
     if (a.ybar && (!a.Tlim || m - 1 < a.Tlim[b])) {
@@ -771,74 +821,60 @@ __device__ __forceinline__ void adj_cs_body(const AdjArgs &a, const int w) {
         gs += tp[2] ? 2.0f * a.yraw[o] * gy : gy;
       }
     }
-    seeds[i] = gs;
+    S.seeds[i] = gs;
   }
-  // waves with special pixels, with two in a thread
-  const bool wave_sp = __ballot(sr0 >= 0) != 0;
-  const bool wave_sp2 = __ballot(sr1 >= 0) != 0;
-  // output cells of this thread (gradient write-back, dJ/dx)
-  uint32_t omask = 0;
-  if (g.active && g.C0 + g.c >= g.oc0 && g.C0 + g.c < g.oc1) {
+  const int64_t F = (int64_t)a.Nx * Ny, out_bytes = (int64_t)(S.g.or1 - S.g.or0) * Ny * 4;
+  const float *rec0 = adj_cs_rec<R, BATCH>(a, S, m_hi);
+  const uint32_t voff = cs_opaque(S.voff);
+  // lap(u_{m-1}) of the first two steps (SG0: even steps, SG1: odd steps)
+  const __amdgpu_buffer_rsrc_t rs0 = cs_rsrc(rec0, out_bytes);
+  const uint32_t voff0 = adj_cs_rec_off<R, BATCH>(S, voff, m_hi - 1);
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int gr = g.R0 + row0 + r;
-      if (row0 + r < g.RH && gr >= g.or0 && gr < g.or1) omask |= 1u << r;
-    }
-  }
-  const uint32_t voff = cs_out_voff<float>(g, row0, Ny);
-  const int64_t out_bytes = (int64_t)(g.or1 - g.or0) * Ny * 4;
-  // record of step j (read at reverse step m = j + 1): a sample's steps at or
-  // past its length are not recorded, and lambda_m is exactly 0 there, so
-  // those reads are sent out of range (they return 0)
-  const int Lb = (BATCH && a.Tlim) ? a.Tlim[b] : 0x7fffffff;
-  auto rec_off = [&](int j) { return (!BATCH || j < Lb) ? voff : 0x80000000u; };
-  __syncthreads();
+  for (int r = 0; r < R; ++r) S.SG0[r] = cs_rec_load(rs0, voff0 + (uint32_t)(r * Ny * 4));
+  // issued even for a one-step launch (out of range, reads nothing) so
+  // that the loop's wait counts need not cover a path without them
+  const bool two = nsteps > 1;
+  const __amdgpu_buffer_rsrc_t rs1 = cs_rsrc(two ? rec0 - F : rec0, out_bytes);
+  const uint32_t voff1 = two ? adj_cs_rec_off<R, BATCH>(S, voff, m_hi - 2) : 0x80000000u;
+#pragma unroll
+  for (int r = 0; r < R; ++r) S.SG1[r] = cs_rec_load(rs1, voff1 + (uint32_t)(r * Ny * 4));
+#pragma unroll
+  for (int r = 0; r < R; ++r) S.G[r] = 0.0f;
+}
 
-  const int64_t sslot0 =
-      (BATCH && a.seg_soff) ? (int64_t)a.seg_soff[b] : (int64_t)b * a.seg_K;
-  // slice of the record read at reverse step m_hi (the steps below it lie F
-  // values before each other)
-  const float *rec0 =
-      a.seg_lap + (sslot0 + (a.m_hi - 1 - a.seg_n0)) * F + (int64_t)g.or0 * Ny;
-  // lap(u_{m-1}) of the first two steps of this launch (SG0: even steps,
-  // SG1: odd steps)
-  {
-    const __amdgpu_buffer_rsrc_t rs0 = cs_rsrc(rec0, out_bytes);
-    const uint32_t voff0 = rec_off(a.m_hi - 1);
-#pragma unroll
-    for (int r = 0; r < R; ++r) SG0[r] = cs_rec_load(rs0, voff0 + (uint32_t)(r * Ny * 4));
-    // issued even for a one-step launch (out of range, reads nothing) so
-    // that the loop's wait counts need not cover a path without them
-    const bool two = a.nsteps > 1;
-    const __amdgpu_buffer_rsrc_t rs1 = cs_rsrc(two ? rec0 - F : rec0, out_bytes);
-    const uint32_t voff1 = two ? rec_off(a.m_hi - 2) : 0x80000000u;
-#pragma unroll
-    for (int r = 0; r < R; ++r) SG1[r] = cs_rec_load(rs1, voff1 + (uint32_t)(r * Ny * 4));
-  }
-  const int live = cs_live_steps<R>(g, row0, a.nsteps);
-  const float *recp = rec0 - 2 * F;  // the step after next
-  const float kw0 = cs_pick<R>(KW, sr0), kw1 = cs_pick<R>(KW, sr1);
-  const bool gx0 = sl0 >= 0 && sr0 >= 0 && ((omask >> sr0) & 1u);
-  const bool gx1 = sl1 >= 0 && sr1 >= 0 && ((omask >> sr1) & 1u);
-  float *gsrc_row = a.gsrc + ((int64_t)b * a.T + (a.m_hi - 1)) * a.nsrcslot;
+// Reverse steps m_hi .. m_hi - nsteps + 1: after an even number of them the
+// pair (lambda_{m_lo}, lambda_{m_lo + 1}) is (L1, L2), after an odd (L2, L1).
+template <int R, bool BATCH>
+__device__ __forceinline__ void adj_cs_steps(const AdjArgs &a, CsAdj<R> &S, int m_hi, int nsteps) {
+  const CsGeom &g = S.g;
+  const int Ny = a.Ny;
+  const int64_t F = (int64_t)a.Nx * Ny, out_bytes = (int64_t)(g.or1 - g.or0) * Ny * 4;
+  const int live = cs_live_steps<R>(g, S.row0, nsteps);
+  const uint32_t voff = cs_opaque(S.voff);
+  // the step after next
+  const float *recp = adj_cs_rec<R, BATCH>(a, S, m_hi) - 2 * F;
+  const bool gx0 = S.sp.sl0 >= 0 && S.sp.sr0 >= 0 && ((S.omask >> S.sp.sr0) & 1u);
+  const bool gx1 = S.sp.sl1 >= 0 && S.sp.sr1 >= 0 && ((S.omask >> S.sp.sr1) & 1u);
+  float *gsrc_row = a.gsrc + ((int64_t)S.b * a.T + (m_hi - 1)) * a.nsrcslot;
 
-  const float *sd0p = seeds + (sd0 >= 0 ? sd0 * a.nsteps : 0);
-  const float *sd1p = seeds + (sd1 >= 0 ? sd1 * a.nsteps : 0);
+  const float *sd0p = S.seeds + (S.sp.sd0 >= 0 ? S.sp.sd0 * nsteps : 0);
+  const float *sd1p = S.seeds + (S.sp.sd1 >= 0 ? S.sp.sd1 * nsteps : 0);
 
   auto step = [&](const float *P, float *Q, float(&Lc)[R], float(&Ln)[R], float(&SG)[R],
                   int s) {
     // record index m-3-seg_n0 >= 0: m-2 >= m_hi-nsteps+1 >= seg_n0+1
-    const bool prefetch = s + 2 < a.nsteps;
+    const bool prefetch = s + 2 < nsteps;
     const __amdgpu_buffer_rsrc_t rsn = cs_rsrc(recp, out_bytes);
-    const uint32_t pvoff = prefetch ? rec_off(a.m_hi - s - 3) : 0x80000000u;
+    const uint32_t pvoff =
+        prefetch ? adj_cs_rec_off<R, BATCH>(S, voff, m_hi - s - 3) : 0x80000000u;
     if (s < live) {
-      cs_adj_rows<R>(P, Q, Lc, Ln, KA1, KW, g.base, g.CS);
-      if (wave_sp) {
-        cs_adj_special<R>(Ln, Q + g.base, sr0, kw0, sd0 >= 0 ? sd0p[s] : 0.0f,
-                          gx0 ? gsrc_row + sl0 : nullptr);
-        if (wave_sp2)
-          cs_adj_special<R>(Ln, Q + g.base, sr1, kw1, sd1 >= 0 ? sd1p[s] : 0.0f,
-                            gx1 ? gsrc_row + sl1 : nullptr);
+      cs_adj_rows<R>(P, Q, Lc, Ln, S.KA1, S.KW, g.base, g.CS);
+      if (S.wave_sp) {
+        cs_adj_special<R>(Ln, Q + g.base, S.sp.sr0, S.kw0, S.sp.sd0 >= 0 ? sd0p[s] : 0.0f,
+                          gx0 ? gsrc_row + S.sp.sl0 : nullptr);
+        if (S.wave_sp2)
+          cs_adj_special<R>(Ln, Q + g.base, S.sp.sr1, S.kw1, S.sp.sd1 >= 0 ? sd1p[s] : 0.0f,
+                            gx1 ? gsrc_row + S.sp.sl1 : nullptr);
       }
     }
     // gradient sum, then refill SG with lap(u) of step m-2 (the record is
@@ -854,8 +890,8 @@ __device__ __forceinline__ void adj_cs_body(const AdjArgs &a, const int w) {
     // would copy the fresh loads (waiting for them) at its back edge.
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      G[r] = __builtin_fmaf(SG[r], Ln[r], G[r]);
-      asm volatile("" : "+v"(G[r]));
+      S.G[r] = __builtin_fmaf(SG[r], Ln[r], S.G[r]);
+      asm volatile("" : "+v"(S.G[r]));
       SG[r] = cs_rec_load(rsn, pvoff + (uint32_t)(r * Ny * 4));
     }
     recp -= F;
@@ -865,26 +901,48 @@ __device__ __forceinline__ void adj_cs_body(const AdjArgs &a, const int w) {
 
   WT_TS(1);
   int s = 0;
-  for (; s + 1 < a.nsteps; s += 2) {
-    step(buf0, buf1, L1, L2, SG0, s);   // lambda_m -> L2
-    step(buf1, buf0, L2, L1, SG1, s + 1);
+  for (; s + 1 < nsteps; s += 2) {
+    step(S.buf0, S.buf1, S.L1, S.L2, S.SG0, s);   // lambda_m -> L2
+    step(S.buf1, S.buf0, S.L2, S.L1, S.SG1, s + 1);
   }
-  if (s < a.nsteps) step(buf0, buf1, L1, L2, SG0, s);
+  if (s < nsteps) step(S.buf0, S.buf1, S.L1, S.L2, S.SG0, s);
   WT_TS(2);
+}
+
+// Linear cell.  LDS holds w*lambda.  Work item w of the launch `a` (BATCH:
+// the batched kernel, with per-sample lengths and record slots).
+template <int NT, int R, bool BATCH>
+__device__ __forceinline__ void adj_cs_body(const AdjArgs &a, const int w) {
+  WT_TS(0);
+  const int b = w / a.ntiles, ti = w - (w / a.ntiles) * a.ntiles;
+  // lambda_m = 0 for every m of this launch when the sample ends before it
+  if (BATCH && a.Tlim && a.m_hi - a.nsteps + 1 > a.Tlim[b]) return;
+  __shared__ int tb_sp[CS_MAX_TABLE * CS_SP_W];
+  __shared__ int seed_px[CS_MAX_SEEDS];
+  __shared__ int nseeds;
+  CsAdj<R> S;
+  S.Lb = (BATCH && a.Tlim) ? a.Tlim[b] : 0x7fffffff;
+  adj_cs_setup<R, false>(a, S, b, ti, a.in1, a.in2, tb_sp, seed_px, &nseeds);
+  adj_cs_start<R, BATCH>(a, S, a.m_hi, a.nsteps, tb_sp, seed_px, nseeds);
+  __syncthreads();
+  adj_cs_steps<R, BATCH>(a, S, a.m_hi, a.nsteps);
+  const CsGeom &g = S.g;
   const bool odd = (a.nsteps & 1) != 0;
   if (g.active) {
     // running gradient sums: all loads first, then the stores
-    const int64_t q0 = boff + (int64_t)(g.R0 + row0) * Ny + (g.C0 + g.c);
+    const int64_t q0 =
+        ((int64_t)b * a.Nx + (g.R0 + S.row0)) * a.Ny + (g.C0 + g.c);
     float gold[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) gold[r] = ((omask >> r) & 1u) ? a.gacc[q0 + (int64_t)r * Ny] : 0.0f;
+    for (int r = 0; r < R; ++r)
+      gold[r] = ((S.omask >> r) & 1u) ? a.gacc[q0 + (int64_t)r * a.Ny] : 0.0f;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      if ((omask >> r) & 1u) {
-        const int64_t q = q0 + (int64_t)r * Ny;
-        a.out1[q] = odd ? L2[r] : L1[r];
-        a.out2[q] = odd ? L1[r] : L2[r];
-        a.gacc[q] = gold[r] + G[r];
+      if ((S.omask >> r) & 1u) {
+        const int64_t q = q0 + (int64_t)r * a.Ny;
+        a.out1[q] = odd ? S.L2[r] : S.L1[r];
+        a.out2[q] = odd ? S.L1[r] : S.L2[r];
+        a.gacc[q] = gold[r] + S.G[r];
       }
     }
   }
@@ -894,6 +952,170 @@ __device__ __forceinline__ void adj_cs_body(const AdjArgs &a, const int w) {
 template <int NT, int R>
 __global__ __launch_bounds__(NT) void k_adj_cs(AdjArgs a) {
   adj_cs_body<NT, R, false>(a, xcd_remap(blockIdx.x, gridDim.x));
+}
+
+// Reverse steps of the chunk that starts at m: chunks end at multiples of
+// a.group steps, so that the gradient is summed over the same spans whatever
+// the record's segments are.
+__device__ __forceinline__ int adj_walk_steps(const AdjArgs &a, int m) {
+  const int lo = a.group > 0 ? (m - 1) / a.group * a.group : 0;
+  return min(a.nsteps, m - lo);
+}
+
+// Adds a chunk's gradient sums to the running ones (the output rows have one
+// owner from the first chunk to the last).
+template <int R>
+__device__ __forceinline__ void adj_walk_sum(const AdjArgs &a, const float (&G)[R],
+                                             uint32_t omask, int64_t q0) {
+  const uint32_t out = cs_opaque(omask);
+  const int64_t q = cs_opaque(q0);
+  float gold[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    gold[r] = ((out >> r) & 1u) ? a.gacc[q + (int64_t)r * a.Ny] : 0.0f;
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    if ((out >> r) & 1u) a.gacc[q + (int64_t)r * a.Ny] = gold[r] + G[r];
+}
+
+// The resident adjoint: k_fwd_cs_walk's scheme for the reverse sweep.  The
+// record of a chunk's first steps and its probe seeds are read before the
+// wait for the neighbours.  The gradient is summed chunk by chunk, as the
+// launches of the other path do, in registers where there is room (KEEP).
+// (us per pass, a launch per chunk and resident: 150 x 150, 64 samples, 1000
+// steps 9876 and 8729, 100 x 100, 4 samples, forward and backward 1259 and
+// 1126, 500 steps of one sample 1210 and 1063.)
+template <int NT, int R>
+__global__ __launch_bounds__(NT) void k_adj_cs_walk(AdjArgs a) {
+  const int tid = threadIdx.x;
+  const int64_t BF = (int64_t)a.B * a.Nx * a.Ny;
+  __shared__ int tb_sp[CS_MAX_TABLE * CS_SP_W];
+  __shared__ int seed_px[CS_MAX_SEEDS];
+  __shared__ int nseeds;
+  __shared__ int msg;
+  int w = xcd_remap(blockIdx.x, gridDim.x);
+  if (tid == 0) msg = atomicCAS(a.prog + w * CS_WALK_W, 0, 1);
+  __syncthreads();
+  if (msg != 0) return;  // a neighbour took it over
+  constexpr bool KEEP = R <= 6;
+  CsAdj<R> S;
+  float GT[R];
+  int64_t q0;
+  int chunk = 0, m = a.T, got;
+  {
+    const int b = w / a.ntiles, ti = w - b * a.ntiles;
+    const int nbr = tid < 64 ? cs_walk_neighbours(a.tiles, a.ntiles, ti) : 0;
+    adj_cs_setup<R, true>(a, S, b, ti, a.in1, a.in2, tb_sp, seed_px, &nseeds);
+    const CsGeom &g = S.g;
+    q0 = ((int64_t)b * a.Nx + (g.R0 + S.row0)) * a.Ny + (g.C0 + g.c);
+    uint32_t halo = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      GT[r] = 0.0f;
+      if (g.active && S.row0 + r < g.RH && !((S.omask >> r) & 1u)) halo |= 1u << r;
+    }
+    int nsteps = adj_walk_steps(a, m);
+    adj_cs_start<R, false>(a, S, m, nsteps, tb_sp, seed_px, nseeds);
+    __syncthreads();
+    while (true) {
+      adj_cs_steps<R, false>(a, S, m, nsteps);
+      m -= nsteps;
+      if (KEEP) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) GT[r] = GT[r] + S.G[r];
+      }
+      if (m > 0) cs_walk_store<R>(a, S.L1, S.L2, w, chunk, nsteps, S.omask, q0);
+      if (!KEEP) adj_walk_sum<R>(a, S.G, S.omask, q0);
+      if (m == 0) break;
+      ++chunk;
+      nsteps = adj_walk_steps(a, m);
+      adj_cs_start<R, false>(a, S, m, nsteps, tb_sp, seed_px, nseeds);
+      if (tid < 64) {
+        const int r = cs_walk_wait(a.prog, a.ntiles, b, nbr, chunk);
+        if (tid == 0) msg = r;
+      }
+      __syncthreads();
+      got = msg;
+      if (got != -1) break;
+      const float *in1 = a.out1 + ((chunk - 1) & 1) * 2 * BF, *in2 = in1 + BF;
+      const uint32_t hm = cs_opaque(halo);
+      int64_t q = cs_opaque(q0);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        if ((hm >> r) & 1u) {
+          S.L1[r] = cs_dev_load(in1 + q);
+          S.L2[r] = cs_dev_load(in2 + q);
+        }
+        q += a.Ny;
+      }
+      if (g.active) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) S.buf0[g.base + r] = S.KW[r] * S.L1[r];
+      }
+      __syncthreads();
+    }
+    if (KEEP) adj_walk_sum<R>(a, GT, S.omask, q0);
+    if (m == 0) return;
+  }
+  // Work items taken over: from here on every chunk of this workgroup starts
+  // with a whole set-up (of a work item that nobody else touches any more).
+  __shared__ int own_w[CS_WALK_MAX], own_n[CS_WALK_MAX];
+  int nown = 1, at = 0;
+  while (true) {
+    if (got == -2) {  // given up: the gradient's first cell of the tile becomes NaN
+      const int32_t *td = a.tiles + w % a.ntiles * TILE_W;
+      if (tid == 0)
+        a.gacc[((int64_t)(w / a.ntiles) * a.Nx + td[4]) * a.Ny + td[6]] = __builtin_nanf("");
+      return;
+    }
+    if (got >= 0) {
+      if (tid == 0) {
+        own_w[at] = w;
+        own_n[at] = chunk;
+        own_w[nown] = got;
+        own_n[nown] = 0;
+      }
+      ++nown;
+    } else {
+      const float *in1 = chunk ? a.out1 + ((chunk - 1) & 1) * 2 * BF : a.in1;
+      m = a.T;
+      for (int i = 0; i < chunk; ++i) m -= adj_walk_steps(a, m);
+      const int nsteps = adj_walk_steps(a, m);
+      adj_cs_setup<R, true>(a, S, w / a.ntiles, w % a.ntiles, in1, in1 + BF, tb_sp, seed_px,
+                            &nseeds);
+      adj_cs_start<R, false>(a, S, m, nsteps, tb_sp, seed_px, nseeds);
+      __syncthreads();
+      adj_cs_steps<R, false>(a, S, m, nsteps);
+      q0 = ((int64_t)S.b * a.Nx + (S.g.R0 + S.row0)) * a.Ny + (S.g.C0 + S.g.c);
+      adj_walk_sum<R>(a, S.G, S.omask, q0);
+      cs_walk_store<R>(a, S.L1, S.L2, w, chunk, nsteps, S.omask, q0);
+      ++chunk;
+      const bool done = m == nsteps;
+      if (done && --nown == 0) return;
+      if (tid == 0) {
+        own_n[at] = chunk;
+        if (done) {
+          own_w[at] = own_w[nown];
+          own_n[at] = own_n[nown];
+        }
+      }
+    }
+    __syncthreads();
+    at = 0;  // the least advanced one next
+    for (int i = 1; i < nown; ++i)
+      if (own_n[i] < own_n[at]) at = i;
+    w = own_w[at];
+    chunk = own_n[at];
+    if (tid < 64) {
+      const int r =
+          chunk > 0 ? cs_walk_wait(a.prog, a.ntiles, w / a.ntiles,
+                                   cs_walk_neighbours(a.tiles, a.ntiles, w % a.ntiles), chunk)
+                    : -1;
+      if (tid == 0) msg = r;
+    }
+    __syncthreads();
+    got = msg;
+  }
 }
 
 template <int NT, int R>
@@ -1208,35 +1430,9 @@ static hipError_t cs_fwd_dispatch(bool unit_h, int nl, bool rec, const FwdArgs &
                                   int nthreads, size_t shmem, hipStream_t s) {
 #define FT(NL, REC, UH)                                                               \
   do {                                                                                \
-    auto kfn = k_fwd_cs<NT, R, NL, REC, UH>;                                           \
-    static std::atomic<uint64_t> done{0};                                             \
-    hipError_t e = allow_dyn_lds((const void *)kfn, done);                            \
-    if (e != hipSuccess) return e;                                                    \
-    hipLaunchKernelGGL(kfn, dim3(nblocks), dim3(nthreads), shmem, s, a);              \
-  } while (0)
-  if (nl == 0) {
-    if (unit_h) {
-      if (rec) FT(0, true, true); else FT(0, false, true);
-    } else {
-      if (rec) FT(0, true, false); else FT(0, false, false);
-    }
-  } else if (unit_h) {
-    if (rec) FT(8, true, true); else FT(8, false, true);
-  } else {
-    if (rec) FT(8, true, false); else FT(8, false, false);
-  }
-#undef FT
-  return hipGetLastError();
-}
-
-template <int NT, int R>
-static hipError_t cs_walk_dispatch(bool unit_h, int nl, bool rec, const FwdArgs &a, int nblocks,
-                                   int nthreads, size_t shmem, hipStream_t s) {
-#define FT(NL, REC, UH)                                                               \
-  do {                                                                                \
-    auto kfn = k_fwd_cs_walk<NT, R, NL, REC, UH>;                                      \
-    static std::atomic<uint64_t> done{0};                                             \
-    hipError_t e = allow_dyn_lds((const void *)kfn, done);                            \
+    auto kfn = a.prog ? k_fwd_cs_walk<NT, R, NL, REC, UH> : k_fwd_cs<NT, R, NL, REC, UH>; \
+    static std::atomic<uint64_t> done[2];                                             \
+    hipError_t e = allow_dyn_lds((const void *)kfn, done[a.prog != nullptr]);         \
     if (e != hipSuccess) return e;                                                    \
     hipLaunchKernelGGL(kfn, dim3(nblocks), dim3(nthreads), shmem, s, a);              \
   } while (0)
@@ -1258,11 +1454,16 @@ static hipError_t cs_walk_dispatch(bool unit_h, int nl, bool rec, const FwdArgs 
 template <int NT, int R>
 static hipError_t cs_adj_dispatch(const AdjArgs &a, int nblocks, int nthreads, size_t shmem,
                                   hipStream_t s) {
-  auto kfn = k_adj_cs<NT, R>;
-  static std::atomic<uint64_t> done{0};
-  hipError_t e = allow_dyn_lds((const void *)kfn, done);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kfn, dim3(nblocks), dim3(nthreads), shmem, s, a);
+#define AT(KFN)                                                                       \
+  do {                                                                                \
+    auto kfn = KFN<NT, R>;                                                            \
+    static std::atomic<uint64_t> done{0};                                             \
+    hipError_t e = allow_dyn_lds((const void *)kfn, done);                            \
+    if (e != hipSuccess) return e;                                                    \
+    hipLaunchKernelGGL(kfn, dim3(nblocks), dim3(nthreads), shmem, s, a);              \
+  } while (0)
+  if (a.prog) AT(k_adj_cs_walk); else AT(k_adj_cs);
+#undef AT
   return hipGetLastError();
 }
 
@@ -1273,25 +1474,12 @@ hipError_t launch_fwd_cs(int nt, int R, bool unit_h, int nl, bool rec, const Fwd
   int nblocks = a.B * a.ntiles;
   size_t shmem = cs_shmem_bytes(R, RHmax, RWmax, true);
   int nthreads = cs_threads(R, RHmax, RWmax);
-  if (shmem + CS_STATIC_LDS > (size_t)cs_max_dyn_lds() || nthreads > nt) return hipErrorInvalidConfiguration;
-#define X(A, B) \
-  if (nt == A && R == B)                                                                \
-    return cs_fwd_dispatch<A, B>(unit_h, nl, rec, a, nblocks, nthreads, shmem, s);
-  WT_CS_VARIANTS(X)
-#undef X
-  return hipErrorInvalidValue;
-}
-
-hipError_t launch_fwd_cs_walk(int nt, int R, bool unit_h, int nl, bool rec, const FwdArgs &a,
-                              int RHmax, int RWmax, hipStream_t s) {
-  int nblocks = a.B * a.ntiles;
-  size_t shmem = cs_shmem_bytes(R, RHmax, RWmax, true);
-  int nthreads = cs_threads(R, RHmax, RWmax);
-  if (shmem + CS_STATIC_LDS > (size_t)cs_max_dyn_lds() || nthreads > nt || nblocks > CS_WALK_MAX)
+  if (shmem + CS_STATIC_LDS > (size_t)cs_max_dyn_lds() || nthreads > nt ||
+      (a.prog && nblocks > CS_WALK_MAX))
     return hipErrorInvalidConfiguration;
 #define X(A, B) \
   if (nt == A && R == B)                                                                \
-    return cs_walk_dispatch<A, B>(unit_h, nl, rec, a, nblocks, nthreads, shmem, s);
+    return cs_fwd_dispatch<A, B>(unit_h, nl, rec, a, nblocks, nthreads, shmem, s);
   WT_CS_VARIANTS(X)
 #undef X
   return hipErrorInvalidValue;
@@ -1301,7 +1489,9 @@ hipError_t launch_adj_cs(int nt, int R, const AdjArgs &a, int RHmax, int RWmax, 
   int nblocks = a.B * a.ntiles;
   size_t shmem = cs_shmem_bytes(R, RHmax, RWmax, false);
   int nthreads = cs_threads(R, RHmax, RWmax);
-  if (shmem + CS_STATIC_LDS > (size_t)cs_max_dyn_lds() || nthreads > nt) return hipErrorInvalidConfiguration;
+  if (shmem + CS_STATIC_LDS + (a.prog ? CS_WALK_LDS : 0) > (size_t)cs_max_dyn_lds() ||
+      nthreads > nt || (a.prog && nblocks > CS_WALK_MAX))
+    return hipErrorInvalidConfiguration;
 #define X(A, B) if (nt == A && R == B) return cs_adj_dispatch<A, B>(a, nblocks, nthreads, shmem, s);
   WT_CS_VARIANTS(X)
 #undef X

@@ -121,6 +121,7 @@ struct FwdArgs {
 };
 constexpr int CS_WALK_MAX = 256;  // work items of a resident launch, at most
 constexpr int CS_WALK_W = 16;     // ints between its progress words
+constexpr int CS_WALK_LDS = 2112; // LDS of its lists of work items
 
 // Arguments of the fused adjoint kernel (row strips only: C0 = 0, RW = Ny).
 struct AdjArgs {
@@ -150,6 +151,11 @@ struct AdjArgs {
   float *gsrc;       // (B,T,nsrcslot) lambda_m at source pixels
   const int32_t *Tlim;  // per-sample step count, or NULL
   int c2_bstride;       // C2 stride between samples (0 = shared)
+  // resident launch: progress words, as in FwdArgs (out1: two alternating
+  // state pairs, m_hi unused, nsteps the steps of a chunk), and the multiple
+  // of steps at which chunks end (0: any)
+  int *prog;
+  int group;
 };
 
 // One launch over several configurations (batched instances of uneven grid

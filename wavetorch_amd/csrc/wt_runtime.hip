@@ -92,8 +92,6 @@ size_t cs_shmem_bytes(int R, int RH, int RW, bool padded);
 int cs_threads(int R, int RH, int RW);
 hipError_t launch_fwd_cs(int nt, int R, bool unit_h, int nl, bool rec, const FwdArgs &a,
                          int RHmax, int RWmax, hipStream_t s);
-hipError_t launch_fwd_cs_walk(int nt, int R, bool unit_h, int nl, bool rec, const FwdArgs &a,
-                              int RHmax, int RWmax, hipStream_t s);
 hipError_t launch_adj_cs(int nt, int R, const AdjArgs &a, int RHmax, int RWmax, hipStream_t s);
 size_t cs64_shmem_bytes(int R, int RH, int RW, int tb);
 bool cs64_variant_exists(int R, bool fwd);
@@ -1372,13 +1370,12 @@ FwdArgs base_fwd(const Plan &p, const Ws &w, const float *b, const float *c, con
   return a;
 }
 
-// Whether a whole forward of this plan runs as one resident launch: more than
-// one chunk, a workgroup for each CU at most, and progress words that fit one
-// state buffer.
-bool walks(const Plan &p) {
-  const int64_t items = (int64_t)p.B * p.ntiles;
-  return p.tiled && p.tun.kind == 0 && p.T > p.tun.tblock &&
-         items <= std::min(CS_WALK_MAX, device_cus()) &&
+// Whether `ntiles` tiles per sample, in chunks of tb steps, run as one
+// resident launch: more than one chunk, a workgroup for each CU at most, and
+// progress words that fit one state buffer.
+bool walks(const Plan &p, int ntiles, int tb) {
+  const int64_t items = (int64_t)p.B * ntiles;
+  return p.tiled && p.tun.kind == 0 && p.T > tb && items <= std::min(CS_WALK_MAX, device_cus()) &&
          items * CS_WALK_W <= (int64_t)p.B * (int64_t)p.F;
 }
 
@@ -1608,7 +1605,7 @@ int wt_loop_fwd(void *plan, const float *b, const float *c, const float *rho, co
   float *tmp[4] = {bufs[0], bufs[1], bufs[2], bufs[3]};
   float *z = with_grad ? w.ck : bufs[4];
   const bool rec = with_grad && w.rec;
-  if (walks(*p) && (!with_grad || (rec && p->nseg == 1))) {
+  if (walks(*p, p->ntiles, p->tun.tblock) && (!with_grad || (rec && p->nseg == 1))) {
     // the progress words take the state buffer after the (non-recording
     // call's) zero state: one fill for both
     const int64_t words = (int64_t)p->B * p->ntiles * CS_WALK_W;
@@ -1629,8 +1626,7 @@ int wt_loop_fwd(void *plan, const float *b, const float *c, const float *rho, co
       a.rec_K = p->K;
     }
     ProfScope ps(0, s, (int64_t)p->B * p->Nx * p->Ny * p->T);
-    WT_HIP(launch_fwd_cs_walk(p->tun.nt, p->tun.cpt, p->unit_h, p->nl, rec, a, p->RHmax,
-                              p->RWmax, s));
+    WT_HIP(launch_fwd_cs(p->tun.nt, p->tun.cpt, p->unit_h, p->nl, rec, a, p->RHmax, p->RWmax, s));
     return WT_OK;
   }
   WT_HIP(launch_fill(z, 2 * BF, 0.0f, s));
@@ -1722,7 +1718,19 @@ int wt_loop_adj(void *plan, const float *b, const float *c, const float *rho, co
     aa.seg_n0 = n0;
     // adjoint over m = n1 .. n0+1
     int m = n1;
-    if (use_tiled) {
+    if (use_tiled && p->nseg == 1 && walks(*p, p->ntiles_a, p->tb_a) &&
+        cs_shmem_bytes(p->cpt_a, p->RHmax_a, p->RWmax_a, false) + CS_STATIC_LDS + CS_WALK_LDS <=
+            (size_t)max_dyn_lds_dev()) {
+      // one resident launch; its progress words take the plain sweep's
+      // w*lambda buffer (zero)
+      // (the second state pair, first written by the second chunks, is zero)
+      aa.in1 = lam[2]; aa.in2 = lam[3]; aa.out1 = lam[0];
+      aa.nsteps = p->tb_a;
+      aa.prog = (int *)w.wl;
+      aa.group = p->group;
+      ProfScope ps(2, s, (int64_t)p->B * p->Nx * p->Ny * T);
+      WT_HIP(launch_adj_cs(p->nt_a, p->cpt_a, aa, p->RHmax_a, p->RWmax_a, s));
+    } else if (use_tiled) {
       while (m > n0) {
         int k = adj_steps(*p, m, n0);
         aa.in1 = l1; aa.in2 = l2; aa.out1 = l3; aa.out2 = l4;
