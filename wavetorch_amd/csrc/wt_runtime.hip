@@ -630,6 +630,50 @@ static double launch_us(const BlockModel &m, int R, int waves, int occ, int perc
          cells * (m.rec * n * 1e-6 + m.state);
 }
 
+// A chunk of n steps of a resident launch, one workgroup of w waves and R rows
+// per thread on a CU: k = ceil(w/4) waves per SIMD,
+//   ts + tR R k                                     exchange
+//   e + cw w/16 + max(issue R k', row R)            per step
+// (a row takes `issue` of a SIMD, but at least `row` of its wave's time; k' =
+// k less the waves that the halo's cone has left, times `cone`), and the
+// traffic of the record (`rec` per cell and step, rows of tw cells in whole
+// cache lines: 1 + edge 32 / tw) and of the state (`state` per cell, `lines`
+// per cache line of halo and output rows).  Fitted to 10000 forwards, 2000
+// nonlinear ones and 3700 adjoints on the cheapest tilings of 80 to 340
+// random problems each: 5 to 6% rms, the choice 2 to 3% slower on average
+// than the fastest of 18 candidates measured.
+struct WalkModel {
+  double ts, tR, e, cw, issue, row, cone, rec, edge, state, lines;
+  int rows[5];
+};
+static const WalkModel kWalkLin = {2.75, 0.0247, 0.031, 0.126, 0.0179, 0.0532, 1.12, 0.09, 2.0,
+                                   0.0, 6.34e-6, {4, 6, 8, 10, 12}};
+static const WalkModel kWalkLinAdj = {1.71, 0.0411, 0.262, 0.0, 0.0222, 0.0599, 1.2, 0.0835, 2.0,
+                                      3.48e-6, 0.0, {4, 6, 8, 10, 0}};
+static const WalkModel kWalkNl = {2.5, 0.0547, 0.0, 0.372, 0.0545, 0.14, 0.963, 0.152, 2.0, 0.0,
+                                  4.48e-6, {4, 6, 8, 0, 0}};
+
+// (an interior tile of s strips and c columns)
+static double walk_us(const WalkModel &m, int R, int waves, int s, int c, int th, int tw, int RH,
+                      int RW, int n, double cells) {
+  const int nseg = (RH + R - 1) / R, lo = s > 2 ? std::min(n, RH - th) : 0;
+  double live = 0.0;
+  for (int g = 0; g < nseg; ++g) {
+    int q = 0;  // as cs_live_steps
+    if (lo + th < RH) q = std::max(q, g * R - lo - th + 1);
+    if (lo > 0) q = std::max(q, lo - g * R - R + 1);
+    live += std::max(0, n - q);
+  }
+  live /= (double)nseg * n;
+  const int k = (waves + 3) / 4;
+  const double lines = (RH - th) * (RW / 32.0 + 1) + th * (tw / 32.0 + 1) +
+                       th * std::min(c - 1, 2) * (n / 32.0 + 1);
+  const double issue = m.issue * R * k * (1.0 - m.cone * (1.0 - live));
+  return m.ts + m.tR * R * k + n * (m.e + m.cw * waves / 16 + std::max(issue, m.row * R)) +
+         cells * (m.rec * n * 1e-6 * (1.0 + m.edge * 32.0 / tw) + m.state +
+                  lines / ((double)th * tw) * m.lines);
+}
+
 struct BlockChoice {
   double us;
   int s, c, tb, R;
@@ -640,8 +684,9 @@ struct BlockChoice {
 // that many steps per launch.  shmem(R, RH, RW, tb): LDS of the block, static
 // part included.
 template <typename Shmem>
-static std::vector<BlockChoice> cheapest_blocks(const BlockModel &m, int Nx, int Ny, int B,
-                                                int len, int depth, int top, Shmem shmem) {
+static std::vector<BlockChoice> cheapest_blocks(const BlockModel &launches, const WalkModel *walk,
+                                                int Nx, int Ny, int B, int len, int depth, int top,
+                                                Shmem shmem) {
   static const int depths[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 14, 16, 18, 20, 24, 28, 32, 40, 48};
   std::vector<BlockChoice> best;
   auto consider = [&](int s, int c, int tb) {
@@ -649,20 +694,29 @@ static std::vector<BlockChoice> cheapest_blocks(const BlockModel &m, int Nx, int
     const int RH = std::min(Nx, th + (s > 2 ? 2 * tb : s == 2 ? tb : 0));
     const int RW = std::min(Ny, tw + (c > 2 ? 2 * tb : c == 2 ? tb : 0));
     const int percu = (int)(((int64_t)B * s * c + 255) / 256);
-    for (int v = 0; v < 5 && m.rows[v]; ++v) {
-      const int R = m.rows[v], waves = cs_threads(R, RH, RW) / 64;
+    // (a single chunk too: a launch of its own, whose steps are the same)
+    const bool walks =
+        walk && percu == 1 && (int64_t)s * c * CS_WALK_W <= (int64_t)Nx * Ny;
+    const BlockModel &m = launches;
+    const int *rows = walks ? walk->rows : m.rows;
+    for (int v = 0; v < 5 && rows[v]; ++v) {
+      const int R = rows[v], waves = cs_threads(R, RH, RW) / 64;
       if (waves > 16) continue;
-      const size_t lds = shmem(R, RH, RW, tb);
+      const size_t lds = shmem(R, RH, RW, tb) + (walks ? CS_WALK_LDS : 0);
       if (lds > LDS_LIMIT) continue;
       const int occ = std::max(1, std::min((int)(LDS_LIMIT / lds), m.waves[v] * 4 / waves));
       const double cells = (double)B * Nx * Ny;
-      auto launch = [&](int n) { return launch_us(m, R, waves, occ, percu, n, cells); };
+      auto launch = [&](int n) {
+        return walks ? walk_us(*walk, R, waves, s, c, th, tw, RH, RW, n, cells)
+                     : launch_us(m, R, waves, occ, percu, n, cells);
+      };
       // among tilings that the model's whole waves and rounds call equal, the
       // one with the least area computed (halos clipped at the domain's edge;
       // halo rows drop out of the cone step by step, halo columns stay)
       const double area = (Nx + (s > 1 ? 1.0 * tb * (s - 1) : 0.0)) *
                           (Ny + (c > 1 ? 2.0 * tb * (c - 1) : 0.0)) * B;
-      const double us = (len / tb * launch(tb) + (len % tb ? launch(len % tb) : 0.0)) *
+      const double us = (len / tb * launch(tb) + (len % tb ? launch(len % tb) : 0.0) +
+                         (walks ? 8.0 : 0.0)) *
                         (1.0 + 0.06 * area / (256.0 * 1024.0 * R * percu));
       if ((int)best.size() == top && us >= best.back().us) continue;
       const BlockChoice ch{us, s, c, tb, R};
@@ -727,7 +781,7 @@ static void plan_f64(Plan &plan) {
     }
     if (!ok) {
       for (const BlockChoice &ch : cheapest_blocks(
-               fwd ? kModel64 : kModel64Adj, p.Nx, p.Ny, p.B, p.T, 0, 32,
+               fwd ? kModel64 : kModel64Adj, nullptr, p.Nx, p.Ny, p.B, p.T, 0, 32,
                [](int R, int RH, int RW, int tb) {
                  return cs64_shmem_bytes(R, RH, RW, tb) + 16 * 1024;
                })) {
@@ -1107,7 +1161,8 @@ int wt_plan_suggest(const wt_config *cfg, int32_t B, int32_t T, float cmax_geom,
   out->ck_every = K;
   bool ok = false;
   for (const BlockChoice &ch : cheapest_blocks(
-           p->nl ? kModelNl : kModelLin, p->Nx, p->Ny, B, K, 0, 32,
+           p->nl ? kModelNl : kModelLin,
+           K < T ? nullptr : p->nl ? &kWalkNl : &kWalkLin, p->Nx, p->Ny, B, K, 0, 32,
            [](int R, int RH, int RW, int) { return cs_shmem_bytes(R, RH, RW, true) + 8192; })) {
     build_tiles(*p, ch.s, ch.c, ch.tb);
     if (!tiles_ok_cs(*p, 1024, ch.R)) continue;
@@ -1120,7 +1175,8 @@ int wt_plan_suggest(const wt_config *cfg, int32_t B, int32_t T, float cmax_geom,
   if (ok) {
     const bool nl = p->nl != 0;
     for (const BlockChoice &ch : cheapest_blocks(
-             nl ? kModelNlAdj : kModelLinAdj, p->Nx, p->Ny, B, K, a_depth, 32,
+             nl ? kModelNlAdj : kModelLinAdj, K < T || nl ? nullptr : &kWalkLinAdj, p->Nx,
+             p->Ny, B, K, a_depth, 32,
              [nl](int R, int RH, int RW, int) {
                return (nl ? cs_nl_shmem_bytes(R, RH, RW) : cs_shmem_bytes(R, RH, RW, false)) +
                       8192;
