@@ -58,8 +58,18 @@ def traffic_file(workload):
     return os.path.join(ROOT, "profiles", f"traffic_{workload}.json")
 
 
-def class_name(cls, tun, nonlinear=False):
-    """Kernel (as rocprofv3 names it) of a kernel class under plan tuning `tun`."""
+def resident(cls, tun, nonlinear, B, T):
+    """Whether class `cls` of a plan's sweeps runs as one resident launch: a
+    workgroup per CU at most, more than one chunk, and one segment (a forward
+    without a record counts as class 0 and needs no segments)."""
+    a = "a_" if cls == 2 else ""
+    return not (cls == 2 and nonlinear) and tun["ck_every"] >= T and \
+        B * tun[a + "strips"] * tun[a + "tcols"] <= 256 and T > tun[a + "tblock"]
+
+
+def class_name(cls, tun, nonlinear, B, T, unit_h=True, rec=False):
+    """Kernel (as rocprofv3 names it) of a kernel class under plan tuning
+    `tun`; `rec`: class 0 is the forward of a training step with one segment."""
     if tun["plain"]:
         return ["wt::k_loop_fwd_plain", "wt::k_loop_fwd_plain (record)",
                 "wt::k_loop_adj_nl_plain" if nonlinear else "wt::k_loop_adj_plain"][cls]
@@ -69,9 +79,11 @@ def class_name(cls, tun, nonlinear=False):
     if cls == 2:
         if nonlinear:
             return f"wt::k_adj_cs_nl<{tun['a_nt']}, {tun['a_cpt']}, false>"
-        return f"wt::k_adj_cs<{tun['a_nt']}, {tun['a_cpt']}>"
-    return f"wt::k_fwd_cs<{tun['nt']}, {tun['cpt']}, {8 if nonlinear else 0}, " \
-        f"{'true' if cls == 1 else 'false'}>"
+        walk = "_walk" if resident(cls, tun, nonlinear, B, T) else ""
+        return f"wt::k_adj_cs{walk}<{tun['a_nt']}, {tun['a_cpt']}>"
+    walk = "_walk" if cls == 0 and resident(cls, tun, nonlinear, B, T) else ""
+    return f"wt::k_fwd_cs{walk}<{tun['nt']}, {tun['cpt']}, {8 if nonlinear else 0}, " \
+        f"{'true' if cls == 1 or rec else 'false'}, {'true' if unit_h else 'false'}>"
 
 
 def log(*a):
@@ -836,10 +848,14 @@ def main():
     avg_s = ms / max(nl, 1) / 1e3
     per_launch = work / max(nl, 1)
     nonlin = plan.cfg.nonlinear
+
+    def name(c):
+        return class_name(c, plan.tuning, nonlin, B, T, plan.cfg.h == 1.0,
+                          labels is not None and plan.tuning["ck_every"] >= T)
     for c, (m_, n_, w_) in prof.items():
-        log(f"[bench] class {c} {class_name(c, plan.tuning, nonlin)}: {n_} launches, "
+        log(f"[bench] class {c} {name(c)}: {n_} launches, "
             f"{m_:.2f} ms total, {(m_ / max(n_, 1)) * 1e3:.1f} us avg")
-    kname = class_name(cls, plan.tuning, nonlin)
+    kname = name(cls)
     out = {
         "metric": wl["metric"],
         "value": round(value, 3),
@@ -857,8 +873,7 @@ def main():
                    "T": T, "tuning": plan.tuning},
         "roofline": roofline(args.workload, kname, plan.tuning, cls, per_launch, avg_s, nl,
                              {"events_ms_per_step": round(prof_step_s * 1e3, 3),
-                              "kernel_ms_per_step": {class_name(c, plan.tuning, nonlin):
-                                                     round(prof[c][0] / args.steps, 3)
+                              "kernel_ms_per_step": {name(c): round(prof[c][0] / args.steps, 3)
                                                      for c in prof if prof[c][1]}}),
         # the whole step at its algorithmic bytes per cell-step (28 B = 12 forward
         # + 16 adjoint for a training step, 12 B forward only)
