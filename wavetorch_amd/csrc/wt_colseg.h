@@ -305,4 +305,107 @@ __device__ __forceinline__ void cs_zero_lds(T *b0, T *b1, const CsGeom &g, int n
   }
 }
 
+// Resident sweeps: one launch walks all T steps in chunks,
+// each workgroup with its own tile, whose cells and coefficients stay in its
+// registers.  Between two chunks only the halo is read again, from the state
+// that the neighbours stored: that exchange takes about 3 us (the stores'
+// and the flag's way to the memory side, a poll, the halo loads), a launch
+// and its set-up 6 to 10 us.
+//
+// Word w of `prog` (CS_WALK_W ints apart, zero at the start) holds 1 + the
+// chunks that work item w's owner has done, 0 while it has no owner.  Chunk n
+// starts when every tile whose output reaches into this region has n chunks
+// done; tiles reach into each other mutually, so these are then also past
+// reading the state that chunk n overwrites (two pairs of fields alternate).
+// A workgroup raises its word when all of its stores have completed.
+//
+// The device holds all workgroups of such a launch at once, but nothing
+// relies on it (another stream's work may hold compute units): a workgroup
+// that waits for a tile without an owner takes the tile over after
+// CS_WALK_US, and an owner of several works on the one with the fewest
+// chunks.  So the least advanced of all tiles has an owner that works on it,
+// or a neighbour that will take it, or none that waits for it while its own
+// workgroup is still to start; every wait ends.
+constexpr int CS_WALK_US = 50;
+
+// A value the compiler knows nothing about: what is derived from it per row
+// is formed where it is used.  (Of loop-invariant row predicates and offsets
+// it keeps one pair of scalar registers each, and spills 100 of them.)
+template <typename T>
+__device__ __forceinline__ T cs_opaque(T v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+// State shared between the workgroups of one launch: accessed at device
+// scope, the eight dies' L2 caches are not coherent for ordinary accesses.
+template <typename T>
+__device__ __forceinline__ T cs_dev_load(const T *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void cs_dev_store(T *p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// First wave: waits until the tiles of sample b in `nbr` (bit q of lane l:
+// tile l + 64 q) have n chunks done.  -1: they have; -2: given up after about
+// a minute; else the work item without an owner that was taken over.
+__device__ __forceinline__ int cs_walk_wait(int *prog, int ntiles, int b, int nbr, int n) {
+  const int lane = cs_opaque((int)threadIdx.x);
+  nbr = cs_opaque(nbr);
+  const uint64_t t0 = wall_clock64();
+  for (int polls = 0; polls < (1 << 26); ++polls) {
+    bool ok = true;
+    int unowned = -1;
+#pragma unroll
+    for (int q = 0; q < CS_WALK_MAX / 64; ++q)
+      if ((nbr >> q) & 1) {
+        const int j = b * ntiles + lane + 64 * q;
+        const int v = __hip_atomic_load(prog + j * CS_WALK_W, __ATOMIC_RELAXED,
+                                        __HIP_MEMORY_SCOPE_AGENT);
+        if (v < n + 1) ok = false;
+        if (v == 0) unowned = j;
+      }
+    if (__ballot(!ok) == 0) return -1;
+    const uint64_t cand = __ballot(unowned >= 0);
+    if (cand && wall_clock64() - t0 > 100 * CS_WALK_US) {  // the clock runs at 100 MHz
+      const int first = __ffsll((unsigned long long)cand) - 1;
+      int got = -1;
+      if (lane == first && atomicCAS(prog + unowned * CS_WALK_W, 0, 1) == 0) got = unowned;
+      got = __shfl(got, first);
+      if (got >= 0) return got;
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+  return -2;
+}
+
+// First wave: the tiles whose output rows and columns reach into tile ti's
+// region, as cs_walk_wait takes them.
+__device__ __forceinline__ int cs_walk_neighbours(const int32_t *tiles, int ntiles, int ti) {
+  const int32_t *td = tiles + ti * TILE_W;
+  int nbr = 0;
+#pragma unroll
+  for (int q = 0; q < CS_WALK_MAX / 64; ++q) {
+    const int j = threadIdx.x + 64 * q;
+    if (j < ntiles && j != ti) {
+      const int32_t *o = tiles + j * TILE_W;
+      if (o[4] < td[0] + td[1] && o[5] > td[0] && o[6] < td[2] + td[3] && o[7] > td[2])
+        nbr |= 1 << q;
+    }
+  }
+  return nbr;
+}
+
+// After a chunk's state is stored: when every wave's stores have completed,
+// the work item's word.
+__device__ __forceinline__ void cs_walk_raise(int *prog, int w, int chunk) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0)
+    __hip_atomic_store(prog + w * CS_WALK_W, 2 + chunk, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+
 }  // namespace wt

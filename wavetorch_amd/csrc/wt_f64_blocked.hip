@@ -36,6 +36,7 @@ struct F64Blk {
   const double *x;
   double *y, *yraw, *fields, *rec;
   int fstride;
+  int *prog;                // resident forward: progress words, else null
   const double *ybar;       // adjoint: reverse steps m_hi .. m_hi - nsteps + 1
   double *gacc, *gsrc;
   int m_hi;
@@ -50,148 +51,361 @@ __device__ __forceinline__ void b64_store(__amdgpu_buffer_rsrc_t rs, uint32_t of
   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), rs, (int)off, 0, 0);
 }
 
-template <int NT, int R, bool REC, bool UH>
-__global__ __launch_bounds__(NT) void k64_fwd_cs(F64Blk a) {
-  extern __shared__ double smem64[];
-  __shared__ int own[NT];  // source rows of each thread, a bit mask
-  const int tid = threadIdx.x;
-  const int w = xcd_remap(blockIdx.x, gridDim.x);
-  const int b = w / a.ntiles, ti = w - (w / a.ntiles) * a.ntiles;
-  const int32_t *td = a.tiles + ti * TILE_W;
-  const CsGeom g = cs_geom<R>(td, tid);
-  const int NBUF = (g.RW + 2) * g.CS;
-  double *buf0 = smem64, *buf1 = smem64 + NBUF, *xs = smem64 + 2 * NBUF;
-  const int Ny = a.Ny;
-  const int64_t F = (int64_t)a.Nx * Ny, boff = (int64_t)b * F;
-  const int nsp = min(td[9] - td[8], CS_MAX_TABLE), ntp = min(td[11] - td[10], CS_MAX_TABLE);
-  const int row0 = g.k * R;
-  double U0[R], U1[R], KA[R], KB[R], KC[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    double u1 = 0., u2 = 0., v0 = 0., v1 = 0., v2 = 0.;
-    if (g.active && row0 + r < g.RH) {
-      const int64_t q = (int64_t)(g.R0 + row0 + r) * Ny + (g.C0 + g.c);
-      v0 = a.A[q]; v1 = a.Bm[q]; v2 = a.C2[q];
-      if (a.in1) { u1 = a.in1[boff + q]; u2 = a.in2[boff + q]; }
-    }
-    U0[r] = u1; U1[r] = u2; KA[r] = v0; KB[r] = v1; KC[r] = v2;
+// Output rows (bit mask) of a thread whose cells inside the region are vmask.
+template <int R>
+__device__ __forceinline__ uint32_t cs64_out_rows(const CsGeom &g, int row0, uint32_t voff,
+                                                  uint32_t vmask) {
+  uint32_t m = 0;
+  if (voff != 0x80000000u) {
+    const int lo = max(g.or0 - g.R0 - row0, 0), hi = min(g.or1 - g.R0 - row0, R);
+    if (hi > lo) m = ((1u << hi) - 1u) & ~((1u << lo) - 1u) & vmask;
   }
-  for (int i = tid; i < a.nsteps; i += blockDim.x) xs[i] = a.x[(int64_t)b * a.T + a.n0 + i];
-  int spx0 = 0, spx1 = 0, spx2 = 0, te[TAP_W];
-  if (tid < nsp) {
-    const int32_t *e = a.spx + (td[8] + tid) * SPX_W;
-    spx0 = e[0]; spx1 = e[1]; spx2 = e[2];
-  }
-  cs_tap_load(a.taps, td[10], ntp, te);
-  own[tid] = 0;
-  cs_zero_lds<double>(buf0, buf1, g, ((g.RH + R - 1) / R) * R, NBUF);
-  __syncthreads();
-  if (g.active) {
-#pragma unroll
-    for (int r = 0; r < R; ++r) buf0[g.base + r] = U0[r];
-  }
-  // source pixels mark the rows of their owners
-  for (int kk = tid; kk < nsp; kk += blockDim.x) {
-    if (kk != tid) {  // more entries than threads
-      const int32_t *e = a.spx + (td[8] + kk) * SPX_W;
-      spx0 = e[0]; spx1 = e[1]; spx2 = e[2];
-    }
-    int rr;
-    const int t = spx2 > 0 ? cs_owner<R>(g, spx0, spx1, rr) : -1;
-    if (t >= 0) atomicOr(&own[t], 1 << rr);
-  }
-  __syncthreads();
-  const CsTap tap = cs_tap(g, a.taps, td[10], ntp, te);
-  const int srows = own[tid];
-  const bool wave_src = __ballot(srows != 0) != 0;
-  const bool one_src = __ballot((srows & (srows - 1)) != 0) == 0;
-  const uint32_t voff = cs_out_voff<double>(g, row0, Ny);
-  const int64_t out_bytes = (int64_t)(g.or1 - g.or0) * Ny * 8;
+  return m;
+}
 
-  const int live = cs_live_steps<R>(g, row0, a.nsteps);
-  const double *recp = REC ? a.rec + ((int64_t)b * a.T + a.n0) * F + (int64_t)g.or0 * Ny : a.A;
-  const int64_t yo = ((int64_t)b * a.T + a.n0) * a.ntap + tap.pcol;
-  double *yp = a.y ? a.y + yo : nullptr, *yrp = a.yraw ? a.yraw + yo : nullptr;
-  // next snapshot: at step `snap`
-  int snap = a.fields ? a.fstride - 1 - a.n0 % a.fstride : -1;
-  const double *fp = a.fields ? a.fields +
-                                    ((int64_t)b * (a.T / a.fstride) + a.n0 / a.fstride) * F +
-                                    (int64_t)g.or0 * Ny
-                              : a.A;
-
-  auto step = [&](const double *P, double *Q, double(&Uc)[R], double(&Up)[R], int s) {
-    if (s < live) {
-      const __amdgpu_buffer_rsrc_t rsl = cs_rsrc(recp, REC ? out_bytes : 0);
-      const int lfb = g.base - g.CS, rtb = g.base + g.CS;
-      double upv = UH ? P[g.base - 1] : a.t1 * P[g.base - 1];
-      double ctv = UH ? 0.0 : a.t1 * Uc[0];
+// State after nsteps steps to (o1, o2); DEV: the later one to V0 first.
+template <int R, bool DEV>
+__device__ __forceinline__ void cs64_store(const F64Blk &a, const CsGeom &g, double (&V0)[R],
+                                           double (&V1)[R], int nsteps, uint32_t voff,
+                                           uint32_t omask, int64_t q0, int b, double *o1,
+                                           double *o2) {
+  const bool odd = (nsteps & 1) != 0;
+  if (DEV) {
+    if (odd) {
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        const double ct = Uc[r];
-        const double dn = (r < R - 1) ? Uc[r + 1] : P[g.base + R];
-        const double lf = P[lfb + r], rt = P[rtb + r];
-        double lap;
-        if (UH) {  // products with t1 = 1 and t4 = -4 are exact
-          double s0 = upv + lf;
-          s0 = __builtin_fma(-4.0, ct, s0);
-          s0 = s0 + rt;
-          lap = s0 + dn;
-          upv = ct;
-        } else {
-          const double dnv = a.t1 * dn;
-          double s0 = upv + a.t1 * lf;
-          s0 = s0 + a.t4 * ct;
-          s0 = s0 + a.t1 * rt;
-          lap = s0 + dnv;
-          upv = ctv;
-          ctv = dnv;
-        }
-        const double p1 = a.s2 * ct;
-        const double p2 = KB[r] * Up[r];
-        const double p3 = KC[r] * lap;
-        const double v = KA[r] * ((p1 - p2) + p3);
-        Up[r] = v;
-        Q[g.base + r] = v;
-        if (REC) b64_store(rsl, voff + (uint32_t)(r * Ny * 8), lap);
+        const double u = V0[r];
+        V0[r] = V1[r];
+        V1[r] = u;
       }
-      if (wave_src) cs_add_source<R>(Up, Q + g.base, srows, one_src, xs[s]);
-      if (s == snap) {  // the thread's own rows: consecutive lanes, consecutive columns
-        const __amdgpu_buffer_rsrc_t rf = cs_rsrc(fp, out_bytes);
+    }
+    const uint32_t out = cs_opaque(omask);
+    int64_t q = cs_opaque(q0);
 #pragma unroll
-        for (int r = 0; r < R; ++r) b64_store(rf, voff + (uint32_t)(r * Ny * 8), Up[r]);
+    for (int r = 0; r < R; ++r) {
+      if ((out >> r) & 1u) {
+        cs_dev_store(o1 + q, V0[r]);
+        cs_dev_store(o2 + q, V1[r]);
       }
+      q += a.Ny;
     }
-    if (s == snap) {
-      snap += a.fstride;
-      fp += F;
+  } else {
+    const int64_t at = ((int64_t)b * a.Nx + g.or0) * a.Ny;
+    const int64_t out_bytes = (int64_t)(g.or1 - g.or0) * a.Ny * 8;
+    const __amdgpu_buffer_rsrc_t r1 = cs_rsrc(o1 + at, out_bytes), r2 = cs_rsrc(o2 + at, out_bytes);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      b64_store(r1, voff + (uint32_t)(r * a.Ny * 8), odd ? V1[r] : V0[r]);
+      b64_store(r2, voff + (uint32_t)(r * a.Ny * 8), odd ? V0[r] : V1[r]);
     }
-    if (REC) recp += F;
-    __syncthreads();
-    if (tap.pidx >= 0) {
-      const double v = Q[tap.pidx];
-      if (yp) {
-        *yp = tap.pkind ? v * v : v;
-        yp += a.ntap;
-      }
-      if (yrp) {
-        *yrp = v;
-        yrp += a.ntap;
-      }
-    }
-  };
-  int s = 0;
-  for (; s + 1 < a.nsteps; s += 2) {
-    step(buf0, buf1, U0, U1, s);
-    step(buf1, buf0, U1, U0, s + 1);
   }
-  if (s < a.nsteps) step(buf0, buf1, U0, U1, s);
-  const bool odd = (a.nsteps & 1) != 0;
-  const __amdgpu_buffer_rsrc_t r1 = cs_rsrc(a.out1 + boff + (int64_t)g.or0 * Ny, out_bytes);
-  const __amdgpu_buffer_rsrc_t r2 = cs_rsrc(a.out2 + boff + (int64_t)g.or0 * Ny, out_bytes);
+}
+
+template <int R>
+__device__ __forceinline__ void cs64_halo(const F64Blk &a, double (&V0)[R], double (&V1)[R],
+                                          uint32_t halo, int64_t q0, const double *in1,
+                                          const double *in2) {
+  const uint32_t hm = cs_opaque(halo);
+  int64_t q = cs_opaque(q0);
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    b64_store(r1, voff + (uint32_t)(r * Ny * 8), odd ? U1[r] : U0[r]);
-    b64_store(r2, voff + (uint32_t)(r * Ny * 8), odd ? U0[r] : U1[r]);
+    if ((hm >> r) & 1u) {
+      V0[r] = cs_dev_load(in1 + q);
+      V1[r] = cs_dev_load(in2 + q);
+    }
+    q += a.Ny;
+  }
+}
+
+// A forward workgroup's tile and its sweeps: set-up, the steps n0 .. n0 +
+// nsteps - 1 (after an even number u_n is in U0, else in U1) and write-back.
+// DEV: the state is shared with the other workgroups of the launch.
+template <int R, bool REC, bool UH, bool DEV>
+struct Fwd64 {
+  CsGeom g;
+  CsTap tap;
+  int b, row0, srows;
+  uint32_t voff, vmask, omask;  // cs_out_voff; cells of the region; output rows
+  int64_t q0;                   // first cell
+  bool wave_src, one_src;
+  double *buf0, *buf1, *xs;
+  double U0[R], U1[R], KA[R], KB[R], KC[R];
+
+  __device__ __forceinline__ void setup(const F64Blk &a, int w, const double *in1,
+                                        const double *in2) {
+    extern __shared__ double smem64[];
+    __shared__ int own[1024];  // source rows of each thread, a bit mask
+    const int tid = threadIdx.x;
+    b = w / a.ntiles;
+    const int32_t *td = a.tiles + (w - b * a.ntiles) * TILE_W;
+    g = cs_geom<R>(td, tid);
+    const int NBUF = (g.RW + 2) * g.CS;
+    buf0 = smem64;
+    buf1 = smem64 + NBUF;
+    xs = smem64 + 2 * NBUF;
+    const int nsp = min(td[9] - td[8], CS_MAX_TABLE), ntp = min(td[11] - td[10], CS_MAX_TABLE);
+    row0 = g.k * R;
+    q0 = ((int64_t)b * a.Nx + g.R0 + row0) * a.Ny + g.C0 + g.c;
+    vmask = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      double u1 = 0., u2 = 0., v0 = 0., v1 = 0., v2 = 0.;
+      if (g.active && row0 + r < g.RH) {
+        vmask |= 1u << r;
+        const int64_t q = (int64_t)(g.R0 + row0 + r) * a.Ny + (g.C0 + g.c);
+        v0 = a.A[q]; v1 = a.Bm[q]; v2 = a.C2[q];
+        if (in1) {
+          const int64_t o = q0 + (int64_t)r * a.Ny;
+          u1 = DEV ? cs_dev_load(in1 + o) : in1[o];
+          u2 = DEV ? cs_dev_load(in2 + o) : in2[o];
+        }
+      }
+      U0[r] = u1; U1[r] = u2; KA[r] = v0; KB[r] = v1; KC[r] = v2;
+    }
+    int spx0 = 0, spx1 = 0, spx2 = 0, te[TAP_W];
+    if (tid < nsp) {
+      const int32_t *e = a.spx + (td[8] + tid) * SPX_W;
+      spx0 = e[0]; spx1 = e[1]; spx2 = e[2];
+    }
+    cs_tap_load(a.taps, td[10], ntp, te);
+    own[tid] = 0;
+    cs_zero_lds<double>(buf0, buf1, g, ((g.RH + R - 1) / R) * R, NBUF);
+    __syncthreads();
+    fill();
+    // source pixels mark the rows of their owners
+    for (int kk = tid; kk < nsp; kk += blockDim.x) {
+      if (kk != tid) {  // more entries than threads
+        const int32_t *e = a.spx + (td[8] + kk) * SPX_W;
+        spx0 = e[0]; spx1 = e[1]; spx2 = e[2];
+      }
+      int rr;
+      const int t = spx2 > 0 ? cs_owner<R>(g, spx0, spx1, rr) : -1;
+      if (t >= 0) atomicOr(&own[t], 1 << rr);
+    }
+    __syncthreads();
+    tap = cs_tap(g, a.taps, td[10], ntp, te);
+    srows = own[tid];
+    wave_src = __ballot(srows != 0) != 0;
+    one_src = __ballot((srows & (srows - 1)) != 0) == 0;
+    voff = cs_out_voff<double>(g, row0, a.Ny);
+    omask = cs64_out_rows<R>(g, row0, voff, vmask);
+  }
+  __device__ __forceinline__ void fill() {
+    if (g.active) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) buf0[g.base + r] = U0[r];
+    }
+  }
+  // the input samples of a chunk (a barrier must follow)
+  __device__ __forceinline__ void prepare(const F64Blk &a, int n0, int nsteps) {
+    for (int i = cs_opaque((int)threadIdx.x); i < nsteps; i += blockDim.x)
+      xs[i] = a.x[(int64_t)b * a.T + n0 + i];
+  }
+  __device__ __forceinline__ void run(const F64Blk &a, int n0, int nsteps) {
+    const int Ny = a.Ny;
+    const int64_t F = (int64_t)a.Nx * Ny;
+    const int64_t out_bytes = (int64_t)(g.or1 - g.or0) * Ny * 8;
+    const uint32_t voff = cs_opaque(this->voff);
+    const int live = cs_live_steps<R>(g, row0, nsteps);
+    const double *recp = REC ? a.rec + ((int64_t)b * a.T + n0) * F + (int64_t)g.or0 * Ny : a.A;
+    const int64_t yo = ((int64_t)b * a.T + n0) * a.ntap + tap.pcol;
+    double *yp = a.y ? a.y + yo : nullptr, *yrp = a.yraw ? a.yraw + yo : nullptr;
+    // next snapshot: at step `snap`
+    int snap = a.fields ? a.fstride - 1 - n0 % a.fstride : -1;
+    const double *fp = a.fields ? a.fields +
+                                      ((int64_t)b * (a.T / a.fstride) + n0 / a.fstride) * F +
+                                      (int64_t)g.or0 * Ny
+                                : a.A;
+
+    auto step = [&](const double *P, double *Q, double(&Uc)[R], double(&Up)[R], int s) {
+      if (s < live) {
+        const __amdgpu_buffer_rsrc_t rsl = cs_rsrc(recp, REC ? out_bytes : 0);
+        const int lfb = g.base - g.CS, rtb = g.base + g.CS;
+        double upv = UH ? P[g.base - 1] : a.t1 * P[g.base - 1];
+        double ctv = UH ? 0.0 : a.t1 * Uc[0];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const double ct = Uc[r];
+          const double dn = (r < R - 1) ? Uc[r + 1] : P[g.base + R];
+          const double lf = P[lfb + r], rt = P[rtb + r];
+          double lap;
+          if (UH) {  // products with t1 = 1 and t4 = -4 are exact
+            double s0 = upv + lf;
+            s0 = __builtin_fma(-4.0, ct, s0);
+            s0 = s0 + rt;
+            lap = s0 + dn;
+            upv = ct;
+          } else {
+            const double dnv = a.t1 * dn;
+            double s0 = upv + a.t1 * lf;
+            s0 = s0 + a.t4 * ct;
+            s0 = s0 + a.t1 * rt;
+            lap = s0 + dnv;
+            upv = ctv;
+            ctv = dnv;
+          }
+          const double p1 = a.s2 * ct;
+          const double p2 = KB[r] * Up[r];
+          const double p3 = KC[r] * lap;
+          const double v = KA[r] * ((p1 - p2) + p3);
+          Up[r] = v;
+          Q[g.base + r] = v;
+          if (REC) b64_store(rsl, voff + (uint32_t)(r * Ny * 8), lap);
+        }
+        if (wave_src) cs_add_source<R>(Up, Q + g.base, srows, one_src, xs[s]);
+        if (s == snap) {  // the thread's own rows: consecutive lanes, consecutive columns
+          const __amdgpu_buffer_rsrc_t rf = cs_rsrc(fp, out_bytes);
+#pragma unroll
+          for (int r = 0; r < R; ++r) b64_store(rf, voff + (uint32_t)(r * Ny * 8), Up[r]);
+        }
+      }
+      if (s == snap) {
+        snap += a.fstride;
+        fp += F;
+      }
+      if (REC) recp += F;
+      __syncthreads();
+      if (tap.pidx >= 0) {
+        const double v = Q[tap.pidx];
+        if (yp) {
+          *yp = tap.pkind ? v * v : v;
+          yp += a.ntap;
+        }
+        if (yrp) {
+          *yrp = v;
+          yrp += a.ntap;
+        }
+      }
+    };
+    int s = 0;
+    for (; s + 1 < nsteps; s += 2) {
+      step(buf0, buf1, U0, U1, s);
+      step(buf1, buf0, U1, U0, s + 1);
+    }
+    if (s < nsteps) step(buf0, buf1, U0, U1, s);
+  }
+  // u_n to U0 (DEV), and the output rows to (o1, o2)
+  __device__ __forceinline__ void store(const F64Blk &a, int nsteps, double *o1, double *o2) {
+    cs64_store<R, DEV>(a, g, U0, U1, nsteps, voff, omask, q0, b, o1, o2);
+  }
+  // the halo of the next chunk
+  __device__ __forceinline__ void refill(const F64Blk &a, const double *in1, const double *in2) {
+    cs64_halo<R>(a, U0, U1, vmask & ~omask, q0, in1, in2);
+    fill();
+  }
+};
+
+// One launch of nsteps steps.
+template <int NT, int R, bool REC, bool UH>
+__global__ __launch_bounds__(NT) void k64_fwd_cs(F64Blk a) {
+  Fwd64<R, REC, UH, false> S;
+  S.setup(a, xcd_remap(blockIdx.x, gridDim.x), a.in1, a.in2);
+  S.prepare(a, a.n0, a.nsteps);
+  __syncthreads();
+  S.run(a, a.n0, a.nsteps);
+  S.store(a, a.nsteps, a.out1, a.out2);
+}
+
+// The whole forward in one resident launch, in chunks of nsteps steps (the
+// scheme stands in wt_colseg.h); out1: two alternating state pairs.  (150 x
+// 140, 16 samples, 1200 steps: 75 launches of 24.0 us, resident 1377 us.  The
+// adjoint gained nothing from it: its registers spill in the walk, 1784 us
+// against 75 launches of 23.3 us.)
+template <int NT, int R, bool REC, bool UH>
+__global__ __launch_bounds__(NT) void k64_fwd_walk(F64Blk a) {
+  const int tid = threadIdx.x;
+  const int64_t BF = (int64_t)a.B * a.Nx * a.Ny;
+  const int nchunks = (a.T + a.nsteps - 1) / a.nsteps;
+  auto pair = [&](int chunk) { return a.out1 + (chunk & 1) * 2 * BF; };
+  auto steps = [&](int chunk) { return min(a.nsteps, a.T - chunk * a.nsteps); };
+  auto start = [&](int chunk) { return chunk * a.nsteps; };
+  __shared__ int own_w[CS_WALK_MAX], own_n[CS_WALK_MAX];
+  __shared__ int msg;
+  int w = xcd_remap(blockIdx.x, gridDim.x);
+  if (tid == 0) msg = atomicCAS(a.prog + w * CS_WALK_W, 0, 1);
+  __syncthreads();
+  if (msg != 0) return;  // a neighbour took it over
+  Fwd64<R, REC, UH, true> S;
+  int chunk = 0, got;
+  {
+    const int b = w / a.ntiles;
+    const int nbr = tid < 64 ? cs_walk_neighbours(a.tiles, a.ntiles, w - b * a.ntiles) : 0;
+    S.setup(a, w, nullptr, nullptr);
+    S.prepare(a, start(0), steps(0));
+    __syncthreads();
+    while (true) {
+      S.run(a, start(chunk), steps(chunk));
+      if (chunk + 1 == nchunks) return;
+      S.store(a, steps(chunk), pair(chunk), pair(chunk) + BF);
+      cs_walk_raise(a.prog, w, chunk);
+      ++chunk;
+      S.prepare(a, start(chunk), steps(chunk));
+      if (tid < 64) {
+        const int r = cs_walk_wait(a.prog, a.ntiles, b, nbr, chunk);
+        if (tid == 0) msg = r;
+      }
+      __syncthreads();
+      got = msg;
+      if (got != -1) break;
+      S.refill(a, pair(chunk - 1), pair(chunk - 1) + BF);
+      __syncthreads();
+    }
+  }
+  // Work items taken over: from here on every chunk of this workgroup starts
+  // with a whole set-up.
+  int nown = 1, at = 0;
+  while (true) {
+    if (got == -2) {  // given up: probe outputs from this chunk on are NaN
+      const double nan = __builtin_nan("");
+      const int64_t o = (int64_t)(w / a.ntiles) * a.T * a.ntap;
+      for (int64_t i = (int64_t)chunk * a.nsteps * a.ntap + tid; i < (int64_t)a.T * a.ntap;
+           i += blockDim.x) {
+        if (a.y) a.y[o + i] = nan;
+        if (a.yraw) a.yraw[o + i] = nan;
+      }
+      return;
+    }
+    if (got >= 0) {
+      if (tid == 0) {
+        own_w[at] = w;
+        own_n[at] = chunk;
+        own_w[nown] = got;
+        own_n[nown] = 0;
+      }
+      ++nown;
+    } else {
+      const double *in1 = chunk ? pair(chunk - 1) : nullptr;
+      S.setup(a, w, in1, in1 + BF);
+      S.prepare(a, start(chunk), steps(chunk));
+      __syncthreads();
+      S.run(a, start(chunk), steps(chunk));
+      S.store(a, steps(chunk), pair(chunk), pair(chunk) + BF);
+      cs_walk_raise(a.prog, w, chunk);
+      ++chunk;
+      if (chunk == nchunks && --nown == 0) return;
+      if (tid == 0) {
+        own_n[at] = chunk;
+        if (chunk == nchunks) {
+          own_w[at] = own_w[nown];
+          own_n[at] = own_n[nown];
+        }
+      }
+    }
+    __syncthreads();
+    at = 0;  // the least advanced one next
+    for (int i = 1; i < nown; ++i)
+      if (own_n[i] < own_n[at]) at = i;
+    w = own_w[at];
+    chunk = own_n[at];
+    if (tid < 64) {
+      const int r =
+          chunk > 0 ? cs_walk_wait(a.prog, a.ntiles, w / a.ntiles,
+                                   cs_walk_neighbours(a.tiles, a.ntiles, w % a.ntiles), chunk)
+                    : -1;
+      if (tid == 0) msg = r;
+    }
+    __syncthreads();
+    got = msg;
   }
 }
 
@@ -401,8 +615,12 @@ static hipError_t launch64(K kfn, std::atomic<uint64_t> &done, const F64Blk &a, 
 
 template <int R, bool REC, bool UH>
 static hipError_t launch64_fwd(const F64Blk &a, int nthreads, size_t shmem, hipStream_t s) {
-  static std::atomic<uint64_t> done{0};
-  return launch64(k64_fwd_cs<1024, R, REC, UH>, done, a, nthreads, shmem, s);
+  static std::atomic<uint64_t> done[2];
+  if constexpr (R <= 6) {
+    if (a.prog)
+      return launch64(k64_fwd_walk<1024, R, REC, UH>, done[1], a, nthreads, shmem, s);
+  }
+  return launch64(k64_fwd_cs<1024, R, REC, UH>, done[0], a, nthreads, shmem, s);
 }
 
 template <int R>
@@ -421,14 +639,22 @@ static hipError_t launch64_adj(const F64Blk &a, int nthreads, size_t shmem, hipS
   return launch64(k64_adj_cs<1024, R>, done, a, nthreads, shmem, s);
 }
 
+// Whether the forward over these tiles runs as one resident launch: more than
+// one chunk, a workgroup for each CU at most, and at most 6 rows per thread
+// (8 spill 41 registers in the walk).
+static bool walks64(const PlanView &v, const TileView &t) {
+  return v.T > t.tb && (int64_t)v.B * t.ntiles <= std::min(CS_WALK_MAX, device_cus()) && t.R <= 6;
+}
+
 // Workspace layout in doubles.  saved: A, Bm, C2, the probe amplitudes and
 // lap(u_n) of every step; temp: two state pairs and, forward without
-// gradients, the coefficients, or, adjoint, the gradient sum and lambda at
-// the source slots.
+// gradients, the coefficients, then a resident launch's progress words, or,
+// adjoint, the gradient sum and lambda at the source slots.
 struct Blk64 {
+  static constexpr int64_t words = CS_WALK_MAX * CS_WALK_W / 2;
   int64_t F, BF, yraw, rec, gsrc;
   int64_t saved() const { return 3 * F + yraw + rec; }
-  int64_t fwd_temp() const { return 4 * BF + 3 * F; }
+  int64_t fwd_temp() const { return 4 * BF + 3 * F + words; }
   int64_t adj_temp() const { return 5 * BF + gsrc; }
 };
 static Blk64 blk64(const PlanView &v) {
@@ -520,16 +746,22 @@ extern "C" int wt_loop_fwd_rec_f64(void *plan, const wt_scalars_f64 *sc, const d
     a.rec = a.yraw + w.yraw;
   }
   const size_t shmem = cs64_shmem_bytes(t.R, t.RHmax, t.RWmax, t.tb);
+  const bool walk = walks64(v, t);
+  if (walk) {
+    a.prog = (int *)(st + w.fwd_temp() - w.words);
+    WT_HIP(launch_fill64(st + w.fwd_temp() - w.words, w.words, 0.0, s));
+  }
   int pp = 0;
   for (int n = 0; n < v.T; n += t.tb, pp ^= 1) {
     a.n0 = n;
-    a.nsteps = std::min(t.tb, v.T - n);
+    a.nsteps = walk ? t.tb : std::min(t.tb, v.T - n);
     a.out1 = st + 2 * pp * w.BF;
     a.out2 = a.out1 + w.BF;
     hipError_t e = t.R == 4   ? launch64_fwd<4>(with_grad, sc->h == 1.0, a, t.nthreads, shmem, s)
                    : t.R == 6 ? launch64_fwd<6>(with_grad, sc->h == 1.0, a, t.nthreads, shmem, s)
                               : launch64_fwd<8>(with_grad, sc->h == 1.0, a, t.nthreads, shmem, s);
     WT_HIP(e);
+    if (walk) break;
     a.in1 = a.out1;
     a.in2 = a.out2;
   }
