@@ -94,8 +94,8 @@ def auto_interval(cfg: LoopConfig, B: int, T: int, budget: int, K0: int) -> int:
     at most `budget` bytes, else a half, third or quarter of it when that
     does, else K0.  Recording a step in the forward costs a store per cell;
     recomputing it costs the step again: 150x150, batch 64, 3000 steps,
-    training step 14.3 ms at K0 = 64 and 9.9 ms with the whole record
-    (17.4 GB); 100x100, batch 4, 1000 steps 2.80 and 2.00 ms."""
+    training step 13.9 ms at K0 = 64 and 8.7 ms with the whole record
+    (17.4 GB), which also lets each sweep run as one resident launch."""
     step = (8 if cfg.nonlinear else 4) * B * cfg.Nx * (cfg.Ny + 1)
     for n in (1, 2, 3, 4):
         K = -(-T // n)

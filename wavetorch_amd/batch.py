@@ -45,7 +45,7 @@ def _open_interval(instances, K: int, device) -> int:
     instance (lap u, packed by the instances' lengths) takes at most an eighth
     of the device's memory, else K: the adjoint then recomputes nothing (20
     instances of sides 64 to 256 and 1000 to 4000 steps, forward + adjoint
-    15.4 ms at K = 64, 10.8 ms with the 3.9 GB record)."""
+    15.4 ms at K = 64, 10.5 ms with the 3.9 GB record)."""
     T = max(inst.length for inst in instances)
     size = sum(4 * i.cfg.Nx * (i.cfg.Ny + 1) * i.length for i in instances)
     return T if T > K and size <= torch.cuda.get_device_properties(device).total_memory // 8 else K

@@ -888,9 +888,9 @@ __device__ __forceinline__ void adj_walk_sum(const AdjArgs &a, const float (&G)[
 // record of a chunk's first steps and its probe seeds are read before the
 // wait for the neighbours.  The gradient is summed chunk by chunk, as the
 // launches of the other path do, in registers where there is room (KEEP).
-// (us per pass, a launch per chunk and resident: 150 x 150, 64 samples, 1000
-// steps 9876 and 8729, 100 x 100, 4 samples, forward and backward 1259 and
-// 1126, 500 steps of one sample 1210 and 1063.)
+// (us of a training step, a launch per chunk and resident: 150 x 150, 64
+// samples, 3000 steps 9876 and 8729; 100 x 100, 4 samples, 1000 steps 1259
+// and 1126; 500 x 380, one sample, 800 steps 1210 and 1063.)
 template <int NT, int R>
 __global__ __launch_bounds__(NT) void k_adj_cs_walk(AdjArgs a) {
   const int tid = threadIdx.x;

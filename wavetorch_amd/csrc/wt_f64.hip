@@ -1,4 +1,6 @@
-// wt_f64.hip -- the WaveRNN time loop in double precision (gfx950).
+// wt_f64.hip -- the WaveRNN time loop in double precision, a launch per step
+// (gfx950): the nonlinear cell, dJ/db and field seeds (the linear cell's other
+// sweeps run blocked, wt_f64_blocked.hip).
 //
 // The reference computes in float64 when a user calls set_dtype('float64')
 // (utils.py:14-20; its own example configurations train that way).  This path

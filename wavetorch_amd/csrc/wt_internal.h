@@ -242,8 +242,8 @@ extern __device__ unsigned long long *wt_phase_ts;
 // q + e r), within about half an ulp of the IEEE quotient for the
 // normal-range operands met there (1 + q^2, its square, dt^-2 + b dt^-1, the
 // threshold uth).  Four instructions instead of the ten of the IEEE
-// sequence; the forward kernels keep IEEE division (their results are
-// compared bit for bit).
+// sequence; the forward's quotients (wt_colseg.hip) take one correction more
+// and are correctly rounded (they are compared bit for bit).
 __device__ __forceinline__ float adj_div(float a, float b) {
   const float r = __builtin_amdgcn_rcpf(b);
   const float q = a * r;

@@ -924,7 +924,8 @@ static int plan_build(const wt_config *cfg, int32_t B, int32_t T, float cmax_geo
   // Every grid step runs blocked: off h = 1 the forward pays four more VALU
   // operations per cell-step and the adjoint none, against one launch and
   // three field passes per step (150x150, batch 32, 1500 steps, h = 1.43,
-  // training step: 27.0 ms plain, 5.9 ms blocked).  The flat family's
+  // training step with checkpoints every 64 steps: 27.0 ms plain, 5.9 ms
+  // blocked).  The flat family's
   // kernels take h = 1 only.
   bool tiled = !tun.plain && (p->unit_h || tun.kind == 0);
   if (tiled) {

@@ -18,8 +18,8 @@ def to_tensor(x, dtype=None):
 
 def set_dtype(dtype=None):
     """utils.py:14-20.  Modules built after set_dtype('float64') hold float64
-    buffers and run the double-precision time loop (one launch per step,
-    every field kept); float32 runs the temporally blocked kernels."""
+    buffers and run the double-precision time loop (temporally blocked for
+    the linear cell, one launch per step with every field kept otherwise)."""
     if dtype == 'float32' or dtype is None:
         torch.set_default_dtype(torch.float32)
     elif dtype == 'float64':
