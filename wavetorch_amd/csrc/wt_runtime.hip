@@ -640,8 +640,8 @@ static double launch_us(const BlockModel &m, int R, int waves, int occ, int perc
 // cache lines: 1 + edge 32 / tw) and of the state (`state` per cell, `lines`
 // per cache line of halo and output rows).  Fitted to 10000 forwards, 2000
 // nonlinear ones and 3700 adjoints on the cheapest tilings of 80 to 340
-// random problems each: 5 to 6% rms, the choice 2 to 3% slower on average
-// than the fastest of 18 candidates measured.
+// random problems each: 5 to 6% rms, the choice 1.5 to 3% slower on
+// average than the fastest of 18 candidates measured.
 struct WalkModel {
   double ts, tR, e, cw, issue, row, cone, rec, edge, state, lines;
   int rows[5];
@@ -652,6 +652,8 @@ static const WalkModel kWalkLinAdj = {1.71, 0.0411, 0.262, 0.0, 0.0222, 0.0599, 
                                       3.48e-6, 0.0, {4, 6, 8, 10, 0}};
 static const WalkModel kWalkNl = {2.5, 0.0547, 0.0, 0.372, 0.0545, 0.14, 0.963, 0.152, 2.0, 0.0,
                                   4.48e-6, {4, 6, 8, 0, 0}};
+static const WalkModel kWalk64 = {2.22, 0.0423, 0.0, 0.209, 0.0266, 0.0827, 0.929, 0.178, 1.4,
+                                  1.19e-6, 8.6e-6, {4, 6, 0, 0, 0}};
 
 // (an interior tile of s strips and c columns)
 static double walk_us(const WalkModel &m, int R, int waves, int s, int c, int th, int tw, int RH,
@@ -781,7 +783,7 @@ static void plan_f64(Plan &plan) {
     }
     if (!ok) {
       for (const BlockChoice &ch : cheapest_blocks(
-               fwd ? kModel64 : kModel64Adj, nullptr, p.Nx, p.Ny, p.B, p.T, 0, 32,
+               fwd ? kModel64 : kModel64Adj, fwd ? &kWalk64 : nullptr, p.Nx, p.Ny, p.B, p.T, 0, 32,
                [](int R, int RH, int RW, int tb) {
                  return cs64_shmem_bytes(R, RH, RW, tb) + 16 * 1024;
                })) {
