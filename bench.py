@@ -31,7 +31,7 @@ Prints ONE JSON line:
   plain          the same step with the one-launch-per-step kernels
 
 `--dtype float64` times a training workload in double precision instead (the
-per-step float64 kernels; its roofline is algorithmic bytes over the launch
+float64 kernels; its roofline is unavoidable bytes over the launch
 time of the longer sweep, from HIP events).
 """
 from __future__ import annotations
@@ -382,12 +382,14 @@ def run_f64(args, dev):
     """The training step of a "train" workload in float64 (set_dtype('float64'),
     the precision the reference's example configurations train in): geometry
     and loss as torch ops in float64, the double-precision time loop
-    (k64_fwd one launch per step, the adjoint as one k64_adj launch per
-    step over the stored fields).  HIP events on the launch stream bracket
-    the forward sweep and the backward of each timed step; the roofline is
-    that of the sweep that takes longer, at its algorithmic bytes (24 B per
-    cell-step forward: read u_n, u_{n-1}, write u_{n+1}; 32 B adjoint: read
-    lambda_{m+1}, lambda_{m+2}, u_m, write lambda_m)."""
+    (the linear cell temporally blocked, with a record of lap(u); the
+    nonlinear one a launch per step over the stored fields).  HIP events on
+    the launch stream bracket the forward sweep and the backward of each timed
+    step; the roofline is that of the sweep that takes longer: the bytes it
+    cannot avoid, 8 B per cell-step of record for the blocked kernels, the
+    algorithmic 24 B (forward: read u_n, u_{n-1}, write u_{n+1}) and 32 B
+    (adjoint: read lambda_{m+1}, lambda_{m+2}, u_m, write lambda_m) for the
+    others."""
     from wavetorch_amd.utils import normalize_power, set_dtype
     wl = WORKLOADS[args.workload]
     set_dtype("float64")
@@ -422,26 +424,19 @@ def run_f64(args, dev):
             bwd_ms += ev[1].elapsed_time(ev[2]) / args.steps
         log(f"[bench] float64 sweeps: forward {fwd_ms:.2f} ms, backward {bwd_ms:.2f} ms")
         fwd = fwd_ms >= bwd_ms
-        kname = "k64_fwd" if fwd else "k64_adj"
+        blocked = not next(iter(model._plans.values())).cfg.nonlinear
+        kname = ("wt::k64_fwd" if fwd else "wt::k64_adj") + ("_cs" if blocked else "")
         avg_s = (fwd_ms if fwd else bwd_ms) / 1e3 / T
         per_launch = B * Nx * Ny
         byts = (24.0 if fwd else 32.0) * per_launch
-        eff = {"basis": f"{byts / per_launch:g} algorithmic B per cell-step x cells / launch "
-                        "time", "achieved": round(byts / avg_s / 1e9, 1), "unit": "GB/s",
+        eff = {"basis": f"{byts / per_launch:g} algorithmic B per cell-step x cells / time per "
+                        "step (not a bound)", "achieved": round(byts / avg_s / 1e9, 1), "unit": "GB/s",
                "frac_of_hbm_peak": round(byts / avg_s / PEAK_HBM, 4)}
-        # counter bytes (profiles/traffic_<workload>_f64.json, --summarize-pmc)
-        knames = ["wt::k64_fwd"] if fwd else ["wt::k64_adj"]
-        ks = [kernel_counters(f"{args.workload}_f64", k, "float64") for k in knames]
-        traffic_b = (sum(k["hbm_bytes_per_launch"] for k in ks)
-                     if all(k.get("hbm_bytes_per_launch") for k in ks) else None)
-        if traffic_b:
-            roof = {"achieved": round(traffic_b / avg_s / 1e9, 1),
-                    "frac": round(traffic_b / avg_s / PEAK_HBM, 4),
-                    "basis": "HBM bytes counted by FETCH_SIZE + WRITE_SIZE (calibrated) per "
-                             "launch / launch time from HIP events over the sweep"}
-        else:
-            roof = {"achieved": eff["achieved"], "frac": eff["frac_of_hbm_peak"],
-                    "basis": eff["basis"]}
+        must = 8.0 * per_launch / avg_s if blocked else byts / avg_s
+        roof = {"achieved": round(must / 1e9, 1), "frac": round(must / PEAK_HBM, 4),
+                "basis": ("8 B of record per cell-step" if blocked else
+                          f"{byts / per_launch:g} algorithmic B per cell-step") +
+                         " x cells / time per step from HIP events over the sweep"}
         out = {
             "metric": wl["metric"].replace("Gcell-steps/s (", "Gcell-steps/s (float64, "),
             "value": round(cells / dt / 1e9, 3),
@@ -455,8 +450,8 @@ def run_f64(args, dev):
                        "Nx": Nx, "Ny": Ny, "T": T},
             "roofline": {"kernel": kname, "bound": "hbm", "achieved": roof["achieved"],
                          "peak": PEAK_HBM / 1e9, "unit": "GB/s", "frac": roof["frac"],
-                         "basis": roof["basis"], "avg_launch_us": round(avg_s * 1e6, 2),
-                         "traffic": traffic_b, "effective_bw": eff,
+                         "basis": roof["basis"], "us_per_time_step": round(avg_s * 1e6, 2),
+                         "traffic": None, "effective_bw": eff,
                          "forward_ms_per_step": round(fwd_ms, 3),
                          "backward_ms_per_step": round(bwd_ms, 3)},
             "loss_finite": bool(np.isfinite(float(loss.detach()))),
