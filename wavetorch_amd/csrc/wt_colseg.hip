@@ -61,8 +61,9 @@ __device__ __forceinline__ void cs_rec_store(__amdgpu_buffer_rsrc_t rs, uint32_t
 // method ("IA-64 and Elementary Functions", 2000): q = a y, r = a - b q,
 // q + r y, with y = 1/b to the last bit.  Checked on MI355X against the
 // general division for all 2^23 mantissas of the variable operand at 141
-// exponents and 1032 pairs of constants: not one differs.  Outside the normal
-// range the callers see to the operands.
+// exponents and 1032 pairs of constants: not one differs.  Configurations whose
+// operands would leave the normal range run other kernels (quotients_hold in
+// wt_runtime.hip).
 // a / b for a wave-uniform b with rb = 1/b (rounded to nearest)
 __device__ __forceinline__ float nl_div_by(float a, float b, float rb) {
   const float q = a * rb;

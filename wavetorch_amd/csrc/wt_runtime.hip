@@ -798,6 +798,22 @@ static void plan_f64(Plan &plan) {
   }
 }
 
+// Whether the blocked nonlinear forward's quotients (nl_div_by, nl_div and
+// nl_rcp of wt_colseg.hip, exact only where their reciprocals and residuals
+// are normal numbers) hold for this configuration: dt^-2 with room for b/dt
+// and a normal reciprocal, a threshold whose reciprocal is normal and whose
+// residuals do not underflow, and a b0 whose share at the cap of 1 + (u/uth)^2
+// is nothing against dt^-2.  Outside (a threshold of 0, which must give NaN;
+// dt of 1e-19) the per-step kernels with the general division run.
+static bool quotients_hold(const Plan &p) {
+  if (p.nl == 0) return true;
+  const float b0 = (p.nl & 1) ? p.sat_b0 : 0.0f;
+  if (!(p.dtm2 >= 0x1p-122f && p.dtm2 + b0 * p.dtm1 <= 0x1p122f)) return false;
+  if (!(p.nl & 1)) return true;
+  const float uth = std::fabs(p.sat_uth);
+  return uth >= 0x1p-80f && uth <= 0x1p100f && b0 <= p.dtm1 * 0x1p60f;
+}
+
 // Host half of plan creation: validation, special-pixel tables, tiling and
 // variant choice, workspace layout.  No device call except hipGetDevice.
 static int plan_build(const wt_config *cfg, int32_t B, int32_t T, float cmax_geom,
@@ -927,9 +943,8 @@ static int plan_build(const wt_config *cfg, int32_t B, int32_t T, float cmax_geo
   // operations per cell-step and the adjoint none, against one launch and
   // three field passes per step (150x150, batch 32, 1500 steps, h = 1.43,
   // training step with checkpoints every 64 steps: 27.0 ms plain, 5.9 ms
-  // blocked).  The flat family's
-  // kernels take h = 1 only.
-  bool tiled = !tun.plain && (p->unit_h || tun.kind == 0);
+  // blocked).  The flat family's kernels take h = 1 only.
+  bool tiled = !tun.plain && (tun.kind == 0 ? quotients_hold(*p) : p->unit_h);
   if (tiled) {
     int strips = tun.strips, tb = tun.tblock, nt = tun.nt, cpt = tun.cpt;
     // the nonlinear cell forms its coefficients (three divisions) per cell
