@@ -136,12 +136,14 @@ class WaveRNN(torch.nn.Module):
             total = torch.cuda.get_device_properties(device).total_memory
             tun["ck_every"] = auto_interval(cfg, B, T, total // 8, tun["ck_every"])
         tkey = tuple(sorted(tun.items()))
-        key = (cfg, B, T, str(device), tkey, group)
+        key = (cfg, B, T, str(device), tkey, group, self.cell.geom.b.dtype)
         p = self._plans.get(key)
         if p is None:
             if len(self._plans) > 8:
                 self._plans.clear()
-            if not self.tuning:  # no tiling asked for
+            # no tiling asked for: the model's choice (a float64 plan makes its
+            # own, for its own kernels, where none is given)
+            if not self.tuning and self.cell.geom.b.dtype != torch.float64:
                 tun = suggest(cfg, B, T, self.cell.geom.cmax, tun["ck_every"], group)
             p = Plan(cfg, B, T, self.cell.geom.cmax, device, tun, group)
             self._plans[key] = p
