@@ -19,7 +19,7 @@ def test_tiling_of_a_float64_plan(tuning, monkeypatch):
     asked = []
 
     class FakePlan:
-        def __init__(self, cfg, B, T, cmax, device, tuning=None, group=0):
+        def __init__(self, cfg, B, T, cmax, device, tuning=None, group=0, waiting=None):
             asked.append(dict(tuning or {}))
 
         def bytes_rec_f64(self):

@@ -1,0 +1,49 @@
+"""Whole records and the memory they take: one per model at a time, whatever
+the lengths."""
+import pytest
+import torch
+
+from tests.helpers import rel
+from wavetorch_amd import (WaveCell, WaveGeometryFreeForm, WaveIntensityProbe, WaveRNN,
+                           WaveSource)
+
+pytestmark = pytest.mark.gpu
+
+
+def _model(cuda, N=60):
+    geom = WaveGeometryFreeForm((N, N - 8), 1.0, c0=1.0, c1=0.5, abs_N=8, abs_sig=1.0, abs_p=2,
+                                rho="half")
+    return WaveRNN(WaveCell(0.7, geom), WaveSource(N // 4, N // 2),
+                   [WaveIntensityProbe(N - 16, N // 3), WaveIntensityProbe(N - 16, N // 2)]).to(cuda)
+
+
+def _x(cuda, B, T):
+    n = torch.arange(float(T))
+    return torch.stack([torch.sin(0.3 * n + k) * torch.exp(-((n - 60) / 25) ** 2)
+                        for k in range(B)]).to(cuda)
+
+
+def _grad(model, y):
+    model.zero_grad(set_to_none=True)
+    y.sum().backward()
+    return model.cell.geom.rho.grad.cpu().numpy()
+
+
+def test_one_record_at_a_time_over_lengths(cuda):
+    model = _model(cuda)
+    x1, x2 = _x(cuda, 3, 150), _x(cuda, 2, 130)
+    alone = _grad(model, model(x2))
+    y1 = model(x1)
+    y2 = model(x2)  # another length while y1's record waits
+    model._plans.clear()
+    y3 = model(x1)  # and with the waiting record's plan gone
+    used = sorted((p.B, p.T, p.tuning["ck_every"]) for p in model._plans.values())
+    assert (3, 150, 64) in used
+    g1 = _grad(model, y1)
+    assert rel(_grad(model, y2), alone) < 1e-5 and rel(_grad(model, y3), g1) < 1e-5
+    model._plans.clear()
+    y2 = model(x2)  # nothing waits any more
+    y1 = model(x1)
+    assert {(2, 130): 130, (3, 150): 64}.items() <= \
+        {(p.B, p.T): p.tuning["ck_every"] for p in model._plans.values()}.items()
+    assert torch.equal(y1, y3)

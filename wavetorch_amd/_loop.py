@@ -110,7 +110,7 @@ class Plan:
     """Owner of a library plan (validated config + device tables + tiling)."""
 
     def __init__(self, cfg: LoopConfig, B: int, T: int, cmax: float, device, tuning=None,
-                 group: int = 0):
+                 group: int = 0, waiting=None):
         self.cfg, self.B, self.T, self.device = cfg, B, T, device
         c, keep = cfg.to_c()
         tun = None
@@ -136,13 +136,22 @@ class Plan:
         _lib.check(L.wt_workspace_bytes(handle, 0, ctypes.byref(s0), ctypes.byref(t0)),
                    "wt_workspace_bytes")
         self.temp_bytes_nograd = t0.value
-        self._record = None  # weak reference to the last forward's workspace
+        # workspaces that record more than the default 64 steps and wait for
+        # their backward, as weak references; `waiting`: a table that several
+        # plans share (those of one model)
+        self._waiting = {} if waiting is None else waiting
 
     def record_waits(self) -> bool:
-        """True while a workspace of this plan that records more than the
-        default 64 steps waits for its backward."""
-        return (self.tuning["ck_every"] > 64 and self._record is not None
-                and self._record() is not None)
+        """True while a workspace of this plan, or of one that shares its
+        table, records more than the default 64 steps and waits for its
+        backward."""
+        return self.tuning["ck_every"] > 64 and bool(self._waiting)
+
+    def _wait(self, saved):
+        """Counts `saved` among the waiting records for as long as it lives."""
+        if self.tuning["ck_every"] > 64:
+            key, waiting = object(), self._waiting
+            waiting[key] = weakref.ref(saved, lambda _: waiting.pop(key, None))
 
     def bytes_f64(self, with_grad: bool):
         """(saved, temp) bytes of the float64 loop (wt_workspace_bytes_f64)."""
@@ -261,7 +270,7 @@ class WaveLoop(torch.autograd.Function):
         if with_grad:
             ctx.save_for_backward(x, c, b, rho_c if rho_c is not None else x.new_empty(0))
             ctx.ws = saved
-            plan._record = weakref.ref(saved)
+            plan._wait(saved)
             ctx.plan = plan
             ctx.rec64 = rec64
             ctx.has_rho = rho_c is not None

@@ -42,6 +42,7 @@ class WaveRNN(torch.nn.Module):
         self.check_finite = False
         self._nonfinite = None
         self._plans = {}
+        self._waiting = {}  # whole records of all plans that wait for a backward
         self._cfg_cache = None
 
     @property
@@ -145,7 +146,7 @@ class WaveRNN(torch.nn.Module):
             # own, for its own kernels, where none is given)
             if not self.tuning and self.cell.geom.b.dtype != torch.float64:
                 tun = suggest(cfg, B, T, self.cell.geom.cmax, tun["ck_every"], group)
-            p = Plan(cfg, B, T, self.cell.geom.cmax, device, tun, group)
+            p = Plan(cfg, B, T, self.cell.geom.cmax, device, tun, group, self._waiting)
             self._plans[key] = p
         return p
 
@@ -175,9 +176,10 @@ class WaveRNN(torch.nn.Module):
         c = geom.c
         b = geom.b
         rho = geom.rho if self.loop_config().nonlinear else None
-        # one whole record per model at a time: while a forward's record waits
-        # for its backward, further forwards keep checkpoints every 64 steps
-        # (the float64 loop keeps every field and has no interval)
+        # one whole record per model at a time, whatever the lengths and batch
+        # sizes: while a forward's record waits for its backward, further
+        # forwards keep checkpoints every 64 steps (the float64 loop keeps
+        # every field and has no interval)
         plan = self.plan(B, T, x.device, lean=x.dtype == torch.float64)
         if torch.is_grad_enabled() and plan.record_waits():
             plan = self.plan(B, T, x.device, lean=True)
