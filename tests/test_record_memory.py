@@ -1,11 +1,13 @@
 """Whole records and the memory they take: one per model at a time, whatever
-the lengths."""
+the lengths, and calls whose record does not fit run with checkpoints."""
+import weakref
+
 import pytest
 import torch
 
 from tests.helpers import rel
 from wavetorch_amd import (WaveCell, WaveGeometryFreeForm, WaveIntensityProbe, WaveRNN,
-                           WaveSource)
+                           WaveSource, rnn)
 
 pytestmark = pytest.mark.gpu
 
@@ -47,3 +49,22 @@ def test_one_record_at_a_time_over_lengths(cuda):
     assert {(2, 130): 130, (3, 150): 64}.items() <= \
         {(p.B, p.T): p.tuning["ck_every"] for p in model._plans.values()}.items()
     assert torch.equal(y1, y3)
+
+
+def test_retry_holds_nothing_of_the_failed_call(cuda, monkeypatch):
+    model = _model(cuda)
+    held = []
+
+    class Loop:
+        @staticmethod
+        def apply(*args):
+            if not held:
+                saved = torch.empty(1 << 20, device=cuda)
+                held.append(weakref.ref(saved))
+                raise torch.cuda.OutOfMemoryError("out of memory")
+            assert held[0]() is None
+            return rnn_loop.apply(*args)
+
+    rnn_loop = rnn.WaveLoop
+    monkeypatch.setattr(rnn, "WaveLoop", Loop)
+    assert torch.isfinite(model(_x(cuda, 2, 150))).all()

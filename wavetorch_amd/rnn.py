@@ -184,13 +184,15 @@ class WaveRNN(torch.nn.Module):
         if torch.is_grad_enabled() and plan.record_waits():
             plan = self.plan(B, T, x.device, lean=True)
         args = (fields_mode, stride, self._nonfinite_flags(x.device))
+        out = None
         try:
             out = WaveLoop.apply(x, c, b, rho, plan, *args)
         except torch.cuda.OutOfMemoryError:
-            lean = self.plan(B, T, x.device, lean=True)
-            if lean is plan:
-                raise
-            out = WaveLoop.apply(x, c, b, rho, lean, *args)
+            if plan.tuning["ck_every"] <= self.checkpoint_every:
+                raise  # no shorter interval to fall back to
+        if out is None:  # out of the handler, which holds the failed call's buffers
+            plan = self.plan(B, T, x.device, lean=True)
+            out = WaveLoop.apply(x, c, b, rho, plan, *args)
         if fields_mode:
             return out
         shp = self.probes[0].out_shape()  # from tensor shapes: no device read
