@@ -31,6 +31,22 @@ def _grad(model, y):
     return model.cell.geom.rho.grad.cpu().numpy()
 
 
+class _Limit:
+    """At most `nbytes` more device memory for torch than it holds now."""
+
+    def __init__(self, cuda, nbytes):
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        total = torch.cuda.get_device_properties(cuda).total_memory
+        self.fraction = (torch.cuda.memory_reserved(cuda) + nbytes) / total
+
+    def __enter__(self):
+        torch.cuda.set_per_process_memory_fraction(self.fraction)
+
+    def __exit__(self, *exc):
+        torch.cuda.set_per_process_memory_fraction(1.0)
+
+
 def test_one_record_at_a_time_over_lengths(cuda):
     model = _model(cuda)
     x1, x2 = _x(cuda, 3, 150), _x(cuda, 2, 130)
@@ -68,3 +84,18 @@ def test_retry_holds_nothing_of_the_failed_call(cuda, monkeypatch):
     rnn_loop = rnn.WaveLoop
     monkeypatch.setattr(rnn, "WaveLoop", Loop)
     assert torch.isfinite(model(_x(cuda, 2, 150))).all()
+
+
+def test_record_that_leaves_no_room_for_the_backward(cuda):
+    """The forward's own buffers would fit beside the record, the backward's
+    would not: the call runs with checkpoints."""
+    model, x = _model(cuda, 150), _x(cuda, 64, 150)
+    p = model.plan(64, 150, x.device)
+    assert p.tuning["ck_every"] == 150
+    room = p.saved_bytes + p.temp_bytes_nograd + (12 << 20)
+    assert room < p.saved_bytes + p.temp_bytes
+    ref = _grad(model, model(x))
+    with _Limit(cuda, room):
+        y = model(x)
+        g = _grad(model, y)
+    assert rel(g, ref) < 1e-5
