@@ -1,13 +1,16 @@
-"""Whole records and the memory they take: one per model at a time, whatever
-the lengths, and calls whose record does not fit run with checkpoints."""
+"""Whole records and the memory they take: one per model at a time whatever the
+lengths, and calls whose record does not fit run with checkpoints."""
 import weakref
 
+import numpy as np
 import pytest
 import torch
 
 from tests.helpers import rel
 from wavetorch_amd import (WaveCell, WaveGeometryFreeForm, WaveIntensityProbe, WaveRNN,
                            WaveSource, rnn)
+from wavetorch_amd._loop import LoopConfig
+from wavetorch_amd.batch import Instance, InstanceBatch
 
 pytestmark = pytest.mark.gpu
 
@@ -99,3 +102,31 @@ def test_record_that_leaves_no_room_for_the_backward(cuda):
         y = model(x)
         g = _grad(model, y)
     assert rel(g, ref) < 1e-5
+
+
+def test_batch_whose_record_does_not_fit(cuda):
+    rng = np.random.default_rng(3)
+    cfg = LoopConfig(Nx=200, Ny=200, dt=0.7, h=1.0, src_px=((20, 100, 0),), taps=((150, 90, 1),))
+    insts = [Instance(cfg, torch.zeros(200, 200), T, 1.0) for T in (1500, 1200, 900, 600)]
+    f = lambda a: torch.from_numpy(a.astype(np.float32)).to(cuda)
+    cs = [f(rng.uniform(0.5, 1.0, (200, 200))) for _ in insts]
+    xs = [f(rng.standard_normal(i.length)) for i in insts]
+    ys = [f(rng.standard_normal((i.length, 1))) for i in insts]
+
+    def run(bt):
+        bt.set_inputs(cs, xs, ys)
+        bt.fwd_adj()
+        return [t.clone() for o in bt.outputs() for t in o]
+
+    ref = run(InstanceBatch(insts, cuda, checkpoint_every=64))
+    open_ = InstanceBatch(insts, cuda)
+    assert open_.tuning[0]["ck_every"] == 1500
+    del open_
+    with _Limit(cuda, 400 << 20):  # the record takes 675 MB
+        bt = InstanceBatch(insts, cuda)
+        assert bt.tuning[0]["ck_every"] == 64
+        out = run(bt)
+    assert all(torch.equal(a, b) for a, b in zip(ref, out))
+    with _Limit(cuda, 400 << 20):  # what the caller asked for is not changed
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            InstanceBatch(insts, cuda, checkpoint_every=1500)

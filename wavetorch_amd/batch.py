@@ -62,19 +62,18 @@ class InstanceBatch:
     runs forward only and holds no saved workspace (checkpoints and the
     forward's record, the bulk of the memory of a one-segment plan).  A
     checkpoint interval given in `checkpoint_every` or in the tuning holds;
-    left open it is chosen by ``_open_interval``."""
+    left open it is chosen by ``_open_interval``, and 64 steps where the
+    record of the choice does not fit beside what the device holds."""
 
     def __init__(self, instances, device, tuning=None, checkpoint_every=_Open(64),
                  longest_first=True, grad=True):
         self.device = torch.device(device)
         self.instances = list(instances)
-        group = 0
+        self.grad = bool(grad)
         first = tuning[0] if isinstance(tuning, (list, tuple)) else tuning
+        default = every = int(checkpoint_every)
         if grad and isinstance(checkpoint_every, _Open) and not (first or {}).get("ck_every"):
-            group = int(checkpoint_every)  # the gradient sums of the default interval
-            checkpoint_every = _open_interval(self.instances, group, self.device)
-            if checkpoint_every == group:
-                group = 0
+            every = _open_interval(self.instances, default, self.device)
         groups = {}
         for i, inst in enumerate(self.instances):
             if inst.cfg.nonlinear:
@@ -93,6 +92,32 @@ class InstanceBatch:
             for k, i in enumerate(idx):
                 self.where[i] = (g, k)
         self.T = max(inst.length for inst in self.instances)
+        built = False
+        try:
+            # (adjoint launches that end at the default interval's multiples
+            # keep its gradient sums)
+            self._build(tuning, every, default if every != default else 0)
+            built = True
+        except torch.cuda.OutOfMemoryError:
+            if every == default:
+                raise
+        if not built:
+            self._release()
+            self._build(tuning, default, 0)
+
+    def _release(self):
+        """Gives the plan, the workspaces and the buffers back."""
+        if getattr(self, "_graph", None) is not None:
+            _lib.lib().wt_graph_destroy(self._graph)
+            self._graph = None
+        if getattr(self, "handle", None) is not None and self.handle.value:
+            _lib.lib().wt_batch_plan_destroy(self.handle)
+            self.handle = None
+        self.saved = self.temp = None
+        self.buf = []
+
+    def _build(self, tuning, checkpoint_every, group):
+        """The plan, the workspaces and the per-group buffers."""
         G = len(self.groups)
         cfgs = (_lib.WtConfig * G)()
         keep = []
@@ -136,7 +161,6 @@ class InstanceBatch:
         dev = self.device
         # the saved workspace (checkpoints, the forward's record) only when
         # gradients are wanted: forward-only batches run without it
-        self.grad = bool(grad)
         self.saved = (torch.empty(max(s0.value, 1), dtype=torch.uint8, device=dev)
                       if self.grad else None)
         self.temp = torch.empty(max(t0.value, 1), dtype=torch.uint8, device=dev)
@@ -164,12 +188,7 @@ class InstanceBatch:
 
     def __del__(self):
         try:
-            if getattr(self, "_graph", None) is not None:
-                _lib.lib().wt_graph_destroy(self._graph)
-                self._graph = None
-            if getattr(self, "handle", None) is not None and self.handle.value:
-                _lib.lib().wt_batch_plan_destroy(self.handle)
-                self.handle = None
+            self._release()
         except Exception:
             pass
 
