@@ -273,6 +273,12 @@ int wt_autotune(const wt_config *cfg, int32_t B, int32_t T, float cmax,
                 const float *c, const float *rho, const float *x, int32_t reps,
                 double budget_ms, wt_tuning *out, double *best_ms, void *stream);
 
+/* As wt_autotune, for plans that wt_plan_group is given `group` for (0: none). */
+int wt_autotune_group(const wt_config *cfg, int32_t B, int32_t T, float cmax,
+                      const wt_tuning *start, int32_t group, int32_t with_grad, const float *b,
+                      const float *c, const float *rho, const float *x, int32_t reps,
+                      double budget_ms, wt_tuning *out, double *best_ms, void *stream);
+
 /* ------------------------------------------------------------------------ */
 /* The time loop in double precision (set_dtype('float64'), utils.py:14-20)  */
 /* ------------------------------------------------------------------------ */

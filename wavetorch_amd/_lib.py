@@ -143,6 +143,10 @@ _SIGS = {
                                    ctypes.POINTER(WtTuning), c_i32, c_p, c_p, c_p, c_p, c_i32,
                                    ctypes.c_double, ctypes.POINTER(WtTuning),
                                    ctypes.POINTER(ctypes.c_double), c_p]),
+    "wt_autotune_group": (ctypes.c_int, [ctypes.POINTER(WtConfig), c_i32, c_i32, c_f32,
+                                         ctypes.POINTER(WtTuning), c_i32, c_i32, c_p, c_p, c_p,
+                                         c_p, c_i32, ctypes.c_double, ctypes.POINTER(WtTuning),
+                                         ctypes.POINTER(ctypes.c_double), c_p]),
     "wt_batch_plan_create": (ctypes.c_int, [c_i32, ctypes.POINTER(WtConfig),
                                             ctypes.POINTER(c_i32), ctypes.POINTER(c_i32),
                                             ctypes.POINTER(c_f32), ctypes.POINTER(WtTuning),

@@ -112,6 +112,7 @@ class Plan:
     def __init__(self, cfg: LoopConfig, B: int, T: int, cmax: float, device, tuning=None,
                  group: int = 0, waiting=None):
         self.cfg, self.B, self.T, self.device = cfg, B, T, device
+        self.group = int(group)
         c, keep = cfg.to_c()
         tun = None
         if tuning:

@@ -49,14 +49,20 @@ def _store(d):
 
 
 def key(Nx, Ny, B, T, K, arch=None, forward_only=False):
-    """Cache key of a problem shape; K is the checkpoint interval, or "open"
-    for tunings whose search chose it (they carry ``ck_every``)."""
+    """Cache key of a problem shape; K is the checkpoint interval, "open" for
+    tunings whose search chose it (they carry ``ck_every``), or "auto" for
+    those searched at the interval that a model which leaves it open takes."""
     return f"{arch or _arch()}:{Nx}x{Ny}:B{B}:T{T}:K{K}" + (":fwd" if forward_only else "")
 
 
 def lookup(Nx, Ny, B, T, K=64, arch="gfx950", forward_only=False):
+    """The cached tuning of a shape, or None; without one for the default
+    K = 64, that of a model which left K open."""
     with _lock:
-        e = _load().get(key(Nx, Ny, B, T, K, arch, forward_only))
+        d = _load()
+    e = d.get(key(Nx, Ny, B, T, K, arch, forward_only))
+    if e is None and K == 64:
+        e = d.get(key(Nx, Ny, B, T, "auto", arch, forward_only))
     return dict(e["tuning"]) if e else None
 
 
@@ -141,7 +147,9 @@ def tune(model, x, labels=None, steps=2, verbose=False, budget_s=300.0, rounds=2
     between good plans).  Starts from the library's own choice, tries every
     option of one field at a time (the rest fixed), keeps any improvement and
     repeats for `rounds` passes or until `budget_s`; caches the winner under
-    key(Nx, Ny, B, T, K) and returns it.  With `tune_k` the checkpoint
+    key(Nx, Ny, B, T, K) and returns it.  The search runs the interval that
+    the tuned model's calls will: the one set on the model, or, left open, the
+    one that the model chooses for this batch (K = "auto").  With `tune_k` the checkpoint
     interval is searched too, from the model's K (k_options; the winner
     carries ``ck_every`` and is cached under K = "open") -- for
     configurations that leave K open: more memory for fewer recomputed
@@ -153,9 +161,7 @@ def tune(model, x, labels=None, steps=2, verbose=False, budget_s=300.0, rounds=2
     Nx, Ny = model.cell.geom.domain_shape
     K = int(model.checkpoint_every)
     user_k = model._checkpoint_every
-    # the interval searched for is the model's, not the one an open model
-    # would choose per call
-    model.checkpoint_every = None if tune_k else K
+    model.checkpoint_every = None if tune_k else user_k
     t_start = time.perf_counter()
 
     def step():
@@ -239,9 +245,10 @@ def tune(model, x, labels=None, steps=2, verbose=False, budget_s=300.0, rounds=2
     best = _to_tuning(state)
     model.tuning = best
     model.checkpoint_every = user_k
+    kname = "open" if tune_k else "auto" if model.plan(B, T, x.device).group else K
     with _lock:
         d = _load()
-        d[key(Nx, Ny, B, T, "open" if tune_k else K, forward_only=forward_only)] = {
+        d[key(Nx, Ny, B, T, kname, forward_only=forward_only)] = {
             "tuning": best, "ms": best_t * 1e3}
         _store(d)
     return best
@@ -252,7 +259,9 @@ def tune_native(model, x, with_grad=True, reps=2, budget_s=120.0, store=True):
     fields, options and acceptance rule as :func:`tune`, timed with HIP events
     on the loop kernels alone -- forward, and with ``with_grad`` the
     checkpointed adjoint -- rather than on a whole training step) for
-    ``model`` on batch ``x`` at the model's checkpoint interval.  Returns the
+    ``model`` on batch ``x`` at the checkpoint interval that the model's calls
+    take (the one set on it, or, left open, the one that it chooses for this
+    batch: K = "auto").  Returns the
     winning tuning dict (also set as ``model.tuning``) and its time in ms;
     with ``store`` the winner is cached under key(Nx, Ny, B, T, K) like
     :func:`tune`'s."""
@@ -266,14 +275,17 @@ def tune_native(model, x, with_grad=True, reps=2, budget_s=120.0, store=True):
         b = geom.b.detach().contiguous()
         rho = geom.rho.detach().contiguous() if cfg.nonlinear else None
     xx = x.detach().contiguous()
-    K = int(model.checkpoint_every)
-    start = _lib.WtTuning(ck_every=K)
+    plan = model.plan(B, T, x.device)
+    start = _lib.WtTuning(ck_every=plan.tuning["ck_every"])
+    kname = "auto" if plan.group else int(model.checkpoint_every)
+    torch.cuda.empty_cache()  # the search allocates beside torch
     out = _lib.WtTuning()
     ms = ctypes.c_double(0.0)
     cc, keep = cfg.to_c()
     with torch.cuda.device(x.device):
-        _lib.check(_lib.lib().wt_autotune(
-            ctypes.byref(cc), B, T, float(geom.cmax), ctypes.byref(start), int(bool(with_grad)),
+        _lib.check(_lib.lib().wt_autotune_group(
+            ctypes.byref(cc), B, T, float(geom.cmax), ctypes.byref(start), plan.group,
+            int(bool(with_grad)),
             b.data_ptr(), c.data_ptr(), rho.data_ptr() if rho is not None else None,
             xx.data_ptr(), int(reps), float(budget_s * 1e3), ctypes.byref(out),
             ctypes.byref(ms), _lib.stream_ptr(x.device)), "wt_autotune")
@@ -284,7 +296,7 @@ def tune_native(model, x, with_grad=True, reps=2, budget_s=120.0, store=True):
     if store:
         with _lock:
             d = _load()
-            d[key(cfg.Nx, cfg.Ny, B, T, K, forward_only=not with_grad)] = {
+            d[key(cfg.Nx, cfg.Ny, B, T, kname, forward_only=not with_grad)] = {
                 "tuning": best, "ms": ms.value, "search": "wt_autotune"}
             _store(d)
     return best, ms.value

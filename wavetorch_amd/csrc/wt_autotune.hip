@@ -127,10 +127,10 @@ struct Entry {
 std::mutex g_mu;
 std::map<std::string, Entry> g_cache;
 
-std::string cache_key(const wt_config *cfg, int B, int T, int ck, int with_grad) {
+std::string cache_key(const wt_config *cfg, int B, int T, int ck, int group, int with_grad) {
   char buf[256];
-  std::snprintf(buf, sizeof(buf), "%dx%d:B%d:T%d:K%d:g%d:nl%g,%g,%g,%d:s%d:p%d", cfg->Nx,
-                cfg->Ny, B, T, ck, with_grad, cfg->sat_b0, cfg->sat_uth, cfg->c_nl,
+  std::snprintf(buf, sizeof(buf), "%dx%d:B%d:T%d:K%d,%d:g%d:h%g:nl%g,%g,%g,%d:s%d:p%d", cfg->Nx,
+                cfg->Ny, B, T, ck, group, with_grad, cfg->h, cfg->sat_b0, cfg->sat_uth, cfg->c_nl,
                 cfg->c_clamp, cfg->nsrc_px, cfg->ntap);
   return buf;
 }
@@ -141,9 +141,18 @@ extern "C" int wt_autotune(const wt_config *cfg, int32_t B, int32_t T, float cma
                            const wt_tuning *start, int32_t with_grad, const float *b,
                            const float *c, const float *rho, const float *x, int32_t reps,
                            double budget_ms, wt_tuning *out, double *best_ms, void *stream) {
+  return wt_autotune_group(cfg, B, T, cmax, start, 0, with_grad, b, c, rho, x, reps, budget_ms,
+                           out, best_ms, stream);
+}
+
+extern "C" int wt_autotune_group(const wt_config *cfg, int32_t B, int32_t T, float cmax,
+                                 const wt_tuning *start, int32_t group, int32_t with_grad,
+                                 const float *b, const float *c, const float *rho, const float *x,
+                                 int32_t reps, double budget_ms, wt_tuning *out, double *best_ms,
+                                 void *stream) {
   const char *what = "wt_autotune";
-  if (!cfg || !b || !c || !x || !out) {
-    set_error("%s: invalid argument (null pointer)", what);
+  if (!cfg || !b || !c || !x || !out || group < 0) {
+    set_error("%s: invalid argument (null pointer or negative group)", what);
     return WT_EINVAL;
   }
   if (reps < 1 || reps > 100 || !(budget_ms > 0)) {
@@ -160,7 +169,7 @@ extern "C" int wt_autotune(const wt_config *cfg, int32_t B, int32_t T, float cma
   wt_tuning base;
   int rc = wt_plan_resolve(cfg, B, T, cmax, &base_req, &base, nullptr, nullptr);
   if (rc != WT_OK) return rc;
-  const std::string key = cache_key(cfg, B, T, base.ck_every, with_grad);
+  const std::string key = cache_key(cfg, B, T, base.ck_every, group, with_grad);
   {
     std::lock_guard<std::mutex> lk(g_mu);
     auto it = g_cache.find(key);
@@ -220,7 +229,8 @@ extern "C" int wt_autotune(const wt_config *cfg, int32_t B, int32_t T, float cma
     void *plan = nullptr;
     if (wt_plan_create(cfg, B, T, cmax, &t, &plan) != WT_OK) return WT_OK;  // skipped
     int64_t sb = 0, tb = 0;
-    int r = wt_workspace_bytes(plan, with_grad, &sb, &tb);
+    int r = group > 0 ? wt_plan_group(plan, group) : WT_OK;
+    if (r == WT_OK) r = wt_workspace_bytes(plan, with_grad, &sb, &tb);
     if (r == WT_OK && (saved.grow((size_t)std::max<int64_t>(sb, 256)) ||
                        temp.grow((size_t)std::max<int64_t>(tb, 256)))) {
       set_error("%s: hipMalloc of a workspace failed (%lld + %lld bytes)", what, (long long)sb,

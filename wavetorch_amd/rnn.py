@@ -127,24 +127,27 @@ class WaveRNN(torch.nn.Module):
         names a checkpoint interval, the longest one whose record fits an
         eighth of the device's memory is taken (``auto_interval``): the
         forward then records the steps that the adjoint would otherwise
-        recompute.  `lean` asks for K = 64 there instead."""
+        recompute.  `lean` asks for K = 64 there instead (the float64 loop
+        keeps every field and has no interval)."""
         cfg = self.loop_config()
         tun = dict(self.tuning) if self.tuning else {}
         tun["ck_every"] = self.checkpoint_every
         group = 0
-        if not lean and self._checkpoint_every is None and not (self.tuning or {}).get("ck_every"):
+        f64 = self.cell.geom.b.dtype == torch.float64
+        if not (lean or f64) and self._checkpoint_every is None \
+                and not (self.tuning or {}).get("ck_every"):
             group = tun["ck_every"]  # the gradient sums of the default interval
             total = torch.cuda.get_device_properties(device).total_memory
             tun["ck_every"] = auto_interval(cfg, B, T, total // 8, tun["ck_every"])
         tkey = tuple(sorted(tun.items()))
-        key = (cfg, B, T, str(device), tkey, group, self.cell.geom.b.dtype)
+        key = (cfg, B, T, str(device), tkey, group, f64)
         p = self._plans.get(key)
         if p is None:
             if len(self._plans) > 8:
                 self._plans.clear()
             # no tiling asked for: the model's choice (a float64 plan makes its
             # own, for its own kernels, where none is given)
-            if not self.tuning and self.cell.geom.b.dtype != torch.float64:
+            if not self.tuning and not f64:
                 tun = suggest(cfg, B, T, self.cell.geom.cmax, tun["ck_every"], group)
             p = Plan(cfg, B, T, self.cell.geom.cmax, device, tun, group, self._waiting)
             self._plans[key] = p
@@ -178,9 +181,8 @@ class WaveRNN(torch.nn.Module):
         rho = geom.rho if self.loop_config().nonlinear else None
         # one whole record per model at a time, whatever the lengths and batch
         # sizes: while a forward's record waits for its backward, further
-        # forwards keep checkpoints every 64 steps (the float64 loop keeps
-        # every field and has no interval)
-        plan = self.plan(B, T, x.device, lean=x.dtype == torch.float64)
+        # forwards keep checkpoints every 64 steps
+        plan = self.plan(B, T, x.device)
         if torch.is_grad_enabled() and plan.record_waits():
             plan = self.plan(B, T, x.device, lean=True)
         args = (fields_mode, stride, self._nonfinite_flags(x.device))
