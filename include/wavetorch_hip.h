@@ -196,6 +196,16 @@ int wt_plan_suggest(const wt_config *cfg, int32_t B, int32_t T, float cmax_geom,
  * launched. */
 int wt_plan_group(void *plan, int32_t steps);
 
+/* For tests of a plan's resident sweeps (one launch whose workgroups wait for
+ * their neighbours between chunks of steps): starts a workgroup for every
+ * `every`-th tile only, at least one per sample (1, the state after
+ * wt_plan_create: for each), which take the others' tiles over, and with
+ * `give_up` ends every wait at once, as after about a minute otherwise.
+ * Resident sweeps of plans with 4 rows per thread (1024-thread blocks; 8 too
+ * in the float adjoint); launching another one then fails.  Host only; not to
+ * be called while a loop of the plan is being launched. */
+int wt_plan_walk(void *plan, int32_t every, int32_t give_up);
+
 /* Host-only half of wt_plan_create: the same validation (including the CFL
  * check of cell.py:66-73) and tiling/variant choice, with no device work.
  * Writes the resolved tuning to *out and the with-grad workspace sizes of

@@ -94,6 +94,7 @@ _SIGS = {
     "wt_plan_suggest": (ctypes.c_int, [ctypes.POINTER(WtConfig), c_i32, c_i32, c_f32, c_i32,
                                        c_i32, ctypes.POINTER(WtTuning)]),
     "wt_plan_group": (ctypes.c_int, [c_p, c_i32]),
+    "wt_plan_walk": (ctypes.c_int, [c_p, c_i32, c_i32]),
     "wt_plan_destroy": (ctypes.c_int, [c_p]),
     "wt_plan_tuning": (ctypes.c_int, [c_p, ctypes.POINTER(WtTuning)]),
     "wt_workspace_bytes": (ctypes.c_int, [c_p, c_i32, ctypes.POINTER(c_i64),

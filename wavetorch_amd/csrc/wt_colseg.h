@@ -350,8 +350,12 @@ __device__ __forceinline__ void cs_dev_store(T *p, T v) {
 
 // First wave: waits until the tiles of sample b in `nbr` (bit q of lane l:
 // tile l + 64 q) have n chunks done.  -1: they have; -2: given up after about
-// a minute; else the work item without an owner that was taken over.
-__device__ __forceinline__ int cs_walk_wait(int *prog, int ntiles, int b, int nbr, int n) {
+// a minute (HOOK: at once where `give_up` says so); else the work item without
+// an owner that was taken over.
+template <bool HOOK>
+__device__ __forceinline__ int cs_walk_wait(int *prog, int ntiles, int b, int nbr, int n,
+                                            int give_up) {
+  if (HOOK && give_up) return -2;
   const int lane = cs_opaque((int)threadIdx.x);
   nbr = cs_opaque(nbr);
   const uint64_t t0 = wall_clock64();

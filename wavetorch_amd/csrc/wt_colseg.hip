@@ -446,13 +446,13 @@ __device__ __forceinline__ void cs_walk_failed(const FwdArgs &a, int b, int n0) 
   }
 }
 
-template <int NT, int R, int NL, bool REC, bool UH>
+template <int NT, int R, int NL, bool REC, bool UH, bool HOOK = false>
 __global__ __launch_bounds__(NT) void k_fwd_cs_walk(FwdArgs a) {
   const int tid = threadIdx.x;
   const int64_t BF = (int64_t)a.B * a.Nx * a.Ny;
   const int nchunks = (a.T + a.nsteps - 1) / a.nsteps;
   __shared__ int msg;
-  int w = xcd_remap(blockIdx.x, gridDim.x);
+  int w = xcd_remap(blockIdx.x, gridDim.x) * (HOOK ? a.walk.every : 1);
   if (tid == 0) msg = atomicCAS(a.prog + w * CS_WALK_W, 0, 1);
   __syncthreads();
   if (msg != 0) return;  // a neighbour took it over
@@ -474,7 +474,7 @@ __global__ __launch_bounds__(NT) void k_fwd_cs_walk(FwdArgs a) {
       for (int i = tid; i < min(a.nsteps, a.T - n1); i += blockDim.x)
         S.xs[i] = a.x[(int64_t)b * a.T + n1 + i];
       if (tid < 64) {
-        const int r = cs_walk_wait(a.prog, a.ntiles, b, nbr, chunk);
+        const int r = cs_walk_wait<HOOK>(a.prog, a.ntiles, b, nbr, chunk, a.walk.give_up);
         if (tid == 0) msg = r;
       }
       __syncthreads();
@@ -541,8 +541,10 @@ __global__ __launch_bounds__(NT) void k_fwd_cs_walk(FwdArgs a) {
     chunk = own_n[at];
     if (tid < 64) {
       const int ti = w % a.ntiles;
-      const int r = chunk > 0 ? cs_walk_wait(a.prog, a.ntiles, w / a.ntiles,
-                                             cs_walk_neighbours(a.tiles, a.ntiles, ti), chunk)
+      const int r = chunk > 0 ? cs_walk_wait<HOOK>(
+                                    a.prog, a.ntiles, w / a.ntiles,
+                                    cs_walk_neighbours(a.tiles, a.ntiles, ti), chunk,
+                                    a.walk.give_up)
                               : -1;
       if (tid == 0) msg = r;
     }
@@ -892,7 +894,7 @@ __device__ __forceinline__ void adj_walk_sum(const AdjArgs &a, const float (&G)[
 // (us of a training step, a launch per chunk and resident: 150 x 150, 64
 // samples, 3000 steps 9876 and 8729; 100 x 100, 4 samples, 1000 steps 1259
 // and 1126; 500 x 380, one sample, 800 steps 1210 and 1063.)
-template <int NT, int R>
+template <int NT, int R, bool HOOK = false>
 __global__ __launch_bounds__(NT) void k_adj_cs_walk(AdjArgs a) {
   const int tid = threadIdx.x;
   const int64_t BF = (int64_t)a.B * a.Nx * a.Ny;
@@ -900,7 +902,7 @@ __global__ __launch_bounds__(NT) void k_adj_cs_walk(AdjArgs a) {
   __shared__ int seed_px[CS_MAX_SEEDS];
   __shared__ int nseeds;
   __shared__ int msg;
-  int w = xcd_remap(blockIdx.x, gridDim.x);
+  int w = xcd_remap(blockIdx.x, gridDim.x) * (HOOK ? a.walk.every : 1);
   if (tid == 0) msg = atomicCAS(a.prog + w * CS_WALK_W, 0, 1);
   __syncthreads();
   if (msg != 0) return;  // a neighbour took it over
@@ -938,7 +940,7 @@ __global__ __launch_bounds__(NT) void k_adj_cs_walk(AdjArgs a) {
       nsteps = adj_walk_steps(a, m);
       adj_cs_start<R, false>(a, S, m, nsteps, tb_sp, seed_px, nseeds);
       if (tid < 64) {
-        const int r = cs_walk_wait(a.prog, a.ntiles, b, nbr, chunk);
+        const int r = cs_walk_wait<HOOK>(a.prog, a.ntiles, b, nbr, chunk, a.walk.give_up);
         if (tid == 0) msg = r;
       }
       __syncthreads();
@@ -1015,8 +1017,9 @@ __global__ __launch_bounds__(NT) void k_adj_cs_walk(AdjArgs a) {
     chunk = own_n[at];
     if (tid < 64) {
       const int r =
-          chunk > 0 ? cs_walk_wait(a.prog, a.ntiles, w / a.ntiles,
-                                   cs_walk_neighbours(a.tiles, a.ntiles, w % a.ntiles), chunk)
+          chunk > 0 ? cs_walk_wait<HOOK>(a.prog, a.ntiles, w / a.ntiles,
+                                         cs_walk_neighbours(a.tiles, a.ntiles, w % a.ntiles),
+                                         chunk, a.walk.give_up)
                     : -1;
       if (tid == 0) msg = r;
     }
@@ -1335,11 +1338,15 @@ int cs_threads(int R, int RH, int RW) {
 template <int NT, int R>
 static hipError_t cs_fwd_dispatch(bool unit_h, int nl, bool rec, const FwdArgs &a, int nblocks,
                                   int nthreads, size_t shmem, hipStream_t s) {
+  constexpr bool hooks = NT == 1024 && R == 4;
+  const bool hook = a.prog && a.walk.hook();
+  if (hook && !hooks) return hipErrorNotSupported;
 #define FT(NL, REC, UH)                                                               \
   do {                                                                                \
     auto kfn = a.prog ? k_fwd_cs_walk<NT, R, NL, REC, UH> : k_fwd_cs<NT, R, NL, REC, UH>; \
-    static std::atomic<uint64_t> done[2];                                             \
-    hipError_t e = allow_dyn_lds((const void *)kfn, done[a.prog != nullptr]);         \
+    if (hook) kfn = k_fwd_cs_walk<NT, R, NL, REC, UH, hooks>;                         \
+    static std::atomic<uint64_t> done[3];                                             \
+    hipError_t e = allow_dyn_lds((const void *)kfn, done[hook ? 2 : a.prog != nullptr]); \
     if (e != hipSuccess) return e;                                                    \
     hipLaunchKernelGGL(kfn, dim3(nblocks), dim3(nthreads), shmem, s, a);              \
   } while (0)
@@ -1361,15 +1368,20 @@ static hipError_t cs_fwd_dispatch(bool unit_h, int nl, bool rec, const FwdArgs &
 template <int NT, int R>
 static hipError_t cs_adj_dispatch(const AdjArgs &a, int nblocks, int nthreads, size_t shmem,
                                   hipStream_t s) {
-#define AT(KFN)                                                                       \
+  constexpr bool hooks = NT == 1024 && (R == 4 || R == 8);  // sums in registers or not
+  const bool hook = a.prog && a.walk.hook();
+  if (hook && !hooks) return hipErrorNotSupported;
+#define AT(...)                                                                       \
   do {                                                                                \
-    auto kfn = KFN<NT, R>;                                                            \
+    auto kfn = __VA_ARGS__;                                                           \
     static std::atomic<uint64_t> done{0};                                             \
     hipError_t e = allow_dyn_lds((const void *)kfn, done);                            \
     if (e != hipSuccess) return e;                                                    \
     hipLaunchKernelGGL(kfn, dim3(nblocks), dim3(nthreads), shmem, s, a);              \
   } while (0)
-  if (a.prog) AT(k_adj_cs_walk); else AT(k_adj_cs);
+  if (hook) AT(k_adj_cs_walk<NT, R, hooks>);
+  else if (a.prog) AT(k_adj_cs_walk<NT, R>);
+  else AT(k_adj_cs<NT, R>);
 #undef AT
   return hipGetLastError();
 }
@@ -1378,11 +1390,12 @@ static hipError_t cs_adj_dispatch(const AdjArgs &a, int nblocks, int nthreads, s
 // and LDS of the launch; smaller tiles leave threads idle.
 hipError_t launch_fwd_cs(int nt, int R, bool unit_h, int nl, bool rec, const FwdArgs &a,
                          int RHmax, int RWmax, hipStream_t s) {
-  int nblocks = a.B * a.ntiles;
+  const int items = a.B * a.ntiles;
+  const int nblocks = a.prog ? walk_blocks(items, a.walk) : items;
   size_t shmem = cs_shmem_bytes(R, RHmax, RWmax, true);
   int nthreads = cs_threads(R, RHmax, RWmax);
   if (shmem + CS_STATIC_LDS > (size_t)cs_max_dyn_lds() || nthreads > nt ||
-      (a.prog && nblocks > CS_WALK_MAX))
+      (a.prog && items > CS_WALK_MAX))
     return hipErrorInvalidConfiguration;
 #define X(A, B) \
   if (nt == A && R == B)                                                                \
@@ -1393,11 +1406,12 @@ hipError_t launch_fwd_cs(int nt, int R, bool unit_h, int nl, bool rec, const Fwd
 }
 
 hipError_t launch_adj_cs(int nt, int R, const AdjArgs &a, int RHmax, int RWmax, hipStream_t s) {
-  int nblocks = a.B * a.ntiles;
+  const int items = a.B * a.ntiles;
+  const int nblocks = a.prog ? walk_blocks(items, a.walk) : items;
   size_t shmem = cs_shmem_bytes(R, RHmax, RWmax, false);
   int nthreads = cs_threads(R, RHmax, RWmax);
   if (shmem + CS_STATIC_LDS + (a.prog ? CS_WALK_LDS : 0) > (size_t)cs_max_dyn_lds() ||
-      nthreads > nt || (a.prog && nblocks > CS_WALK_MAX))
+      nthreads > nt || (a.prog && items > CS_WALK_MAX))
     return hipErrorInvalidConfiguration;
 #define X(A, B) if (nt == A && R == B) return cs_adj_dispatch<A, B>(a, nblocks, nthreads, shmem, s);
   WT_CS_VARIANTS(X)

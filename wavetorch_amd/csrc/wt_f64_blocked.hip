@@ -37,6 +37,7 @@ struct F64Blk {
   double *y, *yraw, *fields, *rec;
   int fstride;
   int *prog;                // resident forward: progress words, else null
+  WalkStart walk;
   const double *ybar;       // adjoint: reverse steps m_hi .. m_hi - nsteps + 1
   double *gacc, *gsrc;
   int m_hi;
@@ -311,7 +312,7 @@ __global__ __launch_bounds__(NT) void k64_fwd_cs(F64Blk a) {
 // 140, 16 samples, 1200 steps: 75 launches of 24.0 us, resident 1377 us.  The
 // adjoint gained nothing from it: its registers spill in the walk, 1784 us
 // against 75 launches of 23.3 us.)
-template <int NT, int R, bool REC, bool UH>
+template <int NT, int R, bool REC, bool UH, bool HOOK = false>
 __global__ __launch_bounds__(NT) void k64_fwd_walk(F64Blk a) {
   const int tid = threadIdx.x;
   const int64_t BF = (int64_t)a.B * a.Nx * a.Ny;
@@ -321,7 +322,7 @@ __global__ __launch_bounds__(NT) void k64_fwd_walk(F64Blk a) {
   auto start = [&](int chunk) { return chunk * a.nsteps; };
   __shared__ int own_w[CS_WALK_MAX], own_n[CS_WALK_MAX];
   __shared__ int msg;
-  int w = xcd_remap(blockIdx.x, gridDim.x);
+  int w = xcd_remap(blockIdx.x, gridDim.x) * (HOOK ? a.walk.every : 1);
   if (tid == 0) msg = atomicCAS(a.prog + w * CS_WALK_W, 0, 1);
   __syncthreads();
   if (msg != 0) return;  // a neighbour took it over
@@ -341,7 +342,7 @@ __global__ __launch_bounds__(NT) void k64_fwd_walk(F64Blk a) {
       ++chunk;
       S.prepare(a, start(chunk), steps(chunk));
       if (tid < 64) {
-        const int r = cs_walk_wait(a.prog, a.ntiles, b, nbr, chunk);
+        const int r = cs_walk_wait<HOOK>(a.prog, a.ntiles, b, nbr, chunk, a.walk.give_up);
         if (tid == 0) msg = r;
       }
       __syncthreads();
@@ -399,8 +400,9 @@ __global__ __launch_bounds__(NT) void k64_fwd_walk(F64Blk a) {
     chunk = own_n[at];
     if (tid < 64) {
       const int r =
-          chunk > 0 ? cs_walk_wait(a.prog, a.ntiles, w / a.ntiles,
-                                   cs_walk_neighbours(a.tiles, a.ntiles, w % a.ntiles), chunk)
+          chunk > 0 ? cs_walk_wait<HOOK>(a.prog, a.ntiles, w / a.ntiles,
+                                         cs_walk_neighbours(a.tiles, a.ntiles, w % a.ntiles),
+                                         chunk, a.walk.give_up)
                     : -1;
       if (tid == 0) msg = r;
     }
@@ -609,13 +611,20 @@ static hipError_t launch64(K kfn, std::atomic<uint64_t> &done, const F64Blk &a, 
                            size_t shmem, hipStream_t s) {
   hipError_t e = allow_dyn_lds((const void *)kfn, done);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kfn, dim3(a.B * a.ntiles), dim3(nthreads), shmem, s, a);
+  const int items = a.B * a.ntiles;
+  const int nblocks = a.prog ? walk_blocks(items, a.walk) : items;
+  hipLaunchKernelGGL(kfn, dim3(nblocks), dim3(nthreads), shmem, s, a);
   return hipGetLastError();
 }
 
 template <int R, bool REC, bool UH>
 static hipError_t launch64_fwd(const F64Blk &a, int nthreads, size_t shmem, hipStream_t s) {
-  static std::atomic<uint64_t> done[2];
+  static std::atomic<uint64_t> done[3];
+  if (a.prog && a.walk.hook()) {
+    if constexpr (R == 4)
+      return launch64(k64_fwd_walk<1024, R, REC, UH, true>, done[2], a, nthreads, shmem, s);
+    return hipErrorNotSupported;
+  }
   if constexpr (R <= 6) {
     if (a.prog)
       return launch64(k64_fwd_walk<1024, R, REC, UH>, done[1], a, nthreads, shmem, s);
@@ -749,6 +758,8 @@ extern "C" int wt_loop_fwd_rec_f64(void *plan, const wt_scalars_f64 *sc, const d
   const bool walk = walks64(v, t);
   if (walk) {
     a.prog = (int *)(st + w.fwd_temp() - w.words);
+    a.walk = v.walk;
+    a.walk.every = std::min(a.walk.every, t.ntiles);
     WT_HIP(launch_fill64(st + w.fwd_temp() - w.words, w.words, 0.0, s));
   }
   int pp = 0;

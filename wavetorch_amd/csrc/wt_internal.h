@@ -78,6 +78,18 @@ __host__ __device__ inline void cs_layout(int RH, int RW, int R, int maxthr, int
   }
 }
 
+// How a resident launch starts and waits, but for its tests {1, 0}: a
+// workgroup for every `every`-th work item, the others' tiles are taken over
+// (at most a sample's tiles, so that each sample has one), and whether waits
+// are given up at once.  Kernels of their own look at it (template parameter
+// HOOK, for 4 rows per thread): compiled into every walk it moved registers
+// enough to cost the forward 1 to 2.7%.
+struct WalkStart {
+  int every = 1, give_up = 0;
+  bool hook() const { return every != 1 || give_up; }
+};
+inline int walk_blocks(int items, const WalkStart &w) { return (items + w.every - 1) / w.every; }
+
 // Arguments of the fused (temporally blocked) forward kernel.
 struct FwdArgs {
   int B, Nx, Ny, T;
@@ -118,6 +130,7 @@ struct FwdArgs {
   // out1 then starts two alternating state pairs, n0 is 0 and nsteps the
   // steps of a chunk
   int *prog;
+  WalkStart walk;
 };
 constexpr int CS_WALK_MAX = 256;  // work items of a resident launch, at most
 constexpr int CS_WALK_W = 16;     // ints between its progress words
@@ -156,6 +169,7 @@ struct AdjArgs {
   // of steps at which chunks end (0: any)
   int *prog;
   int group;
+  WalkStart walk;
 };
 
 // One launch over several configurations (batched instances of uneven grid
@@ -214,6 +228,7 @@ struct PlanView {
   int nspx, ntap, nslot;
   const int32_t *spx, *taps, *spmap, *mult;
   TileView f64, f64_a;  // blocked double-precision forward and adjoint
+  WalkStart walk;
 };
 int plan_view(const void *plan, PlanView *out);
 int plan_use_f64(void *plan);  // builds f64 and f64_a on first use

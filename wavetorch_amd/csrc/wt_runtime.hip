@@ -167,6 +167,7 @@ struct Plan {
   wt_tuning tun{};
   int K = 64, nseg = 1;
   int group = 0;  // adjoint launches end at multiples of this many steps (0: any)
+  WalkStart walk;
   int nspx = 0, ntap = 0, nslot = 0;
   std::vector<int32_t> h_spx, h_taps, h_tiles, h_mult;
   int32_t *d_spx = nullptr, *d_taps = nullptr, *d_spmap = nullptr, *d_mult = nullptr;
@@ -1331,6 +1332,7 @@ int plan_view(const void *plan, PlanView *out) {
   out->nspx = p->nspx; out->ntap = p->ntap; out->nslot = p->nslot;
   out->spx = p->d_spx; out->taps = p->d_taps; out->spmap = p->d_spmap; out->mult = p->d_mult;
   out->f64 = p->t64; out->f64_a = p->t64_a;
+  out->walk = p->walk;
   return WT_OK;
 }
 }  // namespace wt
@@ -1343,6 +1345,16 @@ int wt_plan_group(void *plan, int32_t steps) {
     return WT_EINVAL;
   }
   ((Plan *)plan)->group = steps;
+  return WT_OK;
+}
+
+int wt_plan_walk(void *plan, int32_t every, int32_t give_up) {
+  if (!plan || every < 1) {
+    set_error("wt_plan_walk: invalid argument");
+    return WT_EINVAL;
+  }
+  ((Plan *)plan)->walk.every = every;
+  ((Plan *)plan)->walk.give_up = give_up;
   return WT_OK;
 }
 
@@ -1451,6 +1463,10 @@ bool walks(const Plan &p, int ntiles, int tb) {
   const int64_t items = (int64_t)p.B * ntiles;
   return p.tiled && p.tun.kind == 0 && p.T > tb && items <= std::min(CS_WALK_MAX, device_cus()) &&
          items * CS_WALK_W <= (int64_t)p.B * (int64_t)p.F;
+}
+
+WalkStart walk_start(const Plan &p, int ntiles) {
+  return {std::min(p.walk.every, ntiles), p.walk.give_up};
 }
 
 // Runs forward steps [n0, n1) from the state (in1, in2) = (u_n0, u_{n0-1}).
@@ -1694,6 +1710,7 @@ int wt_loop_fwd(void *plan, const float *b, const float *c, const float *rho, co
     a.out1 = bufs[0];
     a.nsteps = p->tun.tblock;
     a.prog = (int *)bufs[6];
+    a.walk = walk_start(*p, p->ntiles);
     if (rec) {
       a.rec_lap = w.rec;
       a.rec_u = p->nl ? w.rec + (size_t)p->B * p->K * p->Nx * (p->Ny + 1) : nullptr;
@@ -1801,6 +1818,7 @@ int wt_loop_adj(void *plan, const float *b, const float *c, const float *rho, co
       aa.in1 = lam[2]; aa.in2 = lam[3]; aa.out1 = lam[0];
       aa.nsteps = p->tb_a;
       aa.prog = (int *)w.wl;
+      aa.walk = walk_start(*p, p->ntiles_a);
       aa.group = p->group;
       ProfScope ps(2, s, (int64_t)p->B * p->Nx * p->Ny * T);
       WT_HIP(launch_adj_cs(p->nt_a, p->cpt_a, aa, p->RHmax_a, p->RWmax_a, s));
