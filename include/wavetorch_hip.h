@@ -200,10 +200,13 @@ int wt_plan_group(void *plan, int32_t steps);
  * their neighbours between chunks of steps): starts a workgroup for every
  * `every`-th tile only, at least one per sample (1, the state after
  * wt_plan_create: for each), which take the others' tiles over, and with
- * `give_up` ends every wait at once, as after about a minute otherwise.
- * Resident sweeps of plans with 4 rows per thread (1024-thread blocks; 8 too
- * in the float adjoint); launching another one then fails.  Host only; not to
- * be called while a loop of the plan is being launched. */
+ * `give_up` ends every wait at once, as after about a minute otherwise.  A
+ * sweep with a wait that was given up leaves NaN: in every probe value and
+ * field snapshot of the sample that it had not computed, or in a cell of the
+ * tile's dJ/dc and in dJ/dx for the steps left.  Resident sweeps of
+ * plans with 4 rows per thread (1024-thread blocks; 8 too in the float
+ * adjoint); launching another one then fails.  Host only; not to be called
+ * while a loop of the plan is being launched. */
 int wt_plan_walk(void *plan, int32_t every, int32_t give_up);
 
 /* Host-only half of wt_plan_create: the same validation (including the CFL

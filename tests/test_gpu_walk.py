@@ -1,6 +1,7 @@
 """How resident sweeps start and wait: one launch per sweep; the same bits when
 only every n-th workgroup is started and the others' tiles are taken over,
-forward and adjoint, float32 and float64, odd chunks and remainders."""
+forward and adjoint, float32 and float64, odd chunks and remainders; and NaN
+for what a sweep has not computed when its waits are given up."""
 import ctypes
 
 import numpy as np
@@ -94,6 +95,61 @@ def test_tiles_taken_over_f64(case, tun, every, cuda):
     assert np.array_equal(ref[0].cpu().numpy(), yo)
     for a, b in zip(ref, out):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("tun", TILED)
+@pytest.mark.parametrize("case", ["linear", "nonlinear"])
+def test_forward_given_up(case, tun, cuda):
+    """Every wait ends at once: the first chunk's values stand, NaN for the
+    rest of every probe series and every later field snapshot."""
+    p, nl, plan = _plan(case, tun, cuda)
+    n0 = plan.tuning["tblock"]
+    t = {k: torch.from_numpy(p[k]).to(cuda) for k in ("x", "c", "b", "rho")}
+    rho = t["rho"] if nl else None
+    run = lambda fields, stride: WaveLoop.apply(t["x"], t["c"], t["b"], rho, plan, fields, stride)
+    ref = [run(False, 1), run(True, 1), run(True, 5)]
+    _walk(plan, 1, 1)
+    y, f, f5 = run(False, 1), run(True, 1), run(True, 5)
+    for a, r, k in ((y, ref[0], n0), (f, ref[1], n0), (f5, ref[2], n0 // 5)):
+        assert torch.equal(a[:, :k], r[:, :k]) and torch.isnan(a[:, k:]).all()
+    _walk(plan, 1)
+    assert torch.equal(run(False, 1), ref[0])
+
+
+@pytest.mark.parametrize("rows", [4, 8])
+@pytest.mark.parametrize("tun", TILED)
+def test_adjoint_given_up(tun, rows, cuda):
+    """The gradient of c has a NaN for every tile, that of x a NaN for every
+    step after the first chunk (the last steps)."""
+    p, nl, plan = _plan("linear", tun, cuda, rows)
+    k = plan.tuning["a_tblock"]
+    grads = []
+    for give_up in (0, 1):
+        t = {q: torch.from_numpy(p[q]).to(cuda).requires_grad_(q != "b") for q in ("x", "c", "b")}
+        _walk(plan, 1)
+        y = WaveLoop.apply(t["x"], t["c"], t["b"], None, plan, False, 1)
+        w = torch.from_numpy(np.random.default_rng(5).standard_normal(y.shape)).to(cuda, y.dtype)
+        _walk(plan, 1, give_up)
+        (y * w).sum().backward()
+        grads.append((t["c"].grad, t["x"].grad))
+    (gc, gx), (bc, bx) = grads
+    tiles = plan.tuning["a_strips"] * plan.tuning["a_tcols"]
+    assert int(torch.isnan(bc).sum()) == tiles and torch.isfinite(gc).all()
+    assert torch.equal(bx[:, -k:], gx[:, -k:]) and torch.isnan(bx[:, :-k]).all()
+
+
+@pytest.mark.parametrize("tun", TILED)
+def test_forward_given_up_f64(tun, cuda):
+    p, cfg, h, nl, onl = _setup("linear")
+    plan = Plan(cfg, p["B"], p["T"], 1.0, cuda, dict(TUNINGS[tun], nt=1024, cpt=4,
+                                                     ck_every=p["T"]))
+    n0 = plan.tuning["tblock"]
+    t = [torch.from_numpy(p[k]).to(cuda, torch.float64) for k in ("x", "c", "b")]
+    run = lambda fields: WaveLoop.apply(*t, None, plan, fields, 1)
+    ref = [run(False), run(True)]
+    _walk(plan, 1, 1)
+    for a, r in zip((run(False), run(True)), ref):
+        assert torch.equal(a[:, :n0], r[:, :n0]) and torch.isnan(a[:, n0:]).all()
 
 
 def test_arguments(cuda):

@@ -402,6 +402,21 @@ __device__ __forceinline__ int cs_walk_neighbours(const int32_t *tiles, int ntil
   return nbr;
 }
 
+// A wait of a sweep was given up with steps n0 and later of sample b to do:
+// NaN to all of their probe values and field snapshots.  (A neighbour's later
+// store can only be a value that it could still compute.)
+template <typename Args, typename T>
+__device__ __forceinline__ void cs_walk_failed(const Args &a, int b, int n0, T nan) {
+  auto mark = [&](T *p, int64_t per, int64_t lo, int64_t hi) {
+    if (p)
+      for (int64_t i = lo * per + threadIdx.x; i < hi * per; i += blockDim.x)
+        p[b * hi * per + i] = nan;
+  };
+  mark(a.y, a.ntap, n0, a.T);
+  mark(a.yraw, a.ntap, n0, a.T);
+  mark(a.fields, (int64_t)a.Nx * a.Ny, n0 / a.fstride, a.T / a.fstride);
+}
+
 // After a chunk's state is stored: when every wave's stores have completed,
 // the work item's word.
 __device__ __forceinline__ void cs_walk_raise(int *prog, int w, int chunk) {

@@ -436,16 +436,6 @@ __device__ __forceinline__ void cs_walk_store(const Args &a, float (&V0)[R], flo
   cs_walk_raise(a.prog, w, chunk);
 }
 
-// The wait of a workgroup was given up: probe outputs from step n0 on are NaN.
-__device__ __forceinline__ void cs_walk_failed(const FwdArgs &a, int b, int n0) {
-  const float nan = __builtin_nanf("");
-  for (int64_t i = (int64_t)n0 * a.ntap + threadIdx.x; i < (int64_t)a.T * a.ntap;
-       i += blockDim.x) {
-    if (a.y) a.y[(int64_t)b * a.T * a.ntap + i] = nan;
-    if (a.yraw) a.yraw[(int64_t)b * a.T * a.ntap + i] = nan;
-  }
-}
-
 template <int NT, int R, int NL, bool REC, bool UH, bool HOOK = false>
 __global__ __launch_bounds__(NT) void k_fwd_cs_walk(FwdArgs a) {
   const int tid = threadIdx.x;
@@ -505,7 +495,7 @@ __global__ __launch_bounds__(NT) void k_fwd_cs_walk(FwdArgs a) {
   while (true) {
     // -1: run the chunk that was waited for; >= 0: one more work item
     if (got == -2) {
-      cs_walk_failed(a, w / a.ntiles, chunk * a.nsteps);
+      cs_walk_failed(a, w / a.ntiles, chunk * a.nsteps, __builtin_nanf(""));
       return;
     }
     if (got >= 0) {
@@ -971,10 +961,17 @@ __global__ __launch_bounds__(NT) void k_adj_cs_walk(AdjArgs a) {
   __shared__ int own_w[CS_WALK_MAX], own_n[CS_WALK_MAX];
   int nown = 1, at = 0;
   while (true) {
-    if (got == -2) {  // given up: the gradient's first cell of the tile becomes NaN
+    if (got == -2) {
+      // given up: NaN to the gradient's first cell of the tile (after the sums
+      // above) and to lambda at the source pixels for the steps left
       const int32_t *td = a.tiles + w % a.ntiles * TILE_W;
-      if (tid == 0)
-        a.gacc[((int64_t)(w / a.ntiles) * a.Nx + td[4]) * a.Ny + td[6]] = __builtin_nanf("");
+      const int b = w / a.ntiles;
+      m = a.T;
+      for (int i = 0; i < chunk; ++i) m -= adj_walk_steps(a, m);
+      __syncthreads();
+      if (tid == 0) a.gacc[((int64_t)b * a.Nx + td[4]) * a.Ny + td[6]] = __builtin_nanf("");
+      for (int64_t i = tid; i < (int64_t)m * a.nsrcslot; i += blockDim.x)
+        a.gsrc[(int64_t)b * a.T * a.nsrcslot + i] = __builtin_nanf("");
       return;
     }
     if (got >= 0) {

@@ -356,14 +356,8 @@ __global__ __launch_bounds__(NT) void k64_fwd_walk(F64Blk a) {
   // with a whole set-up.
   int nown = 1, at = 0;
   while (true) {
-    if (got == -2) {  // given up: probe outputs from this chunk on are NaN
-      const double nan = __builtin_nan("");
-      const int64_t o = (int64_t)(w / a.ntiles) * a.T * a.ntap;
-      for (int64_t i = (int64_t)chunk * a.nsteps * a.ntap + tid; i < (int64_t)a.T * a.ntap;
-           i += blockDim.x) {
-        if (a.y) a.y[o + i] = nan;
-        if (a.yraw) a.yraw[o + i] = nan;
-      }
+    if (got == -2) {
+      cs_walk_failed(a, w / a.ntiles, start(chunk), __builtin_nan(""));
       return;
     }
     if (got >= 0) {
