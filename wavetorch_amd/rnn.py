@@ -150,6 +150,8 @@ class WaveRNN(torch.nn.Module):
             if not self.tuning and not f64:
                 tun = suggest(cfg, B, T, self.cell.geom.cmax, tun["ck_every"], group)
             p = Plan(cfg, B, T, self.cell.geom.cmax, device, tun, group, self._waiting)
+            if f64:  # its tilings are built and uploaded here, not in a captured call
+                p.bytes_rec_f64()
             self._plans[key] = p
         return p
 
