@@ -353,6 +353,31 @@ static bool tables_ok_cs(const Plan &p, int R, int nthr) {
   return true;
 }
 
+// Whether no tiling with halos of tb rows passes tables_ok_cs: a pixel shared
+// by several sources, or a row whose surroundings, which the region of its
+// tile holds whatever the tiling, have too many special pixels, probe pixels
+// or taps.  (Trying all tilings of a 300 x 300 grid takes 6 s.)
+static bool tables_too_dense(const Plan &p, int tb) {
+  std::vector<int> px(p.Nx + 1, 0), probe(p.Nx + 1, 0), tap(p.Nx, 0);
+  for (int k = 0; k < p.nspx; ++k) {
+    const int32_t *e = &p.h_spx[k * SPX_W];
+    if (e[2] > 1) return true;
+    ++px[e[0] + 1];
+    probe[e[0] + 1] += e[5] > e[4];
+  }
+  for (int k = 0; k < p.ntap; ++k)
+    if (++tap[p.h_taps[k * TAP_W]] > CS_MAX_TABLE) return true;
+  for (int x = 0; x < p.Nx; ++x) {
+    px[x + 1] += px[x];
+    probe[x + 1] += probe[x];
+  }
+  for (int x = 0; x < p.Nx; ++x) {
+    const int lo = std::max(0, x - tb), hi = std::min(p.Nx, x + tb + 1);
+    if (px[hi] - px[lo] > CS_MAX_TABLE || probe[hi] - probe[lo] > CS_MAX_SEEDS) return true;
+  }
+  return false;
+}
+
 static const int kCsVariants[][2] = {{1024, 4},  {1024, 6},  {1024, 8},  {1024, 10},
                                      {1024, 12}, {512, 16},  {512, 20},  {512, 24}};
 
@@ -970,6 +995,7 @@ static int plan_build(const wt_config *cfg, int32_t B, int32_t T, float cmax_geo
         if (std::min(p->Nx / order[i].first, p->Ny / order[i].second) >= 2 * tb) oi = i;
       }
       strips = order[oi].first;
+      if (tables_too_dense(*p, tb)) oi = order.size();
     } else if (strips <= 0) {
       // row strips: enough workgroups to cover the 256 CUs
       strips = 1;
