@@ -702,6 +702,12 @@ static double walk_us(const WalkModel &m, int R, int waves, int s, int c, int th
                   lines / ((double)th * tw) * m.lines);
 }
 
+// At most walk_us: every row at its least, no halo lines.
+static double walk_us_least(const WalkModel &m, int R, int waves, int tw, int n, double cells) {
+  return m.ts + m.tR * R * ((waves + 3) / 4) + n * (m.e + m.cw * waves / 16 + m.row * R) +
+         cells * (m.rec * n * 1e-6 * (1.0 + m.edge * 32.0 / tw) + m.state);
+}
+
 struct BlockChoice {
   double us;
   int s, c, tb, R;
@@ -717,23 +723,38 @@ static std::vector<BlockChoice> cheapest_blocks(const BlockModel &launches, cons
                                                 Shmem shmem) {
   static const int depths[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 14, 16, 18, 20, 24, 28, 32, 40, 48};
   std::vector<BlockChoice> best;
-  auto consider = [&](int s, int c, int tb) {
-    const int th = (Nx + s - 1) / s, tw = (Ny + c - 1) / c;
+  const double cells = (double)B * Nx * Ny;
+  auto consider = [&](int s, int c, int th, int tw, int percu, int tb) {
     const int RH = std::min(Nx, th + (s > 2 ? 2 * tb : s == 2 ? tb : 0));
     const int RW = std::min(Ny, tw + (c > 2 ? 2 * tb : c == 2 ? tb : 0));
-    const int percu = (int)(((int64_t)B * s * c + 255) / 256);
+    if ((int64_t)RH * RW > 12 * 1024) return;  // more than 12 rows for 1024 threads
     // (a single chunk too: a launch of its own, whose steps are the same)
     const bool walks =
         walk && percu == 1 && (int64_t)s * c * CS_WALK_W <= (int64_t)Nx * Ny;
     const BlockModel &m = launches;
     const int *rows = walks ? walk->rows : m.rows;
+    // Most candidates are out by what their full chunks take at least, first
+    // for any rows per thread (R k >= RH RW / 256), then for R without the
+    // cone and the halo's lines.  (A suggestion for 500 x 380, one sample, 800
+    // steps: 1.19 ms, 0.52 so; 121 x 97, 500 steps: 0.57 and 0.20.)
+    auto out = [&](double us) {
+      return (int)best.size() == top && us > best.back().us * (1.0 + 1e-9);
+    };
+    const double row_cells = RH * (RW / 256.0);
+    const double step_least =
+        walks ? walk->e + std::max(4 * walk->row,
+                                   walk->issue * row_cells *
+                                       (1.0 - walk->cone * (1.0 - th / (RH + 12.0))))
+              : m.cw * percu * row_cells;
+    if (out(len / tb * (tb * (step_least + cells * (walks ? walk->rec : m.rec) * 1e-6) +
+                        (walks ? walk->ts : m.t0))))
+      return;
     for (int v = 0; v < 5 && rows[v]; ++v) {
       const int R = rows[v], waves = cs_threads(R, RH, RW) / 64;
       if (waves > 16) continue;
       const size_t lds = shmem(R, RH, RW, tb) + (walks ? CS_WALK_LDS : 0);
       if (lds > LDS_LIMIT) continue;
       const int occ = std::max(1, std::min((int)(LDS_LIMIT / lds), m.waves[v] * 4 / waves));
-      const double cells = (double)B * Nx * Ny;
       auto launch = [&](int n) {
         return walks ? walk_us(*walk, R, waves, s, c, th, tw, RH, RW, n, cells)
                      : launch_us(m, R, waves, occ, percu, n, cells);
@@ -743,9 +764,13 @@ static std::vector<BlockChoice> cheapest_blocks(const BlockModel &launches, cons
       // halo rows drop out of the cone step by step, halo columns stay)
       const double area = (Nx + (s > 1 ? 1.0 * tb * (s - 1) : 0.0)) *
                           (Ny + (c > 1 ? 2.0 * tb * (c - 1) : 0.0)) * B;
-      const double us = (len / tb * launch(tb) + (len % tb ? launch(len % tb) : 0.0) +
-                         (walks ? 8.0 : 0.0)) *
-                        (1.0 + 0.06 * area / (256.0 * 1024.0 * R * percu));
+      const double worse = 1.0 + 0.06 * area / (256.0 * 1024.0 * R * percu);
+      if (walks && out(len / tb * walk_us_least(*walk, R, waves, tw, tb, cells) * worse))
+        continue;
+      const double full = len / tb * launch(tb);
+      if (out(full * worse)) continue;
+      const double us =
+          (full + (len % tb ? launch(len % tb) : 0.0) + (walks ? 8.0 : 0.0)) * worse;
       if ((int)best.size() == top && us >= best.back().us) continue;
       const BlockChoice ch{us, s, c, tb, R};
       best.insert(std::upper_bound(best.begin(), best.end(), ch,
@@ -756,7 +781,8 @@ static std::vector<BlockChoice> cheapest_blocks(const BlockModel &launches, cons
       if ((int)best.size() > top) best.pop_back();
     }
   };
-  consider(1, 1, depth > 0 ? depth : std::min(len, 256));  // no halo: any depth
+  // (one tile has no halo: any depth)
+  consider(1, 1, Nx, Ny, (B + 255) / 256, depth > 0 ? depth : std::min(len, 256));
   // near-square tilings (at most 2:1) of up to two workgroups per CU, or of
   // four times the tiles that 64 x 64 cells each would make of a large batch
   const int64_t most = std::max<int64_t>(512, (int64_t)B * Nx * Ny / 1024);
@@ -768,15 +794,28 @@ static std::vector<BlockChoice> cheapest_blocks(const BlockModel &launches, cons
       if (s * c == 1 || (int64_t)B * s * c > most) continue;
       if (c > 1 && (Ny + c - 1) / c == (Ny + c - 2) / (c - 1)) continue;
       const int own = std::min(s > 1 ? Nx / s : Nx, c > 1 ? Ny / c : Ny);
+      const int th = (Nx + s - 1) / s, tw = (Ny + c - 1) / c;
+      const int percu = (int)(((int64_t)B * s * c + 255) / 256);
       if (depth > 0) {
-        consider(s, c, depth);
+        consider(s, c, th, tw, percu, depth);
       } else {
         for (int tb : depths)
-          if (tb <= len && tb <= 2 * own) consider(s, c, tb);
+          if (tb <= len && tb <= 2 * own) consider(s, c, th, tw, percu, tb);
       }
     }
   }
   return best;
+}
+
+// The cheapest of cheapest_blocks' choices that `take` holds: mostly the first,
+// which alone is found much faster than the first 32.
+template <typename Shmem, typename Take>
+static bool take_cheapest(const BlockModel &launches, const WalkModel *walk, int Nx, int Ny, int B,
+                          int len, int depth, Shmem shmem, Take take) {
+  for (int top : {1, 32})
+    for (const BlockChoice &ch : cheapest_blocks(launches, walk, Nx, Ny, B, len, depth, top, shmem))
+      if (take(ch)) return true;
+  return false;
 }
 
 static int plan_upload(Plan *p);
@@ -807,16 +846,13 @@ static void plan_f64(Plan &plan) {
       const int R = fwd || tuning->a_cpt <= 0 ? tuning->cpt : tuning->a_cpt;
       ok = tb > 0 && tb <= 256 && take(s, std::max(c, 1), std::min(tb, p.T), R, fwd);
     }
-    if (!ok) {
-      for (const BlockChoice &ch : cheapest_blocks(
-               fwd ? kModel64 : kModel64Adj, fwd ? &kWalk64 : nullptr, p.Nx, p.Ny, p.B, p.T, 0, 32,
-               [](int R, int RH, int RW, int tb) {
-                 return cs64_shmem_bytes(R, RH, RW, tb) + 16 * 1024;
-               })) {
-        ok = take(ch.s, ch.c, ch.tb, ch.R, fwd);
-        if (ok) break;
-      }
-    }
+    if (!ok)
+      ok = take_cheapest(
+          fwd ? kModel64 : kModel64Adj, fwd ? &kWalk64 : nullptr, p.Nx, p.Ny, p.B, p.T, 0,
+          [](int R, int RH, int RW, int tb) {
+            return cs64_shmem_bytes(R, RH, RW, tb) + 16 * 1024;
+          },
+          [&](const BlockChoice &ch) { return take(ch.s, ch.c, ch.tb, ch.R, fwd); });
     if (!ok) {
       plan.t64.R = plan.t64_a.R = 0;
       break;
@@ -1204,36 +1240,30 @@ int wt_plan_suggest(const wt_config *cfg, int32_t B, int32_t T, float cmax_geom,
   const int a_depth = p->tiled && p->unit_h ? p->tb_a : 0;
   *out = wt_tuning{};
   out->ck_every = K;
-  bool ok = false;
-  for (const BlockChoice &ch : cheapest_blocks(
-           p->nl ? kModelNl : kModelLin,
-           K < T ? nullptr : p->nl ? &kWalkNl : &kWalkLin, p->Nx, p->Ny, B, K, 0, 32,
-           [](int R, int RH, int RW, int) { return cs_shmem_bytes(R, RH, RW, true) + 8192; })) {
-    build_tiles(*p, ch.s, ch.c, ch.tb);
-    if (!tiles_ok_cs(*p, 1024, ch.R)) continue;
-    out->strips = ch.s; out->tcols = ch.c; out->tblock = ch.tb;
-    out->nt = 1024; out->cpt = ch.R;
-    ok = true;
-    break;
-  }
-  bool aok = false;
-  if (ok) {
-    const bool nl = p->nl != 0;
-    for (const BlockChoice &ch : cheapest_blocks(
-             nl ? kModelNlAdj : kModelLinAdj, K < T || nl ? nullptr : &kWalkLinAdj, p->Nx,
-             p->Ny, B, K, a_depth, 32,
-             [nl](int R, int RH, int RW, int) {
-               return (nl ? cs_nl_shmem_bytes(R, RH, RW) : cs_shmem_bytes(R, RH, RW, false)) +
-                      8192;
-             })) {
-      build_tiles(*p, ch.s, ch.c, ch.tb);
-      if (!tiles_ok_cs(*p, 1024, ch.R, false)) continue;
-      out->a_strips = ch.s; out->a_tcols = ch.c; out->a_tblock = ch.tb;
-      out->a_nt = 1024; out->a_cpt = ch.R;
-      aok = true;
-      break;
-    }
-  }
+  const bool nl = p->nl != 0;
+  const bool ok = take_cheapest(
+      nl ? kModelNl : kModelLin, K < T ? nullptr : nl ? &kWalkNl : &kWalkLin, p->Nx, p->Ny, B, K,
+      0, [](int R, int RH, int RW, int) { return cs_shmem_bytes(R, RH, RW, true) + 8192; },
+      [&](const BlockChoice &ch) {
+        build_tiles(*p, ch.s, ch.c, ch.tb);
+        if (!tiles_ok_cs(*p, 1024, ch.R)) return false;
+        out->strips = ch.s; out->tcols = ch.c; out->tblock = ch.tb;
+        out->nt = 1024; out->cpt = ch.R;
+        return true;
+      });
+  const bool aok = ok && take_cheapest(
+      nl ? kModelNlAdj : kModelLinAdj, K < T || nl ? nullptr : &kWalkLinAdj, p->Nx, p->Ny, B, K,
+      a_depth,
+      [nl](int R, int RH, int RW, int) {
+        return (nl ? cs_nl_shmem_bytes(R, RH, RW) : cs_shmem_bytes(R, RH, RW, false)) + 8192;
+      },
+      [&](const BlockChoice &ch) {
+        build_tiles(*p, ch.s, ch.c, ch.tb);
+        if (!tiles_ok_cs(*p, 1024, ch.R, false)) return false;
+        out->a_strips = ch.s; out->a_tcols = ch.c; out->a_tblock = ch.tb;
+        out->a_nt = 1024; out->a_cpt = ch.R;
+        return true;
+      });
   if (!aok) {  // no block holds this configuration: the library's default
     const int k = out->ck_every;
     *out = wt_tuning{};
