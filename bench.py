@@ -79,11 +79,12 @@ def class_name(cls, tun, nonlinear, B, T, unit_h=True, rec=False):
     if cls == 2:
         if nonlinear:
             return f"wt::k_adj_cs_nl<{tun['a_nt']}, {tun['a_cpt']}, false>"
-        walk = "_walk" if resident(cls, tun, nonlinear, B, T) else ""
-        return f"wt::k_adj_cs{walk}<{tun['a_nt']}, {tun['a_cpt']}>"
-    walk = "_walk" if cls == 0 and resident(cls, tun, nonlinear, B, T) else ""
+        walk, end = ("_walk", ", false>") if resident(cls, tun, nonlinear, B, T) else ("", ">")
+        return f"wt::k_adj_cs{walk}<{tun['a_nt']}, {tun['a_cpt']}{end}"
+    walk, end = ("_walk", ", false>") if cls == 0 and resident(cls, tun, nonlinear, B, T) \
+        else ("", ">")
     return f"wt::k_fwd_cs{walk}<{tun['nt']}, {tun['cpt']}, {8 if nonlinear else 0}, " \
-        f"{'true' if cls == 1 or rec else 'false'}, {'true' if unit_h else 'false'}>"
+        f"{'true' if cls == 1 or rec else 'false'}, {'true' if unit_h else 'false'}{end}"
 
 
 def log(*a):

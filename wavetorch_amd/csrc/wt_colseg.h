@@ -1,5 +1,5 @@
 // wt_colseg.h -- region geometry and memory access shared by the temporally
-// blocked column-segment kernels (wt_colseg.hip in float, wt_f64.hip in
+// blocked column-segment kernels (wt_colseg.hip in float, wt_f64_blocked.hip in
 // double; the thread mapping is described in wt_colseg.hip).  Not part of the
 // public ABI.
 #pragma once

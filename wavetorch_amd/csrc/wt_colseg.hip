@@ -1,9 +1,10 @@
 // wt_colseg.hip -- column-segment, temporally blocked WaveRNN kernels (gfx950).
 //
 // Same contract as the flat kernels of wt_tiled.hip (one workgroup advances
-// one region = tile + halo of one sample by `nsteps` steps, no inter-workgroup
-// synchronisation), with a thread mapping that keeps vertical neighbours in
-// registers:
+// one region = tile + halo of one sample by `nsteps` steps), with a thread
+// mapping that keeps vertical neighbours in registers.  A launch's workgroups
+// do not wait for each other, but for the resident sweeps (k_fwd_cs_walk,
+// k_adj_cs_walk; the scheme stands in wt_colseg.h).
 //
 //   thread t -> column c = t % RW, segment k = t / RW; it owns the R cells
 //   (rows k*R .. k*R+R-1, column c) of the region.  u_n and u_{n-1} of those
