@@ -146,7 +146,8 @@ class Plan:
         """True while a workspace of this plan, or of one that shares its
         table, records more than the default 64 steps and waits for its
         backward."""
-        return self.tuning["ck_every"] > 64 and bool(self._waiting)
+        return (self.tuning["ck_every"] > 64
+                and any(r() is not None for r in list(self._waiting.values())))
 
     def _wait(self, saved):
         """Counts `saved` among the waiting records for as long as it lives."""
