@@ -27,16 +27,19 @@ class _Spy:
         return call
 
 
+def _model(cuda, shape=(60, 52)):
+    geom = WaveGeometryFreeForm(shape, 1.0, c0=1.0, c1=0.5, abs_N=8, abs_sig=1.0, abs_p=2,
+                                rho="half")
+    return WaveRNN(WaveCell(0.7, geom), WaveSource(16, 26), [WaveIntensityProbe(44, 20)]).to(cuda)
+
+
 @pytest.mark.parametrize("native", [False, True])
 @pytest.mark.parametrize("every", [None, 50])
 def test_interval_of_a_tuned_model(every, native, cuda, monkeypatch):
     stored, seen = {}, set()
     monkeypatch.setattr(autotune, "_load", lambda: dict(stored))
     monkeypatch.setattr(autotune, "_store", stored.update)
-    geom = WaveGeometryFreeForm((60, 52), 1.0, c0=1.0, c1=0.5, abs_N=8, abs_sig=1.0, abs_p=2,
-                                rho="half")
-    model = WaveRNN(WaveCell(0.7, geom), WaveSource(16, 26),
-                    [WaveIntensityProbe(44, 20)]).to(cuda)
+    model = _model(cuda)
     model.checkpoint_every = every
     x = torch.randn(3, 150, device=cuda)
     if native:
@@ -59,3 +62,20 @@ def test_interval_of_a_tuned_model(every, native, cuda, monkeypatch):
     assert all(run.tuning[k] == v for k, v in best.items())
     assert list(stored) == [autotune.key(60, 52, 3, 150, every or "auto", "gfx950")]
     assert autotune.lookup(60, 52, 3, 150) == (None if every else best)
+
+
+@pytest.mark.parametrize("native", [False, True])
+def test_search_after_a_tuning_that_does_not_fit(native, cuda, monkeypatch):
+    """The tuning of another shape on the model, which no block holds here."""
+    monkeypatch.setattr(autotune, "_load", dict)
+    monkeypatch.setattr(autotune, "_store", lambda d: None)
+    model = _model(cuda, (150, 120))
+    model.tuning = dict(strips=1, tcols=1, tblock=8, nt=1024, cpt=4)
+    x = torch.randn(2, 100, device=cuda)
+    with pytest.raises(RuntimeError):
+        model(x)
+    if native:
+        best, _ = autotune.tune_native(model, x, reps=1, budget_s=1e-3)
+    else:
+        best = autotune.tune(model, x, steps=1, reps=1, budget_s=0.0)
+    assert model.tuning == best and torch.isfinite(model(x)).all()

@@ -275,9 +275,13 @@ def tune_native(model, x, with_grad=True, reps=2, budget_s=120.0, store=True):
         b = geom.b.detach().contiguous()
         rho = geom.rho.detach().contiguous() if cfg.nonlinear else None
     xx = x.detach().contiguous()
-    plan = model.plan(B, T, x.device)
+    former, model.tuning = model.tuning, None  # (it may be another shape's)
+    try:
+        plan = model.plan(B, T, x.device)
+    finally:
+        model.tuning = former
     start = _lib.WtTuning(ck_every=plan.tuning["ck_every"])
-    kname = "auto" if plan.group else int(model.checkpoint_every)
+    kname = "auto" if plan.group else int(model._checkpoint_every or 64)
     torch.cuda.empty_cache()  # the search allocates beside torch
     out = _lib.WtTuning()
     ms = ctypes.c_double(0.0)
