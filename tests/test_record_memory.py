@@ -130,3 +130,15 @@ def test_batch_whose_record_does_not_fit(cuda):
     with _Limit(cuda, 400 << 20):  # what the caller asked for is not changed
         with pytest.raises(torch.cuda.OutOfMemoryError):
             InstanceBatch(insts, cuda, checkpoint_every=1500)
+
+
+def test_a_given_interval_needs_no_room_for_a_backward(cuda):
+    """A forward at an interval that the caller named runs in the memory it
+    needs itself, as there is nothing to fall back to."""
+    model, x = _model(cuda, 150), _x(cuda, 64, 150)
+    model.checkpoint_every = 150
+    p = model.plan(64, 150, x.device)
+    ref = model(x).detach()
+    with _Limit(cuda, p.saved_bytes + p.temp_bytes_nograd + (12 << 20)):
+        y = model(x)
+    assert torch.equal(y, ref)

@@ -261,10 +261,11 @@ class WaveLoop(torch.autograd.Function):
                 _lib.ptr(saved), _lib.ptr(temp), s), "wt_loop_fwd_f64")
         else:
             saved = _buf(plan.saved_bytes, dev) if with_grad else None
-            # the forward's scratch; beside a record of more than the default 64
-            # steps as large as the backward's, so that a record which leaves
-            # no room for that one fails here, where the caller can fall back
-            whole = with_grad and plan.tuning["ck_every"] > 64
+            # the forward's scratch; beside a record longer than the default
+            # interval that the caller left open (`group`) as large as the
+            # backward's, so that a record which leaves no room for that one
+            # fails here, where the caller can fall back
+            whole = with_grad and 0 < plan.group < plan.tuning["ck_every"]
             temp = _buf(max(plan.temp_bytes_nograd, plan.temp_bytes if whole else 0), dev)
             _lib.check(_lib.lib().wt_loop_fwd(
                 plan.handle, b.data_ptr(), c.data_ptr(), _lib.ptr(rho_c), x.data_ptr(),
